@@ -30,6 +30,8 @@ SIGNATURES = {
     'flyhip_sblocal_bwd': [c_vp] * 14 + [c_int] * 7 + [c_float, c_int, c_vp],
     'flyhip_sblocal_bwd_prep': [c_vp] * 18 + [c_i64] + [c_int] * 7 + [c_float, c_vp],
     'flyhip_sblocal_bwd_pieces': [c_vp] * 12 + [c_i64] + [c_int] * 7 + [c_float, c_int, c_float, c_u64, c_vp],
+    'flyhip_sblocal_bwd_far_floats': [c_int] * 5,
+    'flyhip_sblocal_bwd_far': [c_vp] * 12 + [c_i64] + [c_int] * 8 + [c_i64] * 24 + [c_float, c_vp],
     'flyhip_sbblocksparse_bwd_pieces': [c_vp] * 15 + [c_int] * 2 + [c_vp, c_i64] + [c_int] * 6 + [c_float, c_int, c_float, c_u64, c_vp],
     'flyhip_sbblocksparse_fwd': [c_vp] * 15 + [c_int] * 2 + [c_vp] * 4 + [c_int] * 8 + [c_i64] * 12 + [c_float, c_int, c_float, c_u64, c_vp],
     'flyhip_local_fwd_lse': [c_vp] * 6 + [c_int] * 7 + [c_i64] * 12 + [c_float, c_int, c_vp],
@@ -72,6 +74,7 @@ def load():
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = c_int
+    lib.flyhip_sblocal_bwd_far_floats.restype = c_i64
     lib.flyhip_sb_workspace_bytes.argtypes = [c_int] * 9
     lib.flyhip_sb_workspace_bytes.restype = c_i64
     lib.flyhip_sblocal_bwd_prep_scratch.argtypes = [c_int] * 5

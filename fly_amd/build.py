@@ -8,7 +8,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libflyhip.so')
-SOURCES = ['api.cpp', 'sblocal.hip', 'sblocal_prep.hip', 'blocksparse.hip']
+SOURCES = ['api.cpp', 'sblocal.hip', 'sblocal_prep.hip', 'sblocal_far.hip', 'blocksparse.hip']
 # packed-fp32 VALU forms are switched off for every kernel of this library; MFMA accumulators stay in
 # ordinary VGPRs (the softmax arithmetic reads them between products, and every trip through the
 # accumulation registers costs a move per value)
@@ -41,7 +41,7 @@ def build(verbose=False):
             print(' '.join(cmd))
         return obj
 
-    with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as pool:
+    with ThreadPoolExecutor(max_workers=len(SOURCES)) as pool:
         objs = list(pool.map(compile_one, SOURCES))
     cmd = [hipcc, '--offload-arch=gfx950', '-shared', '-fPIC', '-o', LIB] + objs
     res = subprocess.run(cmd, capture_output=True, text=True)

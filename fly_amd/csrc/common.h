@@ -361,6 +361,43 @@ __device__ __forceinline__ void dma_to_lds(const void* lane_src, const char* wav
                  : "=&s"(saved_m0) : "v"(lane_src), "s"(base) : "memory");
 }
 
+// ROWS x W tile of 2-byte elements, global -> registers -> LDS (row indices clamped to the last row: rows past
+// the end re-read it, which callers mask, so the loads need no branches and never leave the tensor)
+template <int ROWS, int W, int NT>
+struct Tile16 {
+    static constexpr int C8 = W / 8, N = (ROWS * C8 + NT - 1) / NT;
+    uintx4 r[N];
+    // the same with a wave-uniform tile base and per-thread byte offsets computed once (all rows exist)
+    __device__ __forceinline__ void offsets(uint32_t (&off)[N], long row_stride, int tid) const {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int idx = (tid + NT * j) % (ROWS * C8), row = idx / C8, c8 = idx % C8;
+            off[j] = (uint32_t)((row * row_stride + 8 * c8) * 2);
+        }
+    }
+    __device__ __forceinline__ void fetch_at(const uint16_t* tile_base, const uint32_t (&off)[N]) {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            r[j] = *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(tile_base) + off[j]);
+    }
+    // (a tile with fewer pieces than threads wraps around: every thread loads and stores, see TileKV16)
+    __device__ __forceinline__ void fetch(const uint16_t* src, long row_stride, int row0, int last_row, int tid) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int idx = (tid + NT * j) % (ROWS * C8), row = idx / C8, c8 = idx % C8;
+            r[j] = *reinterpret_cast<const uintx4*>(src + (long)min(row0 + row, last_row) * row_stride + 8 * c8);
+        }
+    }
+    template <int LD>
+    __device__ __forceinline__ void stash(uint16_t* dst, int tid) const {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int idx = (tid + NT * j) % (ROWS * C8), row = idx / C8, c8 = idx % C8;
+            *reinterpret_cast<uintx4*>(dst + row * LD + 8 * c8) = r[j];
+        }
+    }
+};
+
 // Transposed operand reads (ds_read_b64_tr_b16): within each group of 16 lanes, lane s passes the address of four
 // consecutive 16-bit elements -- row s / 4, columns 4 (s % 4) .. + 3 of a 4 x 16 block -- and lane l receives column l of
 // the four rows.

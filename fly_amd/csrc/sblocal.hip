@@ -23,6 +23,7 @@
 // columns = queries) so that r indexes the lane's query and the four register elements index
 // consecutive keys/features -- which is exactly the operand layout the next product needs.
 #include "common.h"
+#include "local.h"
 #include <hip/hip_ext.h>
 #include <math.h>
 #include <type_traits>
@@ -1143,43 +1144,6 @@ __global__ __launch_bounds__(NT) void sb_kfeat_x3_kernel(KvArgs a) {
 // rounded to bf16 for their products.  The query projection sqrt(t) P q also runs on the bf16 MFMA
 // without losing precision: q is bf16 already and P is split into a bf16 head and a bf16 remainder
 // (two MFMAs per step; the split represents P to 2^-17).
-
-// ROWS x W tile of 2-byte elements, global -> registers -> LDS (rows clamped like RowTile)
-
-template <int ROWS, int W, int NT>
-struct Tile16 {
-    static constexpr int C8 = W / 8, N = (ROWS * C8 + NT - 1) / NT;
-    uintx4 r[N];
-    // the same with a wave-uniform tile base and per-thread byte offsets computed once (all rows exist)
-    __device__ __forceinline__ void offsets(uint32_t (&off)[N], long row_stride, int tid) const {
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            const int idx = (tid + NT * j) % (ROWS * C8), row = idx / C8, c8 = idx % C8;
-            off[j] = (uint32_t)((row * row_stride + 8 * c8) * 2);
-        }
-    }
-    __device__ __forceinline__ void fetch_at(const uint16_t* tile_base, const uint32_t (&off)[N]) {
-#pragma unroll
-        for (int j = 0; j < N; ++j)
-            r[j] = *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(tile_base) + off[j]);
-    }
-    // (a tile with fewer pieces than threads wraps around: every thread loads and stores, see TileKV16)
-    __device__ __forceinline__ void fetch(const uint16_t* src, long row_stride, int row0, int last_row, int tid) {
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            const int idx = (tid + NT * j) % (ROWS * C8), row = idx / C8, c8 = idx % C8;
-            r[j] = *reinterpret_cast<const uintx4*>(src + (long)min(row0 + row, last_row) * row_stride + 8 * c8);
-        }
-    }
-    template <int LD>
-    __device__ __forceinline__ void stash(uint16_t* dst, int tid) const {
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            const int idx = (tid + NT * j) % (ROWS * C8), row = idx / C8, c8 = idx % C8;
-            *reinterpret_cast<uintx4*>(dst + row * LD + 8 * c8) = r[j];
-        }
-    }
-};
 
 // The K tile (TK rows of E, row-major) and the V tile (D rows of TK, contiguous) of one step as ONE
 // list of 16-byte pieces dealt to the threads round-robin, so that every thread issues the same
@@ -2982,17 +2946,6 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
 //   P = exp2(sc S - lse log2e) where the pair is in the band, dS = P (G - delta)   (lse, delta: of the query)
 //   d x^T[e][outer] += Y^T[e][inner] . {P, dS}[inner][outer]   (Y^T fragments by transposing LDS reads)
 // Query-major: d q from (K, dS).  Key-major: d v from (d out, P) and d k from (Q, dS).
-struct LocalBwdArgs {
-    const void* q; const void* k; const void* v; const void* go; const void* out;
-    const float* lse; float* delta;                 // (B, H, T); delta is written by the query-major launch
-    const int64_t* lens;
-    void* dq; void* dk; void* dv;
-    int B, H, T, S, lc;
-    long q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss;
-    long dq_sb, dq_sh, dq_ss, dk_sb, dk_sh, dk_ss, dv_sb, dv_sh, dv_ss;
-    float temp;
-    int n_xcd;
-};
 template <typename T> __device__ __forceinline__ float unpack_lo(uint32_t w);
 template <typename T> __device__ __forceinline__ float unpack_hi(uint32_t w);
 template <> __device__ __forceinline__ float unpack_lo<bf16_t>(uint32_t w) { return __uint_as_float(w << 16); }
@@ -3001,7 +2954,10 @@ template <> __device__ __forceinline__ float unpack_lo<f16_t>(uint32_t w) { retu
 template <> __device__ __forceinline__ float unpack_hi<f16_t>(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)); }
 template <int E> constexpr size_t local_bwd_smem() { return (size_t)2 * (TKL * 2 * (E + 8) * 2 + 2 * TKL * sizeof(float)); }
 
-template <typename T, int E, bool KEYMAJOR, int QB>
+// EXACT (bfloat16): the exact part of a Scatterbrain-local backward.  lse is the log-normaliser of all keys and delta is
+// given; P and dS enter the second products in two bf16 pieces (2^-17: the sums are exact to the rounding of the
+// results, as they were when this part ran in float32), and the low-rank part of the gradient is added in the epilogue.
+template <typename T, int E, bool KEYMAJOR, int QB, bool EXACT = false>
 __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
     static_assert(sizeof(T) == 2 && E % 32 == 0, "2-byte inputs, whole MFMA steps");
     constexpr int LD = E + 8, KS = E / 32, EB = E / 16;
@@ -3080,6 +3036,9 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
         l_own[qq] = d_own[qq] = 0.f;
         if (!KEYMAJOR) {
             l_own[qq] = lsep[min(io[qq], a.T - 1)] * LOG2E;
+        }
+        if (EXACT && !KEYMAJOR) d_own[qq] = delp[min(io[qq], a.T - 1)];
+        if (!EXACT && !KEYMAJOR) {
             // delta of the query, g . out, from the output row in the layout of the gradient row; kept for the key-major launch
             const uint16_t* orow = reinterpret_cast<const uint16_t*>(a.out) + b * a.o_sb + h * a.o_sh + row * a.o_ss;
             float dsum = 0.f;
@@ -3161,16 +3120,28 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
                     }
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf) {
-                uint4 pb[KEYMAJOR ? QB : 1], sb[QB];
+                uint4 pb[KEYMAJOR ? QB : 1], sb[QB], pbl[KEYMAJOR ? QB : 1], sbl[QB];     // (..l: the second pieces, EXACT)
 #pragma unroll
                 for (int qq = 0; qq < QB; ++qq) {
-                    sb[qq] = make_uint4(pack_pair<T>(gp[qq][2 * hf][0], gp[qq][2 * hf][1]), pack_pair<T>(gp[qq][2 * hf][2], gp[qq][2 * hf][3]),
-                                        pack_pair<T>(gp[qq][2 * hf + 1][0], gp[qq][2 * hf + 1][1]),
-                                        pack_pair<T>(gp[qq][2 * hf + 1][2], gp[qq][2 * hf + 1][3]));
-                    if (KEYMAJOR)
-                        pb[qq] = make_uint4(pack_pair<T>(s1[qq][2 * hf][0], s1[qq][2 * hf][1]), pack_pair<T>(s1[qq][2 * hf][2], s1[qq][2 * hf][3]),
-                                            pack_pair<T>(s1[qq][2 * hf + 1][0], s1[qq][2 * hf + 1][1]),
-                                            pack_pair<T>(s1[qq][2 * hf + 1][2], s1[qq][2 * hf + 1][3]));
+                    if constexpr (EXACT) {
+                        uintx4 hi, lo;
+                        split2(gp[qq][2 * hf], gp[qq][2 * hf + 1], hi, lo);
+                        sb[qq] = __builtin_bit_cast(uint4, hi);
+                        sbl[qq] = __builtin_bit_cast(uint4, lo);
+                        if (KEYMAJOR) {
+                            split2(s1[qq][2 * hf], s1[qq][2 * hf + 1], hi, lo);
+                            pb[qq] = __builtin_bit_cast(uint4, hi);
+                            pbl[qq] = __builtin_bit_cast(uint4, lo);
+                        }
+                    } else {
+                        sb[qq] = make_uint4(pack_pair<T>(gp[qq][2 * hf][0], gp[qq][2 * hf][1]), pack_pair<T>(gp[qq][2 * hf][2], gp[qq][2 * hf][3]),
+                                            pack_pair<T>(gp[qq][2 * hf + 1][0], gp[qq][2 * hf + 1][1]),
+                                            pack_pair<T>(gp[qq][2 * hf + 1][2], gp[qq][2 * hf + 1][3]));
+                        if (KEYMAJOR)
+                            pb[qq] = make_uint4(pack_pair<T>(s1[qq][2 * hf][0], s1[qq][2 * hf][1]), pack_pair<T>(s1[qq][2 * hf][2], s1[qq][2 * hf][3]),
+                                                pack_pair<T>(s1[qq][2 * hf + 1][0], s1[qq][2 * hf + 1][1]),
+                                                pack_pair<T>(s1[qq][2 * hf + 1][2], s1[qq][2 * hf + 1][3]));
+                    }
                 }
 #pragma unroll
                 for (int eb = 0; eb < EB; ++eb) {
@@ -3178,13 +3149,19 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
                     const uint4 t1 = __builtin_bit_cast(uint4, lds_read_tr8(reinterpret_cast<const char*>(p1),
                                                                              reinterpret_cast<const char*>(p1 + 4 * LD)));
 #pragma unroll
-                    for (int qq = 0; qq < QB; ++qq) acc1[qq][eb] = Frag32<T>::mma(t1, sb[qq], acc1[qq][eb]);
+                    for (int qq = 0; qq < QB; ++qq) {
+                        if (EXACT) acc1[qq][eb] = Frag32<T>::mma(t1, sbl[qq], acc1[qq][eb]);
+                        acc1[qq][eb] = Frag32<T>::mma(t1, sb[qq], acc1[qq][eb]);
+                    }
                     if (KEYMAJOR) {
                         const uint16_t* p2 = Y2 + toff + 32 * hf * LD + 16 * eb;
                         const uint4 t2 = __builtin_bit_cast(uint4, lds_read_tr8(reinterpret_cast<const char*>(p2),
                                                                                  reinterpret_cast<const char*>(p2 + 4 * LD)));
 #pragma unroll
-                        for (int qq = 0; qq < QB; ++qq) acc2[qq][eb] = Frag32<T>::mma(t2, pb[qq], acc2[qq][eb]);
+                        for (int qq = 0; qq < QB; ++qq) {
+                            if (EXACT) acc2[qq][eb] = Frag32<T>::mma(t2, pbl[qq], acc2[qq][eb]);
+                            acc2[qq][eb] = Frag32<T>::mma(t2, pb[qq], acc2[qq][eb]);
+                        }
                     }
                 }
             }
@@ -3197,12 +3174,21 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
         if (io[qq] < R_out) {
             T* d1 = KEYMAJOR ? reinterpret_cast<T*>(a.dk) + b * a.dk_sb + h * a.dk_sh + (long)io[qq] * a.dk_ss
                              : reinterpret_cast<T*>(a.dq) + b * a.dq_sb + h * a.dq_sh + (long)io[qq] * a.dq_ss;
+            const long lr_at = ((long)bh * R_out + io[qq]) * E + 4 * g;
 #pragma unroll
-            for (int eb = 0; eb < EB; ++eb) store4_f32(d1 + 16 * eb + 4 * g, acc1[qq][eb] * a.temp);
+            for (int eb = 0; eb < EB; ++eb) {
+                floatx4 d = acc1[qq][eb] * a.temp;
+                if (EXACT) d += *reinterpret_cast<const floatx4*>((KEYMAJOR ? a.lr_dk : a.lr_dq) + lr_at + 16 * eb);
+                store4_f32(d1 + 16 * eb + 4 * g, d);
+            }
             if (KEYMAJOR) {
                 T* d2 = reinterpret_cast<T*>(a.dv) + b * a.dv_sb + h * a.dv_sh + (long)io[qq] * a.dv_ss;
 #pragma unroll
-                for (int eb = 0; eb < EB; ++eb) store4_f32(d2 + 16 * eb + 4 * g, acc2[qq][eb]);
+                for (int eb = 0; eb < EB; ++eb) {
+                    floatx4 d = acc2[qq][eb];
+                    if (EXACT) d += *reinterpret_cast<const floatx4*>(a.lr_dv + lr_at + 16 * eb);
+                    store4_f32(d2 + 16 * eb + 4 * g, d);
+                }
             }
         }
     }
@@ -4684,9 +4670,9 @@ static bool local_b16_ready(const LocalArgs& a) {
 #ifndef FLY_LOCAL_BWD_QB
 #define FLY_LOCAL_BWD_QB 1
 #endif
-template <typename T, int E, bool KEYMAJOR, int QB>
+template <typename T, int E, bool KEYMAJOR, int QB, bool EXACT = false>
 static int launch_local_bwd_as(const LocalBwdArgs& a, hipStream_t st) {
-    auto kern = local_bwd_b16_kernel<T, E, KEYMAJOR, QB>;
+    auto kern = local_bwd_b16_kernel<T, E, KEYMAJOR, QB, EXACT>;
     constexpr size_t smem = local_bwd_smem<E>();
     static std::atomic<unsigned long long> lds_set{0};     // (devices on which this kernel has its LDS limit)
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_set, "local_bwd_b16")) return rc;
@@ -4705,6 +4691,15 @@ static int launch_local_bwd(const LocalBwdArgs& a, hipStream_t st) {
     // (query-major first: it leaves delta for the key-major launch)
     if (int rc = launch_local_bwd_as<T, E, false, FLY_LOCAL_BWD_QB>(a, st)) return rc;
     return launch_local_bwd_as<T, E, true, FLY_LOCAL_BWD_QB>(a, st);
+}
+
+int launch_local_bwd_exact(const LocalBwdArgs& a, int E, hipStream_t st) {
+    if (E == 32) {
+        if (int rc = launch_local_bwd_as<bf16_t, 32, false, 1, true>(a, st)) return rc;
+        return launch_local_bwd_as<bf16_t, 32, true, 1, true>(a, st);
+    }
+    if (int rc = launch_local_bwd_as<bf16_t, 64, false, 1, true>(a, st)) return rc;
+    return launch_local_bwd_as<bf16_t, 64, true, 1, true>(a, st);
 }
 
 template <typename T, int E>

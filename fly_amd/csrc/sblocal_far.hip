@@ -1,0 +1,728 @@
+// The low-rank part of the Scatterbrain-local backward for bfloat16 inputs, without the "all keys minus the band" of
+// the kernels in sblocal_prep.hip.
+//
+// The reference obtains these gradients from autograd through softmax_kernel (src/models/attention/feature_maps_sb.py:51-82)
+// and sblocal_attention.py:73-122.  With psi_i = Phi(q_i) exp(kappa) / Z_i, phi_s = Phi(k_s) exp(-kappa), c_i = g_i.out_i and
+// df_is = g_i.v_s - c_i, a pair outside the band has the weight psi_i.phi_s, so
+//   u_i  = psi_i o sum_{s outside} df_is phi_s        (gradient w.r.t. the log-features of q_i)
+//   uk_s = phi_s o sum_{i outside} df_is psi_i,   d v_s += sum_{i outside} (psi_i.phi_s) g_i
+// and inside the band the gradient is that of plain local attention with log Z in the place of its log-denominator.
+// Rows are taken in chunks of 64.  Seen from a chunk, every chunk of the other side is
+//   inside  the band for all pairs    -- no low-rank work at all (the kernels that subtract the band's part spend
+//                                        M-wide products on every pair of it: 15 of 17 chunks at a window of 1024),
+//   far     no pair in the band       -- through the sums  KV_c = sum phi v^T, sum phi  (QG_c = sum psi g^T, sum psi c) of the
+//                                        chunks, kept as prefix sums: far = prefix up to the window + suffix after it,
+//   an edge some pairs in the band    -- the pairs outside it one by one (two chunks at a window that is a multiple of 64).
+// Nothing is subtracted from a sum over all keys that contains it many times over, so features in two bf16 pieces
+// (2^-17) and products of pieces with fp32 accumulation are exact to the rounding of the bfloat16 results.
+//
+//   far_chunk_kernel    KV_c and QG_c of every chunk, stabilised by the chunk's own largest log-feature
+//   far_scan_kernel     their inclusive prefix sums in common units, in place
+//   far_lowrank_kernel  query-major and key-major: far and edge terms, chain rule through the feature map -> float32
+//   local_bwd_b16_kernel<EXACT> (sblocal.hip)  the band, plus the low-rank part, rounded once
+//
+// Measured at B=1, H=16, L=16384, window 1024, 256 features, where the backward ran as library products over windows of
+// keys before (20.8 ms): chunks 166, scan 225, low-rank 392 (query-major) and 740 (key-major), band 188 and 272 us.  The
+// chunk sums (66 KB per 64 rows and side at 256 features: written, scanned, read twice) are what the first three move.
+#include "common.h"
+#include "local.h"
+#include <algorithm>
+
+namespace flyhip {
+
+constexpr int FC = 64;                              // rows per chunk
+struct FarArgs {
+    const uint16_t* q; const uint16_t* k; const uint16_t* v; const uint16_t* go; const uint16_t* out;
+    const float* ln; const float* proj; const int64_t* lens;
+    float* c;                                       // (BH, T): g . out
+    float* kscale; float* qscale;                   // (BH, chunks): base-2 log of the units a chunk's sums are kept in
+    float* kv; float* qg;                           // (BH, chunks, M (E + 1)): sums of the chunk [M][E] | [M], then prefix sums
+    float* dq; float* dk; float* dv;                // low-rank part of the gradients, (BH, rows, E)
+    int B, H, T, S, lc, mh_valid, n_kc, n_qc;
+    long q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss;
+    float temp;
+    int n_xcd;
+};
+
+constexpr float FAR_LOG2E = 1.4426950408889634f;
+
+// largest unit of the keys of a (batch, head) (base 2; 0 when no key is valid).  red: NW floats; ends with a barrier.
+template <int NT>
+__device__ __forceinline__ float far_kappa(const FarArgs& a, int bh, float* red, int tid) {
+    float m = -INFINITY;
+    for (int i = tid; i < a.n_kc; i += NT) m = fmaxf(m, a.kscale[(long)bh * a.n_kc + i]);
+    m = wave_max(m);
+    if ((tid & 63) == 0) red[tid >> 6] = m;
+    __syncthreads();
+    m = red[0];
+#pragma unroll
+    for (int i = 1; i < NT / 64; ++i) m = fmaxf(m, red[i]);
+    __syncthreads();
+    return m == -INFINITY ? 0.f : m;
+}
+
+// 64 rows of one side on their way into LDS: x (the rows that have features) and y (values, or output gradients) row-major
+// with padded rows; diag = t log2e |x|^2 / 2, ext = the rest of the row's log-feature bias (-inf: no such row), cs = c
+template <int E, int NT>
+struct FarTile {
+    static constexpr int LD = E + 8;
+    Tile16<FC, E, NT> x, y;
+    float ext, cv;
+    // queries: bias base + kappa - log Z; keys: base - kappa.  base = -log2(2 mh) / 2
+    __device__ __forceinline__ void fetch(const FarArgs& a, bool queries, const uint16_t* xp, long xs, const uint16_t* yp, long ys,
+                                          int bh, int row0, int len, float base, float kappa, int tid) {
+        const int last = (queries ? a.T : a.S) - 1;
+        x.fetch(xp, xs, row0, last, tid);
+        y.fetch(yp, ys, row0, last, tid);
+        ext = -INFINITY;
+        cv = 0.f;
+        if (tid < FC && row0 + tid < len) {
+            const long at = (long)bh * a.T + row0 + tid;
+            ext = queries ? base + kappa - a.ln[at] * FAR_LOG2E : base - kappa;
+            if (queries && a.c) cv = a.c[at];
+        }
+    }
+    __device__ __forceinline__ void stash(const FarArgs& a, uint16_t* Xs, uint16_t* Ys, float* diag, float* exts, float* cs, int tid) const {
+        x.template stash<LD>(Xs, tid);
+        y.template stash<LD>(Ys, tid);
+        constexpr int C8 = E / 8;
+#pragma unroll
+        for (int j = 0; j < Tile16<FC, E, NT>::N; ++j) {
+            const int idx = tid + NT * j;
+            float sq = 0.f;
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                const float lo = __uint_as_float(x.r[j][n] << 16), hi = __uint_as_float(x.r[j][n] & 0xffff0000u);
+                sq += lo * lo + hi * hi;
+            }
+#pragma unroll
+            for (int off = 1; off < C8; off <<= 1) sq += __shfl_xor(sq, off);          // the C8 lanes of a row
+            if (idx % C8 == 0 && idx < FC * C8) diag[idx / C8] = 0.5f * a.temp * FAR_LOG2E * sq;
+        }
+        if (tid < FC) { exts[tid] = ext; cs[tid] = cv; }
+    }
+};
+
+// this wave's 16 rows of sqrt(t) log2e P in three bf16 pieces (exact): lane (r16, g) holds columns 32 ks + 8 g .. + 7 of row r16
+template <int KS>
+struct FarProj {
+    uintx4 h[KS], m[KS], l[KS];
+    __device__ __forceinline__ void load(const float* proj, int row, int E, float scale, int g) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const float* src = proj + (long)row * E + 32 * ks + 8 * g;
+            split3(*reinterpret_cast<const floatx4*>(src) * scale, *reinterpret_cast<const floatx4*>(src + 4) * scale, h[ks], m[ks], l[ks]);
+        }
+    }
+    // rows of x . P^T: result rows = rows of x, columns (lane r16) = rows of P
+    __device__ __forceinline__ floatx4 rows_by_features(const uint16_t* x0) const {
+        floatx4 d = Frag<float>::zero();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const uintx4 xf = *reinterpret_cast<const uintx4*>(x0 + 32 * ks);
+            d = mma_bf16(xf, l[ks], d);
+            d = mma_bf16(xf, m[ks], d);
+            d = mma_bf16(xf, h[ks], d);
+        }
+        return d;
+    }
+    // the same transposed: result rows = rows of P, columns = rows of x
+    __device__ __forceinline__ floatx4 features_by_rows(const uint16_t* x0) const {
+        floatx4 d = Frag<float>::zero();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const uintx4 xf = *reinterpret_cast<const uintx4*>(x0 + 32 * ks);
+            d = mma_bf16(l[ks], xf, d);
+            d = mma_bf16(m[ks], xf, d);
+            d = mma_bf16(h[ks], xf, d);
+        }
+        return d;
+    }
+};
+
+// ---------------------------------------------------------------------------------------
+// sums of the chunks
+// ---------------------------------------------------------------------------------------
+// One chunk per workgroup, 16 projection rows (32 features, exp(+.) and exp(-.)) per wave.  The projection is formed with
+// the chunk's rows as result rows, which leaves a lane with one feature of 16 rows: the operand of F^T Y as it stands.
+template <int E, int M>
+__global__ __launch_bounds__(2 * M) void far_chunk_kernel(FarArgs a) {
+    constexpr int NW = M / 32, NT = 64 * NW, MH = M / 2, KS = E / 32, EB = E / 16, LD = E + 8, PER = M * (E + 1);
+    __shared__ __attribute__((aligned(16))) uint16_t Xs[FC * LD], Ys[FC * LD];
+    __shared__ __attribute__((aligned(16))) float diag[FC], exts[FC], cs[FC];
+    __shared__ float red[NW];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
+    const bool queries = (int)blockIdx.x >= a.n_kc;
+    const int c = queries ? blockIdx.x - a.n_kc : blockIdx.x;
+    const int len = queries ? a.T : (a.lens ? min((int)a.lens[b], a.S) : a.S);
+    const uint16_t* xp = queries ? a.q + b * a.q_sb + h * a.q_sh : a.k + b * a.k_sb + h * a.k_sh;
+    const uint16_t* yp = queries ? a.go + b * a.g_sb + h * a.g_sh : a.v + b * a.v_sb + h * a.v_sh;
+    const long xs = queries ? a.q_ss : a.k_ss, ys = queries ? a.g_ss : a.v_ss;
+    FarTile<E, NT> t;
+    Tile16<FC, E, NT> o;
+    FarArgs na = a;
+    na.c = nullptr;                                 // (formed here)
+    t.fetch(na, queries, xp, xs, yp, ys, bh, c * FC, len, -0.5f * __log2f(2.0f * a.mh_valid), 0.f, tid);
+    if (queries) o.fetch(a.out + b * a.o_sb + h * a.o_sh, a.o_ss, c * FC, a.T - 1, tid);
+    FarProj<KS> P;
+    P.load(a.proj, 16 * w + r16, E, sqrtf(a.temp) * FAR_LOG2E, g);
+    t.stash(a, Xs, Ys, diag, exts, cs, tid);
+    if (queries) {
+        // c = g . out, C8 lanes per row
+        constexpr int C8 = E / 8;
+        __syncthreads();                            // (cs was zeroed by stash)
+#pragma unroll
+        for (int j = 0; j < Tile16<FC, E, NT>::N; ++j) {
+            const int idx = tid + NT * j, row = idx / C8;
+            float d = 0.f;
+#pragma unroll
+            for (int n = 0; n < 4; ++n)
+                d += __uint_as_float(o.r[j][n] << 16) * __uint_as_float(t.y.r[j][n] << 16) +
+                     __uint_as_float(o.r[j][n] & 0xffff0000u) * __uint_as_float(t.y.r[j][n] & 0xffff0000u);
+#pragma unroll
+            for (int off = 1; off < C8; off <<= 1) d += __shfl_xor(d, off);
+            if (idx % C8 == 0 && idx < FC * C8) {
+                cs[row] = d;
+                if (c * FC + row < a.T) a.c[(long)bh * a.T + c * FC + row] = d;
+            }
+        }
+    }
+    __syncthreads();
+
+    const bool fvalid = 16 * w + r16 < a.mh_valid;
+    floatx4 dd[4], bias[4];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+        dd[kb] = P.rows_by_features(Xs + (16 * kb + r16) * LD + 8 * g);
+        bias[kb] = *reinterpret_cast<const floatx4*>(exts + 16 * kb + 4 * g) - *reinterpret_cast<const floatx4*>(diag + 16 * kb + 4 * g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, fvalid ? fabsf(dd[kb][i]) + bias[kb][i] : -INFINITY);
+    }
+    mx = wave_max(mx);
+    if (lane == 0) red[w] = mx;
+    __syncthreads();
+    float unit = red[0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) unit = fmaxf(unit, red[i]);
+    if (tid == 0) (queries ? a.qscale : a.kscale)[(long)bh * (queries ? a.n_qc : a.n_kc) + c] = unit;
+    const float shift = unit == -INFINITY ? 0.f : unit;
+
+    floatx4 acc[2][EB];
+    float tot[2] = {0.f, 0.f};
+#pragma unroll
+    for (int sg = 0; sg < 2; ++sg)
+#pragma unroll
+        for (int eb = 0; eb < EB; ++eb) acc[sg][eb] = Frag<float>::zero();
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+        uintx4 fh[2], fl[2];
+#pragma unroll
+        for (int sg = 0; sg < 2; ++sg) {
+            floatx4 f[2];
+#pragma unroll
+            for (int hb = 0; hb < 2; ++hb) {
+                const int kb = 2 * t2 + hb;
+                const floatx4 wr = *reinterpret_cast<const floatx4*>(cs + 16 * kb + 4 * g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float x = __builtin_amdgcn_exp2f((sg ? -dd[kb][i] : dd[kb][i]) + bias[kb][i] - shift);
+                    f[hb][i] = fvalid ? x : 0.f;
+                    tot[sg] += queries ? f[hb][i] * wr[i] : f[hb][i];
+                }
+            }
+            split2(f[0], f[1], fh[sg], fl[sg]);
+        }
+#pragma unroll
+        for (int eb = 0; eb < EB; ++eb) {
+            const uint16_t* yq = Ys + (32 * t2 + 4 * g + (r16 >> 2)) * LD + 16 * eb + 4 * (r16 & 3);
+            const uintx4 yt = lds_read_tr8(reinterpret_cast<const char*>(yq), reinterpret_cast<const char*>(yq + 16 * LD));
+#pragma unroll
+            for (int sg = 0; sg < 2; ++sg) {
+                acc[sg][eb] = mma_bf16(fl[sg], yt, acc[sg][eb]);
+                acc[sg][eb] = mma_bf16(fh[sg], yt, acc[sg][eb]);
+            }
+        }
+    }
+    float* dst = (queries ? a.qg + ((long)bh * a.n_qc + c) * PER : a.kv + ((long)bh * a.n_kc + c) * PER);
+#pragma unroll
+    for (int sg = 0; sg < 2; ++sg) {
+#pragma unroll
+        for (int eb = 0; eb < EB; ++eb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[(sg * MH + 16 * w + 4 * g + i) * E + 16 * eb + r16] = acc[sg][eb][i];
+        const float s = group_sum(tot[sg]);
+        if (g == 0) dst[M * E + sg * MH + 16 * w + r16] = s;
+    }
+}
+
+// inclusive prefix sums over the chunks of a (batch, head), in place, in the common units of the features (exp(kappa)
+// taken out of the keys and put into the queries); eight chunks of loads in flight per thread
+constexpr int FAR_SCAN_NT = 256;
+__global__ __launch_bounds__(FAR_SCAN_NT) void far_scan_kernel(FarArgs a, int per4) {
+    __shared__ float red[FAR_SCAN_NT / 64];
+    const int bh = blockIdx.z, e = blockIdx.x * FAR_SCAN_NT + threadIdx.x;
+    const bool queries = blockIdx.y != 0;
+    const float kappa = far_kappa<FAR_SCAN_NT>(a, bh, red, threadIdx.x);
+    if (e >= per4) return;
+    const int n = queries ? a.n_qc : a.n_kc;
+    const float* unit = (queries ? a.qscale : a.kscale) + (long)bh * n;
+    const float ref = queries ? kappa : -kappa;
+    floatx4* p = reinterpret_cast<floatx4*>(queries ? a.qg : a.kv) + (long)bh * n * per4 + e;
+    floatx4 run = Frag<float>::zero();
+    int c = 0;
+    for (; c + 8 <= n; c += 8) {
+        floatx4 x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = p[(long)(c + j) * per4];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            run += x[j] * __builtin_amdgcn_exp2f(unit[c + j] + ref);
+            p[(long)(c + j) * per4] = run;
+        }
+    }
+    for (; c < n; ++c) {
+        run += p[(long)c * per4] * __builtin_amdgcn_exp2f(unit[c] + ref);
+        p[(long)c * per4] = run;
+    }
+}
+
+// ---------------------------------------------------------------------------------------
+// far and edge terms of 64 outer rows
+// ---------------------------------------------------------------------------------------
+// 16 projection rows (32 features) per wave, all 64 outer rows: every feature of an edge chunk is formed once per
+// workgroup and goes from registers into the products.  Sums over features (chain rule, d v) are per wave until the end.
+template <int E, int M>
+constexpr size_t far_lowrank_smem() {
+    const size_t tiles = (size_t)2 * FC * (E + 8) * 2, inner = tiles + 2 * 8 * 64 * 16, red = (size_t)(M / 32) * FC * 16 * 4;
+    return tiles + (inner > red ? inner : red) + sizeof(float) * (6 * FC + (M / 32) * (FC + 1));
+}
+
+template <int E, int M, bool KEYMAJOR>
+__global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(2, 2))) void far_lowrank_kernel(FarArgs a) {
+    constexpr int NW = M / 32, NT = 64 * NW, MH = M / 2, KS = E / 32, EB = E / 16, LD = E + 8, PER = M * (E + 1);
+    constexpr size_t TILES = (size_t)2 * FC * LD * 2, INNER = TILES + 2 * 8 * 64 * 16, RED = (size_t)NW * FC * 16 * 4;
+    extern __shared__ __attribute__((aligned(128))) char far_smem[];
+    uint16_t* Xo = reinterpret_cast<uint16_t*>(far_smem);
+    uint16_t* Yo = Xo + FC * LD;
+    uint16_t* Xi = Yo + FC * LD;                                                    // inner chunk, then df; the reduction overlays both
+    uint16_t* Yi = Xi + FC * LD;
+    uintx4* DF = reinterpret_cast<uintx4*>(Yi + FC * LD);                           // [piece][step, outer block][lane]
+    float* red = reinterpret_cast<float*>(Xi);
+    float* diago = reinterpret_cast<float*>(far_smem + TILES + (INNER > RED ? INNER : RED));
+    float* exto = diago + FC; float* co = exto + FC;
+    float* diagi = co + FC; float* exti = diagi + FC; float* ci = exti + FC;
+    float* us = ci + FC;                                                            // [NW][FC]
+    float* kred = us + NW * FC;                                                     // [NW]
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    const int Lo = KEYMAJOR ? a.S : a.T;
+    const int n_oc = KEYMAJOR ? a.n_kc : a.n_qc, n_ic = KEYMAJOR ? a.n_qc : a.n_kc;
+    const int n_items = a.B * a.H * n_oc;
+    const int per_xcd = (n_items + a.n_xcd - 1) / a.n_xcd;
+    const int item = (blockIdx.x % a.n_xcd) * per_xcd + blockIdx.x / a.n_xcd;      // neighbouring tiles share a die's L2
+    if (item >= n_items) return;                                                    // workgroup-uniform
+    const int oc = item % n_oc, bh = item / n_oc, b = bh / a.H, h = bh % a.H;
+    const int o0 = oc * FC;
+    const int klen = a.lens ? min((int)a.lens[b], a.S) : a.S;
+    const int len_o = KEYMAJOR ? klen : a.T, len_i = KEYMAJOR ? a.T : klen;
+    const uint16_t* qp = a.q + b * a.q_sb + h * a.q_sh;
+    const uint16_t* kp = a.k + b * a.k_sb + h * a.k_sh;
+    const uint16_t* vp = a.v + b * a.v_sb + h * a.v_sh;
+    const uint16_t* gp = a.go + b * a.g_sb + h * a.g_sh;
+    const uint16_t* xop = KEYMAJOR ? kp : qp; const uint16_t* yop = KEYMAJOR ? vp : gp;
+    const uint16_t* xip = KEYMAJOR ? qp : kp; const uint16_t* yip = KEYMAJOR ? gp : vp;
+    const long xos = KEYMAJOR ? a.k_ss : a.q_ss, yos = KEYMAJOR ? a.v_ss : a.g_ss;
+    const long xis = KEYMAJOR ? a.q_ss : a.k_ss, yis = KEYMAJOR ? a.g_ss : a.v_ss;
+    // the pair (outer o, inner n) is in the band when n - o lies in [-A, Bq)
+    const int lc_lo = a.lc / 2, lc_hi = (a.lc + 1) / 2;
+    const int A = KEYMAJOR ? lc_hi - 1 : lc_lo, Bq = KEYMAJOR ? lc_lo + 1 : lc_hi;
+    // inner chunks [c0, c1) meet the band of some row; [e0, e1) lie inside the band of every row; the rest are far
+    const int c0 = min(n_ic, max(0, o0 - A) / FC);
+    const int c1 = max(c0, min(n_ic, (max(0, o0 + FC - 1 + Bq) + FC - 1) / FC));
+    const int e0 = min(c1, max(c0, (max(0, o0 + FC - 1 - A) + FC - 1) / FC));
+    const int e1 = max(e0, min(c1, max(0, o0 + Bq) / FC));
+
+    const float base = -0.5f * __log2f(2.0f * a.mh_valid);
+    const float kappa = far_kappa<NT>(a, bh, kred, tid);
+    FarTile<E, NT> t;
+    t.fetch(a, !KEYMAJOR, xop, xos, yop, yos, bh, o0, len_o, base, kappa, tid);
+    FarProj<KS> P;
+    P.load(a.proj, 16 * w + r16, E, sqrtf(a.temp) * FAR_LOG2E, g);
+    t.stash(a, Xo, Yo, diago, exto, co, tid);
+    int ic = c0 < e0 ? c0 : e1;                                                     // edges: c0 .. e0 - 1, e1 .. c1 - 1
+    constexpr bool AHEAD = !KEYMAJOR || NW >= 4;                                    // (registers for the next chunk's rows)
+    if (AHEAD && ic < c1) t.fetch(a, KEYMAJOR, xip, xis, yip, yis, bh, ic * FC, len_i, base, kappa, tid);
+    __syncthreads();
+
+    // own features: result rows = features 16 w + 4 g + i (sign sg), columns = outer rows 16 ob + r16
+    floatx4 fo[KEYMAJOR ? 1 : 2][4];
+    uintx4 foh[KEYMAJOR ? 4 : 1], fol[KEYMAJOR ? 4 : 1];                            // key-major: as two-piece operands, slots (sg, 4 g + i)
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) {
+        const floatx4 dd = P.features_by_rows(Xo + (16 * ob + r16) * LD + 8 * g);
+        const float bias = exto[16 * ob + r16] - diago[16 * ob + r16];
+        floatx4 f0, f1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool ok = 16 * w + 4 * g + i < a.mh_valid;
+            f0[i] = ok ? __builtin_amdgcn_exp2f(bias + dd[i]) : 0.f;
+            f1[i] = ok ? __builtin_amdgcn_exp2f(bias - dd[i]) : 0.f;
+        }
+        if (KEYMAJOR) split2(f0, f1, foh[KEYMAJOR ? ob : 0], fol[KEYMAJOR ? ob : 0]);
+        else { fo[0][ob] = f0; fo[KEYMAJOR ? 0 : 1][ob] = f1; }
+    }
+
+    // far terms from the prefix sums of the inner side: pre(c0) + (all - pre(c1))
+    const float* pre = (KEYMAJOR ? a.qg : a.kv) + (long)bh * n_ic * PER;
+    const float* p0 = c0 > 0 ? pre + (long)(c0 - 1) * PER : nullptr;
+    const float* p1 = c1 < n_ic ? pre + (long)max(c1 - 1, 0) * PER : nullptr;       // (c1 = 0: nothing to take off)
+    const float* pn = c1 < n_ic ? pre + (long)(n_ic - 1) * PER : nullptr;
+    if (c1 == 0) p1 = nullptr;
+    auto far4 = [&](long at) __attribute__((always_inline)) {
+        floatx4 x = Frag<float>::zero();
+        if (pn) x = *reinterpret_cast<const floatx4*>(pn + at);
+        if (p1) x -= *reinterpret_cast<const floatx4*>(p1 + at);
+        if (p0) x += *reinterpret_cast<const floatx4*>(p0 + at);
+        return x;
+    };
+    floatx4 acc2[2][4];                                                             // [sign][outer block], rows = features
+#pragma unroll
+    for (int sg = 0; sg < 2; ++sg) {
+#pragma unroll
+        for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] = Frag<float>::zero();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const long at = (long)(sg * MH + 16 * w + r16) * E + 32 * ks + 8 * g;
+            uintx4 fh, fl;
+            split2(far4(at), far4(at + 4), fh, fl);
+#pragma unroll
+            for (int ob = 0; ob < 4; ++ob) {
+                const uintx4 yo = *reinterpret_cast<const uintx4*>(Yo + (16 * ob + r16) * LD + 32 * ks + 8 * g);
+                acc2[sg][ob] = mma_bf16(fl, yo, acc2[sg][ob]);
+                acc2[sg][ob] = mma_bf16(fh, yo, acc2[sg][ob]);
+            }
+        }
+        const floatx4 vec = far4((long)M * E + sg * MH + 16 * w + 4 * g);
+#pragma unroll
+        for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] -= vec * (KEYMAJOR ? 1.0f : co[16 * ob + r16]);
+    }
+    floatx4 acc3[KEYMAJOR ? EB : 1][KEYMAJOR ? 4 : 1];                              // d v: rows = value dims, columns = keys
+    if (KEYMAJOR) {
+#pragma unroll
+        for (int eb = 0; eb < EB; ++eb) {
+            floatx4 x[2];
+#pragma unroll
+            for (int sg = 0; sg < 2; ++sg)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const long at = (long)(sg * MH + 16 * w + 4 * g + i) * E + 16 * eb + r16;
+                    float s = 0.f;
+                    if (pn) s = pn[at];
+                    if (p1) s -= p1[at];
+                    if (p0) s += p0[at];
+                    x[sg][i] = s;
+                }
+            uintx4 th, tl;
+            split2(x[0], x[1], th, tl);
+#pragma unroll
+            for (int ob = 0; ob < 4; ++ob) {
+                floatx4 d = Frag<float>::zero();
+                d = mma_bf16(tl, foh[KEYMAJOR ? ob : 0], d);
+                d = mma_bf16(th, fol[KEYMAJOR ? ob : 0], d);
+                acc3[KEYMAJOR ? eb : 0][KEYMAJOR ? ob : 0] = mma_bf16(th, foh[KEYMAJOR ? ob : 0], d);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    while (ic < c1) {
+        const int n0 = ic * FC;
+        if (!AHEAD) t.fetch(a, KEYMAJOR, xip, xis, yip, yis, bh, n0, len_i, base, kappa, tid);
+        t.stash(a, Xi, Yi, diagi, exti, ci, tid);
+        int nx = ic + 1;
+        if (nx == e0) nx = max(nx, e1);                                             // (over the chunks inside the band)
+        if (AHEAD && nx < c1) t.fetch(a, KEYMAJOR, xip, xis, yip, yis, bh, nx * FC, len_i, base, kappa, tid);
+        __syncthreads();
+        // df = g.v - c on the pairs outside the band, 0 inside: inner rows 32 st + 16 hb + 4 g + i, outer row 16 ob + r16 --
+        // eight contraction slots of the products below -- in two pieces
+        for (int it = w; it < 8; it += NW) {
+            const int st = it >> 2, ob = it & 3;
+            floatx4 s[2] = {Frag<float>::zero(), Frag<float>::zero()};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const uintx4 yo = *reinterpret_cast<const uintx4*>(Yo + (16 * ob + r16) * LD + 32 * ks + 8 * g);
+#pragma unroll
+                for (int hb = 0; hb < 2; ++hb)
+                    s[hb] = mma_bf16(*reinterpret_cast<const uintx4*>(Yi + (32 * st + 16 * hb + r16) * LD + 32 * ks + 8 * g), yo, s[hb]);
+            }
+#pragma unroll
+            for (int hb = 0; hb < 2; ++hb) {
+                const int row = 32 * st + 16 * hb + 4 * g;
+                const floatx4 cq = *reinterpret_cast<const floatx4*>(ci + row);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int rel = n0 + row + i - (o0 + 16 * ob + r16);
+                    s[hb][i] = (unsigned)(rel + A) < (unsigned)(A + Bq) ? 0.f : s[hb][i] - (KEYMAJOR ? cq[i] : co[16 * ob + r16]);
+                }
+            }
+            uintx4 hi, lo;
+            split2(s[0], s[1], hi, lo);
+            DF[it * 64 + lane] = hi;
+            DF[(8 + it) * 64 + lane] = lo;
+        }
+        __syncthreads();
+        // acc2^T[feature][outer] += F^T[feature][inner] df[inner][outer]
+        const bool fvalid = 16 * w + r16 < a.mh_valid;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            uintx4 fh[2], fl[2];
+            floatx4 f0[2], f1[2];
+#pragma unroll
+            for (int hb = 0; hb < 2; ++hb) {
+                const int kb = 2 * st + hb;
+                const floatx4 dd = P.rows_by_features(Xi + (16 * kb + r16) * LD + 8 * g);
+                const floatx4 bias = *reinterpret_cast<const floatx4*>(exti + 16 * kb + 4 * g) - *reinterpret_cast<const floatx4*>(diagi + 16 * kb + 4 * g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    f0[hb][i] = fvalid ? __builtin_amdgcn_exp2f(bias[i] + dd[i]) : 0.f;
+                    f1[hb][i] = fvalid ? __builtin_amdgcn_exp2f(bias[i] - dd[i]) : 0.f;
+                }
+            }
+            split2(f0[0], f0[1], fh[0], fl[0]);
+            split2(f1[0], f1[1], fh[1], fl[1]);
+#pragma unroll
+            for (int ob = 0; ob < 4; ++ob) {
+                const uintx4 dh = DF[(4 * st + ob) * 64 + lane], dl = DF[(8 + 4 * st + ob) * 64 + lane];
+#pragma unroll
+                for (int sg = 0; sg < 2; ++sg) {
+                    acc2[sg][ob] = mma_bf16(fl[sg], dh, acc2[sg][ob]);
+                    acc2[sg][ob] = mma_bf16(fh[sg], dl, acc2[sg][ob]);
+                    acc2[sg][ob] = mma_bf16(fh[sg], dh, acc2[sg][ob]);
+                }
+            }
+        }
+        if (KEYMAJOR) {
+            // this wave's features of the low-rank weights outside the band: result rows = queries, columns = keys; then
+            // d v^T[d][key] += g^T[d][query] W[query][key]
+#pragma unroll
+            for (int st = 0; st < 2; ++st) {
+                uintx4 wh[2], wl[2];
+#pragma unroll
+                for (int hb = 0; hb < 2; ++hb) {
+                    const int row = 32 * st + 16 * hb + r16;
+                    const floatx4 dd = P.features_by_rows(Xi + row * LD + 8 * g);
+                    const float bias = exti[row] - diagi[row];
+                    floatx4 f0, f1;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const bool ok = 16 * w + 4 * g + i < a.mh_valid;
+                        f0[i] = ok ? __builtin_amdgcn_exp2f(bias + dd[i]) : 0.f;
+                        f1[i] = ok ? __builtin_amdgcn_exp2f(bias - dd[i]) : 0.f;
+                    }
+                    split2(f0, f1, wh[hb], wl[hb]);
+                }
+                __builtin_amdgcn_sched_barrier(0);          // (the steps' operands do not fit the registers side by side)
+#pragma unroll
+                for (int ob = 0; ob < 4; ++ob) {
+                    floatx4 wt[2];
+#pragma unroll
+                    for (int hb = 0; hb < 2; ++hb) {
+                        wt[hb] = Frag<float>::zero();
+                        wt[hb] = mma_bf16(wl[hb], foh[KEYMAJOR ? ob : 0], wt[hb]);
+                        wt[hb] = mma_bf16(wh[hb], fol[KEYMAJOR ? ob : 0], wt[hb]);
+                        wt[hb] = mma_bf16(wh[hb], foh[KEYMAJOR ? ob : 0], wt[hb]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int rel = n0 + 32 * st + 16 * hb + 4 * g + i - (o0 + 16 * ob + r16);
+                            if ((unsigned)(rel + A) < (unsigned)(A + Bq)) wt[hb][i] = 0.f;
+                        }
+                    }
+                    uintx4 bh_, bl_;
+                    split2(wt[0], wt[1], bh_, bl_);
+#pragma unroll
+                    for (int eb = 0; eb < EB; ++eb) {
+                        const uint16_t* yq = Yi + (32 * st + 4 * g + (r16 >> 2)) * LD + 16 * eb + 4 * (r16 & 3);
+                        const uintx4 yt = lds_read_tr8(reinterpret_cast<const char*>(yq), reinterpret_cast<const char*>(yq + 16 * LD));
+                        floatx4& d = acc3[KEYMAJOR ? eb : 0][KEYMAJOR ? ob : 0];
+                        d = mma_bf16(yt, bl_, d);
+                        d = mma_bf16(yt, bh_, d);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+        __syncthreads();                                                            // the inner chunk and df are free
+        ic = nx;
+    }
+
+    // u = F_o o acc2; d x = sqrt(t) P^T (u+ - u-) - t x sum u
+    floatx4 du[4];
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) {
+        floatx4 f0, f1;
+        if (KEYMAJOR) {
+            const uintx4 xh = foh[KEYMAJOR ? ob : 0], xl = fol[KEYMAJOR ? ob : 0];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t h0 = xh[i >> 1], l0 = xl[i >> 1], h1 = xh[2 + (i >> 1)], l1 = xl[2 + (i >> 1)];
+                f0[i] = (i & 1) ? __uint_as_float(h0 & 0xffff0000u) + __uint_as_float(l0 & 0xffff0000u) : __uint_as_float(h0 << 16) + __uint_as_float(l0 << 16);
+                f1[i] = (i & 1) ? __uint_as_float(h1 & 0xffff0000u) + __uint_as_float(l1 & 0xffff0000u) : __uint_as_float(h1 << 16) + __uint_as_float(l1 << 16);
+            }
+        } else { f0 = fo[0][ob]; f1 = fo[KEYMAJOR ? 0 : 1][ob]; }
+        const floatx4 up = f0 * acc2[0][ob], un = f1 * acc2[1][ob];
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s += up[i] + un[i];
+        s = group_sum(s);
+        if (g == 0) us[w * FC + 16 * ob + r16] = s;
+        du[ob] = up - un;
+    }
+    // the wave's 16 rows of P as one 32-slot step: slots (0, 4 g + i) and (1, 4 g + i) carry different piece products
+    uintx4 bo[4][2];
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) {
+        uint2 dh, dl;
+        split2_4(du[ob], dh, dl);
+        bo[ob][0] = uintx4{dh.x, dh.y, dh.x, dh.y};
+        bo[ob][1] = uintx4{dl.x, dl.y, dh.x, dh.y};
+    }
+    const float stemp = sqrtf(a.temp);
+    constexpr int QUADS = FC * 4;                                                   // groups of four columns of a 16-column block, per 64 rows
+#pragma unroll
+    for (int pass = 0; pass < (KEYMAJOR ? 2 : 1); ++pass)
+#pragma unroll
+        for (int eb = 0; eb < EB; ++eb) {
+            floatx4 d[4];
+            if (pass == 0) {
+                floatx4 pv;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) pv[i] = a.proj[(long)(16 * w + 4 * g + i) * E + 16 * eb + r16] * stemp;
+                uint2 ph, pm, pl;
+                split3_4(pv, ph, pm, pl);
+                const uintx4 a0 = {ph.x, ph.y, pm.x, pm.y}, a1 = {ph.x, ph.y, pl.x, pl.y};
+#pragma unroll
+                for (int ob = 0; ob < 4; ++ob) d[ob] = mma_bf16(a0, bo[ob][0], mma_bf16(a1, bo[ob][1], Frag<float>::zero()));
+            } else {
+#pragma unroll
+                for (int ob = 0; ob < 4; ++ob) d[ob] = acc3[KEYMAJOR ? eb : 0][KEYMAJOR ? ob : 0];
+            }
+#pragma unroll
+            for (int ob = 0; ob < 4; ++ob) *reinterpret_cast<floatx4*>(red + ((w * FC + 16 * ob + r16) * 16 + 4 * g)) = d[ob];
+            __syncthreads();
+            float* dst = pass == 0 ? (KEYMAJOR ? a.dk : a.dq) : a.dv;
+            for (int x = tid; x < QUADS; x += NT) {
+                const int row = x >> 2, qd = x & 3;
+                floatx4 s = *reinterpret_cast<const floatx4*>(red + (row * 16 + 4 * qd));
+                float usum = us[row];
+#pragma unroll
+                for (int v = 1; v < NW; ++v) {
+                    s += *reinterpret_cast<const floatx4*>(red + ((v * FC + row) * 16 + 4 * qd));
+                    usum += us[v * FC + row];
+                }
+                if (pass == 0) {
+                    const uint2 xr = *reinterpret_cast<const uint2*>(Xo + row * LD + 16 * eb + 4 * qd);
+                    const floatx4 xf = {__uint_as_float(xr.x << 16), __uint_as_float(xr.x & 0xffff0000u),
+                                        __uint_as_float(xr.y << 16), __uint_as_float(xr.y & 0xffff0000u)};
+                    s -= xf * (a.temp * usum);
+                }
+                if (o0 + row < Lo) *reinterpret_cast<floatx4*>(dst + ((long)bh * Lo + o0 + row) * E + 16 * eb + 4 * qd) = s;
+            }
+            __syncthreads();
+        }
+}
+
+template <int E, int M, bool KEYMAJOR>
+static int launch_lowrank(const FarArgs& a, hipStream_t st) {
+    auto kern = far_lowrank_kernel<E, M, KEYMAJOR>;
+    constexpr size_t smem = far_lowrank_smem<E, M>();
+    static std::atomic<unsigned long long> lds_set{0};     // (devices on which this kernel has its LDS limit)
+    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_set, "far_lowrank")) return rc;
+    const long items = (long)a.B * a.H * (KEYMAJOR ? a.n_kc : a.n_qc);
+    const long grid = (items + a.n_xcd - 1) / a.n_xcd * a.n_xcd;
+    if (grid > 2147483647L) return fail(ERR_ARG, "sblocal_bwd_far: too many workgroups");
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(2 * M), smem, st, a);
+    return check_launch("far_lowrank_kernel");
+}
+
+template <int E, int M>
+static int launch_far(const FarArgs& a, const LocalBwdArgs& band, hipStream_t st) {
+    const int BH = a.B * a.H, per4 = M * (E + 1) / 4;
+    hipLaunchKernelGGL((far_chunk_kernel<E, M>), dim3(a.n_kc + a.n_qc, BH), dim3(2 * M), 0, st, a);
+    if (int rc = check_launch("far_chunk_kernel")) return rc;
+    hipLaunchKernelGGL(far_scan_kernel, dim3((per4 + FAR_SCAN_NT - 1) / FAR_SCAN_NT, 2, BH), dim3(FAR_SCAN_NT), 0, st, a, per4);
+    if (int rc = check_launch("far_scan_kernel")) return rc;
+    if (int rc = launch_lowrank<E, M, false>(a, st)) return rc;
+    if (int rc = launch_lowrank<E, M, true>(a, st)) return rc;
+    return launch_local_bwd_exact(band, E, st);
+}
+
+// floats of each piece of the workspace, in order: c, kscale, qscale, kv, qg, dq, dk, dv
+static void far_pieces(int64_t BH, int64_t T, int64_t S, int64_t E, int64_t M, int64_t (&n)[8]) {
+    const int64_t kc = (S + FC - 1) / FC, qc = (T + FC - 1) / FC, per = M * (E + 1);
+    const int64_t want[8] = {BH * T, BH * kc, BH * qc, BH * kc * per, BH * qc * per, BH * T * E, BH * S * E, BH * S * E};
+    for (int i = 0; i < 8; ++i) n[i] = (want[i] + 63) / 64 * 64;
+}
+
+}  // namespace flyhip
+
+using namespace flyhip;
+
+extern "C" int64_t flyhip_sblocal_bwd_far_floats(int BH, int T, int S, int E, int M) {
+    if (BH <= 0 || T <= 0 || S <= 0 || E <= 0 || M <= 0) return -1;
+    int64_t n[8], sum = 0;
+    far_pieces(BH, T, S, E, M, n);
+    for (int64_t x : n) sum += x;
+    return sum;
+}
+
+extern "C" int flyhip_sblocal_bwd_far(const void* q, const void* k, const void* v, const void* out, const void* grad_out,
+                                      const float* log_norm, const float* proj, const int64_t* key_lengths,
+                                      void* dq, void* dk, void* dv, float* workspace, int64_t workspace_floats,
+                                      int B, int H, int T, int S, int E, int M, int mh_valid, int local_context,
+                                      int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss,
+                                      int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb, int64_t o_sh, int64_t o_ss,
+                                      int64_t g_sb, int64_t g_sh, int64_t g_ss,
+                                      int64_t dq_sb, int64_t dq_sh, int64_t dq_ss, int64_t dk_sb, int64_t dk_sh, int64_t dk_ss,
+                                      int64_t dv_sb, int64_t dv_sh, int64_t dv_ss,
+                                      float softmax_temp, void* stream) {
+    FLY_REQUIRE(q && k && v && out && grad_out && log_norm && proj && dq && dk && dv && workspace, "sblocal_bwd_far: null pointer");
+    FLY_REQUIRE(B > 0 && H > 0 && T > 0 && S > 0 && (int64_t)B * H <= 65535, "sblocal_bwd_far: empty problem or more than 65535 (batch, head) pairs");
+    FLY_REQUIRE(local_context >= 1, "sblocal_bwd_far: local_context must be >= 1");
+    FLY_REQUIRE(softmax_temp > 0.f, "sblocal_bwd_far: softmax_temp must be positive");
+    FLY_REQUIRE(mh_valid >= 1 && 2 * mh_valid <= M, "sblocal_bwd_far: %d projection rows do not fit %d features", mh_valid, M);
+    FLY_REQUIRE(((q_sb | q_sh | q_ss | k_sb | k_sh | k_ss | v_sb | v_sh | v_ss | g_sb | g_sh | g_ss | o_sb | o_sh | o_ss) % 8) == 0,
+                "sblocal_bwd_far: input strides must be multiples of 8 elements (16-byte loads)");
+    FLY_REQUIRE(((dq_sb | dq_sh | dq_ss | dk_sb | dk_sh | dk_ss | dv_sb | dv_sh | dv_ss) % 4) == 0,
+                "sblocal_bwd_far: output strides must be multiples of 4 elements (8-byte stores)");
+    FLY_REQUIRE(((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
+                  reinterpret_cast<uintptr_t>(grad_out) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(proj) |
+                  reinterpret_cast<uintptr_t>(workspace)) % 16) == 0 &&
+                ((reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv)) % 8) == 0,
+                "sblocal_bwd_far: pointers must be 16-byte (inputs) and 8-byte (outputs) aligned");
+    const int64_t need = flyhip_sblocal_bwd_far_floats(B * H, T, S, E, M);
+    FLY_REQUIRE(workspace_floats >= need, "sblocal_bwd_far: workspace of %lld floats, %lld needed", (long long)workspace_floats, (long long)need);
+    int64_t n[8];
+    far_pieces((int64_t)B * H, T, S, E, M, n);
+    float* p[8];
+    float* at = workspace;
+    for (int i = 0; i < 8; ++i) { p[i] = at; at += n[i]; }
+    FarArgs a{reinterpret_cast<const uint16_t*>(q), reinterpret_cast<const uint16_t*>(k), reinterpret_cast<const uint16_t*>(v),
+              reinterpret_cast<const uint16_t*>(grad_out), reinterpret_cast<const uint16_t*>(out), log_norm, proj, key_lengths,
+              p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7],
+              B, H, T, S, local_context, mh_valid, (S + FC - 1) / FC, (T + FC - 1) / FC,
+              q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss, softmax_temp, machine().xcds};
+    LocalBwdArgs band{q, k, v, grad_out, out, log_norm, p[0], key_lengths, dq, dk, dv, B, H, T, S, local_context,
+                      q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss,
+                      dq_sb, dq_sh, dq_ss, dk_sb, dk_sh, dk_ss, dv_sb, dv_sh, dv_ss, softmax_temp, 0, p[5], p[6], p[7]};
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (int rc_capture = refuse_capture(st)) return rc_capture;
+    if (E == 32 && M == 32) return launch_far<32, 32>(a, band, st);
+    if (E == 32 && M == 64) return launch_far<32, 64>(a, band, st);
+    if (E == 64 && M == 32) return launch_far<64, 32>(a, band, st);
+    if (E == 64 && M == 64) return launch_far<64, 64>(a, band, st);
+    if (E == 64 && M == 128) return launch_far<64, 128>(a, band, st);
+    if (E == 64 && M == 256) return launch_far<64, 256>(a, band, st);
+    return fail(ERR_UNSUPPORTED, "sblocal_bwd_far: (head dim, features) = (%d, %d) not in "
+                                 "{(32,32), (32,64), (64,32), (64,64), (64,128), (64,256)}", E, M);
+}

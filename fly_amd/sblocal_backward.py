@@ -228,6 +228,75 @@ def _backward_hip(Q, K, V, G, O, LN, P, lens_b, H, local_context, t, dims, piece
     return dq[..., :E], dk[..., :E], dv[..., :D]
 
 
+# (head dim, features) of the kernels of flyhip_sblocal_bwd_far
+_FAR_KERNEL_DIMS = ((32, 32), (32, 64), (64, 32), (64, 64), (64, 128), (64, 256))
+_FAR_WORKSPACE_FLOATS = 1 << 30            # workspace of one launch sequence; larger problems go through it in slices
+
+
+def _far_kernel_dims(E, D, M):
+    for dim, mk in _FAR_KERNEL_DIMS:
+        if max(E, D) <= dim and M <= mk:
+            return dim, mk
+    return None
+
+
+def _far_pays(rows, local_context, M):
+    """Whether bfloat16 tensors go to _backward_far where the kernels that subtract the band from the sums over all keys
+    (_backward_hip, on widened copies) could take them too.  Their M-wide products on every pair of the band cost in
+    proportion to the window, the chunk sums of the far path per row: at 200704 rows, 128 features 773 against 943 us at
+    window 256, 774 against 745 at 49; at 131072 rows, 64 features 376 against 464 us at window 128; 262144 rows, 128 features,
+    window 1024: 1263 against 2401.  Small problems, where launches and the copies count: 73 against 134 us at 8000 rows,
+    window 100."""
+    return M > 128 or local_context >= 96 or rows <= 16384
+
+
+def _backward_far(query, key, value, P, local_context, t, key_lengths, out, log_norm, grad_out, dims):
+    """d query, d key, d value for bfloat16 GPU tensors as they lie in memory (flyhip_sblocal_bwd_far): pairs outside the
+    band through prefix sums over chunks of 64 rows, the chunks at the band's edges pair by pair, the band itself on the
+    kernels of plain local attention.  The chunk sums take M (E + 1) floats per 64 rows of either side, so problems of
+    more than _FAR_WORKSPACE_FLOATS go through in slices of the batch (of the heads where one batch entry is too large)."""
+    from . import _lib
+    B, T, H, E = query.shape
+    S, D = key.shape[1], value.shape[3]
+    dim, mk = dims
+
+    def prep(x):
+        if x.shape[-1] != dim:
+            x = torch.nn.functional.pad(x, (0, dim - x.shape[-1]))
+        ready = x.stride(-1) == 1 and all(st % 8 == 0 for st in x.stride()[:-1]) and x.data_ptr() % 16 == 0
+        return x if ready else x.contiguous()
+    q, k, v, o, g = prep(query), prep(key), prep(value), prep(out), prep(grad_out.to(query.dtype))
+    mh = P.shape[0]
+    proj = P.contiguous() if P.shape == (mk // 2, dim) else _fit(torch.nn.functional.pad(P, (0, 0, 0, mk // 2 - mh)), dim)
+    ln = log_norm.reshape(B, H, T).float().contiguous()
+    lens = None if key_lengths is None else key_lengths.to(device=query.device, dtype=torch.int64).contiguous()
+    new = query.new_empty
+    dq, dk, dv = new(B, T, H, dim), new(B, S, H, dim), new(B, S, H, dim)
+    size = _lib.load().flyhip_sblocal_bwd_far_floats
+    per_head = size(1, T, S, dim, mk)
+    fit = max(1, min(_FAR_WORKSPACE_FLOATS // per_head, 65535))              # (batch, head) pairs per slice
+    nb, nh = (max(1, min(B, fit // H)), H) if fit >= H else (1, fit)
+    ws = torch.empty(size(nb * nh, T, S, dim, mk), dtype=torch.float32, device=query.device)
+
+    def strides(x):
+        return x.stride(0), x.stride(2), x.stride(1)
+    with torch.cuda.device(query.device):
+        st = _lib.stream_ptr(query.device)
+        for b0 in range(0, B, nb):
+            for h0 in range(0, H, nh):
+                b1, h1 = min(B, b0 + nb), min(H, h0 + nh)
+                part = [x[b0:b1, :, h0:h1] for x in (q, k, v, o, g, dq, dk, dv)]
+                ln_ = ln[b0:b1, h0:h1].contiguous()
+                lens_ = None if lens is None else lens[b0:b1]
+                qs, ks, vs, os_, gs, dqs, dks, dvs = part
+                _lib.call('flyhip_sblocal_bwd_far', qs.data_ptr(), ks.data_ptr(), vs.data_ptr(), os_.data_ptr(), gs.data_ptr(),
+                          ln_.data_ptr(), proj.data_ptr(), _lib.ptr(lens_), dqs.data_ptr(), dks.data_ptr(), dvs.data_ptr(),
+                          ws.data_ptr(), ws.numel(), b1 - b0, h1 - h0, T, S, dim, mk, mh, local_context,
+                          *strides(q), *strides(k), *strides(v), *strides(o), *strides(g), *strides(dq), *strides(dk),
+                          *strides(dv), float(t), st)
+    return dq[..., :E], dk[..., :E], dv[..., :D]
+
+
 def _band_terms_hip(Q, K, V, G, psi, phik, LN, c, lens_b, H, local_context, t, dims, dropout=(0.0, 0), attn_mask=None):
     """The five band-limited sums on flyhip_sblocal_bwd_band.  Q, G, psi, LN, c: (BH, T, .); K, V, phik:
     (BH, S, .); float32 on the GPU.  Returns (t sum_s dm k, sum_s df phik, t sum_i dm q, sum_i df psi,
@@ -333,7 +402,12 @@ def sblocal_backward(query, key, value, projection_matrix, local_context, softma
     B, T, H, E = query.shape
     S, D = key.shape[1], value.shape[3]
     t = softmax_temp or 1 / math.sqrt(E)
-    lc_lo, lc_hi = local_context // 2, (local_context + 1) // 2
+    if (query.dtype == torch.bfloat16 and query.is_cuda and band_kernel is None and support is None and dropout[0] == 0
+            and key.dtype == value.dtype == out.dtype == query.dtype):
+        far_dims = _far_kernel_dims(E, D, 2 * projection_matrix.shape[0])
+        if far_dims is not None and _far_pays(B * H * max(T, S), local_context, far_dims[1]):
+            return _backward_far(query, key, value, projection_matrix.float(), local_context, t, key_lengths, out,
+                                 log_normalization, grad_out, far_dims)
     wdt = torch.float64 if query.dtype == torch.float64 else torch.float32
 
     def bh(x):                                   # (B,L,H,C) -> (B*H, L, C)

@@ -277,6 +277,25 @@ int flyhip_sblocal_bwd_pieces(const void* outer_images, const void* inner_images
                               float softmax_temp, int key_major, float dropout_p, uint64_t dropout_seed,
                               void* stream);
 
+/* The whole backward of Scatterbrain-local attention after the feature-map draw for bfloat16 tensors (what autograd does
+ * through sblocal_attention.py:73-122), head dims E in {32,64}, up to 256 features: q, out, grad_out (B,T,H,E), k, v
+ * (B,S,H,E), dq / dk / dv like q / k / v, all addressed through (batch, head, seq) strides with the innermost dim
+ * contiguous; log_norm (B,H,T) from the forward; proj (M/2, E) fp32, rows >= mh_valid zero; key_lengths (B) or NULL.
+ * Pairs outside the band go through sums over chunks of 64 rows (prefix sums) and, where a chunk straddles the band's
+ * edge, one by one; pairs inside it are plain local attention's.  workspace: flyhip_sblocal_bwd_far_floats floats, no
+ * initialisation needed.  (E, M) in {(32,32), (32,64), (64,32), (64,64), (64,128), (64,256)}. */
+int64_t flyhip_sblocal_bwd_far_floats(int BH, int T, int S, int E, int M);
+int flyhip_sblocal_bwd_far(const void* q, const void* k, const void* v, const void* out, const void* grad_out,
+                           const float* log_norm, const float* proj, const int64_t* key_lengths,
+                           void* dq, void* dk, void* dv, float* workspace, int64_t workspace_floats,
+                           int B, int H, int T, int S, int E, int M, int mh_valid, int local_context,
+                           int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss,
+                           int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb, int64_t o_sh, int64_t o_ss,
+                           int64_t g_sb, int64_t g_sh, int64_t g_ss,
+                           int64_t dq_sb, int64_t dq_sh, int64_t dq_ss, int64_t dk_sb, int64_t dk_sh, int64_t dk_ss,
+                           int64_t dv_sb, int64_t dv_sh, int64_t dv_ss,
+                           float softmax_temp, void* stream);
+
 /* flyhip_sblocal_bwd_pieces for Scatterbrain attention on a block-sparse support (the reference takes these
  * gradients from autograd through src/models/attention/sbblocksparse_attention.py:161-212): the exact weights live on
  * the nonzero blocks (16 x 16 or 32 x 32) of a layout instead of a band.  tl_ptr (H * ceil(outer rows / 64) + 1),

@@ -998,3 +998,43 @@ def test_attention_dropout_module_and_refusals():
         sblocal_forward(q2.to(dev), k2.to(dev), v2.to(dev), P2.to(dev), 64, dropout_p=0.1, dropout_seed=1)
     with pytest.raises(NotImplementedError):
         attn(qd, kd, vd, need_weights=True)
+
+
+@pytest.mark.parametrize('case', [
+    dict(B=1, T=300, S=300, H=1, E=64, mh=128, lc=64, lens=None, scale=0.35),          # whole chunks at the band's edges
+    dict(B=2, T=200, S=333, H=2, E=64, mh=64, lc=100, lens=[333, 150], scale=0.35),    # ragged, padded keys
+    dict(B=1, T=700, S=500, H=2, E=64, mh=128, lc=257, lens=None, scale=1.0),          # queries past the last key
+    dict(B=1, T=130, S=700, H=1, E=32, mh=32, lc=12, lens=None, scale=0.4),            # window inside one chunk
+    dict(B=2, T=64, S=64, H=1, E=64, mh=16, lc=200, lens=[64, 1], scale=0.4),          # one chunk, window over everything
+    dict(B=1, T=65, S=129, H=1, E=32, mh=16, lc=1, lens=None, scale=0.4),              # one key a query
+    dict(B=1, T=1000, S=1000, H=2, E=64, mh=100, lc=333, lens=[1000], scale=0.35),     # projection rows that are padding
+    dict(B=3, T=90, S=1000, H=1, E=64, mh=3, lc=40, lens=[1000, 1, 500], scale=0.4),
+], ids=lambda c: f"T{c['T']}-S{c['S']}-E{c['E']}-mh{c['mh']}-lc{c['lc']}")
+def test_bf16_gradients_through_chunk_sums(case, monkeypatch):
+    """flyhip_sblocal_bwd_far (far pairs through prefix sums over chunks, edge chunks pair by pair, the band on the local
+    attention kernels) against autograd through the oracle in float64 on the same bfloat16 inputs; the same numbers when
+    the problem goes through in slices of one (batch, head).  Bar (2-norm): the gradients are rounded to bfloat16 (2^-9), and
+    so is the forward's output inside g.out, which d query and d key see once more where g.v - g.out cancels."""
+    import importlib
+    from fly_amd import sblocal_attention_fn
+    sbb = importlib.import_module('fly_amd.sblocal_backward')
+    B, T, S, H, E, mh, lc = (case[x] for x in ('B', 'T', 'S', 'H', 'E', 'mh', 'lc'))
+    g = torch.Generator().manual_seed(T + S + E)
+    q, k, v, w = (torch.randn(B, L, H, E, generator=g) for L in (T, S, S, T))
+    q, k, v, w = (q * case['scale']).bfloat16(), (k * case['scale']).bfloat16(), v.bfloat16(), w.bfloat16()
+    P = osb.gaussian_orthogonal_random_matrix(mh, E, generator=g)
+    lens = None if case['lens'] is None else torch.tensor(case['lens'])
+    dev = torch.device('cuda:0')
+    monkeypatch.setattr(sbb, '_far_pays', lambda *a: True)
+    qg, kg, vg = (x.to(dev).requires_grad_() for x in (q, k, v))
+    out, _ = sblocal_attention_fn(qg, kg, vg, P.to(dev), lc, None, None if lens is None else lens.to(dev))
+    got = torch.autograd.grad(out, (qg, kg, vg), w.to(dev), retain_graph=True)
+    qd, kd, vd = (x.double().requires_grad_() for x in (q, k, v))
+    ref_out, _ = osb.sblocal_attention(qd, kd, vd, P.double(), lc, key_lengths=lens)
+    ref = torch.autograd.grad(ref_out, (qd, kd, vd), w.double())
+    for a, r in zip(got, ref):
+        err = float((a.double().cpu() - r).norm() / r.norm())
+        assert a.dtype == torch.bfloat16 and err <= 6e-3, err
+    monkeypatch.setattr(sbb, '_FAR_WORKSPACE_FLOATS', 1)
+    for a, b in zip(got, torch.autograd.grad(out, (qg, kg, vg), w.to(dev))):
+        assert torch.equal(a, b)
