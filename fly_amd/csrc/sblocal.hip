@@ -2540,23 +2540,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 // The band kernel without its low-rank half: per (batch, head, 64-query tile) scores^T = (t log2e) K q
 // on fp32 MFMA, band / length masks, online softmax, P V; key tiles double-buffered through LDS.
 // A query without any valid key gets a zero output row.
-struct LocalArgs {
-    const void* q; const void* k; const void* v; const int64_t* lens; void* out;
-    int B, H, T, S, lc;
-    long q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss;
-    float temp;
-    float* lse;                     // optional (B, H, T): log of the softmax denominator, for the backward pass
-    int n_xcd;                      // dies the dispatcher deals workgroup ids to (set at launch)
-    // dropout of the probabilities (drop_thresh != 0): pair (query i, key s) of (b, h) is kept when the hash of
-    // (seed, row = (b H + h) T + i, s) reaches the threshold, and scaled by 1 / (1 - p); the denominator sums all
-    uint32_t drop_seed, drop_thresh; float drop_scale;
-    // optional additive mask (T, S), float32, rows contiguous: added to q.k before the temperature.  Entries of -1e24
-    // absorb the product (every masked score is the same float), so a query whose visible keys are all masked gets
-    // equal weights 1 / local_context -- over the positions of its band that fall outside the keys as well, which
-    // count in the denominator only; its lse entry is -inf, the marker the backward kernel reads.
-    const float* add_mask;
-};
-
 template <typename T, int E, int D>
 __global__ __launch_bounds__(NT) void local_fwd_kernel(LocalArgs a) {
     constexpr int LDK = E + 4, LDV = D + 4, EC = E / 16, DB = D / 16, KB = TK / 16;
@@ -5609,7 +5592,9 @@ extern "C" int flyhip_local_fwd_masked(const void* q, const void* k, const void*
         case 128: return launch_local<TT, 128>(a, st);                                              \
         default: return fail(ERR_UNSUPPORTED, "local_fwd: head dim E=%d not in {32,64,128}", E);     \
     }
-    if (dtype == F32) { LOCAL_DISPATCH(float) }
+    if (dtype == F32 && (E == 32 || E == 64)) return launch_local_fwd_x3(a, E, st);
+    if (dtype == F32 && E == 128) return launch_local<float, 128>(a, st);      // (piece tiles would leave one workgroup per compute unit)
+    if (dtype == F32) return fail(ERR_UNSUPPORTED, "local_fwd: head dim E=%d not in {32,64,128}", E);
 #define LOCAL_DISPATCH_B16(TT)                                                                      \
     switch (E) {                                                                                    \
         case 32: return launch_local_b16<TT, 32>(a, st);                                            \
@@ -5628,6 +5613,62 @@ extern "C" int flyhip_local_fwd_masked(const void* q, const void* k, const void*
     return fail(ERR_UNSUPPORTED, "local_fwd supports float32, bfloat16 and float16, got dtype code %d", dtype);
 }
 
+extern "C" int flyhip_local_bwd_masked(const void* q, const void* k, const void* v, const void* out, const void* grad_out,
+                               const float* lse, const int64_t* key_lengths, const float* attn_mask, float* delta,
+                               void* dq, void* dk, void* dv,
+                               int B, int H, int T, int S, int E, int local_context,
+                               int64_t q_sb, int64_t q_sh, int64_t q_ss,
+                               int64_t k_sb, int64_t k_sh, int64_t k_ss,
+                               int64_t v_sb, int64_t v_sh, int64_t v_ss,
+                               int64_t o_sb, int64_t o_sh, int64_t o_ss,
+                               int64_t g_sb, int64_t g_sh, int64_t g_ss,
+                               int64_t dq_sb, int64_t dq_sh, int64_t dq_ss,
+                               int64_t dk_sb, int64_t dk_sh, int64_t dk_ss,
+                               int64_t dv_sb, int64_t dv_sh, int64_t dv_ss,
+                               float softmax_temp, int dtype, float dropout_p, uint64_t dropout_seed, void* stream) {
+    FLY_REQUIRE(q && k && v && out && grad_out && lse && delta && dq && dk && dv, "local_bwd: null pointer");
+    FLY_REQUIRE(B > 0 && H > 0 && T > 0 && S > 0, "local_bwd: empty problem");
+    FLY_REQUIRE(local_context >= 1, "local_bwd: local_context must be >= 1");
+    FLY_REQUIRE(softmax_temp > 0.f, "local_bwd: softmax_temp must be positive");
+    FLY_REQUIRE(dropout_p >= 0.f && dropout_p < 1.f, "local_bwd: dropout_p %g not in [0, 1)", (double)dropout_p);
+    FLY_REQUIRE((long)B * H * T <= 4294967295L, "local_bwd: more than 2^32 query rows");
+    FLY_REQUIRE(((q_sb | q_sh | q_ss | k_sb | k_sh | k_ss | v_sb | v_sh | v_ss | g_sb | g_sh | g_ss | o_sb | o_sh | o_ss) %
+                 (dtype == F32 ? 4 : 8)) == 0,
+                "local_bwd: input strides must be multiples of 16 bytes (16-byte loads)");
+    FLY_REQUIRE(((dq_sb | dq_sh | dq_ss | dk_sb | dk_sh | dk_ss | dv_sb | dv_sh | dv_ss) % 4) == 0,
+                "local_bwd: output strides must be multiples of 4 elements (8-byte stores)");
+    FLY_REQUIRE(((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
+                  reinterpret_cast<uintptr_t>(grad_out) | reinterpret_cast<uintptr_t>(out)) % 16) == 0 &&
+                ((reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv)) % 8) == 0,
+                "local_bwd: pointers must be 16-byte (inputs) and 8-byte (outputs) aligned");
+    FLY_REQUIRE(dtype != F32 || ((reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv)) % 16) == 0,
+                "local_bwd: float32 outputs must be 16-byte aligned");
+    LocalBwdArgs a{q, k, v, grad_out, out, lse, delta, key_lengths, dq, dk, dv, B, H, T, S, local_context,
+                   q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss,
+                   dq_sb, dq_sh, dq_ss, dk_sb, dk_sh, dk_ss, dv_sb, dv_sh, dv_ss, softmax_temp, 0};
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (int rc_capture = refuse_capture(st)) return rc_capture;
+#define LOCAL_BWD_DISPATCH(TT)                                                                      \
+    switch (E) {                                                                                    \
+        case 32: return launch_local_bwd<TT, 32>(a, st);                                            \
+        case 64: return launch_local_bwd<TT, 64>(a, st);                                            \
+        case 128: return launch_local_bwd<TT, 128>(a, st);                                          \
+        default: return fail(ERR_UNSUPPORTED, "local_bwd: head dim E=%d not in {32,64,128}", E);     \
+    }
+    const DropArgs drop = drop_args(dropout_p, dropout_seed);
+    a.add_mask = attn_mask;
+    a.drop_seed = drop.seed; a.drop_thresh = drop.thresh; a.drop_scale = drop.scale;
+    if (dtype == F32) {
+        if (E == 32 || E == 64) return launch_local_bwd_x3(a, E, st);
+        return fail(ERR_UNSUPPORTED, "local_bwd: float32 head dim E=%d not in {32,64}", E);
+    }
+    if (attn_mask || drop.thresh != 0u) return fail(ERR_UNSUPPORTED, "local_bwd: attn_mask and dropout for float32 only");
+    if (dtype == BF16) { LOCAL_BWD_DISPATCH(bf16_t) }
+    if (dtype == F16) { LOCAL_BWD_DISPATCH(f16_t) }
+#undef LOCAL_BWD_DISPATCH
+    return fail(ERR_UNSUPPORTED, "local_bwd supports float32, bfloat16 and float16, got dtype code %d", dtype);
+}
+
 extern "C" int flyhip_local_bwd(const void* q, const void* k, const void* v, const void* out, const void* grad_out,
                                const float* lse, const int64_t* key_lengths, float* delta,
                                void* dq, void* dk, void* dv,
@@ -5641,34 +5682,9 @@ extern "C" int flyhip_local_bwd(const void* q, const void* k, const void* v, con
                                int64_t dk_sb, int64_t dk_sh, int64_t dk_ss,
                                int64_t dv_sb, int64_t dv_sh, int64_t dv_ss,
                                float softmax_temp, int dtype, void* stream) {
-    FLY_REQUIRE(q && k && v && out && grad_out && lse && delta && dq && dk && dv, "local_bwd: null pointer");
-    FLY_REQUIRE(B > 0 && H > 0 && T > 0 && S > 0, "local_bwd: empty problem");
-    FLY_REQUIRE(local_context >= 1, "local_bwd: local_context must be >= 1");
-    FLY_REQUIRE(softmax_temp > 0.f, "local_bwd: softmax_temp must be positive");
-    FLY_REQUIRE(((q_sb | q_sh | q_ss | k_sb | k_sh | k_ss | v_sb | v_sh | v_ss | g_sb | g_sh | g_ss | o_sb | o_sh | o_ss) % 8) == 0,
-                "local_bwd: input strides must be multiples of 8 elements (16-byte loads)");
-    FLY_REQUIRE(((dq_sb | dq_sh | dq_ss | dk_sb | dk_sh | dk_ss | dv_sb | dv_sh | dv_ss) % 4) == 0,
-                "local_bwd: output strides must be multiples of 4 elements (8-byte stores)");
-    FLY_REQUIRE(((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
-                  reinterpret_cast<uintptr_t>(grad_out) | reinterpret_cast<uintptr_t>(out)) % 16) == 0 &&
-                ((reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv)) % 8) == 0,
-                "local_bwd: pointers must be 16-byte (inputs) and 8-byte (outputs) aligned");
-    LocalBwdArgs a{q, k, v, grad_out, out, lse, delta, key_lengths, dq, dk, dv, B, H, T, S, local_context,
-                   q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss,
-                   dq_sb, dq_sh, dq_ss, dk_sb, dk_sh, dk_ss, dv_sb, dv_sh, dv_ss, softmax_temp, 0};
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    if (int rc_capture = refuse_capture(st)) return rc_capture;
-#define LOCAL_BWD_DISPATCH(TT)                                                                      \
-    switch (E) {                                                                                    \
-        case 32: return launch_local_bwd<TT, 32>(a, st);                                            \
-        case 64: return launch_local_bwd<TT, 64>(a, st);                                            \
-        case 128: return launch_local_bwd<TT, 128>(a, st);                                          \
-        default: return fail(ERR_UNSUPPORTED, "local_bwd: head dim E=%d not in {32,64,128}", E);     \
-    }
-    if (dtype == BF16) { LOCAL_BWD_DISPATCH(bf16_t) }
-    if (dtype == F16) { LOCAL_BWD_DISPATCH(f16_t) }
-#undef LOCAL_BWD_DISPATCH
-    return fail(ERR_UNSUPPORTED, "local_bwd supports bfloat16 and float16, got dtype code %d", dtype);
+    return flyhip_local_bwd_masked(q, k, v, out, grad_out, lse, key_lengths, nullptr, delta, dq, dk, dv, B, H, T, S, E, local_context,
+                                   q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, g_sb, g_sh, g_ss,
+                                   dq_sb, dq_sh, dq_ss, dk_sb, dk_sh, dk_ss, dv_sb, dv_sh, dv_ss, softmax_temp, dtype, 0.f, 0, stream);
 }
 
 extern "C" int flyhip_local_fwd(const void* q, const void* k, const void* v, const int64_t* key_lengths, void* out,

@@ -8,7 +8,7 @@ import torch.nn.functional as F
 
 from . import _lib
 from .sblocal_attention import _HEAD_DIMS, _round_up_choice, _vector_ready
-from .sblocal_backward import BandWindows, _band_kernel_dims, _band_terms_hip
+from .sblocal_backward import BandWindows
 
 
 def _additive_mask(attn_mask, T, S, device):
@@ -81,22 +81,26 @@ def local_backward(query, key, value, local_context, softmax_temp, key_lengths, 
     (sblocal_backward.BandWindows); with
     P = softmax over the band, g = d out and delta_i = sum_s P_is g_i.v_s:
     d v_s = sum_i P_is g_i,  d(t q_i.k_s) = P_is (g_i.v_s - delta_i).  Queries without any visible
-    key get zero gradients.  bfloat16 and float16 GPU tensors with the forward's out and lse, no attn_mask and no
-    dropout: flyhip_local_bwd, on the matrix pipe of the input type (_local_backward_2byte).  Otherwise, given the
-    forward's out and lse (local_forward(..., return_lse=True)), GPU tensors
-    and head dims <= 64, the sums run in float32 on the backward band kernel of
-    Scatterbrain-local attention with its feature operands zero (flyhip_sblocal_bwd_band: P_is =
-    exp(t q_i.k_s - lse_i), delta_i = g_i.out_i); otherwise as batched library products on the GPU (host tensors are
+    key get zero gradients.  GPU tensors with the forward's out and lse (local_forward(..., return_lse=True)) run on
+    flyhip_local_bwd: 2-byte tensors without attn_mask and dropout on the matrix pipe of their type, head dims up to 64 of
+    float32 (and of 2-byte tensors with a mask or dropout, widened) from three bf16 pieces per operand
+    (P_is = exp(t q_i.k_s - lse_i), delta_i = g_i.out_i); otherwise as batched library products on the GPU (host tensors are
     accepted in float64 only: the check of these formulas against autograd).  dropout = (p, seed) of the forward:
     with M the kept / (1 - p) mask, d v_s = sum_i M_is P_is g_i and d(t q_i.k_s) = P_is (M_is g_i.v_s - delta_i),
-    delta_i = g_i.out_i as before; on the band kernel only.  attn_mask: the forward's additive matrix (the scores are
-    t (q.k + mask); a query with lse = -inf weighs its visible keys 1 / local_context each); on the band kernel only."""
+    delta_i = g_i.out_i as before; on the kernels only.  attn_mask: the forward's additive matrix (the scores are
+    t (q.k + mask); a query with lse = -inf weighs its visible keys 1 / local_context each); on the kernels only."""
     B, T, H, E = query.shape
     S, D = key.shape[1], value.shape[3]
     t = softmax_temp or 1 / math.sqrt(E)
-    if (query.dtype in (torch.bfloat16, torch.float16) and query.is_cuda and out is not None and lse is not None
-            and attn_mask is None and dropout[0] == 0 and max(E, D) <= _HEAD_DIMS[-1]):
-        return _local_backward_2byte(query, key, value, local_context, t, key_lengths, grad_out, out, lse)
+    on_kernels = query.is_cuda and out is not None and lse is not None and query.dtype != torch.float64
+    plain = attn_mask is None and dropout[0] == 0
+    if on_kernels and query.dtype in (torch.bfloat16, torch.float16) and plain and max(E, D) <= _HEAD_DIMS[-1]:
+        return _local_backward_kernels(query, key, value, local_context, t, key_lengths, grad_out, out, lse)
+    if on_kernels and max(E, D) <= 64:
+        # float32 (2-byte tensors with a mask or dropout are widened)
+        q, k, v, g, o = (x.float() for x in (query, key, value, grad_out, out))
+        grads = _local_backward_kernels(q, k, v, local_context, t, key_lengths, g, o, lse, dropout, attn_mask)
+        return tuple(x.to(query.dtype) for x in grads)
     wdt = torch.float64 if query.dtype == torch.float64 else torch.float32
 
     def bh(x):                                   # (B,L,H,C) -> (B*H, L, C)
@@ -109,20 +113,12 @@ def local_backward(query, key, value, local_context, softmax_temp, key_lengths, 
     if not Q.is_cuda and wdt != torch.float64:
         # host tensors are accepted for one purpose: checking the written-out gradient formulas in float64 against autograd
         raise NotImplementedError('local_backward runs on the GPU; host tensors only in float64 (the check of the formulas)')
-    dims = _band_kernel_dims(E, D, 0)
-    if out is not None and lse is not None and Q.is_cuda and wdt == torch.float32 and dims is not None:
-        zq, zk = Q.new_zeros(B * H, T, dims[1]), Q.new_zeros(B * H, S, dims[1])
-        delta = (G * bh(out)).sum(-1, keepdim=True)
-        lens_b = None if key_lengths is None else key_lengths.to(device=Q.device, dtype=torch.int64).contiguous()
-        dQ, _, dK, _, dV = _band_terms_hip(Q, K, V, G, zq, zk, lse.reshape(B * H, T, 1), delta, lens_b, H,
-                                           local_context, t, dims, dropout, _additive_mask(attn_mask, T, S, Q.device))
-        return back(dQ, query), back(dK, key), back(dV, value)
     if attn_mask is not None:
-        raise NotImplementedError('the gradients of local attention with an attn_mask run on the band kernel only: '
-                                  'float32 or bfloat16 GPU tensors, head dims <= 64, the forward\'s out and lse given')
+        raise NotImplementedError('the gradients of local attention with an attn_mask run on the kernels only: '
+                                  'float32 or 2-byte GPU tensors, head dims <= 64, the forward\'s out and lse given')
     if dropout[0] > 0:
-        raise NotImplementedError('the gradients of dropped local attention run on the band kernel only: float32 or '
-                                  'bfloat16 GPU tensors, head dims <= 64, the forward\'s out and lse given')
+        raise NotImplementedError('the gradients of dropped local attention run on the kernels only: float32 or '
+                                  '2-byte GPU tensors, head dims <= 64, the forward\'s out and lse given')
     lens = None
     if key_lengths is not None:
         lens = key_lengths.to(Q.device).repeat_interleave(H).view(B * H, 1, 1)
@@ -145,22 +141,24 @@ def local_backward(query, key, value, local_context, softmax_temp, key_lengths, 
     return back(dQ, query), back(dK, key), back(dV, value)
 
 
-def _local_backward_2byte(query, key, value, local_context, t, key_lengths, grad_out, out, lse):
-    """local_backward for bfloat16 / float16 GPU tensors on flyhip_local_bwd: the band softmax is formed again from the
-    forward's lse on the matrix pipe of the input type; delta_i = g_i . out_i is formed by the first launch."""
+def _local_backward_kernels(query, key, value, local_context, t, key_lengths, grad_out, out, lse, dropout=(0.0, 0), attn_mask=None):
+    """local_backward on flyhip_local_bwd_masked: the band softmax is formed again from the forward's lse; delta_i = g_i . out_i
+    is formed by the first launch."""
     B, T, H, E = query.shape
     S, D = key.shape[1], value.shape[3]
     dim = _round_up_choice(max(E, D), _HEAD_DIMS, 'head dimension')
+    unit = 16 // query.element_size()             # elements of a 16-byte load
 
     def prep(x):
         if x.shape[-1] != dim:
             x = F.pad(x, (0, dim - x.shape[-1]))      # zero columns change no dot product
-        ready = _vector_ready(x) and all(st % 8 == 0 for st in x.stride()[:-1])
+        ready = _vector_ready(x) and all(st % unit == 0 for st in x.stride()[:-1])
         return x if ready else x.contiguous()
     q, k, v, g, o = prep(query), prep(key), prep(value), prep(grad_out.to(query.dtype)), prep(out.to(query.dtype))
     delta = torch.empty(B, H, T, dtype=torch.float32, device=query.device)     # g . out per query, filled by the kernels
     lse_ = lse.reshape(B, H, T).float().contiguous()
     lens = None if key_lengths is None else key_lengths.to(device=query.device, dtype=torch.int64).contiguous()
+    add = _additive_mask(attn_mask, T, S, query.device)
     dq = torch.empty(B, T, H, dim, dtype=query.dtype, device=query.device)
     dk = torch.empty(B, S, H, dim, dtype=query.dtype, device=query.device)
     dv = torch.empty(B, S, H, dim, dtype=query.dtype, device=query.device)
@@ -168,10 +166,11 @@ def _local_backward_2byte(query, key, value, local_context, t, key_lengths, grad
     def strides(x):
         return x.stride(0), x.stride(2), x.stride(1)
     with torch.cuda.device(query.device):
-        _lib.call('flyhip_local_bwd', q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), g.data_ptr(),
-                  lse_.data_ptr(), _lib.ptr(lens), delta.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+        _lib.call('flyhip_local_bwd_masked', q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), g.data_ptr(),
+                  lse_.data_ptr(), _lib.ptr(lens), _lib.ptr(add), delta.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                   B, H, T, S, dim, local_context, *strides(q), *strides(k), *strides(v), *strides(o), *strides(g),
-                  *strides(dq), *strides(dk), *strides(dv), t, _lib.dtype_code(q), _lib.stream_ptr(query.device))
+                  *strides(dq), *strides(dk), *strides(dv), t, _lib.dtype_code(q), float(dropout[0]), int(dropout[1]),
+                  _lib.stream_ptr(query.device))
     return dq[..., :E], dk[..., :E], dv[..., :D]
 
 

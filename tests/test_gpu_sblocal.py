@@ -1038,3 +1038,27 @@ def test_bf16_gradients_through_chunk_sums(case, monkeypatch):
     monkeypatch.setattr(sbb, '_FAR_WORKSPACE_FLOATS', 1)
     for a, b in zip(got, torch.autograd.grad(out, (qg, kg, vg), w.to(dev))):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize('B,T,S,H,E,D,lc,lens', [
+    (1, 1, 1, 1, 64, 64, 1, None), (2, 33, 31, 1, 32, 32, 7, [31, 2]), (1, 64, 64, 2, 64, 64, 64, None), (1, 65, 97, 1, 64, 48, 33, None),
+    (2, 300, 500, 3, 64, 64, 98, [500, 211]), (1, 700, 200, 1, 24, 32, 150, None), (1, 513, 513, 2, 64, 64, 512, None)])
+def test_local_attention_float32_on_bf16_pieces(B, T, S, H, E, D, lc, lens):
+    """float32 LocalAttention forms every product from three bf16 pieces per operand (what is left out is 2^-24 of a
+    product): output and gradients against the oracle in float64, at edges of its 16-row blocks and 32-row tiles, as
+    close as float32 products are -- 2^-24 per term, accumulated over up to 512 keys and 64 dims in float32: 2e-6 (2-norm)."""
+    from fly_amd import LocalAttention, LengthMask
+    g = torch.Generator().manual_seed(T + S + E)
+    q, k, v, w = (torch.randn(B, L, H, C, generator=g) for L, C in ((T, E), (S, E), (S, D), (T, D)))
+    lengths = None if lens is None else torch.tensor(lens)
+    qd, kd, vd = (x.double().requires_grad_() for x in (q, k, v))
+    ref_out = osb.local_attention(qd, kd, vd, lc, key_lengths=lengths)
+    ref = torch.autograd.grad(ref_out, (qd, kd, vd), w.double())
+    dev = torch.device('cuda:0')
+    qg, kg, vg = (x.to(dev).requires_grad_() for x in (q, k, v))
+    mask = None if lengths is None else LengthMask(lengths.to(dev), max_len=S)
+    out, _ = LocalAttention(lc)(qg, kg, vg, key_padding_mask=mask)
+    got = torch.autograd.grad(out, (qg, kg, vg), w.to(dev))
+    for a, r in zip((out,) + got, (ref_out,) + ref):
+        scale = max(float(r.detach().norm()), 1e-2 * r.numel() ** 0.5)      # (d query is zero where every query sees one key)
+        assert float((a.detach().double().cpu() - r.detach()).norm()) <= 2e-6 * scale
