@@ -16,14 +16,16 @@
 // Nothing is subtracted from a sum over all keys that contains it many times over, so features in two bf16 pieces
 // (2^-17) and products of pieces with fp32 accumulation are exact to the rounding of the bfloat16 results.
 //
-//   far_chunk_kernel    KV_c and QG_c of every chunk, stabilised by the chunk's own largest log-feature
-//   far_scan_kernel     their inclusive prefix sums in common units, in place
+//   far_chunk_kernel    KV_c and QG_c summed over the chunks of a segment, every prefix of it kept, stabilised by the largest
+//                       log-feature so far
+//   far_scan_kernel     inclusive prefix sums over the segments in common units, in place of their last chunks' sums
 //   far_lowrank_kernel  query-major and key-major: far and edge terms, chain rule through the feature map -> float32
 //   local_bwd_b16_kernel<EXACT> (sblocal.hip)  the band, plus the low-rank part, rounded once
 //
 // Measured at B=1, H=16, L=16384, window 1024, 256 features, where the backward ran as library products over windows of
-// keys before (20.8 ms): chunks 166, scan 225, low-rank 392 (query-major) and 740 (key-major), band 188 and 272 us.  The
-// chunk sums (66 KB per 64 rows and side at 256 features: written, scanned, read twice) are what the first three move.
+// keys before (20.8 ms): chunks 185, scan 19, low-rank 316 (query-major) and 730 (key-major), band 204 and 295 us.  The
+// chunk sums (66 KB per 64 rows and side at 256 features) bound the first two: a scan over every chunk instead of every
+// segment moved 1.1 GB in 225 us.
 #include "common.h"
 #include "local.h"
 #include <algorithm>
@@ -36,9 +38,10 @@ struct FarArgs {
     const float* ln; const float* proj; const int64_t* lens;
     float* c;                                       // (BH, T): g . out
     float* kscale; float* qscale;                   // (BH, chunks): base-2 log of the units a chunk's sums are kept in
-    float* kv; float* qg;                           // (BH, chunks, M (E + 1)): sums of the chunk [M][E] | [M], then prefix sums
+    float* kv; float* qg;                           // (BH, chunks, M (E + 1)): prefix sums [M][E] | [M], see FarPrefix
     float* dq; float* dk; float* dv;                // low-rank part of the gradients, (BH, rows, E)
     int B, H, T, S, lc, mh_valid, n_kc, n_qc;
+    int seg;                                        // chunks whose sums one workgroup adds up
     long q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss;
     float temp;
     int n_xcd;
@@ -143,8 +146,11 @@ struct FarProj {
 // ---------------------------------------------------------------------------------------
 // sums of the chunks
 // ---------------------------------------------------------------------------------------
-// One chunk per workgroup, 16 projection rows (32 features, exp(+.) and exp(-.)) per wave.  The projection is formed with
-// the chunk's rows as result rows, which leaves a lane with one feature of 16 rows: the operand of F^T Y as it stands.
+// A segment of `seg` chunks per workgroup, 16 projection rows (32 features, exp(+.) and exp(-.)) per wave.  The projection
+// is formed with a chunk's rows as result rows, which leaves a lane with one feature of 16 rows: the operand of F^T Y as it
+// stands.  The sums stay in the accumulators from chunk to chunk and are written after each: the prefix sum inside the
+// segment, in units of the largest log-feature so far (a whole power of two, so that moving to a larger one is exact).
+// The scan then has the segments' last chunks to read and write instead of every one.
 template <int E, int M>
 __global__ __launch_bounds__(2 * M) void far_chunk_kernel(FarArgs a) {
     constexpr int NW = M / 32, NT = 64 * NW, MH = M / 2, KS = E / 32, EB = E / 16, LD = E + 8, PER = M * (E + 1);
@@ -153,8 +159,10 @@ __global__ __launch_bounds__(2 * M) void far_chunk_kernel(FarArgs a) {
     __shared__ float red[NW];
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
     const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
-    const bool queries = (int)blockIdx.x >= a.n_kc;
-    const int c = queries ? blockIdx.x - a.n_kc : blockIdx.x;
+    const int k_segs = (a.n_kc + a.seg - 1) / a.seg;
+    const bool queries = (int)blockIdx.x >= k_segs;
+    const int n_c = queries ? a.n_qc : a.n_kc;
+    const int c_lo = (queries ? blockIdx.x - k_segs : blockIdx.x) * a.seg, c_hi = min(c_lo + a.seg, n_c);
     const int len = queries ? a.T : (a.lens ? min((int)a.lens[b], a.S) : a.S);
     const uint16_t* xp = queries ? a.q + b * a.q_sb + h * a.q_sh : a.k + b * a.k_sb + h * a.k_sh;
     const uint16_t* yp = queries ? a.go + b * a.g_sb + h * a.g_sh : a.v + b * a.v_sb + h * a.v_sh;
@@ -163,102 +171,123 @@ __global__ __launch_bounds__(2 * M) void far_chunk_kernel(FarArgs a) {
     Tile16<FC, E, NT> o;
     FarArgs na = a;
     na.c = nullptr;                                 // (formed here)
-    t.fetch(na, queries, xp, xs, yp, ys, bh, c * FC, len, -0.5f * __log2f(2.0f * a.mh_valid), 0.f, tid);
-    if (queries) o.fetch(a.out + b * a.o_sb + h * a.o_sh, a.o_ss, c * FC, a.T - 1, tid);
+    const float base = -0.5f * __log2f(2.0f * a.mh_valid);
+    const uint16_t* op = a.out + b * a.o_sb + h * a.o_sh;
+    t.fetch(na, queries, xp, xs, yp, ys, bh, c_lo * FC, len, base, 0.f, tid);
+    if (queries) o.fetch(op, a.o_ss, c_lo * FC, a.T - 1, tid);
     FarProj<KS> P;
     P.load(a.proj, 16 * w + r16, E, sqrtf(a.temp) * FAR_LOG2E, g);
-    t.stash(a, Xs, Ys, diag, exts, cs, tid);
-    if (queries) {
-        // c = g . out, C8 lanes per row
-        constexpr int C8 = E / 8;
-        __syncthreads();                            // (cs was zeroed by stash)
-#pragma unroll
-        for (int j = 0; j < Tile16<FC, E, NT>::N; ++j) {
-            const int idx = tid + NT * j, row = idx / C8;
-            float d = 0.f;
-#pragma unroll
-            for (int n = 0; n < 4; ++n)
-                d += __uint_as_float(o.r[j][n] << 16) * __uint_as_float(t.y.r[j][n] << 16) +
-                     __uint_as_float(o.r[j][n] & 0xffff0000u) * __uint_as_float(t.y.r[j][n] & 0xffff0000u);
-#pragma unroll
-            for (int off = 1; off < C8; off <<= 1) d += __shfl_xor(d, off);
-            if (idx % C8 == 0 && idx < FC * C8) {
-                cs[row] = d;
-                if (c * FC + row < a.T) a.c[(long)bh * a.T + c * FC + row] = d;
-            }
-        }
-    }
-    __syncthreads();
-
     const bool fvalid = 16 * w + r16 < a.mh_valid;
-    floatx4 dd[4], bias[4];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-        dd[kb] = P.rows_by_features(Xs + (16 * kb + r16) * LD + 8 * g);
-        bias[kb] = *reinterpret_cast<const floatx4*>(exts + 16 * kb + 4 * g) - *reinterpret_cast<const floatx4*>(diag + 16 * kb + 4 * g);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, fvalid ? fabsf(dd[kb][i]) + bias[kb][i] : -INFINITY);
-    }
-    mx = wave_max(mx);
-    if (lane == 0) red[w] = mx;
-    __syncthreads();
-    float unit = red[0];
-#pragma unroll
-    for (int i = 1; i < NW; ++i) unit = fmaxf(unit, red[i]);
-    if (tid == 0) (queries ? a.qscale : a.kscale)[(long)bh * (queries ? a.n_qc : a.n_kc) + c] = unit;
-    const float shift = unit == -INFINITY ? 0.f : unit;
-
     floatx4 acc[2][EB];
-    float tot[2] = {0.f, 0.f};
+    float tot[2] = {0.f, 0.f}, unit = -INFINITY;
 #pragma unroll
     for (int sg = 0; sg < 2; ++sg)
 #pragma unroll
         for (int eb = 0; eb < EB; ++eb) acc[sg][eb] = Frag<float>::zero();
+#pragma unroll 1
+    for (int c = c_lo; c < c_hi; ++c) {
+        t.stash(a, Xs, Ys, diag, exts, cs, tid);
+        if (queries) {
+            // c = g . out, C8 lanes per row
+            constexpr int C8 = E / 8;
+            __syncthreads();                        // (cs was zeroed by stash)
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
-        uintx4 fh[2], fl[2];
+            for (int j = 0; j < Tile16<FC, E, NT>::N; ++j) {
+                const int idx = tid + NT * j, row = idx / C8;
+                float d = 0.f;
 #pragma unroll
-        for (int sg = 0; sg < 2; ++sg) {
-            floatx4 f[2];
+                for (int n = 0; n < 4; ++n)
+                    d += __uint_as_float(o.r[j][n] << 16) * __uint_as_float(t.y.r[j][n] << 16) +
+                         __uint_as_float(o.r[j][n] & 0xffff0000u) * __uint_as_float(t.y.r[j][n] & 0xffff0000u);
 #pragma unroll
-            for (int hb = 0; hb < 2; ++hb) {
-                const int kb = 2 * t2 + hb;
-                const floatx4 wr = *reinterpret_cast<const floatx4*>(cs + 16 * kb + 4 * g);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float x = __builtin_amdgcn_exp2f((sg ? -dd[kb][i] : dd[kb][i]) + bias[kb][i] - shift);
-                    f[hb][i] = fvalid ? x : 0.f;
-                    tot[sg] += queries ? f[hb][i] * wr[i] : f[hb][i];
+                for (int off = 1; off < C8; off <<= 1) d += __shfl_xor(d, off);
+                if (idx % C8 == 0 && idx < FC * C8) {
+                    cs[row] = d;
+                    if (c * FC + row < a.T) a.c[(long)bh * a.T + c * FC + row] = d;
                 }
             }
-            split2(f[0], f[1], fh[sg], fl[sg]);
         }
+        if (c + 1 < c_hi) {                         // (workgroup-uniform)
+            t.fetch(na, queries, xp, xs, yp, ys, bh, (c + 1) * FC, len, base, 0.f, tid);
+            if (queries) o.fetch(op, a.o_ss, (c + 1) * FC, a.T - 1, tid);
+        }
+        __syncthreads();
+
+        floatx4 dd[4];
+        float mx = -INFINITY;
+        auto bias_of = [&](int kb) __attribute__((always_inline)) {
+            return *reinterpret_cast<const floatx4*>(exts + 16 * kb + 4 * g) - *reinterpret_cast<const floatx4*>(diag + 16 * kb + 4 * g);
+        };
 #pragma unroll
-        for (int eb = 0; eb < EB; ++eb) {
-            const uint16_t* yq = Ys + (32 * t2 + 4 * g + (r16 >> 2)) * LD + 16 * eb + 4 * (r16 & 3);
-            const uintx4 yt = lds_read_tr8(reinterpret_cast<const char*>(yq), reinterpret_cast<const char*>(yq + 16 * LD));
+        for (int kb = 0; kb < 4; ++kb) {
+            dd[kb] = P.rows_by_features(Xs + (16 * kb + r16) * LD + 8 * g);
+            const floatx4 bias = bias_of(kb);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, fvalid ? fabsf(dd[kb][i]) + bias[i] : -INFINITY);
+        }
+        mx = wave_max(mx);
+        if (lane == 0) red[w] = mx;
+        __syncthreads();
+        const float before = unit;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) unit = fmaxf(unit, ceilf(red[i]));
+        if (tid == 0) (queries ? a.qscale : a.kscale)[(long)bh * n_c + c] = unit;
+        const float shift = unit == -INFINITY ? 0.f : unit;
+        if (unit > before && before != -INFINITY) { // (workgroup-uniform; sums in other units before)
+            const float f = __builtin_amdgcn_exp2f(before - unit);
 #pragma unroll
             for (int sg = 0; sg < 2; ++sg) {
-                acc[sg][eb] = mma_bf16(fl[sg], yt, acc[sg][eb]);
-                acc[sg][eb] = mma_bf16(fh[sg], yt, acc[sg][eb]);
+                tot[sg] *= f;
+#pragma unroll
+                for (int eb = 0; eb < EB; ++eb) acc[sg][eb] *= f;
             }
         }
-    }
-    float* dst = (queries ? a.qg + ((long)bh * a.n_qc + c) * PER : a.kv + ((long)bh * a.n_kc + c) * PER);
 #pragma unroll
-    for (int sg = 0; sg < 2; ++sg) {
+        for (int t2 = 0; t2 < 2; ++t2) {
+            uintx4 fh[2], fl[2];
 #pragma unroll
-        for (int eb = 0; eb < EB; ++eb)
+            for (int sg = 0; sg < 2; ++sg) {
+                floatx4 f[2];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) dst[(sg * MH + 16 * w + 4 * g + i) * E + 16 * eb + r16] = acc[sg][eb][i];
-        const float s = group_sum(tot[sg]);
-        if (g == 0) dst[M * E + sg * MH + 16 * w + r16] = s;
+                for (int hb = 0; hb < 2; ++hb) {
+                    const int kb = 2 * t2 + hb;
+                    const floatx4 wr = *reinterpret_cast<const floatx4*>(cs + 16 * kb + 4 * g);
+                    const floatx4 bias = bias_of(kb);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float x = __builtin_amdgcn_exp2f((sg ? -dd[kb][i] : dd[kb][i]) + bias[i] - shift);
+                        f[hb][i] = fvalid ? x : 0.f;
+                        tot[sg] += queries ? f[hb][i] * wr[i] : f[hb][i];
+                    }
+                }
+                split2(f[0], f[1], fh[sg], fl[sg]);
+            }
+#pragma unroll
+            for (int eb = 0; eb < EB; ++eb) {
+                const uint16_t* yq = Ys + (32 * t2 + 4 * g + (r16 >> 2)) * LD + 16 * eb + 4 * (r16 & 3);
+                const uintx4 yt = lds_read_tr8(reinterpret_cast<const char*>(yq), reinterpret_cast<const char*>(yq + 16 * LD));
+#pragma unroll
+                for (int sg = 0; sg < 2; ++sg) {
+                    acc[sg][eb] = mma_bf16(yt, fl[sg], acc[sg][eb]);     // (transposed: a lane's results are four columns of one feature)
+                    acc[sg][eb] = mma_bf16(yt, fh[sg], acc[sg][eb]);
+                }
+            }
+        }
+        float* dst = (queries ? a.qg : a.kv) + ((long)bh * n_c + c) * PER;
+        const uint32_t lane_at = (uint32_t)((16 * w + r16) * E + 4 * g);
+#pragma unroll
+        for (int sg = 0; sg < 2; ++sg) {
+#pragma unroll
+            for (int eb = 0; eb < EB; ++eb) *reinterpret_cast<floatx4*>(dst + sg * MH * E + lane_at + 16 * eb) = acc[sg][eb];
+            const float s = group_sum(tot[sg]);
+            if (g == 0) dst[M * E + sg * MH + 16 * w + r16] = s;
+        }
+        __syncthreads();                            // the tiles are free
     }
 }
 
-// inclusive prefix sums over the chunks of a (batch, head), in place, in the common units of the features (exp(kappa)
-// taken out of the keys and put into the queries); eight chunks of loads in flight per thread
+// inclusive prefix sums over the segments of a (batch, head), in place of the sums of their last chunks, in the common
+// units of the features (exp(kappa) taken out of the keys and put into the queries); eight loads in flight per thread
 constexpr int FAR_SCAN_NT = 256;
 __global__ __launch_bounds__(FAR_SCAN_NT) void far_scan_kernel(FarArgs a, int per4) {
     __shared__ float red[FAR_SCAN_NT / 64];
@@ -266,27 +295,55 @@ __global__ __launch_bounds__(FAR_SCAN_NT) void far_scan_kernel(FarArgs a, int pe
     const bool queries = blockIdx.y != 0;
     const float kappa = far_kappa<FAR_SCAN_NT>(a, bh, red, threadIdx.x);
     if (e >= per4) return;
-    const int n = queries ? a.n_qc : a.n_kc;
-    const float* unit = (queries ? a.qscale : a.kscale) + (long)bh * n;
+    const int n_c = queries ? a.n_qc : a.n_kc, n = (n_c + a.seg - 1) / a.seg;
+    const float* unit = (queries ? a.qscale : a.kscale) + (long)bh * n_c;
     const float ref = queries ? kappa : -kappa;
-    floatx4* p = reinterpret_cast<floatx4*>(queries ? a.qg : a.kv) + (long)bh * n * per4 + e;
+    floatx4* p = reinterpret_cast<floatx4*>(queries ? a.qg : a.kv) + (long)bh * n_c * per4 + e;
     floatx4 run = Frag<float>::zero();
-    int c = 0;
-    for (; c + 8 <= n; c += 8) {
+    for (int s0 = 0; s0 < n; s0 += 8) {
         floatx4 x[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = p[(long)(c + j) * per4];
+        int at[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            run += x[j] * __builtin_amdgcn_exp2f(unit[c + j] + ref);
-            p[(long)(c + j) * per4] = run;
+            at[j] = min((s0 + j + 1) * a.seg, n_c) - 1;     // (past the end: the last chunk, not used)
+            x[j] = p[(long)at[j] * per4];
         }
-    }
-    for (; c < n; ++c) {
-        run += p[(long)c * per4] * __builtin_amdgcn_exp2f(unit[c] + ref);
-        p[(long)c * per4] = run;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (s0 + j < n) {
+                run += x[j] * __builtin_amdgcn_exp2f(unit[at[j]] + ref);
+                p[(long)at[j] * per4] = run;
+            }
     }
 }
+
+// the sum over the chunks 0 .. c of a (batch, head) in common units, from what the two kernels above leave: at a
+// segment's last chunk as it stands, elsewhere the previous segment's end plus the prefix sum inside the segment
+struct FarPrefix {
+    const float* whole = nullptr; const float* part = nullptr;
+    float f = 0.f;
+    __device__ __forceinline__ FarPrefix(const float* sums, const float* unit, float ref, long per, int c, int n_c, int seg) {
+        if (c < 0) return;                          // (no chunk: 0)
+        const int s = c / seg;
+        if (c == min((s + 1) * seg, n_c) - 1) { whole = sums + c * per; return; }
+        if (s > 0) whole = sums + ((long)s * seg - 1) * per;
+        part = sums + c * per;
+        f = __builtin_amdgcn_exp2f(unit[c] + ref);
+    }
+    // x[j] += sign * (entry at `lane + step(j)`), all loads of a source in flight together (the branches are uniform)
+    template <typename V, int N, typename Step>
+    __device__ __forceinline__ void add(V (&x)[N], float sign, uint32_t lane, Step step) const {
+        if (whole) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) x[j] += *reinterpret_cast<const V*>(whole + lane + step(j)) * sign;
+        }
+        if (part) {
+            const float fs = sign * f;
+#pragma unroll
+            for (int j = 0; j < N; ++j) x[j] += *reinterpret_cast<const V*>(part + lane + step(j)) * fs;
+        }
+    }
+};
 
 // ---------------------------------------------------------------------------------------
 // far and edge terms of 64 outer rows
@@ -300,7 +357,7 @@ constexpr size_t far_lowrank_smem() {
 }
 
 template <int E, int M, bool KEYMAJOR>
-__global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(2, 2))) void far_lowrank_kernel(FarArgs a) {
+__global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR && M >= 128 ? 4 : 2, !KEYMAJOR && M >= 128 ? 8 : 2))) void far_lowrank_kernel(FarArgs a) {
     constexpr int NW = M / 32, NT = 64 * NW, MH = M / 2, KS = E / 32, EB = E / 16, LD = E + 8, PER = M * (E + 1);
     constexpr size_t TILES = (size_t)2 * FC * LD * 2, INNER = TILES + 2 * 8 * 64 * 16, RED = (size_t)NW * FC * 16 * 4;
     extern __shared__ __attribute__((aligned(128))) char far_smem[];
@@ -356,46 +413,52 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     __syncthreads();
 
     // own features: result rows = features 16 w + 4 g + i (sign sg), columns = outer rows 16 ob + r16
-    floatx4 fo[KEYMAJOR ? 1 : 2][4];
-    uintx4 foh[KEYMAJOR ? 4 : 1], fol[KEYMAJOR ? 4 : 1];                            // key-major: as two-piece operands, slots (sg, 4 g + i)
-#pragma unroll
-    for (int ob = 0; ob < 4; ++ob) {
+    auto own_features = [&](int ob, floatx4& f0, floatx4& f1) __attribute__((always_inline)) {
         const floatx4 dd = P.features_by_rows(Xo + (16 * ob + r16) * LD + 8 * g);
         const float bias = exto[16 * ob + r16] - diago[16 * ob + r16];
-        floatx4 f0, f1;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const bool ok = 16 * w + 4 * g + i < a.mh_valid;
             f0[i] = ok ? __builtin_amdgcn_exp2f(bias + dd[i]) : 0.f;
             f1[i] = ok ? __builtin_amdgcn_exp2f(bias - dd[i]) : 0.f;
         }
-        if (KEYMAJOR) split2(f0, f1, foh[KEYMAJOR ? ob : 0], fol[KEYMAJOR ? ob : 0]);
-        else { fo[0][ob] = f0; fo[KEYMAJOR ? 0 : 1][ob] = f1; }
+    };
+    // key-major: needed throughout, as two-piece operands, slots (sg, 4 g + i); query-major: formed where they are used
+    uintx4 foh[KEYMAJOR ? 4 : 1], fol[KEYMAJOR ? 4 : 1];
+    if (KEYMAJOR) {
+#pragma unroll
+        for (int ob = 0; ob < 4; ++ob) {
+            floatx4 f0, f1;
+            own_features(ob, f0, f1);
+            split2(f0, f1, foh[KEYMAJOR ? ob : 0], fol[KEYMAJOR ? ob : 0]);
+        }
     }
 
     // far terms from the prefix sums of the inner side: pre(c0) + (all - pre(c1))
     const float* pre = (KEYMAJOR ? a.qg : a.kv) + (long)bh * n_ic * PER;
-    const float* p0 = c0 > 0 ? pre + (long)(c0 - 1) * PER : nullptr;
-    const float* p1 = c1 < n_ic ? pre + (long)max(c1 - 1, 0) * PER : nullptr;       // (c1 = 0: nothing to take off)
-    const float* pn = c1 < n_ic ? pre + (long)(n_ic - 1) * PER : nullptr;
-    if (c1 == 0) p1 = nullptr;
-    auto far4 = [&](long at) __attribute__((always_inline)) {
-        floatx4 x = Frag<float>::zero();
-        if (pn) x = *reinterpret_cast<const floatx4*>(pn + at);
-        if (p1) x -= *reinterpret_cast<const floatx4*>(p1 + at);
-        if (p0) x += *reinterpret_cast<const floatx4*>(p0 + at);
-        return x;
+    const float* units = (KEYMAJOR ? a.qscale : a.kscale) + (long)bh * n_ic;
+    const float ref = KEYMAJOR ? kappa : -kappa;
+    const FarPrefix p0(pre, units, ref, PER, c0 - 1, n_ic, a.seg);
+    const FarPrefix p1(pre, units, ref, PER, c1 < n_ic ? c1 - 1 : -1, n_ic, a.seg);
+    const FarPrefix pn(pre, units, ref, PER, c1 < n_ic ? n_ic - 1 : -1, n_ic, a.seg);
+    auto far = [&](auto& x, uint32_t lane_at, auto step) __attribute__((always_inline)) {
+        pn.add(x, 1.f, lane_at, step);
+        p1.add(x, -1.f, lane_at, step);
+        p0.add(x, 1.f, lane_at, step);
     };
     floatx4 acc2[2][4];                                                             // [sign][outer block], rows = features
 #pragma unroll
     for (int sg = 0; sg < 2; ++sg) {
 #pragma unroll
         for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] = Frag<float>::zero();
+        floatx4 x[2 * KS];
+#pragma unroll
+        for (int j = 0; j < 2 * KS; ++j) x[j] = Frag<float>::zero();
+        far(x, (uint32_t)((sg * MH + 16 * w + r16) * E + 8 * g), [](int j) { return 32 * (j >> 1) + 4 * (j & 1); });
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            const long at = (long)(sg * MH + 16 * w + r16) * E + 32 * ks + 8 * g;
             uintx4 fh, fl;
-            split2(far4(at), far4(at + 4), fh, fl);
+            split2(x[2 * ks], x[2 * ks + 1], fh, fl);
 #pragma unroll
             for (int ob = 0; ob < 4; ++ob) {
                 const uintx4 yo = *reinterpret_cast<const uintx4*>(Yo + (16 * ob + r16) * LD + 32 * ks + 8 * g);
@@ -403,28 +466,21 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(2, 2))) v
                 acc2[sg][ob] = mma_bf16(fh, yo, acc2[sg][ob]);
             }
         }
-        const floatx4 vec = far4((long)M * E + sg * MH + 16 * w + 4 * g);
+        floatx4 vec[1] = {Frag<float>::zero()};
+        far(vec, (uint32_t)(M * E + sg * MH + 16 * w + 4 * g), [](int) { return 0; });
 #pragma unroll
-        for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] -= vec * (KEYMAJOR ? 1.0f : co[16 * ob + r16]);
+        for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] -= vec[0] * (KEYMAJOR ? 1.0f : co[16 * ob + r16]);
     }
     floatx4 acc3[KEYMAJOR ? EB : 1][KEYMAJOR ? 4 : 1];                              // d v: rows = value dims, columns = keys
     if (KEYMAJOR) {
 #pragma unroll
         for (int eb = 0; eb < EB; ++eb) {
-            floatx4 x[2];
+            float x[8];
 #pragma unroll
-            for (int sg = 0; sg < 2; ++sg)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const long at = (long)(sg * MH + 16 * w + 4 * g + i) * E + 16 * eb + r16;
-                    float s = 0.f;
-                    if (pn) s = pn[at];
-                    if (p1) s -= p1[at];
-                    if (p0) s += p0[at];
-                    x[sg][i] = s;
-                }
+            for (int j = 0; j < 8; ++j) x[j] = 0.f;
+            far(x, (uint32_t)((16 * w + 4 * g) * E + 16 * eb + r16), [](int j) { return ((j >> 2) * MH + (j & 3)) * E; });
             uintx4 th, tl;
-            split2(x[0], x[1], th, tl);
+            split2(floatx4{x[0], x[1], x[2], x[3]}, floatx4{x[4], x[5], x[6], x[7]}, th, tl);
 #pragma unroll
             for (int ob = 0; ob < 4; ++ob) {
                 floatx4 d = Frag<float>::zero();
@@ -569,7 +625,7 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(2, 2))) v
                 f0[i] = (i & 1) ? __uint_as_float(h0 & 0xffff0000u) + __uint_as_float(l0 & 0xffff0000u) : __uint_as_float(h0 << 16) + __uint_as_float(l0 << 16);
                 f1[i] = (i & 1) ? __uint_as_float(h1 & 0xffff0000u) + __uint_as_float(l1 & 0xffff0000u) : __uint_as_float(h1 << 16) + __uint_as_float(l1 << 16);
             }
-        } else { f0 = fo[0][ob]; f1 = fo[KEYMAJOR ? 0 : 1][ob]; }
+        } else own_features(ob, f0, f1);
         const floatx4 up = f0 * acc2[0][ob], un = f1 * acc2[1][ob];
         float s = 0.f;
 #pragma unroll
@@ -648,7 +704,8 @@ static int launch_lowrank(const FarArgs& a, hipStream_t st) {
 template <int E, int M>
 static int launch_far(const FarArgs& a, const LocalBwdArgs& band, hipStream_t st) {
     const int BH = a.B * a.H, per4 = M * (E + 1) / 4;
-    hipLaunchKernelGGL((far_chunk_kernel<E, M>), dim3(a.n_kc + a.n_qc, BH), dim3(2 * M), 0, st, a);
+    const int k_segs = (a.n_kc + a.seg - 1) / a.seg, q_segs = (a.n_qc + a.seg - 1) / a.seg;
+    hipLaunchKernelGGL((far_chunk_kernel<E, M>), dim3(k_segs + q_segs, BH), dim3(2 * M), 0, st, a);
     if (int rc = check_launch("far_chunk_kernel")) return rc;
     hipLaunchKernelGGL(far_scan_kernel, dim3((per4 + FAR_SCAN_NT - 1) / FAR_SCAN_NT, 2, BH), dim3(FAR_SCAN_NT), 0, st, a, per4);
     if (int rc = check_launch("far_scan_kernel")) return rc;
@@ -662,6 +719,16 @@ static void far_pieces(int64_t BH, int64_t T, int64_t S, int64_t E, int64_t M, i
     const int64_t kc = (S + FC - 1) / FC, qc = (T + FC - 1) / FC, per = M * (E + 1);
     const int64_t want[8] = {BH * T, BH * kc, BH * qc, BH * kc * per, BH * qc * per, BH * T * E, BH * S * E, BH * S * E};
     for (int i = 0; i < 8; ++i) n[i] = (want[i] + 63) / 64 * 64;
+}
+
+// chunks per segment: as many as leave 16 waves per compute unit (the chunk kernel holds 8), at most 16: the scan takes 227 us
+// at one chunk per segment (16 heads of 16384 tokens, 256 features: it moves 1.1 GB), 54 us at 4, 30 at 8, 19 at 16, the
+// chunk kernel the same at each
+constexpr int FAR_MAX_SEG = 16;
+static int far_segment(long BH, int n_kc, int n_qc, int M, int cus) {
+    int seg = FAR_MAX_SEG;
+    while (seg > 1 && BH * ((n_kc + seg - 1) / seg + (n_qc + seg - 1) / seg) * (M / 32) < 16L * cus) seg /= 2;
+    return seg;
 }
 
 }  // namespace flyhip
@@ -711,7 +778,7 @@ extern "C" int flyhip_sblocal_bwd_far(const void* q, const void* k, const void* 
               reinterpret_cast<const uint16_t*>(grad_out), reinterpret_cast<const uint16_t*>(out), log_norm, proj, key_lengths,
               p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7],
               B, H, T, S, local_context, mh_valid, (S + FC - 1) / FC, (T + FC - 1) / FC,
-              q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss, softmax_temp, machine().xcds};
+              far_segment(B * H, (S + FC - 1) / FC, (T + FC - 1) / FC, M, machine().cus), q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss, softmax_temp, machine().xcds};
     LocalBwdArgs band{q, k, v, grad_out, out, log_norm, p[0], key_lengths, dq, dk, dv, B, H, T, S, local_context,
                       q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, g_sb, g_sh, g_ss, o_sb, o_sh, o_ss,
                       dq_sb, dq_sh, dq_ss, dk_sb, dk_sh, dk_ss, dv_sb, dv_sh, dv_ss, softmax_temp, 0, p[5], p[6], p[7]};

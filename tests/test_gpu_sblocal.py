@@ -1009,6 +1009,8 @@ def test_attention_dropout_module_and_refusals():
     dict(B=1, T=65, S=129, H=1, E=32, mh=16, lc=1, lens=None, scale=0.4),              # one key a query
     dict(B=1, T=1000, S=1000, H=2, E=64, mh=100, lc=333, lens=[1000], scale=0.35),     # projection rows that are padding
     dict(B=3, T=90, S=1000, H=1, E=64, mh=3, lc=40, lens=[1000, 1, 500], scale=0.4),
+    dict(B=16, T=323, S=270, H=8, E=64, mh=128, lc=90, lens=[270, 1, 65, 140] * 4, scale=0.35, slices=False),   # segments of 4 chunks, 2 left over
+    dict(B=20, T=200, S=330, H=8, E=64, mh=100, lc=64, lens=None, scale=1.0, slices=False),                     # rescaled inside a segment
 ], ids=lambda c: f"T{c['T']}-S{c['S']}-E{c['E']}-mh{c['mh']}-lc{c['lc']}")
 def test_bf16_gradients_through_chunk_sums(case, monkeypatch):
     """flyhip_sblocal_bwd_far (far pairs through prefix sums over chunks, edge chunks pair by pair, the band on the local
@@ -1035,6 +1037,8 @@ def test_bf16_gradients_through_chunk_sums(case, monkeypatch):
     for a, r in zip(got, ref):
         err = float((a.double().cpu() - r).norm() / r.norm())
         assert a.dtype == torch.bfloat16 and err <= 6e-3, err
+    if not case.get('slices', True):             # (slices of a large problem are summed in shorter segments: other roundings)
+        return
     monkeypatch.setattr(sbb, '_FAR_WORKSPACE_FLOATS', 1)
     for a, b in zip(got, torch.autograd.grad(out, (qg, kg, vg), w.to(dev))):
         assert torch.equal(a, b)
