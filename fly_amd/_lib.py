@@ -45,6 +45,7 @@ SIGNATURES = {
     'flyhip_bs_sdd_dsoftmax': [c_vp] * 8 + [c_int] * 6 + [c_i64] * 6 + [c_float, c_int, c_vp],
     'flyhip_bs_sdd_kmajor': [c_vp] * 8 + [c_int] * 8 + [c_i64] * 6 + [c_int, c_vp],
     'flyhip_bs_dsd': [c_vp] * 9 + [c_int] * 6 + [c_i64] * 9 + [c_int, c_vp],
+    'flyhip_bs_dds_bias': [c_vp] * 9 + [c_int] * 8 + [c_i64] * 9 + [c_int, c_vp],
     'flyhip_bs_dds': [c_vp] * 8 + [c_int] * 8 + [c_i64] * 9 + [c_int, c_vp],
     'flyhip_bs_attn_lse': [c_vp] * 8 + [c_int, c_vp, c_i64] + [c_int] * 5 + [c_i64] * 12 + [c_float, c_int, c_vp],
     'flyhip_bs_attn_masks': [c_vp] * 8 + [c_int, c_vp, c_i64, c_vp, c_i64] + [c_int] * 5 + [c_i64] * 12 + [c_float, c_int, c_vp],

@@ -9,7 +9,7 @@ import torch.nn.functional as F
 from torch.nn import init
 
 from .blocksparse_attention import instantiate
-from .blocksparse_matmul import matmul
+from .blocksparse_matmul import KMAJOR_MIN_K, matmul
 from .blocksparse_utils import densify_tensor
 
 
@@ -132,11 +132,13 @@ class BlockSparseLinear(nn.Module):
             op = None
             if self.backend == 'triton':
                 op = matmul(self.layout.cpu(), self.block_size, 'dds', trans_a=False, trans_b=True)
+                op.ragged_rows = True
             self.ops_cache[self.backend] = op
             return op
 
     def forward(self, x):
         """x (..., in_features) -> (..., out_features)."""
+        bias = self.bias
         if self.backend == 'dense':
             pad_in = self.in_features_extended - x.shape[-1]
             dense = densify_tensor(self.weight.view(1, self.nnz_blocks, self.block_size, self.block_size),
@@ -148,14 +150,27 @@ class BlockSparseLinear(nn.Module):
             lead = x.shape[:-1]
             tokens = x.reshape(-1, x.shape[-1])
             n_tok = tokens.shape[0]
-            # one zero-padding for both axes: features up to the padded fan-in, tokens up to whole blocks
+            # one zero-padding for both axes: features up to the padded fan-in; tokens up to whole blocks only where the
+            # weight gradient's kernel asks for them (the products and the split-K gradient take any number of tokens: for
+            # one image of 196 tokens the copies cost 8 of 29 us)
             pad_in = max(self.in_features_extended - tokens.shape[1], 0)
             pad_tok = -n_tok % self.block_size
+            if not (torch.is_grad_enabled() and self.weight.requires_grad) or (
+                    self.block_size == 32 and n_tok >= KMAJOR_MIN_K
+                    and (torch.is_autocast_enabled() or x.dtype in (torch.bfloat16, torch.float16))):
+                pad_tok = 0
             if pad_in or pad_tok:
                 tokens = F.pad(tokens, (0, pad_in, 0, pad_tok))
             # (views only, and slices only where something is cut off: under autograd a select or a slice of the
             #  result, also one that keeps everything, costs a zero-fill and a copy of the whole tensor on the way back)
-            y = self.get_ops()(tokens.view(1, 1, *tokens.shape), self.weight)
+            op = self.get_ops()
+            tokens = tokens.view(1, 1, *tokens.shape)
+            if bias is not None and self.out_features == self.out_features_extended:
+                # (in the dtype of the product: under autocast half precision)
+                y = op(tokens, self.weight, bias.to(torch.float16 if torch.is_autocast_enabled() else tokens.dtype))
+                bias = None
+            else:
+                y = op(tokens, self.weight)
             y = y.view(y.shape[2], y.shape[3])
             if pad_tok:
                 y = y[:n_tok]
@@ -163,4 +178,4 @@ class BlockSparseLinear(nn.Module):
         if y.shape[-1] != self.out_features:
             y = y[..., :self.out_features]
         # the bias joins in the dtype of the product (under autocast the product is half precision)
-        return y if self.bias is None else y + self.bias.to(y.dtype)
+        return y if bias is None else y + bias.to(y.dtype)

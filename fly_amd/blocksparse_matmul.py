@@ -32,9 +32,11 @@ class _MatmulFn(torch.autograd.Function):
     permuted roles exactly as blocksparse_matmul.py:562-587 does."""
 
     @staticmethod
-    def forward(ctx, a, b, op):
+    def forward(ctx, a, b, op, bias=None):
         ctx.save_for_backward(a, b)
         ctx.op = op
+        if bias is not None:                         # ('dds' only)
+            return op._dds(a, b, op.trans_a, op.trans_b, False, bias)
         return op._run(op.mode, a, b, op.trans_a, op.trans_b, False)
 
     @staticmethod
@@ -49,7 +51,8 @@ class _MatmulFn(torch.autograd.Function):
         if ctx.needs_input_grad[1]:
             mode_db = mode[2] + mode[1] + mode[0]
             db = op._run(mode_db, a, dc, not op.trans_a, False, op.trans_b)
-        return da, db, None
+        dbias = dc.flatten(0, 2).sum(0) if ctx.needs_input_grad[3] else None
+        return da, db, None, dbias
 
 
 class matmul:
@@ -70,6 +73,9 @@ class matmul:
         assert layout.ndim in (2, 3), "Layout should be a 2 or 3 dimensional tensor of 0s and 1s"
         self.block, self.mode, self.trans_a, self.trans_b = block, mode, trans_a, trans_b
         self.lut_cache = dict()
+        # 'dds': the gradient of the sparse operand may contract over any number of rows its kernel takes (the linear layer
+        # sets it; a caller's own product keeps the multiple-of-16 rule)
+        self.ragged_rows = False
         self.layout = _as_heads(layout)            # (H, block-rows, block-cols), integral; 2-D means one head
         self.spdims = self.layout.shape
         if mode != 'sdd':
@@ -109,10 +115,16 @@ class matmul:
         return self._table('rows' if by_rows else 'cols', device)
 
     # ------------------------------------------------------------------ call
-    def __call__(self, a, b):
+    def __call__(self, a, b, bias=None):
+        """bias: mode 'dds' with one head only, a vector of N values of the product's dtype added to every row (in
+        float32, before the product is rounded)."""
         original_dims = max(a.ndim, b.ndim)
         a, b = self._validate_inputs(a, b)
-        c = _MatmulFn.apply(a, b, self)
+        if bias is not None:
+            n = self.spdims[-2 if self.trans_b else -1] * self.block
+            if self.mode != 'dds' or self.spdims[0] != 1 or tuple(bias.shape) != (n,) or bias.dtype != a.dtype or bias.device != a.device:
+                raise ValueError(f"bias needs mode 'dds' with one head and a vector of {n} values of {a.dtype}")
+        c = _MatmulFn.apply(a, b, self, bias)
         for _ in range(c.ndim - original_dims):
             c = c.squeeze(0)
         return c
@@ -157,7 +169,10 @@ class matmul:
         if K != Kb:
             raise ValueError(f"Size of tensor A along the {_dim_to_name(a_dim)} dim ({K}) must match size "
                              f"of tensor B along the {_dim_to_name(b_dim)} dim ({Kb})")
-        if K % 16 != 0:
+        kmajor = (trans_a and not trans_b and self.block == 32 and a.dtype in (torch.bfloat16, torch.float16)
+                  and K >= KMAJOR_MIN_K and a.stride(3) == 1 and b.stride(3) == 1
+                  and all(s % 8 == 0 for s in a.stride()[:3] + b.stride()[:3]))
+        if K % 16 != 0 and not (kmajor and self.ragged_rows):
             raise ValueError('Reduction size for SDD must be a multiple of 16')
         H, p, r = self.spdims
         Z = a.shape[0]
@@ -168,9 +183,7 @@ class matmul:
                              f'{tuple(self.spdims)} with block {self.block}')
         if int(self.layout.sum()) == 0:              # a layout without blocks: nothing to compute or launch
             return torch.empty((Z, 0, self.block, self.block), dtype=a.dtype, device=a.device)
-        if (trans_a and not trans_b and self.block == 32 and a.dtype in (torch.bfloat16, torch.float16)
-                and K >= KMAJOR_MIN_K and a.stride(3) == 1 and b.stride(3) == 1
-                and all(s % 8 == 0 for s in a.stride()[:3] + b.stride()[:3])):
+        if kmajor:
             return self._sdd_kmajor(a, b, Z, K)
         (lut,) = self._table('sdd', a.device)
         row_ptr, row_blk, row_col = self._table('rows', a.device)
@@ -228,13 +241,16 @@ class matmul:
                       _lib.dtype_code(b), _lib.stream_ptr(b.device))
         return c
 
-    def _dds(self, a, b, trans_a, trans_b, trans_c):
+    def _dds(self, a, b, trans_a, trans_b, trans_c, bias=None):
         if trans_a and trans_c and not trans_b:
             # (a^T b)^T = b^T a: the same numbers as a dsd with the sparse operand transposed, which has
             # a tiled kernel (this is the gradient of the second operand of an sdd, e.g. dK = dS^T Q)
             return self._dsd(b, a, True, False, False)
         a = _dense_operand(a)
         b = b.contiguous()
+        if bias is not None:
+            bias = bias.contiguous()
+            bias = bias if bias.data_ptr() % 16 == 0 else bias.clone()
         H, p, r = self.spdims
         by_rows = trans_b
         seg_ptr, seg_blk, seg_inner = self._table('rows' if by_rows else 'cols', a.device)
@@ -247,7 +263,7 @@ class matmul:
         c = torch.empty((Z, H, N, M) if trans_c else (Z, H, M, N), dtype=a.dtype, device=a.device)
         c_sm, c_sn = (c.stride(3), c.stride(2)) if trans_c else (c.stride(2), c.stride(3))
         with torch.cuda.device(a.device):
-            _lib.call('flyhip_bs_dds', a.data_ptr(), b.data_ptr(), c.data_ptr(),
+            _lib.call('flyhip_bs_dds_bias', a.data_ptr(), b.data_ptr(), _lib.ptr(bias), c.data_ptr(),
                       seg_ptr.data_ptr(), seg_blk.data_ptr(), seg_inner.data_ptr(),
                       grp_row0.data_ptr(), grp_n.data_ptr(), grp_row0.shape[0],
                       int(self.layout.sum(-1 if by_rows else -2).max()),

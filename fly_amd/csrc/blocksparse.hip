@@ -622,6 +622,7 @@ struct DxdArgs {
     long c_sz, c_sh, c_sm, c_sn;
     int Z;
     int n_xcd;          // dies the dispatcher deals workgroup ids to (set where the kernel is launched)
+    const void* bias;   // DDS, optional: one value per output column
 };
 
 template <typename T, int BLK>
@@ -963,6 +964,11 @@ __global__ __launch_bounds__(256) void bs_dds_kernel(DxdArgs a) {
 #pragma unroll
         for (int tn = 0; tn < NTL; ++tn) {
             const long n = (long)bcol * BLK + subn * TILE + 16 * tn + 4 * g;
+            if (a.bias) {
+                const T* bp = reinterpret_cast<const T*>(a.bias) + (long)head * a.per_head * BLK + n;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[tm][tn][i] += Elem<T>::to_f32(bp[i]);
+            }
             store_tile_row<T>(cp + m * a.c_sm + n * a.c_sn, a.c_sn, acc[tm][tn], 4);
         }
     }
@@ -984,6 +990,7 @@ struct DdsGroupArgs {
     long sp_sz, dn_sz, dn_sh, dn_sm, c_sz, c_sh, c_sm;
     int n_xcd;          // dies the dispatcher deals workgroup ids to (set where the kernel is launched)
     int n_grp;          // groups (the weight-stationary kernel deals (token stream, group) pairs itself)
+    const void* bias;   // optional: one value per output column, added before the result is rounded
 };
 constexpr int DDS_MAX_STEPS = 128;   // longest reduction list the tiled kernel accepts
 #ifndef FLY_DDS_STATIONARY
@@ -995,6 +1002,15 @@ constexpr int DDS_MAX_STEPS = 128;   // longest reduction list the tiled kernel 
 #ifndef FLY_DDS_DIST
 #define FLY_DDS_DIST 2               // steps the loads of the 128-token kernel run ahead of its MFMAs
 #endif
+
+// eight consecutive values of an optional bias vector, added to b0 | b1
+template <typename T>
+__device__ __forceinline__ void bias8(const void* bias, long at, floatx4& b0, floatx4& b1) {
+    if (bias == nullptr) return;                            // (uniform)
+    const T* p = reinterpret_cast<const T*>(bias) + at;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { b0[i] += Elem<T>::to_f32(p[i]); b1[i] += Elem<T>::to_f32(p[4 + i]); }
+}
 
 template <typename T, bool WT, int DIST = FLY_DDS_DIST>     // WT: blocks are [k][n] (y = x W) and are transposed on their way into LDS
 __global__ __launch_bounds__(256) void bs_dds32_kernel(DdsGroupArgs a) {
@@ -1125,8 +1141,12 @@ __global__ __launch_bounds__(256) void bs_dds32_kernel(DdsGroupArgs a) {
 #pragma unroll
             for (int o2 = 0; o2 < 2; ++o2) {
                 const int ob = 2 * wn + o2;
-                if (m < a.M && ob < gn)
-                    store8_f32(cp + m * a.c_sm + (long)(bcol0 + ob) * 32 + 8 * g, acc[tm][2 * o2], acc[tm][2 * o2 + 1]);
+                if (m < a.M && ob < gn) {
+                    const long n = (long)(bcol0 + ob) * 32 + 8 * g;
+                    floatx4 b0 = Frag<float>::zero(), b1 = Frag<float>::zero();
+                    bias8<T>(a.bias, head * (long)a.per_head * 32 + n, b0, b1);
+                    store8_f32(cp + m * a.c_sm + n, acc[tm][2 * o2] + b0, acc[tm][2 * o2 + 1] + b1);
+                }
             }
 #pragma unroll
             for (int tn = 0; tn < 4; ++tn) acc[tm][tn] = Frag<float>::zero();
@@ -1180,6 +1200,95 @@ __global__ __launch_bounds__(256) void bs_dds32_kernel(DdsGroupArgs a) {
             drain_loads_but<8 * (DIST - 1)>();              // the set parked next iteration has arrived
             __syncthreads();
         }
+    }
+}
+
+// DDS for few tokens, 32 x 32 blocks of a 2-byte type.  The grouped kernel above gives a workgroup 128 tokens and up to
+// four block-rows: one image of 196 tokens through the narrowing layer of a channel MLP (24 block-rows of 36 blocks) left 16
+// workgroups that walk the whole list, 20.2 us; 7.6 us here.  Here a workgroup owns 32 tokens of ONE block-row and its eight waves share the reduction list
+// (wave w: entries w, w + 8, ...), operands straight from memory in MFMA order, the loads of four entries in flight; the
+// partial sums meet in LDS.  What bounds it is the latency of two dependent loads and the reduction.
+template <typename T, bool WT>
+__global__ __launch_bounds__(512) void bs_dds32w_kernel(DdsGroupArgs a) {
+    constexpr int NW = 8, AHEAD = 4;
+    __shared__ __attribute__((aligned(16))) floatx4 red[NW][4][64];             // [wave][token half, output half][lane]
+    __shared__ __attribute__((aligned(16))) uint16_t wt[WT ? NW : 1][WT ? AHEAD : 1][WT ? 32 * 32 : 8];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    const int seg = blockIdx.x, z = blockIdx.z, head = seg / a.per_head, bcol = seg % a.per_head;
+    const long m0 = (long)blockIdx.y * 32;
+    const int p0 = a.seg_ptr[seg], nin = a.seg_ptr[seg + 1] - p0;
+    const uint16_t* spz = reinterpret_cast<const uint16_t*>(a.sp) + z * a.sp_sz;
+    const uint16_t* xp = reinterpret_cast<const uint16_t*>(a.dn) + z * a.dn_sz + head * a.dn_sh;
+    const uint16_t* xrow[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) xrow[i] = xp + min(m0 + 16 * i + r16, (long)a.M - 1) * a.dn_sm;         // clamped: masked at the store
+    // products are formed transposed, weight rows dealt so that result row 4 g + i of half j is output 8 g + 4 j + i: a
+    // lane ends up with eight consecutive outputs of one token
+    floatx4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) { acc[i][0] = Frag<float>::zero(); acc[i][1] = Frag<float>::zero(); }
+    const int mine = (nin - w + NW - 1) / NW;                                  // (w < NW: >= 0)
+    for (int t0 = 0; t0 < mine; t0 += 64) {
+        const int at = p0 + min(w + NW * (t0 + lane), nin - 1);                // this wave's next 64 entries, one a lane
+        const int l_in = a.seg_inner[at], l_blk = a.seg_blk[at];
+        const int nt = min(mine - t0, 64);
+        for (int t = 0; t < nt; t += AHEAD) {
+            uintx4 fx[AHEAD][2], fw[AHEAD][2];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {                                  // (past the end: the last entry again, not used)
+                const int tu = min(t + u, nt - 1);
+                const long in0 = (long)__builtin_amdgcn_readlane(l_in, tu) * 32;
+                const uint16_t* blk = spz + (long)__builtin_amdgcn_readlane(l_blk, tu) * 1024;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if (!WT) {
+                        fx[u][i] = *reinterpret_cast<const uintx4*>(xrow[i] + in0 + 8 * g);
+                        fw[u][i] = *reinterpret_cast<const uintx4*>(blk + (8 * (r16 >> 2) + 4 * i + (r16 & 3)) * 32 + 8 * g);
+                    } else {                                                   // contraction slots {4 g + i, 16 + 4 g + i}
+                        const uint2 lo = *reinterpret_cast<const uint2*>(xrow[i] + in0 + 4 * g), hi = *reinterpret_cast<const uint2*>(xrow[i] + in0 + 16 + 4 * g);
+                        fx[u][i] = uintx4{lo.x, lo.y, hi.x, hi.y};
+                        fw[u][i] = *reinterpret_cast<const uintx4*>(blk + 8 * lane + 512 * i);
+                    }
+                }
+            }
+            if (WT) {                                                          // [k][n] blocks: transposed by LDS reads of the wave's own copy
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) *reinterpret_cast<uintx4*>(&wt[WT ? w : 0][WT ? u : 0][WT ? 8 * lane + 512 * i : 0]) = fw[u][i];
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // (read back by other lanes of the wave only)
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const uint16_t* q = &wt[WT ? w : 0][WT ? u : 0][WT ? (4 * g + (r16 >> 2)) * 32 + 8 * (r16 & 3) + 4 * j : 0];
+                        fw[u][j] = lds_read_tr8(reinterpret_cast<const char*>(q), reinterpret_cast<const char*>(q + (WT ? 16 * 32 : 0)));
+                    }
+            }
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u)
+                if (t + u < nt) {                                              // (wave-uniform)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) acc[i][j] = mma32<T>(fw[u][j], fx[u][i], acc[i][j]);
+                }
+            if (WT) { asm volatile("" ::: "memory"); __builtin_amdgcn_wave_barrier(); }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) red[w][2 * i + j][lane] = acc[i][j];
+    __syncthreads();
+    if (w < 2) {                                                               // wave i finishes token half i
+        floatx4 s0 = Frag<float>::zero(), s1 = Frag<float>::zero();
+        bias8<T>(a.bias, (long)seg * 32 + 8 * g, s0, s1);
+#pragma unroll
+        for (int v = 0; v < NW; ++v) { s0 += red[v][2 * w][lane]; s1 += red[v][2 * w + 1][lane]; }
+        const long m = m0 + 16 * w + r16;
+        if (m < a.M) store8_f32(reinterpret_cast<T*>(a.c) + z * a.c_sz + head * a.c_sh + m * a.c_sm + (long)bcol * 32 + 8 * g, s0, s1);
     }
 }
 
@@ -1240,12 +1349,19 @@ __global__ __launch_bounds__(256) void bs_dds32s_kernel(DdsGroupArgs a, int n_st
     }
     __syncthreads();
 
-    floatx4 acc[4][8];
-#pragma unroll
-    for (int tm = 0; tm < 4; ++tm)
-#pragma unroll
-        for (int n = 0; n < 8; ++n) acc[tm][n] = Frag<float>::zero();
     const bool col_live = 8 * r16 < 32 * gn;                // this lane's eight outputs exist in the group
+    floatx4 bias_lo = Frag<float>::zero(), bias_hi = Frag<float>::zero();       // what the sums start from
+    if (col_live) bias8<T>(a.bias, ((long)head * a.per_head + bcol0) * 32 + 8 * r16, bias_lo, bias_hi);
+    floatx4 acc[4][8];
+    auto reset = [&](int tm) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            const float x = n < 4 ? bias_lo[n & 3] : bias_hi[n & 3];
+            acc[tm][n] = floatx4{x, x, x, x};
+        }
+    };
+#pragma unroll
+    for (int tm = 0; tm < 4; ++tm) reset(tm);
     // lane holds y[m = 64 w + 16 tm + 4 g + i][n0 + 8 r16 .. + 7]: one 16-byte store per (tm, i), 256 bytes per row and
     // instruction
     auto store_tile = [&](int tile) __attribute__((always_inline)) {
@@ -1262,8 +1378,7 @@ __global__ __launch_bounds__(256) void bs_dds32s_kernel(DdsGroupArgs a, int n_st
                     store8_f32(base + m * a.c_sm, lo, hi);
                 }
             }
-#pragma unroll
-            for (int n = 0; n < 8; ++n) acc[tm][n] = Frag<float>::zero();
+            reset(tm);
         }
     };
     if (nin == 0) {                                         // no input block: zero rows
@@ -1378,12 +1493,19 @@ __global__ __launch_bounds__(512) void bs_dds32d_kernel(DdsGroupArgs a, int n_st
     }
     __syncthreads();
 
+    const bool col_live = 8 * r16 < 32 * gn;                // this lane's eight outputs exist in the group
+    floatx4 bias_lo = Frag<float>::zero(), bias_hi = Frag<float>::zero();       // what the sums start from
+    if (col_live) bias8<T>(a.bias, ((long)head * a.per_head + bcol0) * 32 + 8 * r16, bias_lo, bias_hi);
     floatx4 acc[4][8];
+    auto reset = [&](int tm) __attribute__((always_inline)) {
 #pragma unroll
-    for (int tm = 0; tm < 4; ++tm)
+        for (int n = 0; n < 8; ++n) {
+            const float x = n < 4 ? bias_lo[n & 3] : bias_hi[n & 3];
+            acc[tm][n] = floatx4{x, x, x, x};
+        }
+    };
 #pragma unroll
-        for (int n = 0; n < 8; ++n) acc[tm][n] = Frag<float>::zero();
-    const bool col_live = 8 * r16 < 32 * gn;
+    for (int tm = 0; tm < 4; ++tm) reset(tm);
     auto store_tile = [&](int tile) __attribute__((always_inline)) {
         const long m0 = ((long)ty + (long)tile * gy) * 512 + 64 * w + 4 * g;
         T* base = cp + (long)bcol0 * 32 + 8 * r16;
@@ -1398,8 +1520,7 @@ __global__ __launch_bounds__(512) void bs_dds32d_kernel(DdsGroupArgs a, int n_st
                     store8_f32(base + m * a.c_sm, lo, hi);
                 }
             }
-#pragma unroll
-            for (int n = 0; n < 8; ++n) acc[tm][n] = Frag<float>::zero();
+            reset(tm);
         }
     };
     if (nin == 0) {                                         // no input block: zero rows
@@ -1518,13 +1639,20 @@ __global__ __launch_bounds__(512) void bs_dds32c_kernel(DdsGroupArgs a, int n_st
     __syncthreads();
 
     floatx4 acc[4][8];
-#pragma unroll
-    for (int tm = 0; tm < 4; ++tm)
-#pragma unroll
-        for (int n = 0; n < 8; ++n) acc[tm][n] = Frag<float>::zero();
     // The group's 32 gn outputs are dealt to NT = 2 gn tiles of 16: tile n holds outputs NT r + n (r = 0..15), so no MFMA
     // column is padding whatever the group's size, and a lane ends up with NT consecutive outputs of four tokens.
     const int NT = 2 * gn;
+    // what the sums start from (WT: zero -- eight registers more would spill, and gradients have no bias)
+    float bias[8];
+#pragma unroll
+    for (int n = 0; n < 8; ++n)
+        bias[n] = !WT && a.bias && n < NT ? Elem<T>::to_f32(reinterpret_cast<const T*>(a.bias)[((long)head * a.per_head + bcol0) * 32 + NT * r16 + n]) : 0.f;
+    auto reset = [&](int tm) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < 8; ++n) acc[tm][n] = floatx4{bias[n], bias[n], bias[n], bias[n]};
+    };
+#pragma unroll
+    for (int tm = 0; tm < 4; ++tm) reset(tm);
     auto store_tile = [&](int tile) __attribute__((always_inline)) {
         const long m0 = ((long)ty + (long)tile * gy) * 512 + 64 * w + 4 * g;
         T* base = cp + (long)bcol0 * 32 + NT * r16;
@@ -1543,8 +1671,7 @@ __global__ __launch_bounds__(512) void bs_dds32c_kernel(DdsGroupArgs a, int n_st
                     else __builtin_nontemporal_store(p0_, dst);
                 }
             }
-#pragma unroll
-            for (int n = 0; n < 8; ++n) acc[tm][n] = Frag<float>::zero();
+            reset(tm);
         }
     };
     if (nin == 0) {                                         // no input block: zero rows
@@ -2963,7 +3090,7 @@ extern "C" int flyhip_bs_dsd(const void* a_sp, const void* b, void* c,
     return check_launch("bs_dsd_kernel");
 }
 
-extern "C" int flyhip_bs_dds(const void* a, const void* b_sp, void* c,
+extern "C" int flyhip_bs_dds_bias(const void* a, const void* b_sp, const void* bias, void* c,
                              const int32_t* seg_ptr, const int32_t* seg_blk, const int32_t* seg_inner,
                              const int32_t* grp_row0, const int32_t* grp_n, int n_grp, int max_seg_len,
                              int n_seg, int cols_per_head, int Z, int M, int blk, int trans_b,
@@ -2989,6 +3116,22 @@ extern "C" int flyhip_bs_dds(const void* a, const void* b_sp, void* c,
         const Machine& mach = machine();
         ga.n_xcd = mach.xcds;
         ga.n_grp = n_grp;
+        ga.bias = bias;
+        // few tokens: 32 tokens of one block-row per workgroup while those are at most two per compute unit.  Measured (us,
+        // this / the 128-token tiles): 24 block-rows of 36 blocks, 196 tokens (168 workgroups) 7.6 / 20.2; 24 of 9 blocks,
+        // 300 tokens (240) 7.1 / 11.2; transposed, 32 of 48, 400 tokens (416) 20 / 30; past the line 96 of 9 blocks, 196 tokens
+        // (672) 12.3 / 11.7; transposed, 32 of 48, 784 tokens (800) 37 / 31
+        if ((long)n_seg * ((M + 31) / 32) * Z <= 2L * mach.cus) {
+            dim3 grid((unsigned)n_seg, (unsigned)((M + 31) / 32), Z);
+            if (dtype == BF16) {
+                if (trans_b) hipLaunchKernelGGL((bs_dds32w_kernel<bf16_t, false>), grid, dim3(512), 0, st, ga);
+                else hipLaunchKernelGGL((bs_dds32w_kernel<bf16_t, true>), grid, dim3(512), 0, st, ga);
+            } else {
+                if (trans_b) hipLaunchKernelGGL((bs_dds32w_kernel<f16_t, false>), grid, dim3(512), 0, st, ga);
+                else hipLaunchKernelGGL((bs_dds32w_kernel<f16_t, true>), grid, dim3(512), 0, st, ga);
+            }
+            return check_launch("bs_dds32w_kernel");
+        }
         // groups whose weights fit the LDS (four output blocks times the longest reduction list) and enough tokens to
         // amortise bringing them in: the weight-stationary kernel, two workgroups per compute unit
         if (FLY_DDS_STATIONARY == 2 && max_seg_len > 0 && max_seg_len <= DDS_STAT_STEPS && (long)M >= 512L * 8) {
@@ -3016,8 +3159,9 @@ extern "C" int flyhip_bs_dds(const void* a, const void* b_sp, void* c,
 #undef DDS_DMA
             return check_launch("bs_dds32d_kernel");
         }
-        if (FLY_DDS_STATIONARY == 2 && max_seg_len > DDS_STAT_STEPS && max_seg_len <= DDS_MAX_STEPS && (long)M >= 512L * 8) {
-            // longer lists: the same workgroup shape with the weights passing through LDS in chunks
+        if (FLY_DDS_STATIONARY == 2 && max_seg_len > DDS_STAT_STEPS && max_seg_len <= DDS_MAX_STEPS && (long)M >= 512L * 8 &&
+            (trans_b || !bias)) {
+            // longer lists: the same workgroup shape with the weights passing through LDS in chunks ([k][n] blocks: no bias)
             const long tiles = (M + 511) / 512;
             long n_streams = 1, best = -1;
             for (long n = 1; n <= tiles && n * n_grp * Z <= 4L * mach.cus + (long)n_grp * Z; ++n) {
@@ -3083,12 +3227,25 @@ extern "C" int flyhip_bs_dds(const void* a, const void* b_sp, void* c,
     }
     DxdArgs args{b_sp, a, c, seg_ptr, seg_blk, seg_inner, n_seg, cols_per_head, M, trans_b,
                  b_sz, a_sz, a_sh, a_sm, a_sk, c_sz, c_sh, c_sm, c_sn};
+    args.bias = bias;
     const int tile = blk >= 32 ? 32 : 16;
     const long nblocks = waves_to_blocks((long)((M + 31) / 32) * n_seg * (blk / tile));
     FLY_REQUIRE(nblocks <= 2147483647L, "bs_dds: too many blocks");
     dim3 grid((unsigned)nblocks, Z);
     BS_DISPATCH(bs_dds_kernel, grid, args)
     return check_launch("bs_dds_kernel");
+}
+
+extern "C" int flyhip_bs_dds(const void* a, const void* b_sp, void* c,
+                             const int32_t* seg_ptr, const int32_t* seg_blk, const int32_t* seg_inner,
+                             const int32_t* grp_row0, const int32_t* grp_n, int n_grp, int max_seg_len,
+                             int n_seg, int cols_per_head, int Z, int M, int blk, int trans_b,
+                             int64_t a_sz, int64_t a_sh, int64_t a_sm, int64_t a_sk,
+                             int64_t b_sz,
+                             int64_t c_sz, int64_t c_sh, int64_t c_sm, int64_t c_sn,
+                             int dtype, void* stream) {
+    return flyhip_bs_dds_bias(a, b_sp, nullptr, c, seg_ptr, seg_blk, seg_inner, grp_row0, grp_n, n_grp, max_seg_len, n_seg,
+                              cols_per_head, Z, M, blk, trans_b, a_sz, a_sh, a_sm, a_sk, b_sz, c_sz, c_sh, c_sm, c_sn, dtype, stream);
 }
 
 template <typename T>

@@ -552,6 +552,17 @@ int flyhip_bs_dds(const void* a, const void* b_sp, void* c,
                   int64_t c_sz, int64_t c_sh, int64_t c_sm, int64_t c_sn,
                   int dtype, void* stream);
 
+/* flyhip_bs_dds with `bias` (or NULL) added to every row: n_seg * blk values of the operands' type, one per output column,
+ * head by head (16-byte aligned); added to the float32 sum before the result is rounded. */
+int flyhip_bs_dds_bias(const void* a, const void* b_sp, const void* bias, void* c,
+                       const int32_t* seg_ptr, const int32_t* seg_blk, const int32_t* seg_inner,
+                       const int32_t* grp_row0, const int32_t* grp_n, int n_grp, int max_seg_len,
+                       int n_seg, int cols_per_head, int Z, int M, int blk, int trans_b,
+                       int64_t a_sz, int64_t a_sh, int64_t a_sm, int64_t a_sk,
+                       int64_t b_sz,
+                       int64_t c_sz, int64_t c_sh, int64_t c_sm, int64_t c_sn,
+                       int dtype, void* stream);
+
 /* Fused block-sparse attention: out = softmax(scale * q k^T + key mask) v over the nonzero blocks of
  * the layout, in one pass -- the SDD -> block softmax -> DSD sequence of BlockSparseAttention.forward
  * (ref: src/models/attention/blocksparse_attention.py:134-160) without the (Z, nnz, blk, blk) score

@@ -1284,3 +1284,40 @@ def test_sbblocksparse_long_lists_in_parts():
     plain = tuple(x.to(DEV) for x in tile_mask_table(layout, 32))
     out1, ln1 = sbblocksparse_forward(q.to(DEV), k.to(DEV), v.to(DEV), P.to(DEV), plain)
     assert rel_err(out, out1) <= 1e-5 and rel_err(ln, ln1) <= 1e-5
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('n_in,n_out,tokens', [(96, 64, 1), (64, 96, 33), (320, 160, 31), (1024, 256, 196), (256, 1024, 511),
+                                               (256, 1024, 520), (1024, 256, 4099), (256, 1024, 4100)])
+def test_linear_layer_any_token_count(n_in, n_out, tokens, dtype):
+    """Products of a block-sparse linear layer with its bias, and its gradients, at token counts that fill no tile: the kernel
+    that splits the reduction list over waves, the tiled one and the weight-stationary ones, on [n][k] blocks (forward) and [k][n]
+    ones (gradient), with an empty block-row, against float64 products of the same values.  Bar (2-norm): one rounding of each
+    result (2^-9 bfloat16, 2^-12 float16, relative) and of the bias gradient's partial sums."""
+    from fly_amd import BlockSparseLinear
+    g = torch.Generator().manual_seed(n_in + tokens)
+
+    class Random:
+        block = 32
+
+        def make_layout(self, rows, cols):
+            layout = (torch.rand(rows // 32, cols // 32, generator=g) < 0.6).long()
+            layout[0] = 1
+            layout[-1] = 0 if rows > 64 else 1
+            return layout
+    lin = BlockSparseLinear(n_in, n_out, Random()).to(DEV).to(dtype)
+    x = torch.randn(tokens, n_in, generator=g).to(dtype)
+    w = torch.randn(tokens, n_out, generator=g).to(dtype)
+    xg = x.to(DEV).requires_grad_()
+    y = lin(xg)
+    got = (y,) + torch.autograd.grad(y, (xg, lin.weight, lin.bias), w.to(DEV))
+    with torch.no_grad():
+        short = lin(xg)              # (no padded tokens: possibly another kernel)
+    xd, wd, bd = x.double().requires_grad_(), lin.weight.detach().double().cpu().requires_grad_(), lin.bias.detach().double().cpu().requires_grad_()
+    brow, bcol = lin.layout.cpu().nonzero(as_tuple=True)
+    dense = torch.zeros(n_out // 32, n_in // 32, 32, 32, dtype=torch.float64).index_put((brow, bcol), wd[0])
+    ref = xd @ dense.permute(0, 2, 1, 3).reshape(n_out, n_in).t() + bd
+    want = (ref,) + torch.autograd.grad(ref, (xd, wd, bd), w.double())
+    bar = 3e-3 if dtype == torch.bfloat16 else 4e-4
+    for a, r in zip(got + (short,), want + (ref,)):
+        assert a.dtype == dtype and float((a.detach().double().cpu() - r.detach()).norm()) <= bar * float(r.detach().norm())
