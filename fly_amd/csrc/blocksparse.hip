@@ -1957,15 +1957,15 @@ __global__ __launch_bounds__(64 * NW) void bs_attn32_kernel(const AttnArgs a) {
                 for (int ks = 0; ks < KS; ++ks) sc[kt][qt] = mma32<T>(fk[kt][ks], fq[qt][ks], sc[kt][qt]);
             }
     };
-    // DROP: the probabilities that go to the product with V, the dropped ones zeroed (the denominator sums all of them)
-    auto dropped = [&](float (&e0)[4], float (&e1)[4], uint32_t row_hash, int inner) __attribute__((always_inline)) {
-        const uint32_t col0 = (uint32_t)inner * 32u + 4u * g;
+    // DROP: the probabilities that go to the product with V, the dropped ones zeroed (the denominator sums all of them).  A
+    // packed pair is a pair of columns with one hash: three 16-bit vector instructions instead of a compare, a select and a
+    // second rounding per element
+    auto dropped = [&](uintx4 p, uint32_t row_hash, int inner) __attribute__((always_inline)) {
+        const uint32_t pair0 = (uint32_t)inner * 16u + 2u * g;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (!drop_keep(row_hash, col0 + i, a.drop_thresh)) e0[i] = 0.f;
-            if (!drop_keep(row_hash, col0 + 16u + i, a.drop_thresh)) e1[i] = 0.f;
-        }
-        return uintx4{pack2<T>(e0[0], e0[1]), pack2<T>(e0[2], e0[3]), pack2<T>(e1[0], e1[1]), pack2<T>(e1[2], e1[3])};
+        for (int i = 0; i < 4; ++i)                       // columns 4 g + 2 (i & 1) + 16 (i >> 1)
+            p[i] = drop_packed(p[i], drop_mix(row_hash + (pair0 + (i & 1) + 8u * (i >> 1)) * 0x632BE5ABu), a.drop_thresh);
+        return p;
     };
     // online softmax of sc and O^T += V^T P with the V tile that follows the K tile at `tile`; `inner` = its block-column
     auto soft_pv = [&](const char* tile, int inner) __attribute__((always_inline)) {
@@ -2002,7 +2002,7 @@ __global__ __launch_bounds__(64 * NW) void bs_attn32_kernel(const AttnArgs a) {
                     e1[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s1[i], scale2, nm));
                 }
                 pb[qt] = uintx4{pack2<T>(e0[0], e0[1]), pack2<T>(e0[2], e0[3]), pack2<T>(e1[0], e1[1]), pack2<T>(e1[2], e1[3])};
-                if (DROP) pd[qt] = dropped(e0, e1, drop_row[qt], inner);
+                if (DROP) pd[qt] = dropped(pb[qt], drop_row[qt], inner);
             }
         } else {
             floatx4 mk[2] = {Frag<float>::zero(), Frag<float>::zero()};
@@ -2034,7 +2034,7 @@ __global__ __launch_bounds__(64 * NW) void bs_attn32_kernel(const AttnArgs a) {
                     e1[i] = __builtin_amdgcn_exp2f(t1[i] - mref);
                 }
                 pb[qt] = uintx4{pack2<T>(e0[0], e0[1]), pack2<T>(e0[2], e0[3]), pack2<T>(e1[0], e1[1]), pack2<T>(e1[2], e1[3])};
-                if (DROP) pd[qt] = dropped(e0, e1, drop_row[qt], inner);
+                if (DROP) pd[qt] = dropped(pb[qt], drop_row[qt], inner);
             }
         }
         // the row sums come from the matrix pipe as well: a row of ones times the rounded probabilities
@@ -2864,17 +2864,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
 #pragma unroll
             for (int qq = 0; qq < 2; ++qq)
 #pragma unroll
-                for (int hb = 0; hb < 2; ++hb)
+                for (int hb = 0; hb < 2; ++hb) {
+                    uint32_t r01 = 0u, r23 = 0u;         // key-major: 16 bits a query, see drop_halves_of_column
+                    if (KEYMAJOR && DROP)
+                        drop_halves_of_column(__float_as_uint((r16 & 1) ? hh4[hb][2] : hh4[hb][0]), __float_as_uint((r16 & 1) ? hh4[hb][3] : hh4[hb][1]),
+                                              (uint32_t)bo_c * 32u + 16u * qq + r16, r01, r23);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float lrow = KEYMAJOR ? ln4[hb][i] : l_own[qq], drow = KEYMAJOR ? dl4[hb][i] : d_own[qq];
                         const float pr = __builtin_amdgcn_exp2f(fmaf(s1[qq][hb][i], sc, -lrow));   // (a row without scores: lse2 = +inf)
                         if (DROP) {
                             // (query, key) of the element: the inner row 8 g + 4 hb + i of the tile, the outer row 16 qq + r16
-                            const uint32_t inner_row = (uint32_t)inner_cur * 32u + 8u * g + 4u * hb + i;
-                            const uint32_t outer_row = (uint32_t)bo_c * 32u + 16u * qq + r16;
-                            const uint32_t rhash = KEYMAJOR ? __float_as_uint(hh4[hb][i]) : h_own[qq];
-                            const float m = drop_keep(rhash, KEYMAJOR ? outer_row : inner_row, a.drop_thresh) ? a.drop_scale : 0.f;
+                            bool keep;
+                            if (KEYMAJOR) {
+                                const uint32_t pair = i < 2 ? r01 : r23;
+                                keep = ((i & 1) ? pair >> 16 : pair & 0xffffu) >= a.drop_thresh;
+                            } else {
+                                keep = drop_keep(h_own[qq], (uint32_t)inner_cur * 32u + 8u * g + 4u * hb + i, a.drop_thresh);
+                            }
+                            const float m = keep ? a.drop_scale : 0.f;
                             s1[qq][hb][i] = m * pr;
                             gp[qq][hb][i] = pr * (m * gp[qq][hb][i] - drow);
                         } else {
@@ -2882,6 +2890,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
                             gp[qq][hb][i] = pr * (gp[qq][hb][i] - drow);
                         }
                     }
+                }
             uintx4 pb[KEYMAJOR ? 2 : 1], sb[2];
 #pragma unroll
             for (int qq = 0; qq < 2; ++qq) {

@@ -330,6 +330,30 @@ __device__ __forceinline__ bool drop_keep(uint32_t row_hash, uint32_t col, uint3
     const uint32_t h = drop_mix(row_hash + (col >> 1) * 0x632BE5ABu);
     return ((col & 1u) ? (h >> 16) : (h & 0xffffu)) >= thresh;
 }
+// The same decisions where a lane's four elements share a column and differ in their rows: lanes 2 c and 2 c + 1 of a quad
+// hold columns of one pair and need the two halves of the same four hashes, so each forms two of them (the even lane rows
+// 0 and 1, the odd lane rows 2 and 3; mine0 / mine1 = their row hashes) and hands over the halves the other needs.  Returns the
+// 16 bits of rows 0 | 1 and 2 | 3, to be compared with the threshold.
+__device__ __forceinline__ void drop_halves_of_column(uint32_t mine0, uint32_t mine1, uint32_t col, uint32_t& r01, uint32_t& r23) {
+    const bool odd = (col & 1u) != 0u;
+    const uint32_t add = (col >> 1) * 0x632BE5ABu;
+    const uint32_t h0 = drop_mix(mine0 + add), h1 = drop_mix(mine1 + add);
+    const uint32_t low = 0x05040100u, high = 0x07060302u;               // v_perm selectors: both low halves, both high halves
+    const uint32_t keep = __builtin_amdgcn_perm(h1, h0, odd ? high : low);
+    const uint32_t give = __builtin_amdgcn_perm(h1, h0, odd ? low : high);
+    const uint32_t got = (uint32_t)__builtin_amdgcn_mov_dpp((int)give, 0xB1, 0xf, 0xf, true);   // quad_perm(1, 0, 3, 2)
+    r01 = odd ? got : keep;
+    r23 = odd ? keep : got;
+}
+// 16-bit halves of `packed` where the half of `hash` at the same place is below thresh (>= 1): set to zero.  packed times
+// min(hash - (thresh - 1) saturated at 0, 1); written out because the compiler makes compares and selects of it.
+__device__ __forceinline__ uint32_t drop_packed(uint32_t packed, uint32_t hash, uint32_t thresh) {
+    const uint32_t below = (thresh - 1u) * 0x10001u, one = 0x10001u;
+    uint32_t kept;
+    asm("v_pk_sub_u16 %0, %1, %2 clamp\n\tv_pk_min_u16 %0, %0, %3\n\tv_pk_mul_lo_u16 %0, %0, %4"
+        : "=&v"(kept) : "v"(hash), "v"(below), "v"(one), "v"(packed));
+    return kept;
+}
 // host side: the kernels' dropout arguments from a probability and a 64-bit seed (p = 0: thresh = 0 = off)
 struct DropArgs { uint32_t seed, thresh; float scale; };
 inline DropArgs drop_args(float p, uint64_t seed) {
