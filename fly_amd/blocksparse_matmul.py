@@ -207,15 +207,12 @@ class matmul:
         grp_row0, grp_n = self._table('grp_rows', a.device)
         nnz = int(self.layout.sum())
         max_row_nnz = int(self.layout.sum(-1).max())
-        tiles = grp_row0.shape[0] * ((max_row_nnz + 3) // 4) * Z
-        slices = max(1, min(K // 256, -(-2048 // tiles)))       # about eight workgroups per CU
-        k_slice = -(-(-(-K // slices)) // 32) * 32
         c32 = torch.zeros((Z, nnz, 32, 32), dtype=torch.float32, device=a.device)
         with torch.cuda.device(a.device):
             _lib.call('flyhip_bs_sdd_kmajor', a.data_ptr(), b.data_ptr(), c32.data_ptr(),
                       row_ptr.data_ptr(), row_blk.data_ptr(), row_col.data_ptr(),
                       grp_row0.data_ptr(), grp_n.data_ptr(), grp_row0.shape[0], max_row_nnz,
-                      p, nnz, Z, K, k_slice, 32, a.stride(0), a.stride(1), a.stride(2),
+                      p, nnz, Z, K, 0, 32, a.stride(0), a.stride(1), a.stride(2),
                       b.stride(0), b.stride(1), b.stride(2), _lib.dtype_code(a), _lib.stream_ptr(a.device))
         return c32.to(a.dtype)
 

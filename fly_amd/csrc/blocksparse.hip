@@ -479,120 +479,127 @@ __global__ __launch_bounds__(256) void bs_sdd32u_kernel(const SddUniArgs a) {
 // ---------------------------------------------------------------------------------------
 // SDD with the contraction index slowest in both operands: sparse = A^T B, A (K x M), B (K x N)
 // ---------------------------------------------------------------------------------------
-// The weight gradient of a block-sparse linear layer: K = tokens (tens of thousands), M / N = output /
-// input features, 32x32 blocks of a 2-byte type.  One workgroup per (group of <= 4 consecutive
-// block-rows with identical column lists, chunk of <= 4 of their block-columns, slice of K): a
-// 128 x 128 output tile, the 2 x 2 waves owning 64 x 64 each.  Per step of 32 tokens the 32 x 128
-// tiles of A and B are loaded with 16-byte pieces along the features and kept row-major in LDS; the
-// MFMA fragments, whose contraction index runs down the rows, are two transposing 8-byte LDS reads
-// each (ds_read_b64_tr_b16), so nothing is transposed with 2-byte stores; the
-// slices' partial blocks meet in an fp32 buffer through hardware float atomics (the caller zeroes
-// it and rounds it to the output type afterwards).
+// The weight gradient of a block-sparse linear layer: K = tokens (tens of thousands), M / N = output / input features, 32x32
+// blocks of a 2-byte type.  One workgroup of eight waves per (group of <= 4 consecutive block-rows with identical column
+// lists, chunk of <= 2 NP of their block-columns, slice of K): a 128 x 64 NP output tile, wave (wm, wn) owning 64 rows and
+// every fourth 16-column tile.  What bounds it is the operands' way into LDS: a 128 x 128 tile per workgroup reads the
+// output gradient once for every four columns of a list (262 us for the widening layer of a channel MLP at 50176 tokens: 9
+// columns in chunks of 4, 4 and 1), so a chunk takes up to ten.  Per step of 32 tokens the tiles go from memory straight
+// into LDS, three steps ahead in four stages; the MFMA fragments, whose contraction index runs down the rows, are two
+// transposing 8-byte LDS reads each.  A holds [token][128 features], B [pair of list entries][token][64 features] (both
+// entries of a pair in one 128-byte line where they are neighbours), 32-byte pieces XOR-swizzled by the token so that the
+// eight rows a half-wave reads together cover all banks.  Measured (us, before / now, with the zero fill and the rounding):
+// 768 -> 3072 features 269 / 185, 3072 -> 768 234 / 220, 1024 -> 4096 345 / 285, 768 -> 768 127 / 74 at 50176 tokens; 106 / 58, 104 / 59, 141 / 69,
+// 46 / 43 at 8192; 32 / 34, 43 / 36, 36 / 34, 43 / 33 at 512.  The slices' partial blocks meet in an fp32 buffer through hardware
+// float atomics (the caller zeroes it and rounds it to the output type afterwards).
 struct SddKArgs {
     const void* a; const void* b; float* c32;
     const int32_t* seg_ptr; const int32_t* seg_blk; const int32_t* seg_inner;
     const int32_t* grp_row0; const int32_t* grp_n;
     int per_head, K, k_slice, chunks, nnz;
     long a_sz, a_sh, a_sk, b_sz, b_sh, b_sk;
+    int n_grp, slices, n_xcd;
 };
-constexpr int SDDK_LD = 144;    // LDS row stride in elements ([token][128 features + 16]: the four token rows a
-                                // 16-lane group reads together start 32 bytes apart modulo 256)
+constexpr int SDDK_STAGES = 4, SDDK_MAX_PAIRS = 5;
+constexpr int sddk_stage_bytes(int np) { return 8192 + 4096 * np; }
 
-template <typename T>
-__global__ __launch_bounds__(256) void bs_sdd32k_kernel(const SddKArgs a) {
-    constexpr int LD = SDDK_LD;
-    __shared__ __attribute__((aligned(16))) uint16_t at[2][32 * LD];
-    __shared__ __attribute__((aligned(16))) uint16_t bt[2][32 * LD];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, g = lane >> 4;
-    const int wm = w >> 1, wn = w & 1;
-    const int grp = blockIdx.x / a.chunks, chunk = blockIdx.x % a.chunks, z = blockIdx.z;
+template <typename T, int NP>
+__global__ __launch_bounds__(512) void bs_sdd32k_kernel(const SddKArgs a) {
+    constexpr int NI = (8 + 4 * NP + 7) / 8;                // transfers of 1 KB a wave and step
+    constexpr int STAGE = sddk_stage_bytes(NP);
+    extern __shared__ __attribute__((aligned(128))) char sddk_smem[];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    const int wm = w & 1, wn = w >> 1, z = blockIdx.z;
+    // (slice, group, chunk) dealt to the dies in contiguous runs: the groups that read one slice of the inputs share an L2
+    const int n_items = a.n_grp * a.chunks * a.slices, per_xcd = (n_items + a.n_xcd - 1) / a.n_xcd;
+    const int item = (blockIdx.x % a.n_xcd) * per_xcd + blockIdx.x / a.n_xcd;
+    if (blockIdx.x / a.n_xcd >= per_xcd || item >= n_items) return;             // workgroup-uniform
+    const int chunk = item % a.chunks, grp = item / a.chunks % a.n_grp, slice = item / (a.chunks * a.n_grp);
     const int row0 = a.grp_row0[grp], gn = a.grp_n[grp];
     const int head = row0 / a.per_head, brow0 = row0 % a.per_head;
     const int p0 = a.seg_ptr[row0], nin = a.seg_ptr[row0 + 1] - p0;
-    const int j0 = chunk * 4, jn = min(4, nin - j0);       // this chunk's block-columns: list entries j0 .. j0 + jn - 1
-    if (jn <= 0) return;                                    // workgroup-uniform
-    const int k0 = blockIdx.y * a.k_slice, k1 = min(a.K, k0 + a.k_slice);
-    if (k0 >= k1) return;
-    const uint16_t* ap = reinterpret_cast<const uint16_t*>(a.a) + z * a.a_sz + head * a.a_sh + (long)brow0 * 32;
-    const uint16_t* bp = reinterpret_cast<const uint16_t*>(a.b) + z * a.b_sz + head * a.b_sh;
+    const int j0 = chunk * 2 * NP, jn = min(2 * NP, nin - j0);                  // this chunk's list entries j0 .. j0 + jn - 1
+    const int k0 = slice * a.k_slice, k1 = min(a.K, k0 + a.k_slice);
+    if (jn <= 0 || k0 >= k1) return;                                            // workgroup-uniform
+    const char* ap = reinterpret_cast<const char*>(a.a) + 2 * (z * a.a_sz + head * a.a_sh + (long)brow0 * 32);
+    const char* bp = reinterpret_cast<const char*>(a.b) + 2 * (z * a.b_sz + head * a.b_sh);
 
-    // staging: piece c = tid + 256 i (i < 2) of each 32-token x 128-feature tile is token c / 16, features
-    // 8 (c % 16) .. + 7: the tiles stay row-major ([token][feature]) in LDS, one 16-byte store per piece; the
-    // MFMA fragments -- tokens are the contraction index -- come out of them through the transposing read.
-    // Feature block (c % 16) / 4 is output block-row ob (A) or list entry j0 + jb (B); absent blocks read
-    // block 0 of the tile and are zeroed when parked
-    int fcol_a[2], fcol_b[2];                               // feature offset of the piece in its operand
-    bool live_a[2], live_b[2];
+    // transfer w + 8 i of a step: 0..7 bring four tokens of A each, 8 + 4 r + j tokens 8 j .. 8 j + 7 of pair r of B (one past
+    // the last is the wave's first again: every wave issues NI a step, which is what the waits count).  A lane's 16 bytes:
+    // the token's bytes from `col` on; absent blocks are read from a present one and their products not stored
+    const char* src[NI];
+    long stride[NI];
+    int tok[NI], dst[NI];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int c = tid + 256 * i, fb = (c & 15) >> 2, f8 = 8 * (c & 3);
-        live_a[i] = fb < gn;
-        live_b[i] = fb < jn;
-        fcol_a[i] = 32 * (live_a[i] ? fb : 0) + f8;
-        fcol_b[i] = a.seg_inner[p0 + j0 + (live_b[i] ? fb : 0)] * 32 + f8;
+    for (int i = 0; i < NI; ++i) {
+        const int t = w + 8 * i < 8 + 4 * NP ? w + 8 * i : w;                   // (wave-uniform)
+        if (t < 8) {
+            const int tk = 4 * t + (lane >> 4), c = lane & 15;
+            const int p = (c >> 1) ^ ((tk & 3) + 4 * ((tk >> 3) & 1));
+            tok[i] = tk;
+            src[i] = ap + (p < 2 * gn ? 32 * p : 32 * (p & 1)) + 16 * (c & 1);
+            stride[i] = 2 * a.a_sk;
+            dst[i] = 1024 * t;
+        } else {
+            const int r = (t - 8) >> 2, tk = 8 * ((t - 8) & 3) + (lane >> 3), c = lane & 7;
+            const int p = (c >> 1) ^ (((tk >> 1) & 1) + 2 * ((tk >> 3) & 1));
+            const int inner = a.seg_inner[p0 + j0 + min(2 * r + (p >> 1), jn - 1)];
+            tok[i] = tk;
+            src[i] = bp + (long)inner * 64 + 32 * (p & 1) + 16 * (c & 1);
+            stride[i] = 2 * a.b_sk;
+            dst[i] = 8192 + 4096 * r + 1024 * ((t - 8) & 3);
+        }
     }
-    // two register sets: the loads of step s+2 are issued while step s is multiplied and are parked in LDS
-    // one step later, so every global load has two steps to arrive (every fetch issues the same four
-    // loads per thread on every path, so the wait for the older set can leave the newer one in flight)
-    uintx4 ra0[2], rb0[2], ra1[2], rb1[2];
-    auto fetch = [&](int kt, uintx4 (&ra)[2], uintx4 (&rb)[2]) __attribute__((always_inline)) {
+    auto transfer = [&](int kt, int stage) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int tok = min(kt + ((tid + 256 * i) >> 4), a.K - 1);     // clamped; tokens past k1 are zeroed below
-            ra[i] = *reinterpret_cast<const uintx4*>(ap + (long)tok * a.a_sk + fcol_a[i]);
-            rb[i] = *reinterpret_cast<const uintx4*>(bp + (long)tok * a.b_sk + fcol_b[i]);
-        }
-    };
-    auto stash = [&](int buf, int kt, const uintx4 (&ra)[2], const uintx4 (&rb)[2]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int c = tid + 256 * i, tok = c >> 4, f0 = 8 * (c & 15);
-            const bool in = kt + tok < k1;
-            *reinterpret_cast<uintx4*>(&at[buf][tok * LD + f0]) = (live_a[i] && in) ? ra[i] : uintx4{0, 0, 0, 0};
-            *reinterpret_cast<uintx4*>(&bt[buf][tok * LD + f0]) = (live_b[i] && in) ? rb[i] : uintx4{0, 0, 0, 0};
-        }
+        for (int i = 0; i < NI; ++i)                                            // (clamped; tokens past k1 are zeroed below)
+            dma_to_lds(src[i] + min(kt + tok[i], a.K - 1) * stride[i], sddk_smem + stage * STAGE + dst[i]);
     };
 
-    floatx4 acc[4][4];
+    floatx4 acc[4][NP];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = Frag<float>::zero();
-    const bool wave_active = 2 * wm < gn && 2 * wn < jn;    // its output blocks exist
-
-    auto compute = [&](int buf) __attribute__((always_inline)) {
-        if (wave_active) {
-            uintx4 fa[4], fb[4];
+        for (int j = 0; j < NP; ++j) acc[i][j] = Frag<float>::zero();
+    const int trow = 8 * g + (r16 >> 2);                                        // (+ 4 for the second half: same swizzle)
+    const int aoff = trow * 256 + 8 * (r16 & 3), asw = (trow & 3) + 4 * (g & 1);
+    const int boff = 8192 + trow * 128 + 32 * (wn ^ (((trow >> 1) & 1) + 2 * (g & 1))) + 8 * (r16 & 3);
+    auto compute = [&](const char* st, bool ragged, int left) __attribute__((always_inline)) {
+        uintx4 keep = {~0u, ~0u, ~0u, ~0u};                                     // tokens 8 g .. 8 g + 7 of the step that exist
+        if (ragged) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                fa[i] = frag_down_rows(at[buf], LD, 64 * wm + 16 * i, r16, g);
-                fb[i] = frag_down_rows(bt[buf], LD, 64 * wn + 16 * i, r16, g);
-            }
+            for (int d = 0; d < 4; ++d)
+                keep[d] = (8 * g + 2 * d < left ? 0xffffu : 0u) | (8 * g + 2 * d + 1 < left ? 0xffff0000u : 0u);
+        }
+        uintx4 fa[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) {
+            const char* q = st + aoff + 32 * ((4 * wm + i) ^ asw);
+            fa[i] = lds_read_tr8(q, q + 4 * 256);
+            if (ragged) fa[i] &= keep;
+        }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = mma32<T>(fa[i], fb[j], acc[i][j]);
+        for (int j = 0; j < NP; ++j) {
+            const char* q = st + boff + 4096 * j;
+            uintx4 fb = lds_read_tr8(q, q + 4 * 128);
+            if (ragged) fb &= keep;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i][j] = mma32<T>(fa[i], fb, acc[i][j]);
         }
     };
-    fetch(k0, ra0, rb0);
-    stash(0, k0, ra0, rb0);
-    fetch(k0 + 32, ra1, rb1);                               // set 1 holds odd steps, set 0 even steps
-    drain_loads_but<4>();                                   // only set 1 (four loads a thread) is in flight
-    __syncthreads();
-    for (int kt = k0; kt < k1; kt += 64) {
-        fetch(kt + 64, ra0, rb0);                           // (past the slice: loaded, zeroed, never used)
-        compute(0);
-        stash(1, kt + 32, ra1, rb1);
-        drain_loads_but<4>();                               // set 1 is parked: only set 0 is in flight
-        __syncthreads();
-        fetch(kt + 96, ra1, rb1);
-        if (kt + 32 < k1) compute(1);
-        stash(0, kt + 64, ra0, rb0);
-        drain_loads_but<4>();
-        __syncthreads();
+#pragma unroll
+    for (int d = 0; d < SDDK_STAGES - 1; ++d) transfer(k0 + 32 * d, d);
+    int cur = 0;
+    for (int kt = k0; kt < k1; kt += 32) {
+        drain_loads_but<NI * (SDDK_STAGES - 2)>();                              // this wave's part of the step is in LDS
+        __syncthreads();                                                        // everyone's is; the stage before it is free
+        transfer(kt + 32 * (SDDK_STAGES - 1), (cur + SDDK_STAGES - 1) % SDDK_STAGES);
+        if (kt + 32 <= k1) compute(sddk_smem + cur * STAGE, false, 32);
+        else compute(sddk_smem + cur * STAGE, true, k1 - kt);
+        cur = (cur + 1) % SDDK_STAGES;
     }
-    if (!wave_active) return;
-    // lane holds C[out = 64 wm + 16 i + 4 g + x][in = 64 wn + 16 j + r16]
+    drain_loads();                                                              // nothing may land in LDS after the workgroup has ended
+    // lane holds C[out = 64 wm + 16 i + 4 g + x][in = 16 (wn + 4 j) + r16] of the chunk
     float* cz = a.c32 + (long)z * a.nnz * 1024;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -600,10 +607,10 @@ __global__ __launch_bounds__(256) void bs_sdd32k_kernel(const SddKArgs a) {
         if (ob >= gn) continue;
         const int* blks = a.seg_blk + a.seg_ptr[row0 + ob] + j0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int jb = 2 * wn + (j >> 1);
-            if (jb >= jn) continue;
-            float* cb = cz + (long)blks[jb] * 1024 + (16 * (i & 1) + 4 * g) * 32 + 16 * (j & 1) + r16;
+        for (int j = 0; j < NP; ++j) {
+            const int t = wn + 4 * j;
+            if (t >> 1 >= jn) continue;
+            float* cb = cz + (long)blks[t >> 1] * 1024 + (16 * (i & 1) + 4 * g) * 32 + 16 * (t & 1) + r16;
 #pragma unroll
             for (int x = 0; x < 4; ++x) unsafeAtomicAdd(cb + 32 * x, acc[i][j][x]);
         }
@@ -3029,17 +3036,47 @@ extern "C" int flyhip_bs_sdd_kmajor(const void* a, const void* b, float* c32,
     FLY_REQUIRE(a && b && c32 && row_ptr && row_blk && row_col && grp_row0 && grp_n, "bs_sdd_kmajor: null pointer");
     FLY_REQUIRE(blk == 32 && (dtype == BF16 || dtype == F16), "bs_sdd_kmajor: needs 32x32 blocks of bf16 / fp16");
     FLY_REQUIRE(n_grp > 0 && max_row_nnz > 0 && brows_per_head > 0 && nnz > 0 && K > 0, "bs_sdd_kmajor: bad sizes");
-    FLY_REQUIRE(k_slice >= 32 && k_slice % 32 == 0, "bs_sdd_kmajor: k_slice must be a positive multiple of 32");
+    FLY_REQUIRE(k_slice >= 0 && k_slice % 32 == 0, "bs_sdd_kmajor: k_slice must be a multiple of 32 (0: chosen here)");
     FLY_REQUIRE(((a_sz | a_sh | a_sk | b_sz | b_sh | b_sk) % 8) == 0, "bs_sdd_kmajor: strides must be multiples of 8 elements");
-    const int chunks = (max_row_nnz + 3) / 4, slices = (K + k_slice - 1) / k_slice;
-    FLY_REQUIRE((long)n_grp * chunks <= 2147483647L && slices <= 65535, "bs_sdd_kmajor: too many workgroups");
+    FLY_REQUIRE(((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) % 16) == 0, "bs_sdd_kmajor: operands must be 16-byte aligned");
+    const Machine& mach = machine();
+    const int pairs = (max_row_nnz + 1) / 2, chunks = (pairs + SDDK_MAX_PAIRS - 1) / SDDK_MAX_PAIRS;
+    const int np = std::max(2, (pairs + chunks - 1) / chunks);
+    if (k_slice == 0) {
+        // the slice length that minimises (rounds of workgroups, one per compute unit) x (steps of a slice + the dozen that
+        // filling the stages and the atomics cost)
+        const long tiles = (long)n_grp * chunks * Z;
+        long best = -1;
+        for (int n = 1; n <= std::max(1, K / 64) && (n == 1 || tiles * (n - 1) < 4L * mach.cus); ++n) {
+            const int steps = ((K + n - 1) / n + 31) / 32;
+            const long cost = ((tiles * n + mach.cus - 1) / mach.cus) * (steps + 12);
+            if (best < 0 || cost < best) { best = cost; k_slice = 32 * steps; }
+        }
+    }
+    const int slices = (K + k_slice - 1) / k_slice;
+    const long items = (long)n_grp * chunks * slices;
+    FLY_REQUIRE(items <= 2147483647L - 64, "bs_sdd_kmajor: too many workgroups");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     if (int rc_capture = refuse_capture(st)) return rc_capture;
     SddKArgs args{a, b, c32, row_ptr, row_blk, row_col, grp_row0, grp_n, brows_per_head, K, k_slice, chunks, nnz,
-                  a_sz, a_sh, a_sk, b_sz, b_sh, b_sk};
-    dim3 grid((unsigned)(n_grp * chunks), slices, Z);
-    if (dtype == BF16) hipLaunchKernelGGL((bs_sdd32k_kernel<bf16_t>), grid, dim3(256), 0, st, args);
-    else hipLaunchKernelGGL((bs_sdd32k_kernel<f16_t>), grid, dim3(256), 0, st, args);
+                  a_sz, a_sh, a_sk, b_sz, b_sh, b_sk, n_grp, slices, mach.xcds};
+    dim3 grid((unsigned)((items + mach.xcds - 1) / mach.xcds * mach.xcds), 1, Z);
+#define SDDK_LAUNCH(TT, NP)                                                                                        \
+    {                                                                                                              \
+        auto kern = bs_sdd32k_kernel<TT, NP>;                                                                      \
+        constexpr size_t smem = (size_t)SDDK_STAGES * sddk_stage_bytes(NP);                                        \
+        static std::atomic<unsigned long long> lds_set{0};                                                         \
+        if (int rc2 = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_set, "bs_sdd_kmajor")) return rc2; \
+        hipLaunchKernelGGL(kern, grid, dim3(512), smem, st, args);                                                 \
+    }
+#define SDDK_PAIRS(TT)                                                                                             \
+    {                                                                                                              \
+        if (np == 2) SDDK_LAUNCH(TT, 2) else if (np == 3) SDDK_LAUNCH(TT, 3)                                       \
+        else if (np == 4) SDDK_LAUNCH(TT, 4) else SDDK_LAUNCH(TT, 5)                                               \
+    }
+    if (dtype == BF16) SDDK_PAIRS(bf16_t) else SDDK_PAIRS(f16_t)
+#undef SDDK_PAIRS
+#undef SDDK_LAUNCH
     return check_launch("bs_sdd32k_kernel");
 }
 

@@ -508,7 +508,7 @@ int flyhip_bs_sdd_dsoftmax(const void* dout, const void* v, const void* p, const
  * features -- the weight gradient x^T dy of a block-sparse linear layer, K = tokens (ref: the 'sdd'
  * call of the backward pass, blocksparse_matmul.py:562-587 -> _sdd_matmul :279-346).  32x32 blocks
  * of bf16 / fp16.  c32 is fp32 (Z, nnz, 32, 32), ZEROED by the caller: slices of k_slice tokens
- * (a multiple of 32) are accumulated into it with float atomics; the caller rounds it to the
+ * (a multiple of 32; 0: as many as fill the machine) are accumulated into it with float atomics; the caller rounds it to the
  * output type.  row_ptr / row_blk / row_col as in flyhip_bs_sdd; grp_row0 / grp_n: groups of at most
  * four consecutive block-rows of a head with identical column lists (every block-row in exactly one
  * group); max_row_nnz = the longest column list. */

@@ -1321,3 +1321,19 @@ def test_linear_layer_any_token_count(n_in, n_out, tokens, dtype):
     bar = 3e-3 if dtype == torch.bfloat16 else 4e-4
     for a, r in zip(got + (short,), want + (ref,)):
         assert a.dtype == dtype and float((a.detach().double().cpu() - r.detach()).norm()) <= bar * float(r.detach().norm())
+
+
+@pytest.mark.parametrize('rows,cols,tokens', [(1, 1, 512), (3, 3, 545), (4, 5, 1000), (5, 7, 4097), (4, 9, 640), (6, 11, 2049), (2, 23, 777)])
+def test_weight_gradient_chunks_of_columns(rows, cols, tokens):
+    """a^T b on a full layout of `rows` x `cols` blocks: groups of one to four block-rows, chunks of one to ten block-columns, odd
+    lists, token counts that end inside a step or a slice, against float64.  Bar: one rounding to bfloat16 (2^-9, 2-norm)."""
+    from fly_amd import matmul
+    g = torch.Generator().manual_seed(rows + cols)
+    a, b = (torch.randn(1, 1, tokens, 32 * n, generator=g).bfloat16() for n in (rows, cols))
+    b[:, :, -1] = float('nan')                       # (the last token counts: nothing past it is read in its place)
+    b[:, :, -1, 1:] = 3.0
+    op = matmul(torch.ones(1, rows, cols, dtype=torch.long), 32, 'sdd', trans_a=True)
+    op.ragged_rows = True
+    c = op(a.to(DEV), b.to(DEV))[0].double().cpu().view(rows, cols, 32, 32).permute(0, 2, 1, 3).reshape(32 * rows, 32 * cols)
+    ref = a[0, 0].double().t() @ b[0, 0].double()
+    assert c[:, 0].isnan().all() and float((c - ref)[:, 1:].norm()) <= 3e-3 * float(ref[:, 1:].norm())
