@@ -23,9 +23,10 @@
 //   local_bwd_b16_kernel<EXACT> (sblocal.hip)  the band, plus the low-rank part, rounded once
 //
 // Measured at B=1, H=16, L=16384, window 1024, 256 features, where the backward ran as library products over windows of
-// keys before (20.8 ms): chunks 185, scan 19, low-rank 316 (query-major) and 730 (key-major), band 204 and 295 us.  The
+// keys before (20.8 ms): chunks 187, scan 19, low-rank 310 (query-major) and 600 (key-major), band 200 and 290 us.  The
 // chunk sums (66 KB per 64 rows and side at 256 features) bound the first two: a scan over every chunk instead of every
-// segment moved 1.1 GB in 225 us.
+// segment moved 1.1 GB in 225 us.  The low-rank kernels wait: for the far sums (five trips to the cache, 140 and 190 us of the
+// two), and in the key-major one vector instructions on the edges' features and weights take as long as the products (230 us).
 #include "common.h"
 #include "local.h"
 #include <algorithm>
@@ -330,17 +331,17 @@ struct FarPrefix {
         part = sums + c * per;
         f = __builtin_amdgcn_exp2f(unit[c] + ref);
     }
-    // x[j] += sign * (entry at `lane + step(j)`), all loads of a source in flight together (the branches are uniform)
-    template <typename V, int N, typename Step>
-    __device__ __forceinline__ void add(V (&x)[N], float sign, uint32_t lane, Step step) const {
+    // x[j] += sign * (the four entries from at(j) on), all loads of a source in flight together (the branches are uniform)
+    template <int N, typename At>
+    __device__ __forceinline__ void add(floatx4 (&x)[N], float sign, At at) const {
         if (whole) {
 #pragma unroll
-            for (int j = 0; j < N; ++j) x[j] += *reinterpret_cast<const V*>(whole + lane + step(j)) * sign;
+            for (int j = 0; j < N; ++j) x[j] += *reinterpret_cast<const floatx4*>(whole + at(j)) * sign;
         }
         if (part) {
             const float fs = sign * f;
 #pragma unroll
-            for (int j = 0; j < N; ++j) x[j] += *reinterpret_cast<const V*>(part + lane + step(j)) * fs;
+            for (int j = 0; j < N; ++j) x[j] += *reinterpret_cast<const floatx4*>(part + at(j)) * fs;
         }
     }
 };
@@ -350,16 +351,30 @@ struct FarPrefix {
 // ---------------------------------------------------------------------------------------
 // 16 projection rows (32 features) per wave, all 64 outer rows: every feature of an edge chunk is formed once per
 // workgroup and goes from registers into the products.  Sums over features (chain rule, d v) are per wave until the end.
-template <int E, int M>
+// Key-major (730 -> 600 us at the size above) needs two operands transposed as well, the far sums and the edge features: it
+// takes them by transposing LDS reads of what it has, not by strided loads and a second evaluation.
+// columns of the result reduced over the waves at a time: two 16-column blocks where that takes no more LDS
+template <int E, int M, bool KEYMAJOR>
+constexpr size_t far_reduce_cols() { return KEYMAJOR || M < 256 ? 32 : 16; }
+constexpr int FAR_LDT = 32 + 8;                                                     // row stride of the transposed features, key-major
+// bytes of the region that holds, one after the other, the wave's far rows (key-major), the inner chunk with df, the reduction
+template <int E, int M, bool KEYMAJOR>
+constexpr size_t far_lowrank_shared() {
+    size_t n = (size_t)2 * FC * (E + 8) * 2 + 2 * 8 * 64 * 16;
+    const size_t red = far_reduce_cols<E, M, KEYMAJOR>() * (M / 32) * FC * 4, rows = KEYMAJOR ? (size_t)(M / 32) * 2 * 32 * (E + 8) * 2 : 0;
+    if (n < red) n = red;
+    return n < rows ? rows : n;
+}
+template <int E, int M, bool KEYMAJOR>
 constexpr size_t far_lowrank_smem() {
-    const size_t tiles = (size_t)2 * FC * (E + 8) * 2, inner = tiles + 2 * 8 * 64 * 16, red = (size_t)(M / 32) * FC * 16 * 4;
-    return tiles + (inner > red ? inner : red) + sizeof(float) * (6 * FC + (M / 32) * (FC + 1));
+    return (size_t)2 * FC * (E + 8) * 2 + far_lowrank_shared<E, M, KEYMAJOR>() + sizeof(float) * (6 * FC + (M / 32) * (FC + 1) + 3) / 16 * 16 +
+           (KEYMAJOR ? (size_t)(M / 32) * 2 * 32 * FAR_LDT * 2 : 0);
 }
 
 template <int E, int M, bool KEYMAJOR>
-__global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR && M >= 128 ? 4 : 2, !KEYMAJOR && M >= 128 ? 8 : 2))) void far_lowrank_kernel(FarArgs a) {
+__global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR && M >= 256 ? 4 : 2, !KEYMAJOR && M >= 256 ? 8 : 2))) void far_lowrank_kernel(FarArgs a) {
     constexpr int NW = M / 32, NT = 64 * NW, MH = M / 2, KS = E / 32, EB = E / 16, LD = E + 8, PER = M * (E + 1);
-    constexpr size_t TILES = (size_t)2 * FC * LD * 2, INNER = TILES + 2 * 8 * 64 * 16, RED = (size_t)NW * FC * 16 * 4;
+    constexpr size_t TILES = (size_t)2 * FC * LD * 2;
     extern __shared__ __attribute__((aligned(128))) char far_smem[];
     uint16_t* Xo = reinterpret_cast<uint16_t*>(far_smem);
     uint16_t* Yo = Xo + FC * LD;
@@ -367,12 +382,14 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
     uint16_t* Yi = Xi + FC * LD;
     uintx4* DF = reinterpret_cast<uintx4*>(Yi + FC * LD);                           // [piece][step, outer block][lane]
     float* red = reinterpret_cast<float*>(Xi);
-    float* diago = reinterpret_cast<float*>(far_smem + TILES + (INNER > RED ? INNER : RED));
+    float* diago = reinterpret_cast<float*>(far_smem + TILES + far_lowrank_shared<E, M, KEYMAJOR>());
     float* exto = diago + FC; float* co = exto + FC;
     float* diagi = co + FC; float* exti = diagi + FC; float* ci = exti + FC;
     float* us = ci + FC;                                                            // [NW][FC]
     float* kred = us + NW * FC;                                                     // [NW]
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    // key-major: the wave's features of 32 inner rows, [piece][sign, 16 features][rows]
+    uint16_t* ft = reinterpret_cast<uint16_t*>(far_smem + far_lowrank_smem<E, M, KEYMAJOR>()) - (NW - w) * 2 * 32 * FAR_LDT;
     const int Lo = KEYMAJOR ? a.S : a.T;
     const int n_oc = KEYMAJOR ? a.n_kc : a.n_qc, n_ic = KEYMAJOR ? a.n_qc : a.n_kc;
     const int n_items = a.B * a.H * n_oc;
@@ -441,24 +458,35 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
     const FarPrefix p0(pre, units, ref, PER, c0 - 1, n_ic, a.seg);
     const FarPrefix p1(pre, units, ref, PER, c1 < n_ic ? c1 - 1 : -1, n_ic, a.seg);
     const FarPrefix pn(pre, units, ref, PER, c1 < n_ic ? n_ic - 1 : -1, n_ic, a.seg);
-    auto far = [&](auto& x, uint32_t lane_at, auto step) __attribute__((always_inline)) {
-        pn.add(x, 1.f, lane_at, step);
-        p1.add(x, -1.f, lane_at, step);
-        p0.add(x, 1.f, lane_at, step);
-    };
+    // (every load of a source in flight together: a source is one trip to the cache, and nothing else hides it)
+    floatx4 fx[2 * (2 * KS + 1)];                                                   // [sign][row: 32 ks + 8 g .. + 7 | features 4 g .. + 3]
+#pragma unroll
+    for (int j = 0; j < 2 * (2 * KS + 1); ++j) fx[j] = Frag<float>::zero();
+    {
+        const uint32_t row_at = (uint32_t)((16 * w + r16) * E + 8 * g), vec_at = (uint32_t)(16 * w + 4 * g);
+        auto at = [&](int j) __attribute__((always_inline)) {
+            const int sg = j / (2 * KS + 1), n = j % (2 * KS + 1);
+            return n < 2 * KS ? row_at + sg * MH * E + 32 * (n >> 1) + 4 * (n & 1) : vec_at + M * E + sg * MH;
+        };
+        pn.add(fx, 1.f, at);
+        p1.add(fx, -1.f, at);
+        p0.add(fx, 1.f, at);
+    }
     floatx4 acc2[2][4];                                                             // [sign][outer block], rows = features
+    uint16_t* fw = Xi + w * 2 * 32 * LD;                                            // key-major: the wave's far rows, [piece][sign, 16 features][E]
 #pragma unroll
     for (int sg = 0; sg < 2; ++sg) {
 #pragma unroll
         for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] = Frag<float>::zero();
-        floatx4 x[2 * KS];
-#pragma unroll
-        for (int j = 0; j < 2 * KS; ++j) x[j] = Frag<float>::zero();
-        far(x, (uint32_t)((sg * MH + 16 * w + r16) * E + 8 * g), [](int j) { return 32 * (j >> 1) + 4 * (j & 1); });
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             uintx4 fh, fl;
-            split2(x[2 * ks], x[2 * ks + 1], fh, fl);
+            split2(fx[sg * (2 * KS + 1) + 2 * ks], fx[sg * (2 * KS + 1) + 2 * ks + 1], fh, fl);
+            if (KEYMAJOR) {
+                uint16_t* d = fw + (16 * sg + r16) * LD + 32 * ks + 8 * g;
+                *reinterpret_cast<uintx4*>(d) = fh;
+                *reinterpret_cast<uintx4*>(d + 32 * LD) = fl;
+            }
 #pragma unroll
             for (int ob = 0; ob < 4; ++ob) {
                 const uintx4 yo = *reinterpret_cast<const uintx4*>(Yo + (16 * ob + r16) * LD + 32 * ks + 8 * g);
@@ -466,21 +494,18 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
                 acc2[sg][ob] = mma_bf16(fh, yo, acc2[sg][ob]);
             }
         }
-        floatx4 vec[1] = {Frag<float>::zero()};
-        far(vec, (uint32_t)(M * E + sg * MH + 16 * w + 4 * g), [](int) { return 0; });
 #pragma unroll
-        for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] -= vec[0] * (KEYMAJOR ? 1.0f : co[16 * ob + r16]);
+        for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] -= fx[sg * (2 * KS + 1) + 2 * KS] * (KEYMAJOR ? 1.0f : co[16 * ob + r16]);
     }
     floatx4 acc3[KEYMAJOR ? EB : 1][KEYMAJOR ? 4 : 1];                              // d v: rows = value dims, columns = keys
     if (KEYMAJOR) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                          // (read by other lanes of the wave only)
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int eb = 0; eb < EB; ++eb) {
-            float x[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) x[j] = 0.f;
-            far(x, (uint32_t)((16 * w + 4 * g) * E + 16 * eb + r16), [](int j) { return ((j >> 2) * MH + (j & 3)) * E; });
-            uintx4 th, tl;
-            split2(floatx4{x[0], x[1], x[2], x[3]}, floatx4{x[4], x[5], x[6], x[7]}, th, tl);
+            const uint16_t* q = fw + (4 * g + (r16 >> 2)) * LD + 16 * eb + 4 * (r16 & 3);
+            const uintx4 th = lds_read_tr8(reinterpret_cast<const char*>(q), reinterpret_cast<const char*>(q + 16 * LD));
+            const uintx4 tl = lds_read_tr8(reinterpret_cast<const char*>(q + 32 * LD), reinterpret_cast<const char*>(q + 48 * LD));
 #pragma unroll
             for (int ob = 0; ob < 4; ++ob) {
                 floatx4 d = Frag<float>::zero();
@@ -490,6 +515,7 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        __syncthreads();                                                            // the far rows lie where the inner chunk goes
     }
 
     while (ic < c1) {
@@ -547,6 +573,16 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
             }
             split2(f0[0], f0[1], fh[0], fl[0]);
             split2(f1[0], f1[1], fh[1], fl[1]);
+            if (KEYMAJOR) {
+#pragma unroll
+                for (int sg = 0; sg < 2; ++sg)
+#pragma unroll
+                    for (int hb = 0; hb < 2; ++hb) {
+                        uint16_t* d = ft + (16 * sg + r16) * FAR_LDT + 16 * hb + 4 * g;
+                        *reinterpret_cast<uint2*>(d) = make_uint2(fh[sg][2 * hb], fh[sg][2 * hb + 1]);
+                        *reinterpret_cast<uint2*>(d + 32 * FAR_LDT) = make_uint2(fl[sg][2 * hb], fl[sg][2 * hb + 1]);
+                    }
+            }
 #pragma unroll
             for (int ob = 0; ob < 4; ++ob) {
                 const uintx4 dh = DF[(4 * st + ob) * 64 + lane], dl = DF[(8 + 4 * st + ob) * 64 + lane];
@@ -557,27 +593,20 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
                     acc2[sg][ob] = mma_bf16(fh[sg], dh, acc2[sg][ob]);
                 }
             }
-        }
-        if (KEYMAJOR) {
-            // this wave's features of the low-rank weights outside the band: result rows = queries, columns = keys; then
-            // d v^T[d][key] += g^T[d][query] W[query][key]
-#pragma unroll
-            for (int st = 0; st < 2; ++st) {
+            if (KEYMAJOR) {
+                // this wave's features of the low-rank weights outside the band: result rows = queries, columns = keys; then
+                // d v^T[d][key] += g^T[d][query] W[query][key].  The operand is the one above transposed
                 uintx4 wh[2], wl[2];
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // (read by other lanes of the wave only)
+                __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int hb = 0; hb < 2; ++hb) {
-                    const int row = 32 * st + 16 * hb + r16;
-                    const floatx4 dd = P.features_by_rows(Xi + row * LD + 8 * g);
-                    const float bias = exti[row] - diagi[row];
-                    floatx4 f0, f1;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const bool ok = 16 * w + 4 * g + i < a.mh_valid;
-                        f0[i] = ok ? __builtin_amdgcn_exp2f(bias + dd[i]) : 0.f;
-                        f1[i] = ok ? __builtin_amdgcn_exp2f(bias - dd[i]) : 0.f;
-                    }
-                    split2(f0, f1, wh[hb], wl[hb]);
+                    const uint16_t* q = ft + (4 * g + (r16 >> 2)) * FAR_LDT + 16 * hb + 4 * (r16 & 3);
+                    wh[hb] = lds_read_tr8(reinterpret_cast<const char*>(q), reinterpret_cast<const char*>(q + 16 * FAR_LDT));
+                    wl[hb] = lds_read_tr8(reinterpret_cast<const char*>(q + 32 * FAR_LDT), reinterpret_cast<const char*>(q + 48 * FAR_LDT));
                 }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_sched_barrier(0);          // (the steps' operands do not fit the registers side by side)
 #pragma unroll
                 for (int ob = 0; ob < 4; ++ob) {
@@ -612,6 +641,13 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
         ic = nx;
     }
 
+    // the wave's rows of sqrt(t) P, asked for before the barriers of the reduction
+    floatx4 pv[EB];
+    const float stemp = sqrtf(a.temp);
+#pragma unroll
+    for (int eb = 0; eb < EB; ++eb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pv[eb][i] = a.proj[(long)(16 * w + 4 * g + i) * E + 16 * eb + r16] * stemp;
     // u = F_o o acc2; d x = sqrt(t) P^T (u+ - u-) - t x sum u
     floatx4 du[4];
 #pragma unroll
@@ -643,19 +679,19 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
         bo[ob][0] = uintx4{dh.x, dh.y, dh.x, dh.y};
         bo[ob][1] = uintx4{dl.x, dl.y, dh.x, dh.y};
     }
-    const float stemp = sqrtf(a.temp);
-    constexpr int QUADS = FC * 4;                                                   // groups of four columns of a 16-column block, per 64 rows
+    constexpr int RC = far_reduce_cols<E, M, KEYMAJOR>(), RB = RC / 16;             // columns and 16-column blocks at a time
+    constexpr int QUADS = FC * RC / 4;                                              // groups of four columns, per 64 rows
 #pragma unroll
     for (int pass = 0; pass < (KEYMAJOR ? 2 : 1); ++pass)
 #pragma unroll
-        for (int eb = 0; eb < EB; ++eb) {
+        for (int e2 = 0; e2 < EB / RB; ++e2) {
+#pragma unroll
+          for (int eh = 0; eh < RB; ++eh) {
+            const int eb = RB * e2 + eh;
             floatx4 d[4];
             if (pass == 0) {
-                floatx4 pv;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) pv[i] = a.proj[(long)(16 * w + 4 * g + i) * E + 16 * eb + r16] * stemp;
                 uint2 ph, pm, pl;
-                split3_4(pv, ph, pm, pl);
+                split3_4(pv[eb], ph, pm, pl);
                 const uintx4 a0 = {ph.x, ph.y, pm.x, pm.y}, a1 = {ph.x, ph.y, pl.x, pl.y};
 #pragma unroll
                 for (int ob = 0; ob < 4; ++ob) d[ob] = mma_bf16(a0, bo[ob][0], mma_bf16(a1, bo[ob][1], Frag<float>::zero()));
@@ -664,16 +700,18 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
                 for (int ob = 0; ob < 4; ++ob) d[ob] = acc3[KEYMAJOR ? eb : 0][KEYMAJOR ? ob : 0];
             }
 #pragma unroll
-            for (int ob = 0; ob < 4; ++ob) *reinterpret_cast<floatx4*>(red + ((w * FC + 16 * ob + r16) * 16 + 4 * g)) = d[ob];
+            for (int ob = 0; ob < 4; ++ob) *reinterpret_cast<floatx4*>(red + ((eh * NW + w) * FC + 16 * ob + r16) * 16 + 4 * g) = d[ob];
+          }
             __syncthreads();
             float* dst = pass == 0 ? (KEYMAJOR ? a.dk : a.dq) : a.dv;
             for (int x = tid; x < QUADS; x += NT) {
-                const int row = x >> 2, qd = x & 3;
-                floatx4 s = *reinterpret_cast<const floatx4*>(red + (row * 16 + 4 * qd));
+                const int row = (x >> 2) % FC, qd = x & 3, eh = x / (4 * FC), eb = RB * e2 + eh;
+                const float* rp = red + (eh * NW * FC + row) * 16 + 4 * qd;
+                floatx4 s = *reinterpret_cast<const floatx4*>(rp);
                 float usum = us[row];
 #pragma unroll
                 for (int v = 1; v < NW; ++v) {
-                    s += *reinterpret_cast<const floatx4*>(red + ((v * FC + row) * 16 + 4 * qd));
+                    s += *reinterpret_cast<const floatx4*>(rp + v * FC * 16);
                     usum += us[v * FC + row];
                 }
                 if (pass == 0) {
@@ -691,7 +729,7 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
 template <int E, int M, bool KEYMAJOR>
 static int launch_lowrank(const FarArgs& a, hipStream_t st) {
     auto kern = far_lowrank_kernel<E, M, KEYMAJOR>;
-    constexpr size_t smem = far_lowrank_smem<E, M>();
+    constexpr size_t smem = far_lowrank_smem<E, M, KEYMAJOR>();
     static std::atomic<unsigned long long> lds_set{0};     // (devices on which this kernel has its LDS limit)
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_set, "far_lowrank")) return rc;
     const long items = (long)a.B * a.H * (KEYMAJOR ? a.n_kc : a.n_qc);

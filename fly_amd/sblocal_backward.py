@@ -243,11 +243,11 @@ def _far_kernel_dims(E, D, M):
 def _far_pays(rows, local_context, M):
     """Whether bfloat16 tensors go to _backward_far where the kernels that subtract the band from the sums over all keys
     (_backward_hip, on widened copies) could take them too.  Their M-wide products on every pair of the band cost in
-    proportion to the window, the chunk sums of the far path per row: at 200704 rows, 128 features 773 against 943 us at
-    window 256, 774 against 745 at 49; at 131072 rows, 64 features 376 against 464 us at window 128; 262144 rows, 128 features,
-    window 1024: 1263 against 2401.  Small problems, where launches and the copies count: 73 against 134 us at 8000 rows,
-    window 100."""
-    return M > 128 or local_context >= 96 or rows <= 16384
+    proportion to the window, the chunk sums of the far path per row.  Training steps in us, far against subtracting: 200704
+    rows, 128 features 758 / 1065 at window 256, 749 / 860 at 49, 737 / 859 at 12; 64 features 674 / 647 at 49; 32 features
+    796 / 604 at 49; 131072 rows, 64 features 420 / 577 at window 128; 262144 rows, 128 features 1317 / 2682 at window 1024,
+    948 / 1247 at 64.  Small problems, where launches and the copies count: 73 against 134 us at 8000 rows, window 100."""
+    return M >= 128 or local_context >= 96 or rows <= 16384
 
 
 def _backward_far(query, key, value, P, local_context, t, key_lengths, out, log_norm, grad_out, dims):
