@@ -9,7 +9,7 @@ import torch.nn.functional as F
 from torch.nn import init
 
 from .blocksparse_attention import instantiate
-from .blocksparse_matmul import KMAJOR_MIN_K, matmul
+from .blocksparse_matmul import KMAJOR_MIN_K, matmul, rows_as_they_are
 from .blocksparse_utils import densify_tensor
 
 
@@ -158,6 +158,8 @@ class BlockSparseLinear(nn.Module):
             if not (torch.is_grad_enabled() and self.weight.requires_grad) or (
                     self.block_size == 32 and n_tok >= KMAJOR_MIN_K
                     and (torch.is_autocast_enabled() or x.dtype in (torch.bfloat16, torch.float16))):
+                if pad_tok and not pad_in:
+                    tokens = rows_as_they_are(tokens)
                 pad_tok = 0
             if pad_in or pad_tok:
                 tokens = F.pad(tokens, (0, pad_in, 0, pad_tok))

@@ -24,7 +24,16 @@ def _dense_operand(x):
     the two matrix dims is unit-stride or vector alignment fails."""
     if (x.stride(-1) == 1 or x.stride(-2) == 1) and _aligned(x):
         return x
-    return x.contiguous()
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
+def rows_as_they_are(x):
+    """`x` itself where the kernels for 16-bit rows read it in place, else a copy they can: a count of rows that fills no block
+    used to come with a padded copy, so its callers may hand over any strides."""
+    if x.stride(-1) == 1 and all(s % 8 == 0 for s in x.stride()[:-1]) and x.data_ptr() % 16 == 0:
+        return x
+    return x.clone(memory_format=torch.contiguous_format)
 
 
 class _MatmulFn(torch.autograd.Function):
@@ -45,6 +54,8 @@ class _MatmulFn(torch.autograd.Function):
         op = ctx.op
         mode = op.mode
         da = db = None
+        if op.ragged_rows and dc.shape[2] % op.block:
+            dc = rows_as_they_are(dc)
         if ctx.needs_input_grad[0]:
             mode_da = mode[1] + mode[0] + mode[2]
             da = op._run(mode_da, dc, b, False, not op.trans_b, op.trans_a)

@@ -1337,3 +1337,22 @@ def test_weight_gradient_chunks_of_columns(rows, cols, tokens):
     c = op(a.to(DEV), b.to(DEV))[0].double().cpu().view(rows, cols, 32, 32).permute(0, 2, 1, 3).reshape(32 * rows, 32 * cols)
     ref = a[0, 0].double().t() @ b[0, 0].double()
     assert c[:, 0].isnan().all() and float((c - ref)[:, 1:].norm()) <= 3e-3 * float(ref[:, 1:].norm())
+
+
+@pytest.mark.parametrize('offset,width', [(0, 260), (1, 257), (4, 264)])
+def test_linear_layer_ragged_rows_of_a_wider_tensor(offset, width):
+    """Token counts that fill no block, rows that are slices of wider ones (strides and starts the kernels do not read in
+    place), input and output gradient alike: the numbers of contiguous copies, bit for bit except the weight gradient, whose
+    slices add up in any order."""
+    from fly_amd import BlockSparseLinear, FlatBlockButterflySparsityConfig
+    torch.manual_seed(0)
+    lin = BlockSparseLinear(256, 256, FlatBlockButterflySparsityConfig(8, 2, block=32)).to(DEV).bfloat16()
+    wide, grad = (torch.randn(601, width + offset, device=DEV).bfloat16() for _ in range(2))
+    x, w = wide[:, offset:offset + 256], grad[:, offset:offset + 256]
+    got = []
+    for a, b in ((x, w), (x.clone(), w.clone())):
+        a = a.detach().requires_grad_()
+        y = lin(a)
+        got.append((y.detach(),) + torch.autograd.grad(y, (a, lin.weight, lin.bias), b))
+    for n, (u, v) in enumerate(zip(*got)):
+        assert torch.equal(u, v) if n != 2 else rel_err(u, v) <= 2 ** -7
