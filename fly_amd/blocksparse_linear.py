@@ -132,7 +132,6 @@ class BlockSparseLinear(nn.Module):
             op = None
             if self.backend == 'triton':
                 op = matmul(self.layout.cpu(), self.block_size, 'dds', trans_a=False, trans_b=True)
-                op.ragged_rows = True
             self.ops_cache[self.backend] = op
             return op
 
@@ -166,6 +165,7 @@ class BlockSparseLinear(nn.Module):
             # (views only, and slices only where something is cut off: under autograd a select or a slice of the
             #  result, also one that keeps everything, costs a zero-fill and a copy of the whole tensor on the way back)
             op = self.get_ops()
+            op.ragged_rows = True                # (here: a layer saved with its operators may hold one without it)
             tokens = tokens.view(1, 1, *tokens.shape)
             if bias is not None and self.out_features == self.out_features_extended:
                 # (in the dtype of the product: under autocast half precision)

@@ -76,6 +76,10 @@ class matmul:
     ValueError before anything is launched, as the reference's _validate_inputs does (:678-702).
     """
 
+    # 'dds': the gradient of the sparse operand may contract over any number of rows its kernel takes (the linear layer sets
+    # it; a caller's own product keeps the multiple-of-16 rule).  On the class, for operators saved without it
+    ragged_rows = False
+
     def __init__(self, layout, block, mode, trans_a=False, trans_b=False):
         if mode not in ['sdd', 'dsd', 'dds']:
             raise NotImplementedError('Supported modes are: sdd, dsd, dds')
@@ -84,9 +88,6 @@ class matmul:
         assert layout.ndim in (2, 3), "Layout should be a 2 or 3 dimensional tensor of 0s and 1s"
         self.block, self.mode, self.trans_a, self.trans_b = block, mode, trans_a, trans_b
         self.lut_cache = dict()
-        # 'dds': the gradient of the sparse operand may contract over any number of rows its kernel takes (the linear layer
-        # sets it; a caller's own product keeps the multiple-of-16 rule)
-        self.ragged_rows = False
         self.layout = _as_heads(layout)            # (H, block-rows, block-cols), integral; 2-D means one head
         self.spdims = self.layout.shape
         if mode != 'sdd':
