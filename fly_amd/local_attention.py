@@ -7,7 +7,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib
-from .sblocal_attention import _HEAD_DIMS, _round_up_choice, _vector_ready
+from .sblocal_attention import _HEAD_DIMS, _round_up_choice, rows_for_vectors
 from .sblocal_backward import BandWindows
 
 
@@ -52,9 +52,7 @@ def local_forward(query, key, value, local_context, softmax_temp=None, key_lengt
     def prep(x):
         if x.shape[-1] != dim:
             x = F.pad(x, (0, dim - x.shape[-1]))      # zero columns change no dot product
-        # (2-byte rows are loaded 8 elements at a time: strides in multiples of 8)
-        ready = _vector_ready(x) and (x.element_size() == 4 or all(st % 8 == 0 for st in x.stride()[:-1]))
-        return x if ready else x.contiguous()
+        return rows_for_vectors(x, 16 // x.element_size())
     q, k, v = prep(query), prep(key), prep(value)
     lens = None
     if key_lengths is not None:
@@ -147,13 +145,11 @@ def _local_backward_kernels(query, key, value, local_context, t, key_lengths, gr
     B, T, H, E = query.shape
     S, D = key.shape[1], value.shape[3]
     dim = _round_up_choice(max(E, D), _HEAD_DIMS, 'head dimension')
-    unit = 16 // query.element_size()             # elements of a 16-byte load
 
     def prep(x):
         if x.shape[-1] != dim:
             x = F.pad(x, (0, dim - x.shape[-1]))      # zero columns change no dot product
-        ready = _vector_ready(x) and all(st % unit == 0 for st in x.stride()[:-1])
-        return x if ready else x.contiguous()
+        return rows_for_vectors(x, 16 // x.element_size())
     q, k, v, g, o = prep(query), prep(key), prep(value), prep(grad_out.to(query.dtype)), prep(out.to(query.dtype))
     delta = torch.empty(B, H, T, dtype=torch.float32, device=query.device)     # g . out per query, filled by the kernels
     lse_ = lse.reshape(B, H, T).float().contiguous()

@@ -29,6 +29,14 @@ def _vector_ready(x):
             and x.data_ptr() % 16 == 0)
 
 
+def rows_for_vectors(x, unit=4):
+    """`x` itself where rows of `unit` elements a load can be read in place (unit inner stride, other strides in multiples
+    of `unit`, 16-byte aligned base), else a copy that can.  A clone and not ``contiguous()``, which hands back the tensor
+    itself when it is contiguous but starts off the boundary or has an odd stride on a dim of size 1."""
+    ready = _vector_ready(x) and all(s % unit == 0 for s in x.stride()[:-1])
+    return x if ready else x.clone(memory_format=torch.contiguous_format)
+
+
 class SBLocalPlan:
     """The device scratch and the C-ABI calls for one problem shape.  Callers that run the same shape
     repeatedly (serving loops, benchmarks, the module below) keep one plan and call ``run`` with tensors
@@ -333,7 +341,7 @@ def sblocal_forward(query, key, value, projection_matrix, local_context, softmax
     def prep(x):
         if x.shape[-1] != dim:
             x = F.pad(x, (0, dim - x.shape[-1]))      # zero columns change neither dots nor norms
-        return x if _vector_ready(x) else x.contiguous()
+        return rows_for_vectors(x)
     q, k, v = prep(query), prep(key), prep(value)
     proj = _padded_projection(projection_matrix, mh, dim, cache)
     lens = None
@@ -400,7 +408,7 @@ def sbblocksparse_forward(query, key, value, projection_matrix, tables, softmax_
     def prep(x):
         if x.shape[-1] != dim:
             x = F.pad(x, (0, dim - x.shape[-1]))
-        return x if _vector_ready(x) else x.contiguous()
+        return rows_for_vectors(x)
     q, k, v = prep(query), prep(key), prep(value)
     proj = _padded_projection(projection_matrix, mh, dim, cache)
 

@@ -23,6 +23,8 @@ import math
 
 import torch
 
+from .sblocal_attention import rows_for_vectors
+
 
 
 class BandWindows:
@@ -263,11 +265,10 @@ def _backward_far(query, key, value, P, local_context, t, key_lengths, out, log_
     def prep(x):
         if x.shape[-1] != dim:
             x = torch.nn.functional.pad(x, (0, dim - x.shape[-1]))
-        ready = x.stride(-1) == 1 and all(st % 8 == 0 for st in x.stride()[:-1]) and x.data_ptr() % 16 == 0
-        return x if ready else x.contiguous()
+        return rows_for_vectors(x, 8)
     q, k, v, o, g = prep(query), prep(key), prep(value), prep(out), prep(grad_out.to(query.dtype))
     mh = P.shape[0]
-    proj = P.contiguous() if P.shape == (mk // 2, dim) else _fit(torch.nn.functional.pad(P, (0, 0, 0, mk // 2 - mh)), dim)
+    proj = rows_for_vectors(P) if P.shape == (mk // 2, dim) else _fit(torch.nn.functional.pad(P, (0, 0, 0, mk // 2 - mh)), dim)
     ln = log_norm.reshape(B, H, T).float().contiguous()
     lens = None if key_lengths is None else key_lengths.to(device=query.device, dtype=torch.int64).contiguous()
     new = query.new_empty

@@ -1066,3 +1066,56 @@ def test_local_attention_float32_on_bf16_pieces(B, T, S, H, E, D, lc, lens):
     for a, r in zip((out,) + got, (ref_out,) + ref):
         scale = max(float(r.detach().norm()), 1e-2 * r.numel() ** 0.5)      # (d query is zero where every query sees one key)
         assert float((a.detach().double().cpu() - r.detach()).norm()) <= 2e-6 * scale
+
+
+def _in_layout(x, layout):
+    """`x` with the same values in memory a caller may hand over: 'offset' contiguous but three elements off an aligned
+    start, 'odd-batch' a single batch entry whose batch stride is odd, 'heads-first' (B, H, L, E) in memory, 'fused' a third
+    of a projection's output, 'plain' contiguous."""
+    if layout == 'offset':
+        y = x.new_empty(x.numel() + 3)[3:].view(x.shape)
+    elif layout == 'odd-batch':
+        y = x.new_empty(x.numel() + 1).as_strided(x.shape, (x[0].numel() + 1,) + x.stride()[1:])
+    elif layout == 'heads-first':
+        y = x.new_empty(x.shape[0], x.shape[2], x.shape[1], x.shape[3]).transpose(1, 2)
+    elif layout == 'fused':
+        y = x.new_empty(x.shape[0], x.shape[1], 3, x.shape[2], x.shape[3])[:, :, 1]
+    else:
+        return x
+    y.copy_(x)
+    return y.detach()
+
+
+@pytest.mark.parametrize('H', [1, 3])
+@pytest.mark.parametrize('layout', ['offset', 'odd-batch', 'heads-first', 'fused'])
+@pytest.mark.parametrize('kind', ['sblocal-bf16', 'local-fp32', 'local-bf16'])
+def test_inputs_and_gradients_in_any_memory_layout(kind, layout, H):
+    """Kernels that read strides directly, on inputs and output gradients that are no plain contiguous tensors: the output
+    and the gradients are those of plain tensors bit for bit.  The gradient that autograd delivers through a concatenation
+    is contiguous and starts off a 16-byte boundary; an expanded one has no strides at all."""
+    from fly_amd import LocalAttention, sblocal_attention_fn
+    dtype = torch.float32 if kind.endswith('fp32') else torch.bfloat16
+    B, T, S, E, lc = 1, 150, 130, 64, 70
+    q, k, v, P = make_inputs(B, T, S, H, E, E, 64, seed=3, dtype=dtype)
+    w = torch.randn(B, T, H, E, generator=torch.Generator().manual_seed(4)).to(dtype)
+    dev = torch.device('cuda:0')
+
+    def layer(q, k, v):
+        if kind.startswith('sblocal'):
+            return sblocal_attention_fn(q, k, v, P.to(dev), lc)[0]
+        return LocalAttention(lc)(q, k, v)[0]
+    plain = [x.to(dev).requires_grad_() for x in (q, k, v)]
+    want = layer(*plain)
+    want_grads = torch.autograd.grad(want, plain, w.to(dev), retain_graph=True)
+    laid = [_in_layout(x.to(dev), layout).requires_grad_() for x in (q, k, v)]
+    out = layer(*laid)
+    assert torch.equal(out, want)
+    for a, b in zip(torch.autograd.grad(out, laid, _in_layout(w.to(dev), layout), retain_graph=True), want_grads):
+        assert a.dtype == dtype and torch.equal(a, b)
+    joined = torch.cat([torch.zeros(3, device=dev, dtype=dtype), out.flatten()])
+    for a, b in zip(torch.autograd.grad(joined, laid, torch.cat([torch.zeros(3, device=dev, dtype=dtype), w.to(dev).flatten()]),
+                                        retain_graph=True), want_grads):
+        assert torch.equal(a, b)
+    ones = torch.autograd.grad(want, plain, torch.ones_like(want))
+    for a, b in zip(torch.autograd.grad(out.sum(), laid), ones):
+        assert torch.equal(a, b)

@@ -372,3 +372,27 @@ def test_tile_mask_table_against_loops(block):
         assert torch.equal(a_, b_)
     with pytest.raises(ValueError):
         tile_mask_table(layout, 64)
+
+
+@pytest.mark.parametrize('dtype,unit', [(torch.float32, 4), (torch.bfloat16, 8)])
+def test_rows_for_vectors_copies_whatever_a_vector_load_cannot_read(dtype, unit):
+    """The layouts that ``contiguous()`` leaves as they are -- a contiguous tensor that starts off a 16-byte boundary, as
+    autograd delivers it through a concatenation, and an odd stride on a dim of size 1 -- come back as an aligned copy with
+    whole strides; what can be read in place is not copied."""
+    from fly_amd.sblocal_attention import rows_for_vectors
+    ok = torch.randn(2, 5, 3, 32).to(dtype)
+    for same in (ok, ok.permute(1, 0, 2, 3), ok[:, 1:], ok[..., :unit], ok[:1].expand(4, 5, 3, 32)):
+        assert rows_for_vectors(same, unit) is same
+    leaf = torch.zeros(2, 5, 3, 32, dtype=dtype, requires_grad=True)
+    seen = []
+    out = leaf * 1
+    out.register_hook(seen.append)
+    torch.cat([torch.zeros(3, dtype=dtype), out.flatten()]).backward(torch.arange(963).to(dtype))
+    late = seen[0]
+    assert late.is_contiguous() and late.data_ptr() % 16 != 0 and late.contiguous() is late
+    odd = torch.randn(5 * 96 + 7).to(dtype).as_strided((1, 5, 3, 32), (5 * 96 + 3, 96, 32, 1))
+    assert odd.is_contiguous() and odd.contiguous().stride(0) % unit != 0
+    for x in (late, odd, ok.transpose(1, 3).contiguous().transpose(1, 3), ok[..., :1].expand(2, 5, 3, 32), ok.flatten()[:480].view(2, 5, 3, 16)[..., 1:9]):
+        got = rows_for_vectors(x, unit)
+        assert got is not x and torch.equal(got, x) and got.data_ptr() % 16 == 0
+        assert got.stride(-1) == 1 and all(s % unit == 0 for s in got.stride()[:-1])
