@@ -300,6 +300,41 @@ __device__ __forceinline__ void split3(floatx4 x0, floatx4 x1, uintx4& h, uintx4
     split2(r0, r1, m, l);
 }
 
+// an operand of 32 contraction slots as N bf16 pieces, largest first: exact with three, to 2^-17 with two
+template <int N> struct PiecesOf { uintx4 p[N]; };
+using Pieces = PiecesOf<3>;
+template <int N>
+__device__ __forceinline__ PiecesOf<N> split(floatx4 x0, floatx4 x1) {
+    static_assert(N == 2 || N == 3, "two or three pieces");
+    PiecesOf<N> r;
+    if constexpr (N == 3) split3(x0, x1, r.p[0], r.p[1], r.p[2]);
+    else split2(x0, x1, r.p[0], r.p[1]);
+    return r;
+}
+// a . b over 32 contraction slots from the piece products above 2^-24 of it, small terms first
+template <int NA, int NB>
+__device__ __forceinline__ floatx4 mma_pieces(const PiecesOf<NA>& a, const PiecesOf<NB>& b, floatx4 c) {
+#pragma unroll
+    for (int n = 2; n >= 0; --n)
+#pragma unroll
+        for (int i = n; i >= 0; --i)
+            if (i < NA && n - i < NB) c = mma_bf16(a.p[i < NA ? i : 0], b.p[n - i < NB ? n - i : 0], c);
+    return c;
+}
+// (one operand bf16 as it stands)
+template <int N>
+__device__ __forceinline__ floatx4 mma_pieces(const PiecesOf<N>& a, uintx4 b, floatx4 c) {
+#pragma unroll
+    for (int i = N - 1; i >= 0; --i) c = mma_bf16(a.p[i], b, c);
+    return c;
+}
+template <int N>
+__device__ __forceinline__ floatx4 mma_pieces(uintx4 a, const PiecesOf<N>& b, floatx4 c) {
+#pragma unroll
+    for (int i = N - 1; i >= 0; --i) c = mma_bf16(a, b.p[i], c);
+    return c;
+}
+
 // four floats -> bf16 head and rest, four k-slots each
 __device__ __forceinline__ void split2_4(floatx4 x, uint2& hi, uint2& lo) {
     hi = make_uint2(pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]));

@@ -52,16 +52,6 @@ struct PieceTile {
     }
 };
 
-struct Pieces { uintx4 h, m, l; };
-// a . b over 32 contraction slots, small terms first
-__device__ __forceinline__ floatx4 mma_x6(const Pieces& a, const Pieces& b, floatx4 c) {
-    c = mma_bf16(a.l, b.h, c);
-    c = mma_bf16(a.h, b.l, c);
-    c = mma_bf16(a.m, b.m, c);
-    c = mma_bf16(a.m, b.h, c);
-    c = mma_bf16(a.h, b.m, c);
-    return mma_bf16(a.h, b.h, c);
-}
 // row fragment: elements 32 ks + 8 g .. + 7 of `row`; transposed fragment: column 16 cb + r16 of rows {4 g + i, 16 + 4 g + i}
 template <int E>
 __device__ __forceinline__ Pieces lx_rows(const char* st, int row, int ks, int g) {
@@ -79,9 +69,7 @@ __device__ __forceinline__ Pieces lx_cols(const char* st, int cb, int r16, int g
                   lds_read_tr8(p + 2 * PT::PIECE, p + 2 * PT::PIECE + 16 * PT::ROWB)};
 }
 __device__ __forceinline__ Pieces lx_load(const float* p) {
-    Pieces x;
-    split3(*reinterpret_cast<const floatx4*>(p), *reinterpret_cast<const floatx4*>(p + 4), x.h, x.m, x.l);
-    return x;
+    return split<3>(*reinterpret_cast<const floatx4*>(p), *reinterpret_cast<const floatx4*>(p + 4));
 }
 
 template <int E, int QB = 1>
@@ -159,7 +147,7 @@ __global__ __launch_bounds__(LX_NT) void local_fwd_x3_kernel(LocalArgs a) {
                 for (int kb = 0; kb < 2; ++kb) {
                     const Pieces kf = lx_rows<E>(Ks, 16 * kb + r16, ks, g);
 #pragma unroll
-                    for (int qq = 0; qq < QB; ++qq) s[qq][kb] = mma_x6(kf, qp[qq][ks], s[qq][kb]);
+                    for (int qq = 0; qq < QB; ++qq) s[qq][kb] = mma_pieces(kf, qp[qq][ks], s[qq][kb]);
                 }
             if (a.add_mask) {                                // (uniform)
 #pragma unroll
@@ -228,12 +216,12 @@ __global__ __launch_bounds__(LX_NT) void local_fwd_x3_kernel(LocalArgs a) {
             }
             Pieces p[QB];
 #pragma unroll
-            for (int qq = 0; qq < QB; ++qq) split3(s[qq][0], s[qq][1], p[qq].h, p[qq].m, p[qq].l);
+            for (int qq = 0; qq < QB; ++qq) p[qq] = split<3>(s[qq][0], s[qq][1]);
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
                 const Pieces vf = lx_cols<E>(Vs, db, r16, g);
 #pragma unroll
-                for (int qq = 0; qq < QB; ++qq) oacc[qq][db] = mma_x6(vf, p[qq], oacc[qq][db]);
+                for (int qq = 0; qq < QB; ++qq) oacc[qq][db] = mma_pieces(vf, p[qq], oacc[qq][db]);
             }
         }
         if (more) {
@@ -331,7 +319,7 @@ __global__ __launch_bounds__(LX_NT) __attribute__((amdgpu_waves_per_eu(3, 4))) v
             const float* gp_ = x2p + row * x2s + 32 * ks + 8 * g;
             const floatx4 g0 = *reinterpret_cast<const floatx4*>(gp_), g1 = *reinterpret_cast<const floatx4*>(gp_ + 4);
             const floatx4 u0 = *reinterpret_cast<const floatx4*>(orow + 32 * ks + 8 * g), u1 = *reinterpret_cast<const floatx4*>(orow + 32 * ks + 8 * g + 4);
-            split3(g0, g1, x2[ks].h, x2[ks].m, x2[ks].l);
+            x2[ks] = split<3>(g0, g1);
 #pragma unroll
             for (int i = 0; i < 4; ++i) d_own += g0[i] * u0[i] + g1[i] * u1[i];
         }
@@ -371,8 +359,8 @@ __global__ __launch_bounds__(LX_NT) __attribute__((amdgpu_waves_per_eu(3, 4))) v
             for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb) {
-                    s[kb] = mma_x6(lx_rows<E>(Y1, 16 * kb + r16, ks, g), x1[ks], s[kb]);
-                    gv[kb] = mma_x6(lx_rows<E>(Y2, 16 * kb + r16, ks, g), x2[ks], gv[kb]);
+                    s[kb] = mma_pieces(lx_rows<E>(Y1, 16 * kb + r16, ks, g), x1[ks], s[kb]);
+                    gv[kb] = mma_pieces(lx_rows<E>(Y2, 16 * kb + r16, ks, g), x2[ks], gv[kb]);
                 }
             // weights (times M) into s, dS into gv
 #pragma unroll
@@ -402,13 +390,13 @@ __global__ __launch_bounds__(LX_NT) __attribute__((amdgpu_waves_per_eu(3, 4))) v
                     gv[kb][i] = pr * (keep * gv[kb][i] - drow);
                 }
             }
-            Pieces ds, pw;
-            split3(gv[0], gv[1], ds.h, ds.m, ds.l);
-            if (KEYMAJOR) split3(s[0], s[1], pw.h, pw.m, pw.l);
+            const Pieces ds = split<3>(gv[0], gv[1]);
+            Pieces pw;
+            if (KEYMAJOR) pw = split<3>(s[0], s[1]);
 #pragma unroll
             for (int eb = 0; eb < EB; ++eb) {
-                acc1[eb] = mma_x6(lx_cols<E>(Y1, eb, r16, g), ds, acc1[eb]);
-                if (KEYMAJOR) acc2[eb] = mma_x6(lx_cols<E>(Y2, eb, r16, g), pw, acc2[eb]);
+                acc1[eb] = mma_pieces(lx_cols<E>(Y1, eb, r16, g), ds, acc1[eb]);
+                if (KEYMAJOR) acc2[eb] = mma_pieces(lx_cols<E>(Y2, eb, r16, g), pw, acc2[eb]);
             }
         }
         if (more) stash(cur ^ 1);

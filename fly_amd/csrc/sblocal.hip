@@ -2938,8 +2938,8 @@ template <> __device__ __forceinline__ float unpack_hi<f16_t>(uint32_t w) { retu
 template <int E> constexpr size_t local_bwd_smem() { return (size_t)2 * (TKL * 2 * (E + 8) * 2 + 2 * TKL * sizeof(float)); }
 
 // EXACT (bfloat16): the exact part of a Scatterbrain-local backward.  lse is the log-normaliser of all keys and delta is
-// given; P and dS enter the second products in two bf16 pieces (2^-17: the sums are exact to the rounding of the
-// results, as they were when this part ran in float32), and the low-rank part of the gradient is added in the epilogue.
+// given; P and dS enter the second products as three bf16 pieces (exactly), and the low-rank part of the gradient is added
+// in the epilogue.
 template <typename T, int E, bool KEYMAJOR, int QB, bool EXACT = false>
 __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
     static_assert(sizeof(T) == 2 && E % 32 == 0, "2-byte inputs, whole MFMA steps");
@@ -3103,19 +3103,13 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
                     }
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf) {
-                uint4 pb[KEYMAJOR ? QB : 1], sb[QB], pbl[KEYMAJOR ? QB : 1], sbl[QB];     // (..l: the second pieces, EXACT)
+                uint4 pb[KEYMAJOR ? QB : 1], sb[QB];
+                Pieces pbx[KEYMAJOR ? QB : 1], sbx[QB];     // (EXACT)
 #pragma unroll
                 for (int qq = 0; qq < QB; ++qq) {
                     if constexpr (EXACT) {
-                        uintx4 hi, lo;
-                        split2(gp[qq][2 * hf], gp[qq][2 * hf + 1], hi, lo);
-                        sb[qq] = __builtin_bit_cast(uint4, hi);
-                        sbl[qq] = __builtin_bit_cast(uint4, lo);
-                        if (KEYMAJOR) {
-                            split2(s1[qq][2 * hf], s1[qq][2 * hf + 1], hi, lo);
-                            pb[qq] = __builtin_bit_cast(uint4, hi);
-                            pbl[qq] = __builtin_bit_cast(uint4, lo);
-                        }
+                        sbx[qq] = split<3>(gp[qq][2 * hf], gp[qq][2 * hf + 1]);
+                        if (KEYMAJOR) pbx[qq] = split<3>(s1[qq][2 * hf], s1[qq][2 * hf + 1]);
                     } else {
                         sb[qq] = make_uint4(pack_pair<T>(gp[qq][2 * hf][0], gp[qq][2 * hf][1]), pack_pair<T>(gp[qq][2 * hf][2], gp[qq][2 * hf][3]),
                                             pack_pair<T>(gp[qq][2 * hf + 1][0], gp[qq][2 * hf + 1][1]),
@@ -3133,8 +3127,8 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
                                                                              reinterpret_cast<const char*>(p1 + 4 * LD)));
 #pragma unroll
                     for (int qq = 0; qq < QB; ++qq) {
-                        if (EXACT) acc1[qq][eb] = Frag32<T>::mma(t1, sbl[qq], acc1[qq][eb]);
-                        acc1[qq][eb] = Frag32<T>::mma(t1, sb[qq], acc1[qq][eb]);
+                        if constexpr (EXACT) acc1[qq][eb] = mma_pieces(__builtin_bit_cast(uintx4, t1), sbx[qq], acc1[qq][eb]);
+                        else acc1[qq][eb] = Frag32<T>::mma(t1, sb[qq], acc1[qq][eb]);
                     }
                     if (KEYMAJOR) {
                         const uint16_t* p2 = Y2 + toff + 32 * hf * LD + 16 * eb;
@@ -3142,8 +3136,8 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
                                                                                  reinterpret_cast<const char*>(p2 + 4 * LD)));
 #pragma unroll
                         for (int qq = 0; qq < QB; ++qq) {
-                            if (EXACT) acc2[qq][eb] = Frag32<T>::mma(t2, pbl[qq], acc2[qq][eb]);
-                            acc2[qq][eb] = Frag32<T>::mma(t2, pb[qq], acc2[qq][eb]);
+                            if constexpr (EXACT) acc2[qq][eb] = mma_pieces(__builtin_bit_cast(uintx4, t2), pbx[qq], acc2[qq][eb]);
+                            else acc2[qq][eb] = Frag32<T>::mma(t2, pb[qq], acc2[qq][eb]);
                         }
                     }
                 }

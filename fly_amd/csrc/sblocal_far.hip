@@ -11,10 +11,19 @@
 //   inside  the band for all pairs    -- no low-rank work at all (the kernels that subtract the band's part spend
 //                                        M-wide products on every pair of it: 15 of 17 chunks at a window of 1024),
 //   far     no pair in the band       -- through the sums  KV_c = sum phi v^T, sum phi  (QG_c = sum psi g^T, sum psi c) of the
-//                                        chunks, kept as prefix sums: far = prefix up to the window + suffix after it,
-//   an edge some pairs in the band    -- the pairs outside it one by one (two chunks at a window that is a multiple of 64).
-// Nothing is subtracted from a sum over all keys that contains it many times over, so features in two bf16 pieces
-// (2^-17) and products of pieces with fp32 accumulation are exact to the rounding of the bfloat16 results.
+//                                        chunks, kept as prefix sums: the chunks before the window are one of them, those
+//                                        after it the sum over all chunks minus the one that ends with the window,
+//   an edge some pairs in the band    -- the pairs outside it one by one (two chunks at a window that is a multiple of 128,
+//                                        up to four otherwise).
+// The difference is taken in float32, so the chunks after the window carry 2^-24 of the sum over all chunks; the pairs of the
+// band enter no product and are not subtracted one by one.
+// What float32 would hold stays in that precision: far sums, df, low-rank weights, the gradients of the log-features and the
+// band's P and dS enter the products as three bf16 pieces (exactly), features as three with more than 128 of them, else as
+// two (2^-17, as in the kernels in sblocal_prep.hip).  Against float64 on the same output and log-normaliser, over 28 problems of
+// 4 to 32 heads, windows of 12 to 1024: 2-norm error of the bfloat16 gradients 1.5e-3 to 1.9e-3, the rounding of the results,
+// and 0.04 to 0.08 % of them rounded otherwise with 256 features (library products in float32: 0.03 to 0.2 %), 0.06 to 0.4 %
+// with fewer (the kernels in sblocal_prep.hip: 0.08 to 0.6 %).  Two pieces throughout took 1870 us a step instead of 2170 and
+// rounded 0.1 to 0.45 % otherwise with 256 features.
 //
 //   far_chunk_kernel    KV_c and QG_c summed over the chunks of a segment, every prefix of it kept, stabilised by the largest
 //                       log-feature so far
@@ -23,10 +32,10 @@
 //   local_bwd_b16_kernel<EXACT> (sblocal.hip)  the band, plus the low-rank part, rounded once
 //
 // Measured at B=1, H=16, L=16384, window 1024, 256 features, where the backward ran as library products over windows of
-// keys before (20.8 ms): chunks 187, scan 19, low-rank 310 (query-major) and 600 (key-major), band 200 and 290 us.  The
+// keys before (20.8 ms): chunks 211, scan 19, low-rank 357 (query-major) and 788 (key-major), band 235 and 352 us.  The
 // chunk sums (66 KB per 64 rows and side at 256 features) bound the first two: a scan over every chunk instead of every
-// segment moved 1.1 GB in 225 us.  The low-rank kernels wait: for the far sums (five trips to the cache, 140 and 190 us of the
-// two), and in the key-major one vector instructions on the edges' features and weights take as long as the products (230 us).
+// segment moved 1.1 GB in 225 us.  The low-rank kernels wait for the far sums (five trips to the cache), and the key-major one
+// spends most of its time on the edges: their features, the weights of their pairs and the pieces of both.
 #include "common.h"
 #include "local.h"
 #include <algorithm>
@@ -49,6 +58,8 @@ struct FarArgs {
 };
 
 constexpr float FAR_LOG2E = 1.4426950408889634f;
+// bf16 pieces a feature enters the products in (everything else but the bfloat16 tensors themselves: three)
+constexpr int far_pieces_of(int M) { return M > 128 ? 3 : 2; }
 
 // largest unit of the keys of a (batch, head) (base 2; 0 when no key is valid).  red: NW floats; ends with a barrier.
 template <int NT>
@@ -110,36 +121,26 @@ struct FarTile {
 // this wave's 16 rows of sqrt(t) log2e P in three bf16 pieces (exact): lane (r16, g) holds columns 32 ks + 8 g .. + 7 of row r16
 template <int KS>
 struct FarProj {
-    uintx4 h[KS], m[KS], l[KS];
+    Pieces p[KS];
     __device__ __forceinline__ void load(const float* proj, int row, int E, float scale, int g) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const float* src = proj + (long)row * E + 32 * ks + 8 * g;
-            split3(*reinterpret_cast<const floatx4*>(src) * scale, *reinterpret_cast<const floatx4*>(src + 4) * scale, h[ks], m[ks], l[ks]);
+            p[ks] = split<3>(*reinterpret_cast<const floatx4*>(src) * scale, *reinterpret_cast<const floatx4*>(src + 4) * scale);
         }
     }
     // rows of x . P^T: result rows = rows of x, columns (lane r16) = rows of P
     __device__ __forceinline__ floatx4 rows_by_features(const uint16_t* x0) const {
         floatx4 d = Frag<float>::zero();
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const uintx4 xf = *reinterpret_cast<const uintx4*>(x0 + 32 * ks);
-            d = mma_bf16(xf, l[ks], d);
-            d = mma_bf16(xf, m[ks], d);
-            d = mma_bf16(xf, h[ks], d);
-        }
+        for (int ks = 0; ks < KS; ++ks) d = mma_pieces(*reinterpret_cast<const uintx4*>(x0 + 32 * ks), p[ks], d);
         return d;
     }
     // the same transposed: result rows = rows of P, columns = rows of x
     __device__ __forceinline__ floatx4 features_by_rows(const uint16_t* x0) const {
         floatx4 d = Frag<float>::zero();
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const uintx4 xf = *reinterpret_cast<const uintx4*>(x0 + 32 * ks);
-            d = mma_bf16(l[ks], xf, d);
-            d = mma_bf16(m[ks], xf, d);
-            d = mma_bf16(h[ks], xf, d);
-        }
+        for (int ks = 0; ks < KS; ++ks) d = mma_pieces(p[ks], *reinterpret_cast<const uintx4*>(x0 + 32 * ks), d);
         return d;
     }
 };
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(2 * M) void far_chunk_kernel(FarArgs a) {
         }
 #pragma unroll
         for (int t2 = 0; t2 < 2; ++t2) {
-            uintx4 fh[2], fl[2];
+            PiecesOf<far_pieces_of(M)> fp[2];
 #pragma unroll
             for (int sg = 0; sg < 2; ++sg) {
                 floatx4 f[2];
@@ -261,17 +262,15 @@ __global__ __launch_bounds__(2 * M) void far_chunk_kernel(FarArgs a) {
                         tot[sg] += queries ? f[hb][i] * wr[i] : f[hb][i];
                     }
                 }
-                split2(f[0], f[1], fh[sg], fl[sg]);
+                fp[sg] = split<far_pieces_of(M)>(f[0], f[1]);
             }
 #pragma unroll
             for (int eb = 0; eb < EB; ++eb) {
                 const uint16_t* yq = Ys + (32 * t2 + 4 * g + (r16 >> 2)) * LD + 16 * eb + 4 * (r16 & 3);
                 const uintx4 yt = lds_read_tr8(reinterpret_cast<const char*>(yq), reinterpret_cast<const char*>(yq + 16 * LD));
 #pragma unroll
-                for (int sg = 0; sg < 2; ++sg) {
-                    acc[sg][eb] = mma_bf16(yt, fl[sg], acc[sg][eb]);     // (transposed: a lane's results are four columns of one feature)
-                    acc[sg][eb] = mma_bf16(yt, fh[sg], acc[sg][eb]);
-                }
+                for (int sg = 0; sg < 2; ++sg)                          // (transposed: a lane's results are four columns of one feature)
+                    acc[sg][eb] = mma_pieces(yt, fp[sg], acc[sg][eb]);
             }
         }
         float* dst = (queries ? a.qg : a.kv) + ((long)bh * n_c + c) * PER;
@@ -351,30 +350,37 @@ struct FarPrefix {
 // ---------------------------------------------------------------------------------------
 // 16 projection rows (32 features) per wave, all 64 outer rows: every feature of an edge chunk is formed once per
 // workgroup and goes from registers into the products.  Sums over features (chain rule, d v) are per wave until the end.
-// Key-major (730 -> 600 us at the size above) needs two operands transposed as well, the far sums and the edge features: it
-// takes them by transposing LDS reads of what it has, not by strided loads and a second evaluation.
+// Key-major needs two operands transposed as well, the far sums and the edge features: it takes them by transposing LDS reads
+// of what it has, not by strided loads and a second evaluation (730 -> 600 us at the size above with operands in two pieces;
+// 788 as they are now).  The pieces go through one buffer per wave in turn: side by side they would leave one workgroup per
+// compute unit at 128 features, and no room at 256 for the own features' smaller pieces, which do not fit the registers.
 // columns of the result reduced over the waves at a time: two 16-column blocks where that takes no more LDS
-template <int E, int M, bool KEYMAJOR>
+template <int M, bool KEYMAJOR>
 constexpr size_t far_reduce_cols() { return KEYMAJOR || M < 256 ? 32 : 16; }
 constexpr int FAR_LDT = 32 + 8;                                                     // row stride of the transposed features, key-major
-// bytes of the region that holds, one after the other, the wave's far rows (key-major), the inner chunk with df, the reduction
+// bytes of the region that holds, one after the other, the waves' far rows (key-major, one piece at a time), the inner chunk
+// with df and (key-major, one piece at a time) the waves' transposed features, the reduction
 template <int E, int M, bool KEYMAJOR>
 constexpr size_t far_lowrank_shared() {
-    size_t n = (size_t)2 * FC * (E + 8) * 2 + 2 * 8 * 64 * 16;
-    const size_t red = far_reduce_cols<E, M, KEYMAJOR>() * (M / 32) * FC * 4, rows = KEYMAJOR ? (size_t)(M / 32) * 2 * 32 * (E + 8) * 2 : 0;
+    size_t n = (size_t)2 * FC * (E + 8) * 2 + 3 * 8 * 64 * 16 + (KEYMAJOR ? (size_t)(M / 32) * 32 * FAR_LDT * 2 : 0);
+    const size_t red = far_reduce_cols<M, KEYMAJOR>() * (M / 32) * FC * 4, rows = KEYMAJOR ? (size_t)(M / 32) * 32 * (E + 8) * 2 : 0;
     if (n < red) n = red;
     return n < rows ? rows : n;
 }
+// key-major: the second and third pieces of the outer rows' features, where the registers do not hold them
+template <int M, bool KEYMAJOR>
+constexpr size_t far_own_pieces() { return KEYMAJOR && far_pieces_of(M) == 3 ? (size_t)(M / 32) * 2 * 4 * 64 * 16 : 0; }
 template <int E, int M, bool KEYMAJOR>
 constexpr size_t far_lowrank_smem() {
-    return (size_t)2 * FC * (E + 8) * 2 + far_lowrank_shared<E, M, KEYMAJOR>() + sizeof(float) * (6 * FC + (M / 32) * (FC + 1) + 3) / 16 * 16 +
-           (KEYMAJOR ? (size_t)(M / 32) * 2 * 32 * FAR_LDT * 2 : 0);
+    return (size_t)2 * FC * (E + 8) * 2 + far_lowrank_shared<E, M, KEYMAJOR>() + far_own_pieces<M, KEYMAJOR>() +
+           sizeof(float) * (6 * FC + (M / 32) * (FC + 1) + 3) / 16 * 16;
 }
 
 template <int E, int M, bool KEYMAJOR>
 __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR && M >= 256 ? 4 : 2, !KEYMAJOR && M >= 256 ? 8 : 2))) void far_lowrank_kernel(FarArgs a) {
     constexpr int NW = M / 32, NT = 64 * NW, MH = M / 2, KS = E / 32, EB = E / 16, LD = E + 8, PER = M * (E + 1);
     constexpr size_t TILES = (size_t)2 * FC * LD * 2;
+    constexpr int NF = far_pieces_of(M), NR = NF == 3 ? 1 : NF;                      // pieces of a feature; of the own ones, in registers
     extern __shared__ __attribute__((aligned(128))) char far_smem[];
     uint16_t* Xo = reinterpret_cast<uint16_t*>(far_smem);
     uint16_t* Yo = Xo + FC * LD;
@@ -382,14 +388,16 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
     uint16_t* Yi = Xi + FC * LD;
     uintx4* DF = reinterpret_cast<uintx4*>(Yi + FC * LD);                           // [piece][step, outer block][lane]
     float* red = reinterpret_cast<float*>(Xi);
-    float* diago = reinterpret_cast<float*>(far_smem + TILES + far_lowrank_shared<E, M, KEYMAJOR>());
+    char* after = far_smem + TILES + far_lowrank_shared<E, M, KEYMAJOR>();
+    float* diago = reinterpret_cast<float*>(after + far_own_pieces<M, KEYMAJOR>());
     float* exto = diago + FC; float* co = exto + FC;
     float* diagi = co + FC; float* exti = diagi + FC; float* ci = exti + FC;
     float* us = ci + FC;                                                            // [NW][FC]
     float* kred = us + NW * FC;                                                     // [NW]
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
-    // key-major: the wave's features of 32 inner rows, [piece][sign, 16 features][rows]
-    uint16_t* ft = reinterpret_cast<uint16_t*>(far_smem + far_lowrank_smem<E, M, KEYMAJOR>()) - (NW - w) * 2 * 32 * FAR_LDT;
+    uintx4* FO = reinterpret_cast<uintx4*>(after) + w * 2 * 4 * 64 + lane;          // [piece - 1][outer block][lane], see own_pieces
+    // key-major: one piece of the wave's features of 32 inner rows, [sign, 16 features][rows]
+    uint16_t* ft = reinterpret_cast<uint16_t*>(DF + 3 * 8 * 64) + w * 32 * FAR_LDT;
     const int Lo = KEYMAJOR ? a.S : a.T;
     const int n_oc = KEYMAJOR ? a.n_kc : a.n_qc, n_ic = KEYMAJOR ? a.n_qc : a.n_kc;
     const int n_items = a.B * a.H * n_oc;
@@ -440,14 +448,25 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
             f1[i] = ok ? __builtin_amdgcn_exp2f(bias - dd[i]) : 0.f;
         }
     };
-    // key-major: needed throughout, as two-piece operands, slots (sg, 4 g + i); query-major: formed where they are used
-    uintx4 foh[KEYMAJOR ? 4 : 1], fol[KEYMAJOR ? 4 : 1];
+    // key-major: needed throughout, as operands with slots (sg, 4 g + i); query-major: formed where they are used
+    PiecesOf<NR> fo[KEYMAJOR ? 4 : 1];
+    auto own_pieces = [&](int ob) __attribute__((always_inline)) {
+        PiecesOf<NF> r;
+#pragma unroll
+        for (int pc = 0; pc < NF; ++pc) r.p[pc] = pc < NR ? fo[KEYMAJOR ? ob : 0].p[pc < NR ? pc : 0] : FO[(4 * (pc - 1) + ob) * 64];
+        return r;
+    };
     if (KEYMAJOR) {
 #pragma unroll
         for (int ob = 0; ob < 4; ++ob) {
             floatx4 f0, f1;
             own_features(ob, f0, f1);
-            split2(f0, f1, foh[KEYMAJOR ? ob : 0], fol[KEYMAJOR ? ob : 0]);
+            const PiecesOf<NF> f = split<NF>(f0, f1);
+#pragma unroll
+            for (int pc = 0; pc < NF; ++pc) {
+                if (pc < NR) fo[KEYMAJOR ? ob : 0].p[pc < NR ? pc : 0] = f.p[pc];
+                else FO[(4 * (pc - 1) + ob) * 64] = f.p[pc];                        // (read back by the same lane only)
+            }
         }
     }
 
@@ -472,48 +491,57 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
         p1.add(fx, -1.f, at);
         p0.add(fx, 1.f, at);
     }
+    Pieces far[KEYMAJOR ? 2 * KS : 1];
     floatx4 acc2[2][4];                                                             // [sign][outer block], rows = features
-    uint16_t* fw = Xi + w * 2 * 32 * LD;                                            // key-major: the wave's far rows, [piece][sign, 16 features][E]
+    uint16_t* fw = Xi + w * 32 * LD;                                                // key-major: one piece of the wave's far rows, [sign, 16 features][E]
 #pragma unroll
     for (int sg = 0; sg < 2; ++sg) {
 #pragma unroll
         for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] = Frag<float>::zero();
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            uintx4 fh, fl;
-            split2(fx[sg * (2 * KS + 1) + 2 * ks], fx[sg * (2 * KS + 1) + 2 * ks + 1], fh, fl);
-            if (KEYMAJOR) {
-                uint16_t* d = fw + (16 * sg + r16) * LD + 32 * ks + 8 * g;
-                *reinterpret_cast<uintx4*>(d) = fh;
-                *reinterpret_cast<uintx4*>(d + 32 * LD) = fl;
-            }
+            const Pieces fp = split<3>(fx[sg * (2 * KS + 1) + 2 * ks], fx[sg * (2 * KS + 1) + 2 * ks + 1]);
+            if (KEYMAJOR) far[KEYMAJOR ? sg * KS + ks : 0] = fp;
 #pragma unroll
-            for (int ob = 0; ob < 4; ++ob) {
-                const uintx4 yo = *reinterpret_cast<const uintx4*>(Yo + (16 * ob + r16) * LD + 32 * ks + 8 * g);
-                acc2[sg][ob] = mma_bf16(fl, yo, acc2[sg][ob]);
-                acc2[sg][ob] = mma_bf16(fh, yo, acc2[sg][ob]);
-            }
+            for (int ob = 0; ob < 4; ++ob)
+                acc2[sg][ob] = mma_pieces(fp, *reinterpret_cast<const uintx4*>(Yo + (16 * ob + r16) * LD + 32 * ks + 8 * g), acc2[sg][ob]);
         }
 #pragma unroll
         for (int ob = 0; ob < 4; ++ob) acc2[sg][ob] -= fx[sg * (2 * KS + 1) + 2 * KS] * (KEYMAJOR ? 1.0f : co[16 * ob + r16]);
     }
     floatx4 acc3[KEYMAJOR ? EB : 1][KEYMAJOR ? 4 : 1];                              // d v: rows = value dims, columns = keys
     if (KEYMAJOR) {
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                          // (read by other lanes of the wave only)
-        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int eb = 0; eb < EB; ++eb) {
-            const uint16_t* q = fw + (4 * g + (r16 >> 2)) * LD + 16 * eb + 4 * (r16 & 3);
-            const uintx4 th = lds_read_tr8(reinterpret_cast<const char*>(q), reinterpret_cast<const char*>(q + 16 * LD));
-            const uintx4 tl = lds_read_tr8(reinterpret_cast<const char*>(q + 32 * LD), reinterpret_cast<const char*>(q + 48 * LD));
+        for (int eb = 0; eb < EB; ++eb)
+#pragma unroll
+            for (int ob = 0; ob < 4; ++ob) acc3[KEYMAJOR ? eb : 0][KEYMAJOR ? ob : 0] = Frag<float>::zero();
+#pragma unroll
+        for (int pc = 2; pc >= 0; --pc) {                                           // (small terms first)
+#pragma unroll
+            for (int n = 0; n < 2 * KS; ++n)
+                *reinterpret_cast<uintx4*>(fw + (16 * (n / KS) + r16) * LD + 32 * (n % KS) + 8 * g) = far[KEYMAJOR ? n : 0].p[pc];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                      // (read by other lanes of the wave only)
+            __builtin_amdgcn_wave_barrier();
+            uintx4 tp[EB];
+#pragma unroll
+            for (int eb = 0; eb < EB; ++eb) {
+                const uint16_t* q = fw + (4 * g + (r16 >> 2)) * LD + 16 * eb + 4 * (r16 & 3);
+                tp[eb] = lds_read_tr8(reinterpret_cast<const char*>(q), reinterpret_cast<const char*>(q + 16 * LD));
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int ob = 0; ob < 4; ++ob) {
-                floatx4 d = Frag<float>::zero();
-                d = mma_bf16(tl, foh[KEYMAJOR ? ob : 0], d);
-                d = mma_bf16(th, fol[KEYMAJOR ? ob : 0], d);
-                acc3[KEYMAJOR ? eb : 0][KEYMAJOR ? ob : 0] = mma_bf16(th, foh[KEYMAJOR ? ob : 0], d);
+                const PiecesOf<NF> f = own_pieces(ob);
+#pragma unroll
+                for (int eb = 0; eb < EB; ++eb) {
+                    floatx4& d = acc3[KEYMAJOR ? eb : 0][KEYMAJOR ? ob : 0];
+#pragma unroll
+                    for (int pf = NF - 1; pf >= 0; --pf)
+                        if (pc + pf <= 2) d = mma_bf16(tp[eb], f.p[pf], d);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();                                                            // the far rows lie where the inner chunk goes
     }
@@ -527,7 +555,7 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
         if (AHEAD && nx < c1) t.fetch(a, KEYMAJOR, xip, xis, yip, yis, bh, nx * FC, len_i, base, kappa, tid);
         __syncthreads();
         // df = g.v - c on the pairs outside the band, 0 inside: inner rows 32 st + 16 hb + 4 g + i, outer row 16 ob + r16 --
-        // eight contraction slots of the products below -- in two pieces
+        // eight contraction slots of the products below -- in pieces
         for (int it = w; it < 8; it += NW) {
             const int st = it >> 2, ob = it & 3;
             floatx4 s[2] = {Frag<float>::zero(), Frag<float>::zero()};
@@ -548,17 +576,15 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
                     s[hb][i] = (unsigned)(rel + A) < (unsigned)(A + Bq) ? 0.f : s[hb][i] - (KEYMAJOR ? cq[i] : co[16 * ob + r16]);
                 }
             }
-            uintx4 hi, lo;
-            split2(s[0], s[1], hi, lo);
-            DF[it * 64 + lane] = hi;
-            DF[(8 + it) * 64 + lane] = lo;
+            const Pieces df = split<3>(s[0], s[1]);
+#pragma unroll
+            for (int pc = 0; pc < 3; ++pc) DF[(8 * pc + it) * 64 + lane] = df.p[pc];
         }
         __syncthreads();
         // acc2^T[feature][outer] += F^T[feature][inner] df[inner][outer]
         const bool fvalid = 16 * w + r16 < a.mh_valid;
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
-            uintx4 fh[2], fl[2];
             floatx4 f0[2], f1[2];
 #pragma unroll
             for (int hb = 0; hb < 2; ++hb) {
@@ -571,67 +597,59 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
                     f1[hb][i] = fvalid ? __builtin_amdgcn_exp2f(bias[i] - dd[i]) : 0.f;
                 }
             }
-            split2(f0[0], f0[1], fh[0], fl[0]);
-            split2(f1[0], f1[1], fh[1], fl[1]);
-            if (KEYMAJOR) {
-#pragma unroll
-                for (int sg = 0; sg < 2; ++sg)
-#pragma unroll
-                    for (int hb = 0; hb < 2; ++hb) {
-                        uint16_t* d = ft + (16 * sg + r16) * FAR_LDT + 16 * hb + 4 * g;
-                        *reinterpret_cast<uint2*>(d) = make_uint2(fh[sg][2 * hb], fh[sg][2 * hb + 1]);
-                        *reinterpret_cast<uint2*>(d + 32 * FAR_LDT) = make_uint2(fl[sg][2 * hb], fl[sg][2 * hb + 1]);
-                    }
-            }
+            const PiecesOf<NF> fp[2] = {split<NF>(f0[0], f0[1]), split<NF>(f1[0], f1[1])};
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int ob = 0; ob < 4; ++ob) {
-                const uintx4 dh = DF[(4 * st + ob) * 64 + lane], dl = DF[(8 + 4 * st + ob) * 64 + lane];
+                const Pieces df = {{DF[(4 * st + ob) * 64 + lane], DF[(8 + 4 * st + ob) * 64 + lane], DF[(16 + 4 * st + ob) * 64 + lane]}};
 #pragma unroll
-                for (int sg = 0; sg < 2; ++sg) {
-                    acc2[sg][ob] = mma_bf16(fl[sg], dh, acc2[sg][ob]);
-                    acc2[sg][ob] = mma_bf16(fh[sg], dl, acc2[sg][ob]);
-                    acc2[sg][ob] = mma_bf16(fh[sg], dh, acc2[sg][ob]);
-                }
+                for (int sg = 0; sg < 2; ++sg) acc2[sg][ob] = mma_pieces(fp[sg], df, acc2[sg][ob]);
             }
             if (KEYMAJOR) {
                 // this wave's features of the low-rank weights outside the band: result rows = queries, columns = keys; then
-                // d v^T[d][key] += g^T[d][query] W[query][key].  The operand is the one above transposed
-                uintx4 wh[2], wl[2];
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // (read by other lanes of the wave only)
-                __builtin_amdgcn_wave_barrier();
+                // d v^T[d][key] += g^T[d][query] W[query][key].  The operand is the one above transposed, one piece at a time
+                // through the wave's rows in LDS
+                PiecesOf<NF> wp[2];
 #pragma unroll
-                for (int hb = 0; hb < 2; ++hb) {
-                    const uint16_t* q = ft + (4 * g + (r16 >> 2)) * FAR_LDT + 16 * hb + 4 * (r16 & 3);
-                    wh[hb] = lds_read_tr8(reinterpret_cast<const char*>(q), reinterpret_cast<const char*>(q + 16 * FAR_LDT));
-                    wl[hb] = lds_read_tr8(reinterpret_cast<const char*>(q + 32 * FAR_LDT), reinterpret_cast<const char*>(q + 48 * FAR_LDT));
+                for (int pc = 0; pc < NF; ++pc) {
+#pragma unroll
+                    for (int sg = 0; sg < 2; ++sg) {
+                        const uintx4 f = fp[sg].p[pc];
+#pragma unroll
+                        for (int hb = 0; hb < 2; ++hb)
+                            *reinterpret_cast<uint2*>(ft + (16 * sg + r16) * FAR_LDT + 16 * hb + 4 * g) = make_uint2(f[2 * hb], f[2 * hb + 1]);
+                    }
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");              // (read by other lanes of the wave only)
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int hb = 0; hb < 2; ++hb) {
+                        const uint16_t* q = ft + (4 * g + (r16 >> 2)) * FAR_LDT + 16 * hb + 4 * (r16 & 3);
+                        wp[hb].p[pc] = lds_read_tr8(reinterpret_cast<const char*>(q), reinterpret_cast<const char*>(q + 16 * FAR_LDT));
+                    }
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    __builtin_amdgcn_wave_barrier();
                 }
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_sched_barrier(0);          // (the steps' operands do not fit the registers side by side)
 #pragma unroll
                 for (int ob = 0; ob < 4; ++ob) {
                     floatx4 wt[2];
+                    const PiecesOf<NF> own = own_pieces(ob);
 #pragma unroll
                     for (int hb = 0; hb < 2; ++hb) {
-                        wt[hb] = Frag<float>::zero();
-                        wt[hb] = mma_bf16(wl[hb], foh[KEYMAJOR ? ob : 0], wt[hb]);
-                        wt[hb] = mma_bf16(wh[hb], fol[KEYMAJOR ? ob : 0], wt[hb]);
-                        wt[hb] = mma_bf16(wh[hb], foh[KEYMAJOR ? ob : 0], wt[hb]);
+                        wt[hb] = mma_pieces(wp[hb], own, Frag<float>::zero());
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const int rel = n0 + 32 * st + 16 * hb + 4 * g + i - (o0 + 16 * ob + r16);
                             if ((unsigned)(rel + A) < (unsigned)(A + Bq)) wt[hb][i] = 0.f;
                         }
                     }
-                    uintx4 bh_, bl_;
-                    split2(wt[0], wt[1], bh_, bl_);
+                    const Pieces wpc = split<3>(wt[0], wt[1]);
 #pragma unroll
                     for (int eb = 0; eb < EB; ++eb) {
                         const uint16_t* yq = Yi + (32 * st + 4 * g + (r16 >> 2)) * LD + 16 * eb + 4 * (r16 & 3);
                         const uintx4 yt = lds_read_tr8(reinterpret_cast<const char*>(yq), reinterpret_cast<const char*>(yq + 16 * LD));
                         floatx4& d = acc3[KEYMAJOR ? eb : 0][KEYMAJOR ? ob : 0];
-                        d = mma_bf16(yt, bl_, d);
-                        d = mma_bf16(yt, bh_, d);
+                        d = mma_pieces(yt, wpc, d);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -654,12 +672,18 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
     for (int ob = 0; ob < 4; ++ob) {
         floatx4 f0, f1;
         if (KEYMAJOR) {
-            const uintx4 xh = foh[KEYMAJOR ? ob : 0], xl = fol[KEYMAJOR ? ob : 0];
+            const PiecesOf<NF> x = own_pieces(ob);
+            auto slot = [](uint32_t w, int odd) __attribute__((always_inline)) { return __uint_as_float(odd ? w & 0xffff0000u : w << 16); };
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const uint32_t h0 = xh[i >> 1], l0 = xl[i >> 1], h1 = xh[2 + (i >> 1)], l1 = xl[2 + (i >> 1)];
-                f0[i] = (i & 1) ? __uint_as_float(h0 & 0xffff0000u) + __uint_as_float(l0 & 0xffff0000u) : __uint_as_float(h0 << 16) + __uint_as_float(l0 << 16);
-                f1[i] = (i & 1) ? __uint_as_float(h1 & 0xffff0000u) + __uint_as_float(l1 & 0xffff0000u) : __uint_as_float(h1 << 16) + __uint_as_float(l1 << 16);
+                const int n = i >> 1, odd = i & 1;
+                f0[i] = slot(x.p[NF - 1][n], odd);
+                f1[i] = slot(x.p[NF - 1][2 + n], odd);
+#pragma unroll
+                for (int pc = NF - 2; pc >= 0; --pc) {                               // (exact)
+                    f0[i] += slot(x.p[pc][n], odd);
+                    f1[i] += slot(x.p[pc][2 + n], odd);
+                }
             }
         } else own_features(ob, f0, f1);
         const floatx4 up = f0 * acc2[0][ob], un = f1 * acc2[1][ob];
@@ -671,15 +695,16 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
         du[ob] = up - un;
     }
     // the wave's 16 rows of P as one 32-slot step: slots (0, 4 g + i) and (1, 4 g + i) carry different piece products
-    uintx4 bo[4][2];
+    uintx4 bo[4][3];
 #pragma unroll
     for (int ob = 0; ob < 4; ++ob) {
-        uint2 dh, dl;
-        split2_4(du[ob], dh, dl);
+        uint2 dh, dm, dl;
+        split3_4(du[ob], dh, dm, dl);
         bo[ob][0] = uintx4{dh.x, dh.y, dh.x, dh.y};
-        bo[ob][1] = uintx4{dl.x, dl.y, dh.x, dh.y};
+        bo[ob][1] = uintx4{dm.x, dm.y, dm.x, dm.y};
+        bo[ob][2] = uintx4{dl.x, dl.y, dh.x, dh.y};
     }
-    constexpr int RC = far_reduce_cols<E, M, KEYMAJOR>(), RB = RC / 16;             // columns and 16-column blocks at a time
+    constexpr int RC = far_reduce_cols<M, KEYMAJOR>(), RB = RC / 16;             // columns and 16-column blocks at a time
     constexpr int QUADS = FC * RC / 4;                                              // groups of four columns, per 64 rows
 #pragma unroll
     for (int pass = 0; pass < (KEYMAJOR ? 2 : 1); ++pass)
@@ -694,7 +719,7 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
                 split3_4(pv[eb], ph, pm, pl);
                 const uintx4 a0 = {ph.x, ph.y, pm.x, pm.y}, a1 = {ph.x, ph.y, pl.x, pl.y};
 #pragma unroll
-                for (int ob = 0; ob < 4; ++ob) d[ob] = mma_bf16(a0, bo[ob][0], mma_bf16(a1, bo[ob][1], Frag<float>::zero()));
+                for (int ob = 0; ob < 4; ++ob) d[ob] = mma_bf16(a0, bo[ob][0], mma_bf16(a0, bo[ob][1], mma_bf16(a1, bo[ob][2], Frag<float>::zero())));
             } else {
 #pragma unroll
                 for (int ob = 0; ob < 4; ++ob) d[ob] = acc3[KEYMAJOR ? eb : 0][KEYMAJOR ? ob : 0];
