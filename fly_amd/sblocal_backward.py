@@ -266,7 +266,7 @@ def _backward_far(query, key, value, P, local_context, t, key_lengths, out, log_
         if x.shape[-1] != dim:
             x = torch.nn.functional.pad(x, (0, dim - x.shape[-1]))
         return rows_for_vectors(x, 8)
-    q, k, v, o, g = prep(query), prep(key), prep(value), prep(out), prep(grad_out.to(query.dtype))
+    q, k, v, o, g = prep(query), prep(key), prep(value), prep(out), prep(grad_out)
     mh = P.shape[0]
     proj = rows_for_vectors(P) if P.shape == (mk // 2, dim) else _fit(torch.nn.functional.pad(P, (0, 0, 0, mk // 2 - mh)), dim)
     ln = log_norm.reshape(B, H, T).float().contiguous()
@@ -403,8 +403,9 @@ def sblocal_backward(query, key, value, projection_matrix, local_context, softma
     B, T, H, E = query.shape
     S, D = key.shape[1], value.shape[3]
     t = softmax_temp or 1 / math.sqrt(E)
+    # (a gradient of another dtype, float32 say, is not rounded to bfloat16 but widened with the rest)
     if (query.dtype == torch.bfloat16 and query.is_cuda and band_kernel is None and support is None and dropout[0] == 0
-            and key.dtype == value.dtype == out.dtype == query.dtype):
+            and key.dtype == value.dtype == out.dtype == grad_out.dtype == query.dtype):
         far_dims = _far_kernel_dims(E, D, 2 * projection_matrix.shape[0])
         if far_dims is not None and _far_pays(B * H * max(T, S), local_context, far_dims[1]):
             return _backward_far(query, key, value, projection_matrix.float(), local_context, t, key_lengths, out,

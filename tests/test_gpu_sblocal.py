@@ -1091,6 +1091,24 @@ def test_bf16_gradients_with_256_features_keep_float32_precision(window, padded)
         assert share <= 1.5e-3, (name, share)
 
 
+@pytest.mark.parametrize('mh', [32, 128])
+def test_float32_gradient_of_a_bfloat16_output_is_not_rounded(mh):
+    """sblocal_backward with a float32 grad_out for bfloat16 tensors: its low bits reach the gradients.  An output gradient
+    rounded to bfloat16 first would change a third of the results; kept, only roundings at a tie differ (2^-17 operands: 1 %)."""
+    from fly_amd import sblocal_backward, sblocal_forward
+    dev = torch.device('cuda:0')
+    B, L, H, E, lc = 1, 300, 2, 64, 64
+    q, k, v, P = make_inputs(B, L, L, H, E, E, mh, seed=6, dtype=torch.bfloat16)
+    w = torch.randn(B, L, H, E, generator=torch.Generator().manual_seed(7))
+    out, ln = sblocal_forward(q.to(dev), k.to(dev), v.to(dev), P.to(dev), lc)
+    got = sblocal_backward(q.to(dev), k.to(dev), v.to(dev), P.to(dev), lc, None, None, out, ln, w.to(dev))
+    ref = sblocal_backward(q.double(), k.double(), v.double(), P.double(), lc, None, None, out.cpu().double(), ln.cpu().double(), w.double())
+    for name, a, r in zip(('dq', 'dk', 'dv'), got, ref):
+        assert a.dtype == torch.bfloat16
+        share = float((a.cpu() != r.bfloat16()).double().mean())
+        assert share <= 1e-2, (name, share)
+
+
 def _in_layout(x, layout):
     """`x` with the same values in memory a caller may hand over: 'offset' contiguous but three elements off an aligned
     start, 'odd-batch' a single batch entry whose batch stride is odd, 'heads-first' (B, H, L, E) in memory, 'fused' a third
