@@ -242,14 +242,38 @@ def _far_kernel_dims(E, D, M):
     return None
 
 
-def _far_pays(rows, local_context, M):
+def _far_pays(rows, heads, local_context, dims):
     """Whether bfloat16 tensors go to _backward_far where the kernels that subtract the band from the sums over all keys
-    (_backward_hip, on widened copies) could take them too.  Their M-wide products on every pair of the band cost in
-    proportion to the window, the chunk sums of the far path per row.  Training steps in us, far against subtracting: 200704
-    rows, 128 features 758 / 1065 at window 256, 749 / 860 at 49, 737 / 859 at 12; 64 features 674 / 647 at 49; 32 features
-    796 / 604 at 49; 131072 rows, 64 features 420 / 577 at window 128; 262144 rows, 128 features 1317 / 2682 at window 1024,
-    948 / 1247 at 64.  Small problems, where launches and the copies count: 73 against 134 us at 8000 rows, window 100."""
-    return M >= 128 or local_context >= 96 or rows <= 16384
+    (_backward_hip, on widened copies) could take them too; rows = batch x heads x the longer sequence, dims = the padded
+    (head dim, features).  The subtracting kernels form M-wide products on every pair of the band, in proportion to the window,
+    and several heads cost them a permuting copy of every tensor.  The far path costs the chunk sums, two edge chunks per 64
+    rows where the window is a multiple of 128 and up to four otherwise, and a fixed share per wave that does not shrink with
+    the features.  us, far / subtracting (windows 12, 96 or 97, 128, 200, 300, 512, 600 unless given):
+      (64, 128)  one head, 8000 rows: 96/98, 95/97, -, 110/105, 116/106, -, 126/118; 16384: 100/114 .. 131/164;
+                 200704: 677/738, 680/793, 617/796, 774/913, 798/975, 717/1172, 865/1281
+      (64, 64)   one head, 8000: 93/106, 93/105, -, 110/106, 116/105, -, 126/108; 50176: 203/163, 205/181, 181/181, -, -,
+                 209/293; 100352: 342/304, 346/332, -, 403/383, 413/409, -, 438/529; eight heads, 65536: 226/244 .. 242/365
+      (64, 32)   one head, 8000: 108/112, 108/145, -, 129/112, 136/110, -, 147/135; 50176: 231/147, 232/163, 199/163, -, -,
+                 228/242; 100352: 396/272, 397/295, -, 462/343, 478/364, -, 476/475; eight heads, 8000: 110/138 .. 110/127;
+                 65536: 245/223, 244/240, 212/244; twelve, 120000: 466/417, 464/452, -, 554/502, 577/533, -, 630/677
+      (32, 64)   one head, 16384: 72/104 .. 97/105; 100352: 197/180, 202/202, -, 231/243, 238/266, -, 267/362; 31360: 94/99,
+                 95/99, -, 112/106, 118/106, -, 130/140; twelve heads, 120000: 265/288 .. 365/515
+      (32, 32)   one head, 16384: 80/103 .. 109/103; 100352: 213/153, 215/173, -, 247/212, 254/226, -, 277/307; 200704: 354/296,
+                 356/331, 298/332; eight heads, 32768: 89/121 .. 125/147; twelve, 120000: 283/253, 283/274, -, 339/320,
+                 357/343, -, 392/451."""
+    dim, m = dims
+    whole = local_context % 128 == 0
+    few_edges = whole or local_context < 192
+    if m > 64:
+        return m > 128 or rows > 8192 or heads > 1 or few_edges             # (above 128 features there is no other kernel)
+    if heads > 1:
+        if m == 64 or rows <= (49152 if dim == 32 else 16384):
+            return True
+    elif rows <= 16384 and (dim == 32 or (m == 64 and few_edges)):
+        return True
+    if heads == 1 and (dim, m) == (64, 32):
+        return local_context >= (512 if whole else 768)
+    return local_context >= (128 if whole else 512)
 
 
 def _backward_far(query, key, value, P, local_context, t, key_lengths, out, log_norm, grad_out, dims):
@@ -407,7 +431,7 @@ def sblocal_backward(query, key, value, projection_matrix, local_context, softma
     if (query.dtype == torch.bfloat16 and query.is_cuda and band_kernel is None and support is None and dropout[0] == 0
             and key.dtype == value.dtype == out.dtype == grad_out.dtype == query.dtype):
         far_dims = _far_kernel_dims(E, D, 2 * projection_matrix.shape[0])
-        if far_dims is not None and _far_pays(B * H * max(T, S), local_context, far_dims[1]):
+        if far_dims is not None and _far_pays(B * H * max(T, S), H, local_context, far_dims):
             return _backward_far(query, key, value, projection_matrix.float(), local_context, t, key_lengths, out,
                                  log_normalization, grad_out, far_dims)
     wdt = torch.float64 if query.dtype == torch.float64 else torch.float32

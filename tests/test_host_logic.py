@@ -396,3 +396,25 @@ def test_rows_for_vectors_copies_whatever_a_vector_load_cannot_read(dtype, unit)
         got = rows_for_vectors(x, unit)
         assert got is not x and torch.equal(got, x) and got.data_ptr() % 16 == 0
         assert got.stride(-1) == 1 and all(s % unit == 0 for s in got.stride()[:-1])
+
+
+def test_route_of_the_bfloat16_scatterbrain_gradients():
+    """Which (head dim, features) the chunk-sum kernels are built for, and on which side of the rule the measured sizes fall;
+    without another kernel for the features it is always taken."""
+    import importlib
+    sbb = importlib.import_module('fly_amd.sblocal_backward')
+    assert sbb._far_kernel_dims(64, 64, 256) == (64, 256) and sbb._far_kernel_dims(48, 64, 130) == (64, 256)
+    assert sbb._far_kernel_dims(32, 20, 6) == (32, 32) and sbb._far_kernel_dims(32, 32, 66) == (64, 128)
+    assert sbb._far_kernel_dims(65, 64, 64) is None and sbb._far_kernel_dims(64, 64, 258) is None
+    for E in (8, 32, 33, 64):
+        for M in range(2, 258, 2):
+            dim, m = sbb._far_kernel_dims(E, E, M)
+            assert E <= dim and M <= m
+            if sbb._band_kernel_dims(E, E, M) is None:
+                assert all(sbb._far_pays(rows, heads, w, (dim, m)) for rows in (1, 10 ** 5) for heads in (1, 2) for w in (1, 200, 9999))
+    far = lambda rows, heads, w, *dims: sbb._far_pays(rows, heads, w, dims)
+    assert far(200704, 1, 12, 64, 128) and far(8000, 1, 97, 64, 128) and not far(8000, 1, 300, 64, 128)
+    assert far(8000, 1, 97, 64, 64) and not far(50176, 1, 96, 64, 64) and far(50176, 1, 256, 64, 64) and far(65536, 8, 12, 64, 64)
+    assert not far(8000, 1, 300, 64, 32) and far(50176, 1, 512, 64, 32) and not far(100352, 1, 600, 64, 32) and far(65536, 8, 128, 64, 32)
+    assert far(16384, 1, 12, 32, 64) and not far(100352, 1, 12, 32, 64) and far(100352, 1, 600, 32, 64)
+    assert far(32768, 8, 12, 32, 32) and not far(120000, 12, 300, 32, 32) and far(120000, 12, 600, 32, 32)
