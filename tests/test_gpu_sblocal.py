@@ -370,8 +370,8 @@ def test_module_keeps_its_scratch_between_calls():
 ], ids=['square', 'odd-sizes-lengths', 'rows-without-keys', 'bf16', 'bf16-odd-sizes-lengths', 'bf16-rows-without-keys',
         'bf16-long-band', 'fp16', 'fp16-long-band'])
 def test_local_attention_matches_oracle(case):
-    """LocalAttention (local_attention.py:50-92) through flyhip_local_fwd against the oracle: float32 on the fp32 matrix
-    pipe, 2-byte inputs on the 16x16x32 MFMA of their type (64-key tiles; tiles inside every query's band skip the masks:
+    """LocalAttention (local_attention.py:50-92) through flyhip_local_fwd against the oracle: float32 on the bf16 matrix
+    pipe from three pieces per operand, 2-byte inputs on the 16x16x32 MFMA of their type (64-key tiles; tiles inside every query's band skip the masks:
     the long-band cases have them)."""
     from fly_amd import LocalAttention, LengthMask
     c = dict(case)
@@ -619,7 +619,7 @@ def test_local_attention_gradients_on_the_2byte_kernels(case):
 @pytest.mark.parametrize('dtype,tol,E,p_drop', [(torch.float32, 1e-4, 64, 0.25), (torch.bfloat16, 3e-2, 64, 0.1),
                                                  (torch.float32, 1e-4, 24, 0.5)])
 def test_local_attention_dropout_inside_the_kernels(dtype, tol, E, p_drop):
-    """Training-mode dropout of LocalAttention (local_attention.py:91) inside the forward kernel and both band kernels
+    """Training-mode dropout of LocalAttention (local_attention.py:91) inside the forward kernel and both kernels
     of the backward: the mask is the hash of (seed, batch, head, query, key) restated in oracle.sblocal.dropout_keep, so
     output and gradients are compared with float64 autograd through band softmax -> mask / (1 - p) -> product on the
     kernels' own mask -- T != S, key lengths (queries without a visible key), a head dim that needs padding.  The
@@ -669,7 +669,7 @@ def test_local_attention_dropout_inside_the_kernels(dtype, tol, E, p_drop):
                                                 (torch.bfloat16, 3e-2, 64, 0.6)])
 def test_local_attention_with_attn_mask(dtype, tol, E, p_keep):
     """LocalAttention with an attn_mask (local_attention.py:53-56, 68-81): its additive matrix (0 / -1e24) is added
-    inside the forward kernel and both band kernels of the backward.  Output, gradients and need_weights against the
+    inside the forward kernel and both kernels of the backward.  Output, gradients and need_weights against the
     oracle in float64 (autograd through it for the gradients): a random FullMask with queries whose visible keys are
     all hidden (equal weights 1 / local_context there, as the reference's packed softmax gives), T != S, key lengths,
     a head dim that needs padding; then a mask that hides nothing (bit-identical to no mask)."""
@@ -1009,13 +1009,15 @@ def test_attention_dropout_module_and_refusals():
     dict(B=1, T=65, S=129, H=1, E=32, mh=16, lc=1, lens=None, scale=0.4),              # one key a query
     dict(B=1, T=1000, S=1000, H=2, E=64, mh=100, lc=333, lens=[1000], scale=0.35),     # projection rows that are padding
     dict(B=3, T=90, S=1000, H=1, E=64, mh=3, lc=40, lens=[1000, 1, 500], scale=0.4),
+    dict(B=3, T=140, S=200, H=3, E=64, mh=128, lc=64, lens=[200, 70, 131], scale=0.35),   # ragged slices of heads and of the batch
     dict(B=16, T=323, S=270, H=8, E=64, mh=128, lc=90, lens=[270, 1, 65, 140] * 4, scale=0.35, slices=False),   # segments of 4 chunks, 2 left over
     dict(B=20, T=200, S=330, H=8, E=64, mh=100, lc=64, lens=None, scale=1.0, slices=False),                     # rescaled inside a segment
 ], ids=lambda c: f"T{c['T']}-S{c['S']}-E{c['E']}-mh{c['mh']}-lc{c['lc']}")
 def test_bf16_gradients_through_chunk_sums(case, monkeypatch):
     """flyhip_sblocal_bwd_far (far pairs through prefix sums over chunks, edge chunks pair by pair, the band on the local
     attention kernels) against autograd through the oracle in float64 on the same bfloat16 inputs; the same numbers when
-    the problem goes through in slices of one (batch, head).  Bar (2-norm): the gradients are rounded to bfloat16 (2^-9), and
+    the problem goes through in slices: of one (batch, head), of some of the heads, of some of the batch entries, the last
+    slice smaller where they do not divide.  Bar (2-norm): the gradients are rounded to bfloat16 (2^-9), and
     so is the forward's output inside g.out, which d query and d key see once more where g.v - g.out cancels."""
     import importlib
     from fly_amd import sblocal_attention_fn
@@ -1028,9 +1030,21 @@ def test_bf16_gradients_through_chunk_sums(case, monkeypatch):
     lens = None if case['lens'] is None else torch.tensor(case['lens'])
     dev = torch.device('cuda:0')
     monkeypatch.setattr(sbb, '_far_pays', lambda *a: True)
+    far, launches = sbb._backward_far, []
+
+    def counted(*args):
+        from fly_amd import _lib
+        call, names = _lib.call, []
+        with pytest.MonkeyPatch.context() as m:
+            m.setattr(_lib, 'call', lambda name, *a: (names.append(name), call(name, *a)))
+            res = far(*args)
+        launches.append(names.count('flyhip_sblocal_bwd_far'))
+        return res
+    monkeypatch.setattr(sbb, '_backward_far', counted)
     qg, kg, vg = (x.to(dev).requires_grad_() for x in (q, k, v))
     out, _ = sblocal_attention_fn(qg, kg, vg, P.to(dev), lc, None, None if lens is None else lens.to(dev))
     got = torch.autograd.grad(out, (qg, kg, vg), w.to(dev), retain_graph=True)
+    assert launches == [1]
     qd, kd, vd = (x.double().requires_grad_() for x in (q, k, v))
     ref_out, _ = osb.sblocal_attention(qd, kd, vd, P.double(), lc, key_lengths=lens)
     ref = torch.autograd.grad(ref_out, (qd, kd, vd), w.double())
@@ -1039,9 +1053,13 @@ def test_bf16_gradients_through_chunk_sums(case, monkeypatch):
         assert a.dtype == torch.bfloat16 and err <= 6e-3, err
     if not case.get('slices', True):             # (slices of a large problem are summed in shorter segments: other roundings)
         return
-    monkeypatch.setattr(sbb, '_FAR_WORKSPACE_FLOATS', 1)
-    for a, b in zip(got, torch.autograd.grad(out, (qg, kg, vg), w.to(dev))):
-        assert torch.equal(a, b)
+    from fly_amd import _lib
+    dims = sbb._far_kernel_dims(E, E, 2 * mh)
+    for pairs in sorted({1, 2, 2 * H, B * H - 1} - {0}):
+        monkeypatch.setattr(sbb, '_FAR_WORKSPACE_FLOATS', pairs * _lib.load().flyhip_sblocal_bwd_far_floats(1, T, S, *dims))
+        for a, b in zip(got, torch.autograd.grad(out, (qg, kg, vg), w.to(dev), retain_graph=True)):
+            assert torch.equal(a, b)
+        assert launches[-1] == (-(-B // min(B, pairs // H)) if pairs >= H else B * -(-H // pairs))
 
 
 @pytest.mark.parametrize('B,T,S,H,E,D,lc,lens', [
@@ -1066,6 +1084,33 @@ def test_local_attention_float32_on_bf16_pieces(B, T, S, H, E, D, lc, lens):
     for a, r in zip((out,) + got, (ref_out,) + ref):
         scale = max(float(r.detach().norm()), 1e-2 * r.numel() ** 0.5)      # (d query is zero where every query sees one key)
         assert float((a.detach().double().cpu() - r.detach()).norm()) <= 2e-6 * scale
+
+
+@pytest.mark.parametrize('where', ['inside', 'before'])
+def test_bf16_gradients_of_rows_whose_far_keys_are_small(where):
+    """The far keys after a query's window are the sum over all keys minus the one that ends with the window.  Keys inside
+    or before the window with a feature e^8 to e^11 times that of any key after it dominate the total; the difference carries
+    2^-24 of it, 2^-24 e^11 = 3.6e-3 of what remains in one feature of 256.  Every row's d query and every key's gradients
+    against float64, row by row: 2^-9 of the row for the rounding of the results (2-norm), and 2^-8 for the rest."""
+    from fly_amd import sblocal_backward, sblocal_forward
+    dev = torch.device('cuda:0')
+    B, L, H, E, mh, lc = 1, 1000, 1, 64, 128, 128
+    q, k, v, P = make_inputs(B, L, L, H, E, E, mh, seed=12, scale=0.5)
+    k[:] *= 0.1
+    u = torch.nn.functional.normalize(P[5], dim=-1)                  # along one projection row: its features stand out
+    loud = slice(420, 470) if where == 'inside' else slice(0, 64)
+    k[:, loud] = 3.5 * u
+    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    w = torch.randn(B, L, H, E, generator=torch.Generator().manual_seed(13)).bfloat16()
+    out, ln = sblocal_forward(q.to(dev), k.to(dev), v.to(dev), P.to(dev), lc)
+    got = sblocal_backward(q.to(dev), k.to(dev), v.to(dev), P.to(dev), lc, None, None, out, ln, w.to(dev))
+    ref = sblocal_backward(q.double(), k.double(), v.double(), P.double(), lc, None, None, out.cpu().double(), ln.cpu().double(), w.double())
+    logf = (k[0, :, 0].double() @ P.double().t() * E ** -0.25).abs().amax(-1) - k[0, :, 0].double().square().sum(-1) * E ** -0.5 / 2
+    assert 8 < float(logf[loud].max() - logf[600:].max()) < 11
+    for name, a, r in zip(('dq', 'dk', 'dv'), got, ref):
+        err = (a.cpu().double() - r).norm(dim=-1) / r.norm(dim=-1)
+        print(name, float(err.max()))
+        assert float(err.max()) <= 2 ** -9 + 2 ** -8, (name, float(err.max()), int(err.argmax()))
 
 
 @pytest.mark.parametrize('window,padded', [(200, False), (512, False), (37, True)])
