@@ -13,7 +13,7 @@
 // The pieces are formed where a tile is staged into LDS (float rows in memory, piece rows in LDS): a preparation pass would
 // write and read 1.5 times the inputs again, and the passes are within a small factor of the memory they touch.
 //
-// A wave owns 16 QB outer rows (queries; keys when KEYMAJOR) with their operands in registers as pieces and walks 32-row
+// A wave owns 16 outer rows (queries; keys when KEYMAJOR) with their operands in registers as pieces and walks 32-row
 // tiles of the other side -- short tiles, so that a wave skips what lies outside its own rows' bands.  Products are
 // formed transposed (rows = inner, columns = outer): a lane's eight weights of a tile are the contraction slots
 // {4 g + i, 16 + 4 g + i} of the second product, whose other operand comes by transposing LDS reads of the same rows.
@@ -72,10 +72,10 @@ __device__ __forceinline__ Pieces lx_load(const float* p) {
     return split<3>(*reinterpret_cast<const floatx4*>(p), *reinterpret_cast<const floatx4*>(p + 4));
 }
 
-template <int E, int QB = 1>
+template <int E>
 __global__ __launch_bounds__(LX_NT) void local_fwd_x3_kernel(LocalArgs a) {
     using PT = PieceTile<E>;
-    constexpr int KS = E / 32, DB = E / 16, STAGE = 2 * PT::BYTES, QW = 16 * QB, TQB = 4 * QW;
+    constexpr int KS = E / 32, DB = E / 16, STAGE = 2 * PT::BYTES, TQB = 64;
     extern __shared__ __attribute__((aligned(128))) char lx_smem[];
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
     const int n_qt = (a.T + TQB - 1) / TQB;
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(LX_NT) void local_fwd_x3_kernel(LocalArgs a) {
     const int item = (blockIdx.x % a.n_xcd) * per_xcd + blockIdx.x / a.n_xcd;      // neighbouring tiles share a die's L2
     if (item >= n_items) return;                                                    // workgroup-uniform
     const int qt = item % n_qt, bh = item / n_qt, b = bh / a.H, h = bh % a.H;
-    const int q0 = qt * TQB, qw0 = q0 + QW * w;
+    const int q0 = qt * TQB, qw0 = q0 + 16 * w;
     const float* qptr = reinterpret_cast<const float*>(a.q) + b * a.q_sb + h * a.q_sh;
     const float* kptr = reinterpret_cast<const float*>(a.k) + b * a.k_sb + h * a.k_sh;
     const float* vptr = reinterpret_cast<const float*>(a.v) + b * a.v_sb + h * a.v_sh;
@@ -98,26 +98,18 @@ __global__ __launch_bounds__(LX_NT) void local_fwd_x3_kernel(LocalArgs a) {
         rk.fetch(kptr, a.k_ss, kt_lo * LX_TK, a.S - 1, tid);
         rv.fetch(vptr, a.v_ss, kt_lo * LX_TK, a.S - 1, tid);
     }
-    int iq[QB], smin[QB];
-    unsigned span[QB];
-    uint32_t drop_row[QB];
-    Pieces qp[QB][KS];
-    float m_run[QB], ze[QB];
-    floatx4 oacc[QB][DB];
+    const int iq = qw0 + r16;
+    const float* qrow = qptr + (long)min(iq, a.T - 1) * a.q_ss;
+    Pieces qp[KS];
 #pragma unroll
-    for (int qq = 0; qq < QB; ++qq) {
-        iq[qq] = qw0 + 16 * qq + r16;
-        const float* qrow = qptr + (long)min(iq[qq], a.T - 1) * a.q_ss;
+    for (int ks = 0; ks < KS; ++ks) qp[ks] = lx_load(qrow + 32 * ks + 8 * g);
+    float m_run = -1e30f, ze = 0.f;         // (finite, so that the first rescale is exp2(-huge) = 0 and not inf - inf)
+    floatx4 oacc[DB];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) qp[qq][ks] = lx_load(qrow + 32 * ks + 8 * g);
-        m_run[qq] = -1e30f;         // finite, so that the first rescale is exp2(-huge) = 0 and not inf - inf
-        ze[qq] = 0.f;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) oacc[qq][db] = Frag<float>::zero();
-        smin[qq] = max(iq[qq] - lc_lo, 0);
-        span[qq] = iq[qq] < a.T ? (unsigned)max(min(iq[qq] + lc_hi, len) - smin[qq], 0) : 0u;
-        drop_row[qq] = a.drop_thresh != 0u ? drop_row_hash(a.drop_seed, (uint32_t)(bh * a.T + iq[qq])) : 0u;
-    }
+    for (int db = 0; db < DB; ++db) oacc[db] = Frag<float>::zero();
+    const int smin = max(iq - lc_lo, 0);
+    const unsigned span = iq < a.T ? (unsigned)max(min(iq + lc_hi, len) - smin, 0) : 0u;
+    const uint32_t drop_row = a.drop_thresh != 0u ? drop_row_hash(a.drop_seed, (uint32_t)(bh * a.T + iq)) : 0u;
     const float sc = a.temp * LX_LOG2E;
     if (kt_lo < kt_hi) {
         rk.stash(lx_smem, tid);
@@ -134,94 +126,70 @@ __global__ __launch_bounds__(LX_NT) void local_fwd_x3_kernel(LocalArgs a) {
             rv.fetch(vptr, a.v_ss, s_base + LX_TK, a.S - 1, tid);
         }
         // (wave-uniform, scalar) does the tile touch the band of one of the wave's queries; does it lie inside all
-        const bool any = !(s_base + LX_TK - 1 - qw0 < -lc_lo || s_base - (qw0 + QW - 1) >= lc_hi || s_base >= len);
-        const bool inside = s_base - (qw0 + QW - 1) >= -lc_lo && s_base + LX_TK - 1 - qw0 < lc_hi && s_base + LX_TK <= len &&
-                            qw0 + QW - 1 < a.T;
+        const bool any = !(s_base + LX_TK - 1 - qw0 < -lc_lo || s_base - (qw0 + 15) >= lc_hi || s_base >= len);
+        const bool inside = s_base - (qw0 + 15) >= -lc_lo && s_base + LX_TK - 1 - qw0 < lc_hi && s_base + LX_TK <= len &&
+                            qw0 + 15 < a.T;
         if (any) {
-            floatx4 s[QB][2];
-#pragma unroll
-            for (int qq = 0; qq < QB; ++qq) { s[qq][0] = Frag<float>::zero(); s[qq][1] = Frag<float>::zero(); }
+            floatx4 s[2] = {Frag<float>::zero(), Frag<float>::zero()};
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb) {
                     const Pieces kf = lx_rows<E>(Ks, 16 * kb + r16, ks, g);
-#pragma unroll
-                    for (int qq = 0; qq < QB; ++qq) s[qq][kb] = mma_pieces(kf, qp[qq][ks], s[qq][kb]);
+                    s[kb] = mma_pieces(kf, qp[ks], s[kb]);
                 }
             if (a.add_mask) {                                // (uniform)
-#pragma unroll
-                for (int qq = 0; qq < QB; ++qq) {
-                    const float* am = a.add_mask + (long)min(iq[qq], a.T - 1) * a.S;
-#pragma unroll
-                    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int n = s_base + 16 * kb + 4 * g + i;
-                            // (an absorbing entry becomes -2^80: its product with the scale is exact, so the multiply-add
-                            //  of the exponent below gives exactly 0 for a row whose keys are all hidden)
-                            if ((unsigned)(n - smin[qq]) < span[qq]) s[qq][kb][i] = am[n] < -1e20f ? -0x1p80f : s[qq][kb][i] + am[n];
-                        }
-                }
-            }
-            if (!inside) {
-#pragma unroll
-                for (int qq = 0; qq < QB; ++qq)
-#pragma unroll
-                    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (!((unsigned)(s_base + 16 * kb + 4 * g + i - smin[qq]) < span[qq])) s[qq][kb][i] = -INFINITY;
-            }
-            float mx[QB];
-            bool moved = false;
-#pragma unroll
-            for (int qq = 0; qq < QB; ++qq) {
-                mx[qq] = -INFINITY;
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) mx[qq] = fmaxf(mx[qq], s[qq][kb][i]);
-                mx[qq] = group_max(mx[qq]) * sc;
-                moved = moved || mx[qq] > m_run[qq] + 8.f;
-            }
-            if (__builtin_amdgcn_ballot_w64(moved) != 0) {
-#pragma unroll
-                for (int qq = 0; qq < QB; ++qq) {
-                    const float m_new = fmaxf(m_run[qq], mx[qq]);
-                    const float alpha = __builtin_amdgcn_exp2f(m_run[qq] - m_new);
-                    m_run[qq] = m_new;
-                    ze[qq] *= alpha;
-#pragma unroll
-                    for (int db = 0; db < DB; ++db) oacc[qq][db] *= alpha;
-                }
-            }
-#pragma unroll
-            for (int qq = 0; qq < QB; ++qq)
+                const float* am = a.add_mask + (long)min(iq, a.T - 1) * a.S;
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        s[qq][kb][i] = __builtin_amdgcn_exp2f(fmaf(s[qq][kb][i], sc, -m_run[qq]));      // (masked: -inf, weight 0)
-                        ze[qq] += s[qq][kb][i];
+                        const int n = s_base + 16 * kb + 4 * g + i;
+                        // (an absorbing entry becomes -2^80: its product with the scale is exact, so the multiply-add
+                        //  of the exponent below gives exactly 0 for a row whose keys are all hidden)
+                        if ((unsigned)(n - smin) < span) s[kb][i] = am[n] < -1e20f ? -0x1p80f : s[kb][i] + am[n];
                     }
+            }
+            if (!inside) {
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (!((unsigned)(s_base + 16 * kb + 4 * g + i - smin) < span)) s[kb][i] = -INFINITY;
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kb][i]);
+            mx = group_max(mx) * sc;
+            if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0) {
+                const float m_new = fmaxf(m_run, mx);
+                const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+                m_run = m_new;
+                ze *= alpha;
+#pragma unroll
+                for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
+            }
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[kb][i] = __builtin_amdgcn_exp2f(fmaf(s[kb][i], sc, -m_run));      // (masked: -inf, weight 0)
+                    ze += s[kb][i];
+                }
             if (a.drop_thresh != 0u) {                       // (uniform) dropped weights leave the product, not the denominator
 #pragma unroll
-                for (int qq = 0; qq < QB; ++qq)
+                for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (!drop_keep(drop_row[qq], (uint32_t)(s_base + 16 * kb + 4 * g + i), a.drop_thresh)) s[qq][kb][i] = 0.f;
+                    for (int i = 0; i < 4; ++i)
+                        if (!drop_keep(drop_row, (uint32_t)(s_base + 16 * kb + 4 * g + i), a.drop_thresh)) s[kb][i] = 0.f;
             }
-            Pieces p[QB];
-#pragma unroll
-            for (int qq = 0; qq < QB; ++qq) p[qq] = split<3>(s[qq][0], s[qq][1]);
+            const Pieces p = split<3>(s[0], s[1]);
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
                 const Pieces vf = lx_cols<E>(Vs, db, r16, g);
-#pragma unroll
-                for (int qq = 0; qq < QB; ++qq) oacc[qq][db] = mma_pieces(vf, p[qq], oacc[qq][db]);
+                oacc[db] = mma_pieces(vf, p, oacc[db]);
             }
         }
         if (more) {
@@ -231,22 +199,19 @@ __global__ __launch_bounds__(LX_NT) void local_fwd_x3_kernel(LocalArgs a) {
         }
         __syncthreads();
     }
+    float z = group_sum(ze);
+    // every visible key masked: the positions of the band outside the keys carry the same score in the reference's
+    // softmax over the packed band (local_attention.py:68-81), so they count in the denominator
+    const bool all_masked = a.add_mask != nullptr && span > 0u && m_run < -1e20f;
+    if (all_masked) z += (float)(a.lc - (int)span);
+    if (iq < a.T) {
+        const float inv = (z > 0.f ? 1.0f / z : 0.f) * (a.drop_thresh != 0u ? a.drop_scale : 1.0f);
+        float* optr = reinterpret_cast<float*>(a.out) + b * a.o_sb + h * a.o_sh + (long)iq * a.o_ss;
 #pragma unroll
-    for (int qq = 0; qq < QB; ++qq) {
-        float z = group_sum(ze[qq]);
-        // every visible key masked: the positions of the band outside the keys carry the same score in the reference's
-        // softmax over the packed band (local_attention.py:68-81), so they count in the denominator
-        const bool all_masked = a.add_mask != nullptr && span[qq] > 0u && m_run[qq] < -1e20f;
-        if (all_masked) z += (float)(a.lc - (int)span[qq]);
-        if (iq[qq] < a.T) {
-            const float inv = (z > 0.f ? 1.0f / z : 0.f) * (a.drop_thresh != 0u ? a.drop_scale : 1.0f);
-            float* optr = reinterpret_cast<float*>(a.out) + b * a.o_sb + h * a.o_sh + (long)iq[qq] * a.o_ss;
-#pragma unroll
-            for (int db = 0; db < DB; ++db) store4_f32(optr + 16 * db + 4 * g, oacc[qq][db] * inv);
-            if (a.lse && g == 0)        // a query without visible keys has no pair that would read its entry
-                a.lse[((long)b * a.H + h) * a.T + iq[qq]] = all_masked ? -INFINITY
-                                                            : z > 0.f ? m_run[qq] * 0.6931471805599453f + __logf(z) : 0.f;
-        }
+        for (int db = 0; db < DB; ++db) store4_f32(optr + 16 * db + 4 * g, oacc[db] * inv);
+        if (a.lse && g == 0)        // a query without visible keys has no pair that would read its entry
+            a.lse[((long)b * a.H + h) * a.T + iq] = all_masked ? -INFINITY
+                                                        : z > 0.f ? m_run * 0.6931471805599453f + __logf(z) : 0.f;
     }
 }
 
