@@ -22,19 +22,14 @@ def _round_up_choice(n, choices, what):
     raise NotImplementedError(f'{what}={n} exceeds the largest supported size {choices[-1]}')
 
 
-def _vector_ready(x):
-    """16-byte vector access needs a unit inner stride, strides in multiples of 4 elements and an
-    aligned base pointer."""
-    return (x.stride(-1) == 1 and all(s % 4 == 0 for s in x.stride()[:-1])
-            and x.data_ptr() % 16 == 0)
-
-
 def rows_for_vectors(x, unit=4):
-    """`x` itself where rows of `unit` elements a load can be read in place (unit inner stride, other strides in multiples
-    of `unit`, 16-byte aligned base), else a copy that can.  A clone and not ``contiguous()``, which hands back the tensor
-    itself when it is contiguous but starts off the boundary or has an odd stride on a dim of size 1."""
-    ready = _vector_ready(x) and all(s % unit == 0 for s in x.stride()[:-1])
-    return x if ready else x.clone(memory_format=torch.contiguous_format)
+    """`x` itself where 16-byte loads of `unit` elements can read its rows in place (unit inner stride, other strides in
+    multiples of `unit`, 16-byte aligned base), else a copy that they can.  A clone and not ``contiguous()``, which hands back
+    the tensor itself when it is contiguous but starts off the boundary or has an odd stride on a dim of size 1."""
+    strides = x.stride()
+    if strides[-1] == 1 and x.data_ptr() % 16 == 0 and not any(s % unit for s in strides[:-1]):
+        return x
+    return x.clone(memory_format=torch.contiguous_format)
 
 
 class SBLocalPlan:
