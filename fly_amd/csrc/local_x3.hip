@@ -18,6 +18,12 @@
 // formed transposed (rows = inner, columns = outer): a lane's eight weights of a tile are the contraction slots
 // {4 g + i, 16 + 4 g + i} of the second product, whose other operand comes by transposing LDS reads of the same rows.
 // Rows are 2 E bytes per piece with 16-byte chunks XOR-swizzled (x3_swz).
+//
+// Pieces of an infinity are no pieces (inf - inf), a float above the largest bfloat16 becomes one, and piece products of
+// values whose product leaves the float range may do so with either sign.  All of that ends in results that are not finite, so a
+// wave with such a result takes its rows again with float multiply-adds over the pairs of the band (local_*_plain):
+// infinities and NaN then reach what they reach in a float computation over those pairs, at a hundredth of the rate.  The check
+// costs 1.7 % of a training step at window 98 (283 -> 288 us), next to nothing at wider ones.
 #include "common.h"
 #include "local.h"
 
@@ -70,6 +76,125 @@ __device__ __forceinline__ Pieces lx_cols(const char* st, int cb, int r16, int g
 }
 __device__ __forceinline__ Pieces lx_load(const float* p) {
     return split<3>(*reinterpret_cast<const floatx4*>(p), *reinterpret_cast<const floatx4*>(p + 4));
+}
+template <int N>
+__device__ __forceinline__ float sum_of(const floatx4 (&x)[N]) {       // (finite only if all of them are)
+    floatx4 s = x[0];
+#pragma unroll
+    for (int j = 1; j < N; ++j) s += x[j];
+    return (s[0] + s[1]) + (s[2] + s[3]);
+}
+__device__ __forceinline__ bool finite_in_wave(float x) { return __builtin_amdgcn_ballot_w64(!(fabsf(x) < INFINITY)) == 0; }
+// four lanes per row (lane / 4), E / 4 elements each, in groups of four
+template <int E>
+struct RowPart {
+    floatx4 x[E / 16];
+    __device__ __forceinline__ void load(const float* row, int part, float scale = 1.f) {
+#pragma unroll
+        for (int j = 0; j < E / 16; ++j) x[j] = *reinterpret_cast<const floatx4*>(row + (E / 4) * part + 4 * j) * scale;
+    }
+    __device__ __forceinline__ float dot(const RowPart& o) const {
+        float d = 0.f;
+#pragma unroll
+        for (int j = 0; j < E / 16; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d = fmaf(x[j][i], o.x[j][i], d);
+        d += __shfl_xor(d, 1);
+        return d + __shfl_xor(d, 2);
+    }
+    __device__ __forceinline__ void add(float w, const RowPart& o) {
+#pragma unroll
+        for (int j = 0; j < E / 16; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[j][i] = fmaf(w, o.x[j][i], x[j][i]);
+    }
+    __device__ __forceinline__ void store(float* row, int part, float scale) const {
+#pragma unroll
+        for (int j = 0; j < E / 16; ++j) store4_f32(row + (E / 4) * part + 4 * j, x[j] * scale);
+    }
+};
+
+// the wave's 16 queries from q0 on, one pass for the largest score and one for the sums
+template <int E>
+__device__ __forceinline__ void local_fwd_plain(const LocalArgs& a, int b, int h, int q0, int len, int lane) {
+    const int part = lane & 3, bh = b * a.H + h, iq = min(q0 + (lane >> 2), a.T - 1);      // (rows past the end do the last one again)
+    const float* kptr = reinterpret_cast<const float*>(a.k) + b * a.k_sb + h * a.k_sh;
+    const float* vptr = reinterpret_cast<const float*>(a.v) + b * a.v_sb + h * a.v_sh;
+    const int lo = max(iq - a.lc / 2, 0), hi = min(iq + (a.lc + 1) / 2, len);
+    const float sc = a.temp * LX_LOG2E;
+    const uint32_t drop_row = a.drop_thresh != 0u ? drop_row_hash(a.drop_seed, (uint32_t)(bh * a.T + iq)) : 0u;
+    RowPart<E> q, y, acc;
+    q.load(reinterpret_cast<const float*>(a.q) + b * a.q_sb + h * a.q_sh + (long)iq * a.q_ss, part, sc);            // (scaled before the products: they stay in range longer)
+#pragma unroll
+    for (int j = 0; j < E / 16; ++j) acc.x[j] = Frag<float>::zero();
+    auto score = [&](int n) __attribute__((always_inline)) {
+        y.load(kptr + (long)n * a.k_ss, part);
+        const float s = q.dot(y), am = a.add_mask ? a.add_mask[(long)iq * a.S + n] : 0.f;
+        return am < -1e20f ? -0x1p80f * sc : s + am * sc;
+    };
+    float m = -1e30f, z = 0.f;
+#pragma unroll 1
+    for (int n = lo; n < hi; ++n) m = fmaxf(m, score(n));
+#pragma unroll 1
+    for (int n = lo; n < hi; ++n) {
+        const float p = __builtin_amdgcn_exp2f(score(n) - m);
+        z += p;
+        y.load(vptr + (long)n * a.v_ss, part);
+        acc.add(a.drop_thresh == 0u || drop_keep(drop_row, (uint32_t)n, a.drop_thresh) ? p : 0.f, y);
+    }
+    const bool all_masked = a.add_mask != nullptr && hi > lo && m < -1e20f;
+    if (all_masked) z += (float)(a.lc - (hi - lo));
+    if (q0 + (lane >> 2) >= a.T) return;
+    acc.store(reinterpret_cast<float*>(a.out) + b * a.o_sb + h * a.o_sh + (long)iq * a.o_ss, part,
+              (z > 0.f ? 1.0f / z : z == z ? 0.f : z) * (a.drop_thresh != 0u ? a.drop_scale : 1.0f));
+    if (a.lse && part == 0) a.lse[(long)bh * a.T + iq] = all_masked ? -INFINITY : z > 0.f ? m * 0.6931471805599453f + __logf(z) : z == z ? 0.f : z;
+}
+
+// the gradients of the wave's 16 outer rows from o0 on
+template <int E, bool KEYMAJOR>
+__device__ __forceinline__ void local_bwd_plain(const LocalBwdArgs& a, int b, int h, int o0, int len, int lane) {
+    const int part = lane & 3, bh = b * a.H + h, rows = KEYMAJOR ? a.S : a.T, o = min(o0 + (lane >> 2), rows - 1);
+    const float* qptr = reinterpret_cast<const float*>(a.q) + b * a.q_sb + h * a.q_sh;
+    const float* kptr = reinterpret_cast<const float*>(a.k) + b * a.k_sb + h * a.k_sh;
+    const float* vptr = reinterpret_cast<const float*>(a.v) + b * a.v_sb + h * a.v_sh;
+    const float* gptr = reinterpret_cast<const float*>(a.go) + b * a.g_sb + h * a.g_sh;
+    const float* y1p = KEYMAJOR ? qptr : kptr;  const long y1s = KEYMAJOR ? a.q_ss : a.k_ss;
+    const float* y2p = KEYMAJOR ? gptr : vptr;  const long y2s = KEYMAJOR ? a.g_ss : a.v_ss;
+    const int lc_lo = a.lc / 2, lc_hi = (a.lc + 1) / 2;
+    const int lo = max(o - (KEYMAJOR ? lc_hi - 1 : lc_lo), 0);
+    const int hi = KEYMAJOR ? (o < len ? min(o + lc_lo + 1, a.T) : 0) : min(o + lc_hi, len);
+    const float sc = a.temp * LX_LOG2E;
+    RowPart<E> x1, x2, y1, y2, acc1, acc2;
+    x1.load(KEYMAJOR ? kptr + (long)o * a.k_ss : qptr + (long)o * a.q_ss, part, sc);
+    x2.load(KEYMAJOR ? vptr + (long)o * a.v_ss : gptr + (long)o * a.g_ss, part);
+    float l_own = 0.f, d_own = 0.f;
+    if (!KEYMAJOR) {
+        y1.load(reinterpret_cast<const float*>(a.out) + b * a.o_sb + h * a.o_sh + (long)o * a.o_ss, part);
+        d_own = x2.dot(y1);
+        l_own = a.lse[(long)bh * a.T + o] * LX_LOG2E;
+    }
+#pragma unroll
+    for (int j = 0; j < E / 16; ++j) { acc1.x[j] = Frag<float>::zero(); acc2.x[j] = Frag<float>::zero(); }
+#pragma unroll 1
+    for (int n = lo; n < hi; ++n) {
+        const int i = KEYMAJOR ? n : o, key = KEYMAJOR ? o : n;                     // the pair's query and key
+        y1.load(y1p + (long)n * y1s, part);
+        y2.load(y2p + (long)n * y2s, part);
+        const float s = x1.dot(y1), gv = x2.dot(y2);
+        const float lrow = KEYMAJOR ? a.lse[(long)bh * a.T + n] * LX_LOG2E : l_own, drow = KEYMAJOR ? a.delta[(long)bh * a.T + n] : d_own;
+        const float am = a.add_mask ? a.add_mask[(long)i * a.S + key] : 0.f;
+        const float pr = a.add_mask && lrow == -INFINITY ? 1.0f / (float)a.lc
+                                                         : __builtin_amdgcn_exp2f((am < -1e20f ? -0x1p80f * sc : s + am * sc) - lrow);
+        float keep = 1.f;
+        if (a.drop_thresh != 0u)
+            keep = drop_keep(drop_row_hash(a.drop_seed, (uint32_t)(bh * a.T + i)), (uint32_t)key, a.drop_thresh) ? a.drop_scale : 0.f;
+        acc1.add(pr * (keep * gv - drow), y1);
+        if (KEYMAJOR) acc2.add(pr * keep, y2);
+    }
+    if (o0 + (lane >> 2) >= rows) return;
+    acc1.store(KEYMAJOR ? reinterpret_cast<float*>(a.dk) + b * a.dk_sb + h * a.dk_sh + (long)o * a.dk_ss
+                        : reinterpret_cast<float*>(a.dq) + b * a.dq_sb + h * a.dq_sh + (long)o * a.dq_ss, part, a.temp);
+    if (KEYMAJOR) acc2.store(reinterpret_cast<float*>(a.dv) + b * a.dv_sb + h * a.dv_sh + (long)o * a.dv_ss, part, 1.f);
 }
 
 template <int E>
@@ -213,6 +338,10 @@ __global__ __launch_bounds__(LX_NT) void local_fwd_x3_kernel(LocalArgs a) {
             a.lse[((long)b * a.H + h) * a.T + iq] = all_masked ? -INFINITY
                                                         : z > 0.f ? m_run * 0.6931471805599453f + __logf(z) : 0.f;
     }
+    if (!finite_in_wave(sum_of(oacc) + ze)) {
+        drain_loads();                                      // (the results stored above have gone out)
+        local_fwd_plain<E>(a, b, h, qw0, len, lane);
+    }
 }
 
 // Gradients, in the two orientations of local_bwd_b16_kernel (sblocal.hip): with P_is = exp(t (q_i.k_s + mask) - lse_i) and
@@ -221,9 +350,10 @@ __global__ __launch_bounds__(LX_NT) void local_fwd_x3_kernel(LocalArgs a) {
 //   key-major:   d k_s = t sum_i dS_is q_i,  d v_s = sum_i M P g_i
 template <int E> constexpr size_t local_bwd_x3_smem() { return (size_t)2 * (2 * PieceTile<E>::BYTES + 2 * LX_TK * sizeof(float)); }
 
-// (three workgroups per compute unit, as many as their stages allow: the key-major form takes 176 registers of its own accord)
+// (three workgroups per compute unit, as many as their stages allow, four at 32 dims: the key-major form takes 176 registers of its
+// own accord)
 template <int E, bool KEYMAJOR>
-__global__ __launch_bounds__(LX_NT) __attribute__((amdgpu_waves_per_eu(3, 4))) void local_bwd_x3_kernel(LocalBwdArgs a) {
+__global__ __launch_bounds__(LX_NT) __attribute__((amdgpu_waves_per_eu(E == 32 ? 4 : 3, 4))) void local_bwd_x3_kernel(LocalBwdArgs a) {
     using PT = PieceTile<E>;
     constexpr int KS = E / 32, EB = E / 16, STAGE = 2 * PT::BYTES + 2 * LX_TK * (int)sizeof(float), TQB = 64;
     extern __shared__ __attribute__((aligned(128))) char lx_smem[];
@@ -377,6 +507,10 @@ __global__ __launch_bounds__(LX_NT) __attribute__((amdgpu_waves_per_eu(3, 4))) v
 #pragma unroll
             for (int eb = 0; eb < EB; ++eb) store4_f32(d2 + 16 * eb + 4 * g, acc2[eb]);
         }
+    }
+    if (!finite_in_wave(KEYMAJOR ? sum_of(acc1) + sum_of(acc2) : sum_of(acc1))) {
+        drain_loads();                                      // (the results stored above have gone out)
+        local_bwd_plain<E, KEYMAJOR>(a, b, h, ow0, len, lane);
     }
 }
 

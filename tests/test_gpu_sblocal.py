@@ -1205,3 +1205,69 @@ def test_inputs_and_gradients_in_any_memory_layout(kind, layout, H):
     ones = torch.autograd.grad(want, plain, torch.ones_like(want))
     for a, b in zip(torch.autograd.grad(out.sum(), laid), ones):
         assert torch.equal(a, b)
+
+
+def _band_rows(q, k, v, lc, lens, additive, mult):
+    """Local attention in float64 that touches the pairs of the band only, one query at a time: an infinity reaches the
+    queries that see it and no others."""
+    B, T, H, E = q.shape
+    t = E ** -0.5
+    rows = []
+    for b in range(B):
+        for h in range(H):
+            for i in range(T):
+                lo, hi = max(i - lc // 2, 0), min(i + (lc + 1) // 2, int(lens[b]))
+                if hi <= lo:
+                    rows.append(v[b, 0, h] * 0 if bool(v[b, 0, h].isfinite().all()) else torch.zeros(v.shape[-1], dtype=v.dtype))
+                    continue
+                s = t * ((k[b, lo:hi, h] * q[b, i, h]).sum(-1) + additive[i, lo:hi])
+                p = torch.softmax(s, -1) * mult[b, h, i, lo:hi]
+                rows.append((p.unsqueeze(-1) * v[b, lo:hi, h]).sum(0))
+    return torch.stack(rows).view(B, H, T, -1).transpose(1, 2)
+
+
+@pytest.mark.parametrize('E', [64, 32])
+@pytest.mark.parametrize('where,value,masked,p_drop', [
+    (where, value, masked, p_drop)
+    for where, value in (('v', math.inf), ('v', -math.inf), ('k', math.inf), ('q', -math.inf), ('w', math.inf), ('v', 3.4e38), ('k', 3.395e38))
+    for masked, p_drop in ((False, 0.0), (True, 0.0), (False, 0.3))
+    if not (masked and where == 'k')])           # (-1e24 added to an infinite score hides it in the kernels and not in the reference)
+def test_local_attention_float32_with_infinities(where, value, masked, p_drop, E):
+    """An infinity, or a finite float above the largest bfloat16, in an input of float32 LocalAttention: it has no three
+    bf16 pieces.  Output and gradients are those of a float computation over the pairs of the band -- infinite, NaN and
+    finite in the same places (next to an infinite gradient: finite or not), the finite ones as close as elsewhere (float32 sums over at most 40 keys and 64 dims).  With the
+    large finite values the gradients overflow float32, so the output alone is compared."""
+    from fly_amd import FullMask, LengthMask, LocalAttention
+    B, T, S, H, lc, p = 1, 150, 130, 2, 40, p_drop
+    g = torch.Generator().manual_seed(71)
+    x = dict(q=torch.randn(B, T, H, E, generator=g), k=torch.randn(B, S, H, E, generator=g), v=torch.randn(B, S, H, E, generator=g),
+             w=torch.randn(B, T, H, E, generator=g))
+    keep = torch.ones(T, S, dtype=torch.bool)
+    if masked:
+        # (the queries from 140 on see no key at all)
+        keep = (torch.rand(T, S, generator=g) < 0.8) | (torch.arange(S).view(1, S) == torch.arange(T).view(T, 1).clamp(max=119))      # (every query sees a key)
+    x[where][0, 75, 1, 5] = value
+    lens = torch.tensor([120])
+    dev = torch.device('cuda:0')
+    layer = LocalAttention(lc, attention_dropout=p).to(dev).train()
+    qkv = [x[n].to(dev).requires_grad_() for n in 'qkv']
+    torch.manual_seed(3)
+    out, _ = layer(*qkv, attn_mask=FullMask(keep.to(dev)) if masked else None, key_padding_mask=LengthMask(lens.to(dev), max_len=S))
+    got = (out.detach(),) + torch.autograd.grad(out, qkv, x['w'].to(dev))
+    mult = osb.dropout_keep(layer.last_dropout_seed, p, B, H, T, S) if p else torch.ones(B, H, T, S, dtype=torch.float64)
+    ref_in = [x[n].double().requires_grad_() for n in 'qkv']
+    ref_out = _band_rows(*ref_in, lc, lens, (~keep).double() * -1e24, mult)
+    ref = (ref_out.detach(),) + torch.autograd.grad(ref_out, ref_in, x['w'].double())
+    if math.isfinite(value):
+        got, ref = got[:1], ref[:1]
+        assert bool(got[0].isfinite().all())
+    for name, a, r in zip(('out', 'dq', 'dk', 'dv'), got, ref):
+        a = a.double().cpu()
+        assert torch.equal(a.isfinite(), r.isfinite()), (name, int(a.isfinite().sum()), int(r.isfinite().sum()))
+        if where != 'w':         # (there g.out, taken after the sum over the keys, is infinite where the sum of P (g.v) is NaN)
+            assert torch.equal(a == math.inf, r == math.inf) and torch.equal(a == -math.inf, r == -math.inf), name
+        ok = r.isfinite()
+        small = ok & (r.abs() < 1e6)
+        assert float(((a - r).abs() / (1e-5 + 1e-4 * r.abs()))[small].max()) <= 1.0, name
+        if bool((ok & ~small).any()):
+            assert float(((a - r).abs() / r.abs())[ok & ~small].max()) <= 1e-4, name
