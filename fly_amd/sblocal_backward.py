@@ -319,7 +319,8 @@ def _backward_far(query, key, value, P, local_context, t, key_lengths, out, log_
                           ws.data_ptr(), ws.numel(), b1 - b0, h1 - h0, T, S, dim, mk, mh, local_context,
                           *strides(q), *strides(k), *strides(v), *strides(o), *strides(g), *strides(dq), *strides(dk),
                           *strides(dv), float(t), st)
-    return dq[..., :E], dk[..., :E], dv[..., :D]
+    # (contiguous in the inputs' shapes also where the head dim was padded, as the other routes return them)
+    return dq[..., :E].contiguous(), dk[..., :E].contiguous(), dv[..., :D].contiguous()
 
 
 def _band_terms_hip(Q, K, V, G, psi, phik, LN, c, lens_b, H, local_context, t, dims, dropout=(0.0, 0), attn_mask=None):

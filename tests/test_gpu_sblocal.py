@@ -1154,6 +1154,19 @@ def test_float32_gradient_of_a_bfloat16_output_is_not_rounded(mh):
         assert share <= 1e-2, (name, share)
 
 
+@pytest.mark.parametrize('E,D,mh', [(48, 48, 128), (64, 40, 64), (20, 20, 16), (64, 64, 64)])
+def test_bf16_gradients_are_contiguous(E, D, mh):
+    """Gradients of bfloat16 Scatterbrain-local attention come back contiguous, padded head dims or not: a caller may view
+    them flat."""
+    from fly_amd import sblocal_attention_fn
+    dev = torch.device('cuda:0')
+    q, k, v, P = make_inputs(1, 130, 120, 2, E, D, mh, seed=5, dtype=torch.bfloat16)
+    leaves = [x.to(dev).requires_grad_() for x in (q, k, v)]
+    out, _ = sblocal_attention_fn(*leaves, P.to(dev), 64)
+    for x, g in zip(leaves, torch.autograd.grad(out, leaves, torch.ones_like(out))):
+        assert g.shape == x.shape and g.is_contiguous()
+
+
 def _in_layout(x, layout):
     """`x` with the same values in memory a caller may hand over: 'offset' contiguous but three elements off an aligned
     start, 'odd-batch' a single batch entry whose batch stride is odd, 'heads-first' (B, H, L, E) in memory, 'fused' a third
