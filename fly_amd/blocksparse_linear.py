@@ -9,8 +9,9 @@ import torch.nn.functional as F
 from torch.nn import init
 
 from .blocksparse_attention import instantiate
-from .blocksparse_matmul import KMAJOR_MIN_K, matmul, rows_as_they_are
+from .blocksparse_matmul import KMAJOR_MIN_K, matmul
 from .blocksparse_utils import densify_tensor
+from .sblocal_attention import rows_for_vectors
 
 
 class FlatBlockButterflySparsityConfig:
@@ -158,7 +159,7 @@ class BlockSparseLinear(nn.Module):
                     self.block_size == 32 and n_tok >= KMAJOR_MIN_K
                     and (torch.is_autocast_enabled() or x.dtype in (torch.bfloat16, torch.float16))):
                 if pad_tok and not pad_in:
-                    tokens = rows_as_they_are(tokens)
+                    tokens = rows_for_vectors(tokens, 8)
                 pad_tok = 0
             if pad_in or pad_tok:
                 tokens = F.pad(tokens, (0, pad_in, 0, pad_tok))

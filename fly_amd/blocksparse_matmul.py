@@ -4,6 +4,7 @@ import torch
 
 from . import _lib
 from .blocksparse_utils import group_table, sdd_table, segment_table, union_table
+from .sblocal_attention import rows_for_vectors
 
 # Sharing the dense operand's tiles among four block-rows pays when the rows have columns in
 # common: the union tables are passed to the kernels when the layout has at least this many
@@ -28,14 +29,6 @@ def _dense_operand(x):
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
-def rows_as_they_are(x):
-    """`x` itself where the kernels for 16-bit rows read it in place, else a copy they can: a count of rows that fills no block
-    used to come with a padded copy, so its callers may hand over any strides."""
-    if x.stride(-1) == 1 and all(s % 8 == 0 for s in x.stride()[:-1]) and x.data_ptr() % 16 == 0:
-        return x
-    return x.clone(memory_format=torch.contiguous_format)
-
-
 class _MatmulFn(torch.autograd.Function):
     """c = op(a) @ op(b) with one sparse participant; backward re-uses the same three kernels with
     permuted roles exactly as blocksparse_matmul.py:562-587 does."""
@@ -55,7 +48,8 @@ class _MatmulFn(torch.autograd.Function):
         mode = op.mode
         da = db = None
         if op.ragged_rows and dc.shape[2] % op.block:
-            dc = rows_as_they_are(dc)
+            # (a count of rows that fills no block used to come with a padded copy, so callers may hand over any strides)
+            dc = rows_for_vectors(dc, 8)
         if ctx.needs_input_grad[0]:
             mode_da = mode[1] + mode[0] + mode[2]
             da = op._run(mode_da, dc, b, False, not op.trans_b, op.trans_a)

@@ -195,9 +195,6 @@ __device__ __forceinline__ uintx4 frag_down_rows_at(const uint16_t* tile, int ld
     const uintx2 l = __builtin_bit_cast(uintx2, lo), h = __builtin_bit_cast(uintx2, hi);
     return uintx4{l[0], l[1], h[0], h[1]};
 }
-__device__ __forceinline__ uintx4 frag_down_rows(const uint16_t* tile, int ld, int f0, int r16, int g) {
-    return frag_down_rows_at(tile, ld, f0, r16, 8 * g + (r16 >> 2), 8 * g + 4 + (r16 >> 2));
-}
 
 // SDD for layouts whose neighbouring block-rows share most of their columns (band and butterfly
 // patterns do): one workgroup per (batch, head, four consecutive block-rows), wave w owning row

@@ -1167,6 +1167,41 @@ def test_bf16_gradients_are_contiguous(E, D, mh):
         assert g.shape == x.shape and g.is_contiguous()
 
 
+@pytest.mark.parametrize('p_drop,masked', [(0.0, False), (0.25, False), (0.0, True), (0.5, True)])
+@pytest.mark.parametrize('E,M', [(32, 64), (64, 32), (64, 128)])
+def test_band_sums_entry_with_dropout_and_mask(E, M, p_drop, masked):
+    """flyhip_sblocal_bwd_band_masked (and _dropout, _band, which are its forms with fewer arguments) called directly: with the
+    features zero and the log-denominators of local attention its sums are that attention's gradients -- the additive mask
+    with rows whose visible keys are all hidden, the dropout mask formed again from the seed, key lengths, T != S.  Against
+    the gradients of the local attention kernels, which have the oracle for a reference: float32 products on either
+    side, 1e-5 (2-norm)."""
+    from fly_amd.local_attention import local_backward, local_forward
+    from fly_amd.sblocal_backward import _band_terms_hip
+    B, T, S, H, lc = 2, 150, 130, 2, 40
+    g = torch.Generator().manual_seed(81)
+    q, k, v, w = (torch.randn(B, L, H, E, generator=g).cuda() for L in (T, S, S, T))
+    lens = torch.tensor([S, 90]).cuda()
+    add = None
+    if masked:
+        keep = torch.rand(T, S, generator=g) < 0.7
+        keep[20:23] = False
+        add = ((~keep).float() * -1e24).cuda()
+    drop = (p_drop, 1234567 if p_drop else 0)
+    out, lse = local_forward(q, k, v, lc, key_lengths=lens, return_lse=True, dropout=drop, attn_mask=add)
+    want = local_backward(q, k, v, lc, None, lens, w, out=out, lse=lse, dropout=drop, attn_mask=add)
+
+    def bh(x):
+        return x.permute(0, 2, 1, 3).reshape(B * H, x.shape[1], x.shape[3])
+    Q, K, V, G = bh(q), bh(k), bh(v), bh(w)
+    zero_q, zero_k = Q.new_zeros(B * H, T, M), Q.new_zeros(B * H, S, M)
+    delta = (G * bh(out)).sum(-1, keepdim=True)
+    dq, _, dk, _, dv = _band_terms_hip(Q, K, V, G, zero_q, zero_k, lse.reshape(B * H, T, 1), delta, lens, H, lc, E ** -0.5, (E, M),
+                                       drop, add)
+    for name, got, ref in (('dq', dq, want[0]), ('dk', dk, want[1]), ('dv', dv, want[2])):
+        err = float((got - bh(ref)).norm() / bh(ref).norm())
+        assert err <= 1e-5, (name, err)
+
+
 def _in_layout(x, layout):
     """`x` with the same values in memory a caller may hand over: 'offset' contiguous but three elements off an aligned
     start, 'odd-batch' a single batch entry whose batch stride is odd, 'heads-first' (B, H, L, E) in memory, 'fused' a third
