@@ -486,8 +486,8 @@ __global__ __launch_bounds__(256) void bs_sdd32u_kernel(const SddUniArgs a) {
 // transposing 8-byte LDS reads each.  A holds [token][128 features], B [pair of list entries][token][64 features] (both
 // entries of a pair in one 128-byte line where they are neighbours), 32-byte pieces XOR-swizzled by the token so that the
 // eight rows a half-wave reads together cover all banks.  Measured (us, before / now, with the zero fill and the rounding):
-// 768 -> 3072 features 269 / 185, 3072 -> 768 234 / 220, 1024 -> 4096 345 / 285, 768 -> 768 127 / 74 at 50176 tokens; 106 / 58, 104 / 59, 141 / 69,
-// 46 / 43 at 8192; 32 / 34, 43 / 36, 36 / 34, 43 / 33 at 512.  The slices' partial blocks meet in an fp32 buffer through hardware
+// 768 -> 3072 features 267 / 161, 3072 -> 768 229 / 188, 1024 -> 4096 343 / 243, 768 -> 768 124 / 70 at 50176 tokens; 104 / 55, 102 / 57, 139 / 63,
+// 44 / 40 at 8192; 32 to 33 on either side at 512, where the host is the slower one.  The slices' partial blocks meet in an fp32 buffer through hardware
 // float atomics (the caller zeroes it and rounds it to the output type afterwards).
 struct SddKArgs {
     const void* a; const void* b; float* c32;

@@ -8,8 +8,8 @@
 // 4.6e-7 and 6.6e-7 on the fp32 instruction), at 6 / 16 of its matrix time, and with vector instructions free to run
 // beside it, which fp32 MFMAs do not allow.
 // Measured (us, forward / training step; before: the fp32-pipe forward and, for the gradients, the Scatterbrain band kernels
-// with zero features on contiguous copies): B=64 L=3136 window 98: 108 / 587 -> 79 / 311; 16 heads of 16384 tokens, window
-// 1024: 634 / 3496 -> 457 / 1800; head dim 32, 8 heads of 8192, window 512: 57 / 343 -> 45 / 164.
+// with zero features on contiguous copies): B=64 L=3136 window 98: 106 / 585 -> 76 / 289; 16 heads of 16384 tokens, window
+// 1024: 629 / 3485 -> 432 / 1726; head dim 32, 8 heads of 8192, window 512: 54 / 332 -> 41 / 185.
 // The pieces are formed where a tile is staged into LDS (float rows in memory, piece rows in LDS): a preparation pass would
 // write and read 1.5 times the inputs again, and the passes are within a small factor of the memory they touch.
 //
@@ -23,7 +23,7 @@
 // values whose product leaves the float range may do so with either sign.  All of that ends in results that are not finite, so a
 // wave with such a result takes its rows again with float multiply-adds over the pairs of the band (local_*_plain):
 // infinities and NaN then reach what they reach in a float computation over those pairs, at a hundredth of the rate.  The check
-// costs 1.7 % of a training step at window 98 (283 -> 288 us), next to nothing at wider ones.
+// costs 2 % of a training step at window 98 (275 -> 281 us), 1 % at 1024 (1663 -> 1682).
 #include "common.h"
 #include "local.h"
 

@@ -22,7 +22,7 @@
 // two (2^-17, as in the kernels in sblocal_prep.hip).  Against float64 on the same output and log-normaliser, over 28 problems of
 // 4 to 32 heads, windows of 12 to 1024: 2-norm error of the bfloat16 gradients 1.5e-3 to 1.9e-3, the rounding of the results,
 // and 0.04 to 0.08 % of them rounded otherwise with 256 features (library products in float32: 0.03 to 0.2 %), 0.06 to 0.4 %
-// with fewer (the kernels in sblocal_prep.hip: 0.08 to 0.6 %).  Two pieces throughout took 1870 us a step instead of 2170 and
+// with fewer (the kernels in sblocal_prep.hip: 0.08 to 0.6 %).  Two pieces throughout took 1860 us a step instead of 2130 and
 // rounded 0.1 to 0.45 % otherwise with 256 features.
 //
 //   far_chunk_kernel    KV_c and QG_c summed over the chunks of a segment, every prefix of it kept, stabilised by the largest
@@ -32,10 +32,11 @@
 //   local_bwd_b16_kernel<EXACT> (sblocal.hip)  the band, plus the low-rank part, rounded once
 //
 // Measured at B=1, H=16, L=16384, window 1024, 256 features, where the backward ran as library products over windows of
-// keys before (20.8 ms): chunks 211, scan 19, low-rank 357 (query-major) and 788 (key-major), band 235 and 352 us.  The
+// keys before (20.8 ms): chunks 203, scan 19, low-rank 345 (query-major) and 752 (key-major), band 223 and 337 us.  The
 // chunk sums (66 KB per 64 rows and side at 256 features) bound the first two: a scan over every chunk instead of every
 // segment moved 1.1 GB in 225 us.  The low-rank kernels wait for the far sums (five trips to the cache), and the key-major one
-// spends most of its time on the edges: their features, the weights of their pairs and the pieces of both.
+// spends most of its time on the edges: their features, the weights of their pairs and the pieces of both (matrix pipe 26 %,
+// vector ALU 36 %, LDS 27 % of its cycles at two waves per SIMD, which wait for memory or a barrier 47 % of theirs).
 #include "common.h"
 #include "local.h"
 #include <algorithm>
@@ -352,7 +353,7 @@ struct FarPrefix {
 // workgroup and goes from registers into the products.  Sums over features (chain rule, d v) are per wave until the end.
 // Key-major needs two operands transposed as well, the far sums and the edge features: it takes them by transposing LDS reads
 // of what it has, not by strided loads and a second evaluation (730 -> 600 us at the size above with operands in two pieces;
-// 788 as they are now).  The pieces go through one buffer per wave in turn: side by side they would leave one workgroup per
+// 752 as they are now).  The pieces go through one buffer per wave in turn: side by side they would leave one workgroup per
 // compute unit at 128 features, and no room at 256 for the own features' smaller pieces, which do not fit the registers.
 // columns of the result reduced over the waves at a time: two 16-column blocks where that takes no more LDS
 template <int M, bool KEYMAJOR>

@@ -390,8 +390,8 @@ int flyhip_local_fwd_lse(const void* q, const void* k, const void* v, const int6
 /* flyhip_local_fwd_lse with the dropout of LocalAttention.forward (ref: src/models/attention/local_attention.py:91,
  * `self.dropout(torch.softmax(...))`): every weight is dropped with probability dropout_p in [0, 1) after the softmax
  * (lse is that of the undropped softmax) and the kept ones are scaled by 1 / (1 - dropout_p).  The mask is the hash
- * of (seed, (b H + h) T + query, key) that flyhip_sblocal_forward documents; flyhip_sblocal_bwd_band_dropout forms
- * it again.  dropout_p = 0 is flyhip_local_fwd_lse. */
+ * of (seed, (b H + h) T + query, key) that flyhip_sblocal_forward documents; flyhip_local_bwd_masked and
+ * flyhip_sblocal_bwd_band_dropout form it again.  dropout_p = 0 is flyhip_local_fwd_lse. */
 int flyhip_local_fwd_dropout(const void* q, const void* k, const void* v, const int64_t* key_lengths, void* out,
                              float* lse,
                              int B, int H, int T, int S, int E, int D, int local_context,
@@ -406,7 +406,9 @@ int flyhip_local_fwd_dropout(const void* q, const void* k, const void* v, const 
  * finite bias is allowed), added to q.k before the temperature.  -1e24 absorbs the product in float32, so a query
  * whose visible keys are all masked weighs every position of its band 1 / local_context, those outside the keys
  * included (they add nothing to the output), as the reference's softmax over the packed band does; its lse entry is
- * -inf, which flyhip_sblocal_bwd_band_masked reads as that case. */
+ * -inf, which flyhip_local_bwd_masked and flyhip_sblocal_bwd_band_masked read as that case.  float32 with E in {32,64}
+ * runs on the bf16 matrix pipe from three pieces per operand, accurate as fp32 products; rows whose result is not finite
+ * are formed again by float multiply-adds over the pairs of the band (an infinity has no pieces). */
 int flyhip_local_fwd_masked(const void* q, const void* k, const void* v, const int64_t* key_lengths,
                             const float* attn_mask, void* out, float* lse,
                             int B, int H, int T, int S, int E, int D, int local_context,
@@ -422,7 +424,8 @@ int flyhip_local_fwd_masked(const void* q, const void* k, const void* v, const i
  * that the first launch fills from out, the forward's output, and the second reads):
  * dv_s = sum_i P_is g_i, dS_is = P_is (g_i.v_s - delta_i), dq_i = t sum_s dS_is k_s, dk_s = t sum_i dS_is q_i.  Two
  * launches (query-major for dq, key-major for dk and dv): bfloat16 and float16 on the 16x16x32 MFMA of the input type, P
- * and dS rounded to it; float32 (E in {32,64}) on the bf16 pipe from three pieces per operand, accurate as fp32 products.
+ * and dS rounded to it; float32 (E in {32,64}) on the bf16 pipe from three pieces per operand, accurate as fp32 products (rows whose
+ * gradient is not finite by float multiply-adds, as in the forward).
  * q, out, grad_out, dq (B,T,H,E) and k, v, dk, dv (B,S,H,E) via (batch, head, seq) strides in elements, innermost
  * contiguous, E in {32,64,128}; input strides in multiples of 16 bytes and 16-byte aligned pointers, output strides in
  * multiples of 4 elements.  Every row of dq, dk, dv is written (zeros where a row has no pair in the band).
