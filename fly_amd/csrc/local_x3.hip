@@ -6,7 +6,8 @@
 // 2^-24 of it (h h, h m, m h, m m, h l, l h), accumulated in fp32: as accurate as the fp32 instruction (2-norm against
 // float64 at 1300 tokens, windows of 98 and 500: output 1.8e-7 and 3.7e-7, gradients 4.2e-7 and 5.6e-7; 2.4e-7, 4.8e-7,
 // 4.6e-7 and 6.6e-7 on the fp32 instruction), at 6 / 16 of its matrix time, and with vector instructions free to run
-// beside it, which fp32 MFMAs do not allow.
+// beside it, which fp32 MFMAs do not allow.  That holds down to 2^-102: smaller values have pieces below the normal range of
+// bf16, which the matrix pipe takes as zero (an output gradient of 1e-30: 4.8e-7; of 1e-36: 4e-4).
 // Measured (us, forward / training step; before: the fp32-pipe forward and, for the gradients, the Scatterbrain band kernels
 // with zero features on contiguous copies): B=64 L=3136 window 98: 106 / 585 -> 76 / 289; 16 heads of 16384 tokens, window
 // 1024: 629 / 3485 -> 432 / 1726; head dim 32, 8 heads of 8192, window 512: 54 / 332 -> 41 / 185.

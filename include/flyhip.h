@@ -407,7 +407,8 @@ int flyhip_local_fwd_dropout(const void* q, const void* k, const void* v, const 
  * whose visible keys are all masked weighs every position of its band 1 / local_context, those outside the keys
  * included (they add nothing to the output), as the reference's softmax over the packed band does; its lse entry is
  * -inf, which flyhip_local_bwd_masked and flyhip_sblocal_bwd_band_masked read as that case.  float32 with E in {32,64}
- * runs on the bf16 matrix pipe from three pieces per operand, accurate as fp32 products; rows whose result is not finite
+ * runs on the bf16 matrix pipe from three pieces per operand, accurate as fp32 products for values down to 2^-102 (smaller
+ * ones lose their lowest pieces); rows whose result is not finite
  * are formed again by float multiply-adds over the pairs of the band (an infinity has no pieces). */
 int flyhip_local_fwd_masked(const void* q, const void* k, const void* v, const int64_t* key_lengths,
                             const float* attn_mask, void* out, float* lse,
