@@ -420,6 +420,47 @@ __device__ __forceinline__ void dma_to_lds(const void* lane_src, const char* wav
                  : "=&s"(saved_m0) : "v"(lane_src), "s"(base) : "memory");
 }
 
+// The same with the source as a wave-uniform base and a byte offset per lane: nothing of the address is computed per lane.
+__device__ __forceinline__ void dma_to_lds_at(const void* base, uint32_t lane_off, const char* wave_base) {
+    typedef __attribute__((address_space(3))) const char* lds_ptr;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)wave_base);
+    uint32_t saved_m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved_m0) : "v"(lane_off), "s"(base), "s"(dst) : "memory");
+}
+
+// ROWS rows of W 2-byte elements straight into LDS by NT threads, chunk c of a row stored where x3_swz puts it: the transfers
+// fill LDS linearly, so the swizzle is in the addresses they read.  Row indices are clamped to the last row, as in Tile16.
+template <int ROWS, int W, int NT>
+struct RowsToLds {
+    static constexpr int CH = W / 8, N = ROWS * CH / NT, ROWB = 2 * W;
+    static_assert(ROWS * CH % NT == 0, "whole wave transfers");
+    uint32_t off[N];
+    const uint16_t* src; long stride; int last;
+    __device__ __forceinline__ void init(const uint16_t* src_, long stride_, int last_row, int w, int lane) {
+        src = src_; stride = stride_; last = last_row;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int at = (j * (NT / 64) + w) * 64 + lane, row = at / CH, c = x3_swz(row, at % CH, ROWB);
+            off[j] = (uint32_t)((row * stride + 8 * c) * 2);
+        }
+    }
+    __device__ __forceinline__ void fetch(int row0, const char* dst, int w, int lane) const {
+        // (uniform) all rows exist and the offsets fit 32 bits
+        if (row0 + ROWS - 1 <= last && stride < (1 << 24)) {
+            const uint16_t* base = src + row0 * stride;
+#pragma unroll
+            for (int j = 0; j < N; ++j) dma_to_lds_at(base, off[j], dst + (j * (NT / 64) + w) * 1024);
+        } else {
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const int at = (j * (NT / 64) + w) * 64 + lane, row = at / CH, c = x3_swz(row, at % CH, ROWB);
+                dma_to_lds(src + (long)min(row0 + row, last) * stride + 8 * c, dst + (j * (NT / 64) + w) * 1024);
+            }
+        }
+    }
+};
+
 // ROWS x W tile of 2-byte elements, global -> registers -> LDS (row indices clamped to the last row: rows past
 // the end re-read it, which callers mask, so the loads need no branches and never leave the tensor)
 template <int ROWS, int W, int NT>

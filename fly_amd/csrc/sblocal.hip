@@ -2698,12 +2698,15 @@ __global__ __launch_bounds__(NT) void local_fwd_kernel(LocalArgs a) {
 // plain local attention for 2-byte inputs: both products on the 16x16x32 MFMA of the input type
 // ---------------------------------------------------------------------------------------
 // The same work decomposition, masks, online softmax and outputs as local_fwd_kernel; key tiles of 64 keys, K and V
-// row-major in LDS as they are in memory (rows padded by 16 bytes).
-//   scores^T block (hf, b) = K rows {32 hf + 8 (r / 4) + 4 b + r % 4 : r = 0 .. 15} . q : lane (query r16, group g)
-//       receives keys 32 hf + 8 g + 4 b + i, i = 0 .. 3 -- over b = 0, 1 the eight consecutive keys 32 hf + 8 g .. + 7,
-//       which is the contraction slot order of the second product, so the weights go from registers into it;
-//   out^T[d][query] += V^T[d][key] P[key][query], 32 keys per step: V^T fragments by transposing LDS reads
-//       (ds_read_b64_tr_b16: column d of four consecutive key rows per read).
+// row-major in LDS as they are in memory, brought there by transfers that take no registers (RowsToLds).
+//   scores^T block hb = K rows 16 hb .. + 15 . q : lane (query r16, group g) receives keys 16 hb + 4 g + i, i = 0 .. 3;
+//   out^T[d][query] += V^T[d][key] P[key][query], 32 keys (two blocks) per step, contraction slots {4 g + i, 16 + 4 g + i}: the
+//       weights go from registers into it, V^T fragments come by transposing LDS reads (ds_read_b64_tr_b16: column d of
+//       four consecutive key rows per read).
+// With the 16-byte chunks of a row swizzled (x3_swz) neither kind of read meets a bank conflict; rows padded by 16 bytes with
+// eight consecutive keys per lane left 27 % of the gradients' and 11 % of this kernel's cycles in conflicts.  B=2, 12 heads of 10007
+// tokens in a padded batch, window 1024, forward and gradients: 434 -> 348 us, of which the layout and the transfers 60, the
+// loop without a branch around its products 16, two blocks of queries in the query-major gradient 8.
 template <typename T> __device__ __forceinline__ uint32_t pack_pair(float lo, float hi);
 template <> __device__ __forceinline__ uint32_t pack_pair<bf16_t>(float lo, float hi) { return pack_bf16x2(lo, hi); }
 template <> __device__ __forceinline__ uint32_t pack_pair<f16_t>(float lo, float hi) {
@@ -2711,19 +2714,19 @@ template <> __device__ __forceinline__ uint32_t pack_pair<f16_t>(float lo, float
     return (uint32_t)__builtin_bit_cast(uint16_t, l) | ((uint32_t)__builtin_bit_cast(uint16_t, h) << 16);
 }
 constexpr int TKL = 64;                                // keys per tile of local_fwd_b16_kernel
-template <int E> constexpr size_t local_b16_smem() { return (size_t)2 * TKL * 2 * (E + 8) * 2; }
+template <int E> constexpr size_t local_b16_smem() { return (size_t)2 * TKL * 2 * (2 * E); }
 
 // QB: 16-query blocks per wave.  With two, every K and V^T fragment read from LDS feeds two products (the LDS fragment
 // traffic is what bounds the one-block form on long problems); a workgroup then covers 128 queries.
 template <typename T, int E, int D, int QB>
 __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
     static_assert(sizeof(T) == 2 && E % 32 == 0 && D % 16 == 0, "2-byte inputs, whole MFMA steps");
-    constexpr int LDK = E + 8, LDV = D + 8, KS = E / 32, DB = D / 16;
-    constexpr int STAGE = TKL * (LDK + LDV);           // 2-byte elements of a stage
+    static_assert(E == D, "one row width");
+    constexpr int KS = E / 32, DB = D / 16, ROWB = 2 * E, TILE = TKL * ROWB;
     constexpr int QW = 16 * QB, TQB = 4 * QW;          // queries per wave, per workgroup
     constexpr float LOG2E = 1.4426950408889634f;
     extern __shared__ __attribute__((aligned(128))) float smem[];
-    uint16_t* lds = reinterpret_cast<uint16_t*>(smem);
+    const char* lds = reinterpret_cast<const char*>(smem);
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
     const int n_qt = (a.T + TQB - 1) / TQB;
     const int n_items = a.B * a.H * n_qt;
@@ -2741,12 +2744,14 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
     const int q_last = min(q0 + TQB - 1, a.T - 1);
     const int lo = max(0, q0 - lc_lo), hi = min(len, q_last + lc_hi);
     const int kt_lo = lo / TKL, kt_hi = (hi > lo) ? (hi + TKL - 1) / TKL : kt_lo;
-    Tile16<TKL, E, NT> rk;
-    Tile16<TKL, D, NT> rv;
-    if (kt_lo < kt_hi) {
-        rk.fetch(kptr, a.k_ss, kt_lo * TKL, a.S - 1, tid);
-        rv.fetch(vptr, a.v_ss, kt_lo * TKL, a.S - 1, tid);
-    }
+    RowsToLds<TKL, E, NT> rk, rv;
+    rk.init(kptr, a.k_ss, a.S - 1, w, lane);
+    rv.init(vptr, a.v_ss, a.S - 1, w, lane);
+    auto fetch = [&](int kt, int stage) __attribute__((always_inline)) {
+        rk.fetch(kt * TKL, lds + stage * 2 * TILE, w, lane);
+        rv.fetch(kt * TKL, lds + stage * 2 * TILE + TILE, w, lane);
+    };
+    if (kt_lo < kt_hi) fetch(kt_lo, 0);
     // score operands: the query rows as they are in memory, dims 32 c + 8 g .. + 7 (the scale goes into the exponent)
     int iq[QB], smin[QB];
     unsigned span[QB];
@@ -2769,29 +2774,40 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
         drop_row[qq] = a.drop_thresh != 0u ? drop_row_hash(a.drop_seed, (uint32_t)(bh * a.T + iq[qq])) : 0u;
     }
     const float sc = a.temp * LOG2E;
-    // fragment addresses inside a stage: the K row of this lane in block (hf, b), the two V rows of its transposing reads
-    const int koff = (8 * (r16 >> 2) + (r16 & 3)) * LDK + 8 * g;        // + (32 hf + 4 b) LDK + 32 c
-    const int voff = (8 * g + (r16 >> 2)) * LDV + 4 * (r16 & 3);        // + 32 hf LDV (+ 4 LDV) + 16 db
-    if (kt_lo < kt_hi) {
-        rk.template stash<LDK>(lds, tid);
-        rv.template stash<LDV>(lds + TKL * LDK, tid);
-    }
+    // K fragments: chunk 4 c + g of row 16 hb + r16; V fragments by transposing reads: rows 4 g + r16 / 4 (+ 16), half r16 % 2 of
+    // chunk 2 db + (r16 % 4) / 2 (the swizzle depends on the row modulo 16 alone)
+    const int trow = 4 * g + (r16 >> 2);
+    int koff[KS], voff[DB];
+#pragma unroll
+    for (int c = 0; c < KS; ++c) koff[c] = r16 * ROWB + x3_swz(r16, 4 * c + g, ROWB) * 16;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) voff[db] = trow * ROWB + x3_swz(trow, 2 * db + ((r16 & 3) >> 1), ROWB) * 16 + 8 * (r16 & 1);
+    drain_loads();
     __syncthreads();
-    for (int kt = kt_lo; kt < kt_hi; ++kt) {
-        const int s_base = kt * TKL, cur = (kt - kt_lo) & 1;
-        const uint16_t* Ks = lds + cur * STAGE;
-        const uint16_t* Vs = Ks + TKL * LDK;
-        const bool more = kt + 1 < kt_hi;
-        if (more) {
-            rk.fetch(kptr, a.k_ss, s_base + TKL, a.S - 1, tid);
-            rv.fetch(vptr, a.v_ss, s_base + TKL, a.S - 1, tid);
-        }
-        // (wave-uniform, scalar: w is) does the tile touch the band of one of the wave's queries; does it lie inside all
-        const bool any = !(s_base + TKL - 1 - qw0 < -lc_lo || s_base - (qw0 + QW - 1) >= lc_hi || s_base >= len);
+    // the tiles that touch the band of one of the wave's queries lie in a row (wave-uniform, scalar: w is): the loop over them
+    // has no branch around its products, which would cost a copy of every accumulator per tile
+    const int w_last = min(qw0 + QW, a.T) - 1;
+    const int w_lo = w_last < qw0 ? kt_hi : max(kt_lo, max(0, qw0 - lc_lo) / TKL);
+    const int w_hi = w_last < qw0 ? kt_hi : min(kt_hi, (max(0, min(len, w_last + lc_hi)) + TKL - 1) / TKL);
+    int kt = kt_lo;
+    auto begin_tile = [&]() __attribute__((always_inline)) {
+        if (kt + 1 < kt_hi) fetch(kt + 1, (kt + 1 - kt_lo) & 1);
+    };
+    auto end_tile = [&]() __attribute__((always_inline)) {
+        drain_loads();                                       // this wave's share of the next tile is in LDS
+        __syncthreads();
+    };
+    for (; kt < w_lo; ++kt) { begin_tile(); end_tile(); }
+    for (; kt < w_hi; ++kt) {
+        const int s_base = kt * TKL;
+        const char* Ks = lds + ((kt - kt_lo) & 1) * 2 * TILE;
+        const char* Vs = Ks + TILE;
+        begin_tile();
+        // (wave-uniform, scalar) does the tile lie inside the band of all of the wave's queries
         const bool inside = s_base - (qw0 + QW - 1) >= -lc_lo && s_base + TKL - 1 - qw0 < lc_hi && s_base + TKL <= len &&
                             qw0 + QW - 1 < a.T;
-        if (any) {
-            floatx4 s1[QB][4];                           // block 2 hf + b, unscaled
+        {
+            floatx4 s1[QB][4];                           // 16-key block hb, unscaled
 #pragma unroll
             for (int qq = 0; qq < QB; ++qq)
 #pragma unroll
@@ -2800,7 +2816,7 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
             for (int hb = 0; hb < 4; ++hb)
 #pragma unroll
                 for (int c = 0; c < KS; ++c) {
-                    const uint4 kf = *reinterpret_cast<const uint4*>(Ks + koff + (32 * (hb >> 1) + 4 * (hb & 1)) * LDK + 32 * c);
+                    const uint4 kf = *reinterpret_cast<const uint4*>(Ks + 16 * hb * ROWB + koff[c]);
 #pragma unroll
                     for (int qq = 0; qq < QB; ++qq) s1[qq][hb] = Frag32<T>::mma(kf, qb[qq][c], s1[qq][hb]);
                 }
@@ -2812,7 +2828,7 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
                     for (int hb = 0; hb < 4; ++hb)
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const int s = s_base + 32 * (hb >> 1) + 8 * g + 4 * (hb & 1) + i;
+                            const int s = s_base + 16 * hb + 4 * g + i;
                             // (an absorbing entry becomes -2^80: its product with the scale is exact, so the multiply-add
                             //  of the exponent below gives exactly 0 for a row whose keys are all hidden)
                             if ((unsigned)(s - smin[qq]) < span[qq])
@@ -2827,7 +2843,7 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
                     for (int hb = 0; hb < 4; ++hb)
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const int s = s_base + 32 * (hb >> 1) + 8 * g + 4 * (hb & 1) + i;
+                            const int s = s_base + 16 * hb + 4 * g + i;
                             if (!((unsigned)(s - smin[qq]) < span[qq])) s1[qq][hb][i] = -INFINITY;
                         }
             }
@@ -2870,7 +2886,7 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
                     for (int hb = 0; hb < 4; ++hb)
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
-                            if (!drop_keep(drop_row[qq], (uint32_t)(s_base + 32 * (hb >> 1) + 8 * g + 4 * (hb & 1) + i), a.drop_thresh))
+                            if (!drop_keep(drop_row[qq], (uint32_t)(s_base + 16 * hb + 4 * g + i), a.drop_thresh))
                                 s1[qq][hb][i] = 0.f;
             }
 #pragma unroll
@@ -2883,21 +2899,16 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
                                         pack_pair<T>(s1[qq][2 * hf + 1][2], s1[qq][2 * hf + 1][3]));
 #pragma unroll
                 for (int db = 0; db < DB; ++db) {
-                    const uint16_t* vp = Vs + voff + 32 * hf * LDV + 16 * db;
-                    const uint4 va = __builtin_bit_cast(uint4, lds_read_tr8(reinterpret_cast<const char*>(vp),
-                                                                             reinterpret_cast<const char*>(vp + 4 * LDV)));
+                    const char* vp = Vs + 32 * hf * ROWB + voff[db];
+                    const uint4 va = __builtin_bit_cast(uint4, lds_read_tr8(vp, vp + 16 * ROWB));
 #pragma unroll
                     for (int qq = 0; qq < QB; ++qq) oacc[qq][db] = Frag32<T>::mma(va, pb[qq], oacc[qq][db]);
                 }
             }
         }
-        if (more) {
-            uint16_t* nxt = lds + (cur ^ 1) * STAGE;
-            rk.template stash<LDK>(nxt, tid);
-            rv.template stash<LDV>(nxt + TKL * LDK, tid);
-        }
-        __syncthreads();
+        end_tile();
     }
+    for (; kt < kt_hi; ++kt) { begin_tile(); end_tile(); }
 #pragma unroll
     for (int qq = 0; qq < QB; ++qq) {
         float z = group_sum(ze[qq]);
@@ -2935,7 +2946,9 @@ template <> __device__ __forceinline__ float unpack_lo<bf16_t>(uint32_t w) { ret
 template <> __device__ __forceinline__ float unpack_hi<bf16_t>(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 template <> __device__ __forceinline__ float unpack_lo<f16_t>(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(w & 0xffffu)); }
 template <> __device__ __forceinline__ float unpack_hi<f16_t>(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)); }
-template <int E> constexpr size_t local_bwd_smem() { return (size_t)2 * (TKL * 2 * (E + 8) * 2 + 2 * TKL * sizeof(float)); }
+// one stage of inner rows: both tiles, 2 E bytes a row with 16-byte chunks swizzled, then (key-major) lse log2e and -delta
+template <int E> constexpr int local_bwd_stage() { return TKL * 2 * (2 * E) + 2 * TKL * (int)sizeof(float); }
+template <int E> constexpr size_t local_bwd_smem() { return (size_t)2 * local_bwd_stage<E>(); }
 
 // EXACT (bfloat16): the exact part of a Scatterbrain-local backward.  lse is the log-normaliser of all keys and delta is
 // given; P and dS enter the second products as three bf16 pieces (exactly), and the low-rank part of the gradient is added
@@ -2943,8 +2956,7 @@ template <int E> constexpr size_t local_bwd_smem() { return (size_t)2 * (TKL * 2
 template <typename T, int E, bool KEYMAJOR, int QB, bool EXACT = false>
 __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
     static_assert(sizeof(T) == 2 && E % 32 == 0, "2-byte inputs, whole MFMA steps");
-    constexpr int LD = E + 8, KS = E / 32, EB = E / 16;
-    constexpr int STAGE_BYTES = TKL * 2 * LD * 2 + 2 * TKL * (int)sizeof(float);
+    constexpr int KS = E / 32, EB = E / 16, ROWB = 2 * E, TILE = TKL * ROWB, STAGE_BYTES = local_bwd_stage<E>();
     constexpr int QW = 16 * QB, TQB = 4 * QW;          // outer rows per wave, per workgroup
     constexpr float LOG2E = 1.4426950408889634f;
     extern __shared__ __attribute__((aligned(128))) float smem[];
@@ -2977,33 +2989,33 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
     const int o_last = min(min(o0 + TQB - 1, R_out - 1), Lo - 1);
     const int lo = max(0, o0 - A), hi = o_last >= o0 ? min(Ln, o_last + Bq) : 0;
     const int it_lo = lo / TKL, it_hi = (hi > lo) ? (hi + TKL - 1) / TKL : it_lo;
-    Tile16<TKL, E, NT> r1, r2;
-    float rl = 0.f, rd = 0.f;                          // key-major: lse log2e and delta of inner row tid (threads 0 .. 63)
-    auto fetch = [&](int it) __attribute__((always_inline)) {
-        r1.fetch(y1p, y1s, it * TKL, R_in - 1, tid);
-        r2.fetch(y2p, y2s, it * TKL, R_in - 1, tid);
+    RowsToLds<TKL, E, NT> r1, r2;
+    r1.init(y1p, y1s, R_in - 1, w, lane);
+    r2.init(y2p, y2s, R_in - 1, w, lane);
+    float rl = 0.f, rd = 0.f;                          // key-major: lse log2e and -delta of inner row tid (threads 0 .. 63)
+    auto fetch = [&](int it, int stage) __attribute__((always_inline)) {
+        char* st = lds + stage * STAGE_BYTES;
+        r1.fetch(it * TKL, st, w, lane);
+        r2.fetch(it * TKL, st + TILE, w, lane);
         if (KEYMAJOR && tid < TKL) {
             const int i = min(it * TKL + tid, a.T - 1);
-            rl = lsep[i] * LOG2E;
+            rl = lsep[i];
             rd = delp[i];
         }
     };
-    auto stash = [&](int stage) __attribute__((always_inline)) {
-        uint16_t* t1 = reinterpret_cast<uint16_t*>(lds + stage * STAGE_BYTES);
-        r1.template stash<LD>(t1, tid);
-        r2.template stash<LD>(t1 + TKL * LD, tid);
+    auto stash = [&](int stage) __attribute__((always_inline)) {       // (the arithmetic here: the loads have the tile's work to arrive in)
         if (KEYMAJOR && tid < TKL) {
-            float* sc_ = reinterpret_cast<float*>(lds + stage * STAGE_BYTES + TKL * 2 * LD * 2);
-            sc_[tid] = rl;
-            sc_[TKL + tid] = rd;
+            float* sc_ = reinterpret_cast<float*>(lds + stage * STAGE_BYTES + 2 * TILE);
+            sc_[tid] = rl * LOG2E;
+            sc_[TKL + tid] = -rd;
         }
     };
-    if (it_lo < it_hi) fetch(it_lo);
+    if (it_lo < it_hi) fetch(it_lo, 0);
 
     int io[QB], vmin[QB];
     unsigned vspan[QB];
     uint4 x1[QB][KS], x2[QB][KS];
-    float l_own[QB], d_own[QB];
+    float l_own[QB], d_own[QB];                        // query-major: lse log2e and -delta of the lane's queries
     floatx4 acc1[QB][EB], acc2[KEYMAJOR ? QB : 1][KEYMAJOR ? EB : 1];     // d q | d k, and d v
 #pragma unroll
     for (int qq = 0; qq < QB; ++qq) {
@@ -3020,7 +3032,7 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
         if (!KEYMAJOR) {
             l_own[qq] = lsep[min(io[qq], a.T - 1)] * LOG2E;
         }
-        if (EXACT && !KEYMAJOR) d_own[qq] = delp[min(io[qq], a.T - 1)];
+        if (EXACT && !KEYMAJOR) d_own[qq] = -delp[min(io[qq], a.T - 1)];
         if (!EXACT && !KEYMAJOR) {
             // delta of the query, g . out, from the output row in the layout of the gradient row; kept for the key-major launch
             const uint16_t* orow = reinterpret_cast<const uint16_t*>(a.out) + b * a.o_sb + h * a.o_sh + row * a.o_ss;
@@ -3033,8 +3045,9 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
                 for (int x = 0; x < 4; ++x)
                     dsum += unpack_lo<T>(ow[x]) * unpack_lo<T>(gw[x]) + unpack_hi<T>(ow[x]) * unpack_hi<T>(gw[x]);
             }
-            d_own[qq] = group_sum(dsum);
-            if (g == 0 && io[qq] < a.T) a.delta[(long)bh * a.T + io[qq]] = d_own[qq];
+            dsum = group_sum(dsum);
+            d_own[qq] = -dsum;
+            if (g == 0 && io[qq] < a.T) a.delta[(long)bh * a.T + io[qq]] = dsum;
         }
 #pragma unroll
         for (int eb = 0; eb < EB; ++eb) acc1[qq][eb] = Frag<float>::zero();
@@ -3046,94 +3059,118 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
             for (int eb = 0; eb < EB; ++eb) acc2[qq][eb] = Frag<float>::zero();
     }
     const float sc = a.temp * LOG2E;
-    const int foff = (8 * (r16 >> 2) + (r16 & 3)) * LD + 8 * g;         // + (32 hf + 4 b) LD + 32 c   (elements)
-    const int toff = (8 * g + (r16 >> 2)) * LD + 4 * (r16 & 3);         // + 32 hf LD (+ 4 LD) + 16 eb
+    // row fragments (scores, g.v): chunk 4 c + g of row 16 kb + r16; transposing reads: rows 4 g + r16 / 4 (+ 16), half
+    // r16 % 2 of chunk 2 eb + (r16 % 4) / 2.  The swizzle depends on the row modulo 16 alone, so 16 kb (32 hf) are offsets.
+    const int trow = 4 * g + (r16 >> 2);
+    int foff[KS], toff[EB];
+#pragma unroll
+    for (int c = 0; c < KS; ++c) foff[c] = r16 * ROWB + x3_swz(r16, 4 * c + g, ROWB) * 16;
+#pragma unroll
+    for (int eb = 0; eb < EB; ++eb) toff[eb] = trow * ROWB + x3_swz(trow, 2 * eb + ((r16 & 3) >> 1), ROWB) * 16 + 8 * (r16 & 1);
     if (it_lo < it_hi) stash(0);
+    drain_loads();
     __syncthreads();
-    for (int it = it_lo; it < it_hi; ++it) {
-        const int i_base = it * TKL, cur = (it - it_lo) & 1;
-        const uint16_t* Y1 = reinterpret_cast<const uint16_t*>(lds + cur * STAGE_BYTES);
-        const uint16_t* Y2 = Y1 + TKL * LD;
-        const float* Ls = reinterpret_cast<const float*>(lds + cur * STAGE_BYTES + TKL * 2 * LD * 2);
-        const bool more = it + 1 < it_hi;
-        if (more) fetch(it + 1);
-        // (wave-uniform, scalar) does the tile touch the band of one of the wave's outer rows; does it lie inside all
-        const bool any = !(i_base + TKL - 1 - ow0 < -A || i_base - (ow0 + QW - 1) >= Bq || i_base >= Ln || ow0 >= Lo);
-        const bool inside = i_base - (ow0 + QW - 1) >= -A && i_base + TKL - 1 - ow0 < Bq && i_base + TKL <= Ln && ow0 + QW - 1 < Lo;
-        if (any) {
-            floatx4 s1[QB][4], gp[QB][4];                // block 2 hf + b: scores (unscaled) and g.v
+    // the tiles that touch the band of one of the wave's outer rows lie in a row (wave-uniform, scalar): the loop over them has
+    // no branch around its products, which would cost a copy of every accumulator per tile
+    const int w_last = min(ow0 + QW, Lo) - 1;
+    const int w_lo = w_last < ow0 ? it_hi : max(it_lo, (max(0, ow0 - A)) / TKL);
+    const int w_hi = w_last < ow0 ? it_hi : min(it_hi, (max(0, min(Ln, w_last + Bq)) + TKL - 1) / TKL);
+    int it = it_lo;
+    auto begin_tile = [&]() __attribute__((always_inline)) {
+        if (it + 1 < it_hi) fetch(it + 1, (it + 1 - it_lo) & 1);
+    };
+    auto end_tile = [&]() __attribute__((always_inline)) {
+        if (it + 1 < it_hi) stash((it + 1 - it_lo) & 1);
+        drain_loads();                                     // this wave's share of the next tile is in LDS
+        __syncthreads();
+    };
+    for (; it < w_lo; ++it) { begin_tile(); end_tile(); }
+    for (; it < w_hi; ++it) {
+        const char* Y1 = lds + ((it - it_lo) & 1) * STAGE_BYTES;
+        const char* Y2 = Y1 + TILE;
+        const float* Ls = reinterpret_cast<const float*>(Y2 + TILE);
+        begin_tile();
 #pragma unroll
-            for (int qq = 0; qq < QB; ++qq)
+        for (int hf = 0; hf < 2; ++hf) {
+            const int i_base = it * TKL + 32 * hf;
+            // (wave-uniform, scalar) do these 32 rows lie inside the band of all of the wave's outer rows
+            const bool inside = i_base - (ow0 + QW - 1) >= -A && i_base + 31 - ow0 < Bq && i_base + 32 <= Ln && ow0 + QW - 1 < Lo;
+            {
+                floatx4 s1[QB][2], gp[QB][2], ln4[2], dl4[2];        // 16-row block kb: scores (unscaled), g.v - delta
 #pragma unroll
-                for (int hb = 0; hb < 4; ++hb) { s1[qq][hb] = Frag<float>::zero(); gp[qq][hb] = Frag<float>::zero(); }
-#pragma unroll
-            for (int hb = 0; hb < 4; ++hb)
-#pragma unroll
-                for (int c = 0; c < KS; ++c) {
-                    const int off = foff + (32 * (hb >> 1) + 4 * (hb & 1)) * LD + 32 * c;
-                    const uint4 f1 = *reinterpret_cast<const uint4*>(Y1 + off);
-                    const uint4 f2 = *reinterpret_cast<const uint4*>(Y2 + off);
+                for (int kb = 0; kb < 2; ++kb) {
+                    if (KEYMAJOR) {                      // the queries' lse log2e and -delta, by block
+                        ln4[kb] = *reinterpret_cast<const floatx4*>(Ls + 32 * hf + 16 * kb + 4 * g);
+                        dl4[kb] = *reinterpret_cast<const floatx4*>(Ls + TKL + 32 * hf + 16 * kb + 4 * g);
+                    }
 #pragma unroll
                     for (int qq = 0; qq < QB; ++qq) {
-                        s1[qq][hb] = Frag32<T>::mma(f1, x1[qq][c], s1[qq][hb]);
-                        gp[qq][hb] = Frag32<T>::mma(f2, x2[qq][c], gp[qq][hb]);
+                        s1[qq][kb] = Frag<float>::zero();
+                        gp[qq][kb] = KEYMAJOR ? dl4[kb] : floatx4{d_own[qq], d_own[qq], d_own[qq], d_own[qq]};
                     }
                 }
-            floatx4 ln4[4], dl4[4];                      // key-major: the queries' lse log2e and delta, by block
-            if (KEYMAJOR) {
 #pragma unroll
-                for (int hb = 0; hb < 4; ++hb) {
-                    ln4[hb] = *reinterpret_cast<const floatx4*>(Ls + 32 * (hb >> 1) + 8 * g + 4 * (hb & 1));
-                    dl4[hb] = *reinterpret_cast<const floatx4*>(Ls + TKL + 32 * (hb >> 1) + 8 * g + 4 * (hb & 1));
-                }
-            }
-            // weights P into s1, dS into gp
+                for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int qq = 0; qq < QB; ++qq)
+                    for (int c = 0; c < KS; ++c) {
+                        const uint4 f1 = *reinterpret_cast<const uint4*>(Y1 + (32 * hf + 16 * kb) * ROWB + foff[c]);
 #pragma unroll
-                for (int hb = 0; hb < 4; ++hb)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int n = i_base + 32 * (hb >> 1) + 8 * g + 4 * (hb & 1) + i;
-                        const float lrow = KEYMAJOR ? ln4[hb][i] : l_own[qq], drow = KEYMAJOR ? dl4[hb][i] : d_own[qq];
-                        float pr = __builtin_amdgcn_exp2f(fmaf(s1[qq][hb][i], sc, -lrow));
-                        if (!inside && !((unsigned)(n - vmin[qq]) < vspan[qq])) pr = 0.f;
-                        s1[qq][hb][i] = pr;
-                        gp[qq][hb][i] = pr * (gp[qq][hb][i] - drow);
+                        for (int qq = 0; qq < QB; ++qq) s1[qq][kb] = Frag32<T>::mma(f1, x1[qq][c], s1[qq][kb]);
                     }
 #pragma unroll
-            for (int hf = 0; hf < 2; ++hf) {
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int c = 0; c < KS; ++c) {
+                        const uint4 f2 = *reinterpret_cast<const uint4*>(Y2 + (32 * hf + 16 * kb) * ROWB + foff[c]);
+#pragma unroll
+                        for (int qq = 0; qq < QB; ++qq) gp[qq][kb] = Frag32<T>::mma(f2, x2[qq][c], gp[qq][kb]);
+                    }
+                if (!inside) {
+#pragma unroll
+                    for (int qq = 0; qq < QB; ++qq)
+#pragma unroll
+                        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                if (!((unsigned)(i_base + 16 * kb + 4 * g + i - vmin[qq]) < vspan[qq])) s1[qq][kb][i] = -INFINITY;
+                }
+                // weights P into s1, dS into gp
+#pragma unroll
+                for (int qq = 0; qq < QB; ++qq)
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            s1[qq][kb][i] = __builtin_amdgcn_exp2f(fmaf(s1[qq][kb][i], sc, -(KEYMAJOR ? ln4[kb][i] : l_own[qq])));
+                            gp[qq][kb][i] *= s1[qq][kb][i];
+                        }
                 uint4 pb[KEYMAJOR ? QB : 1], sb[QB];
                 Pieces pbx[KEYMAJOR ? QB : 1], sbx[QB];     // (EXACT)
 #pragma unroll
                 for (int qq = 0; qq < QB; ++qq) {
                     if constexpr (EXACT) {
-                        sbx[qq] = split<3>(gp[qq][2 * hf], gp[qq][2 * hf + 1]);
-                        if (KEYMAJOR) pbx[qq] = split<3>(s1[qq][2 * hf], s1[qq][2 * hf + 1]);
+                        sbx[qq] = split<3>(gp[qq][0], gp[qq][1]);
+                        if (KEYMAJOR) pbx[qq] = split<3>(s1[qq][0], s1[qq][1]);
                     } else {
-                        sb[qq] = make_uint4(pack_pair<T>(gp[qq][2 * hf][0], gp[qq][2 * hf][1]), pack_pair<T>(gp[qq][2 * hf][2], gp[qq][2 * hf][3]),
-                                            pack_pair<T>(gp[qq][2 * hf + 1][0], gp[qq][2 * hf + 1][1]),
-                                            pack_pair<T>(gp[qq][2 * hf + 1][2], gp[qq][2 * hf + 1][3]));
+                        sb[qq] = make_uint4(pack_pair<T>(gp[qq][0][0], gp[qq][0][1]), pack_pair<T>(gp[qq][0][2], gp[qq][0][3]),
+                                            pack_pair<T>(gp[qq][1][0], gp[qq][1][1]), pack_pair<T>(gp[qq][1][2], gp[qq][1][3]));
                         if (KEYMAJOR)
-                            pb[qq] = make_uint4(pack_pair<T>(s1[qq][2 * hf][0], s1[qq][2 * hf][1]), pack_pair<T>(s1[qq][2 * hf][2], s1[qq][2 * hf][3]),
-                                                pack_pair<T>(s1[qq][2 * hf + 1][0], s1[qq][2 * hf + 1][1]),
-                                                pack_pair<T>(s1[qq][2 * hf + 1][2], s1[qq][2 * hf + 1][3]));
+                            pb[qq] = make_uint4(pack_pair<T>(s1[qq][0][0], s1[qq][0][1]), pack_pair<T>(s1[qq][0][2], s1[qq][0][3]),
+                                                pack_pair<T>(s1[qq][1][0], s1[qq][1][1]), pack_pair<T>(s1[qq][1][2], s1[qq][1][3]));
                     }
                 }
 #pragma unroll
                 for (int eb = 0; eb < EB; ++eb) {
-                    const uint16_t* p1 = Y1 + toff + 32 * hf * LD + 16 * eb;
-                    const uint4 t1 = __builtin_bit_cast(uint4, lds_read_tr8(reinterpret_cast<const char*>(p1),
-                                                                             reinterpret_cast<const char*>(p1 + 4 * LD)));
+                    const char* p1 = Y1 + 32 * hf * ROWB + toff[eb];
+                    const uint4 t1 = __builtin_bit_cast(uint4, lds_read_tr8(p1, p1 + 16 * ROWB));
 #pragma unroll
                     for (int qq = 0; qq < QB; ++qq) {
                         if constexpr (EXACT) acc1[qq][eb] = mma_pieces(__builtin_bit_cast(uintx4, t1), sbx[qq], acc1[qq][eb]);
                         else acc1[qq][eb] = Frag32<T>::mma(t1, sb[qq], acc1[qq][eb]);
                     }
                     if (KEYMAJOR) {
-                        const uint16_t* p2 = Y2 + toff + 32 * hf * LD + 16 * eb;
-                        const uint4 t2 = __builtin_bit_cast(uint4, lds_read_tr8(reinterpret_cast<const char*>(p2),
-                                                                                 reinterpret_cast<const char*>(p2 + 4 * LD)));
+                        const char* p2 = Y2 + 32 * hf * ROWB + toff[eb];
+                        const uint4 t2 = __builtin_bit_cast(uint4, lds_read_tr8(p2, p2 + 16 * ROWB));
 #pragma unroll
                         for (int qq = 0; qq < QB; ++qq) {
                             if constexpr (EXACT) acc2[qq][eb] = mma_pieces(__builtin_bit_cast(uintx4, t2), pbx[qq], acc2[qq][eb]);
@@ -3143,9 +3180,9 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
                 }
             }
         }
-        if (more) stash(cur ^ 1);
-        __syncthreads();
+        end_tile();
     }
+    for (; it < it_hi; ++it) { begin_tile(); end_tile(); }
 #pragma unroll
     for (int qq = 0; qq < QB; ++qq) {
         if (io[qq] < R_out) {
@@ -4630,11 +4667,13 @@ static int launch_local_b16_as(const LocalArgs& a, hipStream_t st) {
 // 32 queries per wave once workgroups of 128 queries still fill the device twice over (three of them share a compute
 // unit; measured at 2.7 rounds: 0.152 -> 0.129 ms at 16 heads of 16384 tokens; head dims up to 64: the wide form's
 // accumulators and score sets need the registers)
+static bool local_b16_wide(int B, int H, int T) {
+    return FLY_LOCAL_B16_WIDE && (long)B * H * ((T + 127) / 128) >= (long)FLY_LOCAL_B16_WIDE_ROUNDS * 3 * machine().cus;
+}
 template <typename T, int E>
 static int launch_local_b16(const LocalArgs& a, hipStream_t st) {
     if constexpr (E <= 64) {
-        const long wide_items = (long)a.B * a.H * ((a.T + 127) / 128);
-        if (FLY_LOCAL_B16_WIDE && wide_items >= (long)FLY_LOCAL_B16_WIDE_ROUNDS * 3 * machine().cus) return launch_local_b16_as<T, E, 2>(a, st);
+        if (local_b16_wide(a.B, a.H, a.T)) return launch_local_b16_as<T, E, 2>(a, st);
     }
     return launch_local_b16_as<T, E, 1>(a, st);
 }
@@ -4644,9 +4683,6 @@ static bool local_b16_ready(const LocalArgs& a) {
     return FLY_LOCAL_B16 && strides % 8 == 0 && ptrs % 16 == 0;
 }
 
-#ifndef FLY_LOCAL_BWD_QB
-#define FLY_LOCAL_BWD_QB 1
-#endif
 template <typename T, int E, bool KEYMAJOR, int QB, bool EXACT = false>
 static int launch_local_bwd_as(const LocalBwdArgs& a, hipStream_t st) {
     auto kern = local_bwd_b16_kernel<T, E, KEYMAJOR, QB, EXACT>;
@@ -4665,9 +4701,13 @@ static int launch_local_bwd_as(const LocalBwdArgs& a, hipStream_t st) {
 }
 template <typename T, int E>
 static int launch_local_bwd(const LocalBwdArgs& a, hipStream_t st) {
-    // (query-major first: it leaves delta for the key-major launch)
-    if (int rc = launch_local_bwd_as<T, E, false, FLY_LOCAL_BWD_QB>(a, st)) return rc;
-    return launch_local_bwd_as<T, E, true, FLY_LOCAL_BWD_QB>(a, st);
+    // query-major first: it leaves delta for the key-major launch
+    // (query-major with 32 queries per wave on the same rule as the forward, 3 % of the training step at 24 heads of 10007 tokens;
+    //  key-major, with two sums to hold, would be left with two waves per SIMD and gains nothing)
+    int rc;
+    if constexpr (E <= 64) rc = local_b16_wide(a.B, a.H, a.T) ? launch_local_bwd_as<T, E, false, 2>(a, st) : launch_local_bwd_as<T, E, false, 1>(a, st);
+    else rc = launch_local_bwd_as<T, E, false, 1>(a, st);
+    return rc ? rc : launch_local_bwd_as<T, E, true, 1>(a, st);
 }
 
 int launch_local_bwd_exact(const LocalBwdArgs& a, int E, hipStream_t st) {

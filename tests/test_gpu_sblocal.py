@@ -1319,3 +1319,34 @@ def test_local_attention_float32_with_infinities(where, value, masked, p_drop, E
         assert float(((a - r).abs() / (1e-5 + 1e-4 * r.abs()))[small].max()) <= 1.0, name
         if bool((ok & ~small).any()):
             assert float(((a - r).abs() / r.abs())[ok & ~small].max()) <= 1e-4, name
+
+
+@pytest.mark.parametrize('E,far_apart', [(64, False), (32, False), (64, True)])
+def test_local_attention_gradients_with_tiles_moved_straight_into_lds(E, far_apart):
+    """The 2-byte local attention kernels: a last tile that ends inside the 64 rows, key lengths, and enough rows for two blocks
+    of queries per wave in the query-major gradient -- or rows so far apart in memory (2^24 elements) that the offsets of a tile
+    no longer fit 32 bits.  Two (batch, head) pairs against autograd through the oracle."""
+    from fly_amd import LocalAttention, LengthMask
+    dev = torch.device('cuda:0')
+    B, L, H, lc = (1, 83, 2, 50) if far_apart else (8, 3037, 16, 70)
+    print('case', E, far_apart, flush=True)
+    g = torch.Generator().manual_seed(67)
+    q, k, v, w = (torch.randn(B, L, H, E, generator=g).bfloat16() for _ in range(4))
+    lens = torch.full((B,), L)
+    lens[B - 1] = L * 3 // 4
+
+    def place(x):
+        if not far_apart:
+            return x.to(dev)
+        return torch.zeros(L << 24, dtype=x.dtype, device=dev).as_strided((B, L, H, E), (0, 1 << 24, E, 1)).copy_(x)
+
+    leaves = [place(x).requires_grad_() for x in (q, k, v)]
+    out, _ = LocalAttention(lc).to(dev)(*leaves, key_padding_mask=LengthMask(lens.to(dev), max_len=L))
+    grads = torch.autograd.grad(out, leaves, place(w))
+    for b, h in ((0, H - 1), (B - 1, 0)):
+        ref = [x[b:b + 1, :, h:h + 1].double().requires_grad_() for x in (q, k, v)]
+        ref_out = osb.local_attention(*ref, lc, key_lengths=lens[b:b + 1])
+        ref_grads = torch.autograd.grad(ref_out, ref, w[b:b + 1, :, h:h + 1].double())
+        assert rel_err(out[b, :, h].float().cpu(), ref_out[0, :, 0].detach()) <= 2e-2
+        for got, r in zip(grads, ref_grads):
+            assert rel_err(got[b, :, h].float().cpu(), r[0, :, 0]) <= 3e-2
