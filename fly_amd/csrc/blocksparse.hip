@@ -1990,7 +1990,8 @@ __global__ __launch_bounds__(64 * NW) void bs_attn32_kernel(const AttnArgs a) {
             for (int qt = 0; qt < 2; ++qt) {
                 const floatx4 s0 = sc[0][qt], s1 = sc[1][qt];
                 const float mx = group_max_finite(max8_finite(s0, s1)) * scale2;
-                if (__builtin_amdgcn_ballot_w64(mx > m_run[qt] + LAZY) != 0) {      // wave-uniform: some row maximum grew a lot
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(mx > m_run[qt] + LAZY) != 0, 0)) {      // wave-uniform: some row maximum grew a lot
+                    asm volatile("");                        // (stays a branch: the compiler would do the multiplications always)
                     const float m_new = fmaxf(m_run[qt], mx);
                     const float alpha = __builtin_amdgcn_exp2f(m_run[qt] - m_new);
                     m_run[qt] = m_new;
@@ -2022,7 +2023,8 @@ __global__ __launch_bounds__(64 * NW) void bs_attn32_kernel(const AttnArgs a) {
                 float mx = fmaxf(fmaxf(fmaxf(t0[0], t0[1]), t0[2]), fmaxf(fmaxf(t0[3], t1[0]), t1[1]));
                 mx = fmaxf(fmaxf(mx, t1[2]), t1[3]);
                 mx = group_max(mx);
-                if (__builtin_amdgcn_ballot_w64(mx > m_run[qt] + LAZY) != 0) {
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(mx > m_run[qt] + LAZY) != 0, 0)) {
+                    asm volatile("");
                     const float m_new = fmaxf(m_run[qt], mx);
                     const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run[qt] - m_new);
                     m_run[qt] = m_new;
@@ -2059,9 +2061,9 @@ __global__ __launch_bounds__(64 * NW) void bs_attn32_kernel(const AttnArgs a) {
     int inner_cur[CP], inner_n1[CP], blk_cur[CP];
 #pragma unroll
     for (int j = 0; j < CP; ++j) {
-        inner_cur[j] = j < n ? a.uni_inner[p0 + j] : 0;
-        inner_n1[j] = CP + j < n ? a.uni_inner[p0 + CP + j] : 0;
-        blk_cur[j] = j < n ? a.uni_blk[(long)(p0 + j) * NW + w] : -1;
+        inner_cur[j] = j < n ? table_entry(a.uni_inner + p0 + j) : 0;
+        inner_n1[j] = CP + j < n ? table_entry(a.uni_inner + p0 + CP + j) : 0;
+        blk_cur[j] = j < n ? table_entry(a.uni_blk + (long)(p0 + j) * NW + w) : -1;
     }
     if (n > 0) {
 #pragma unroll
@@ -2075,8 +2077,8 @@ __global__ __launch_bounds__(64 * NW) void bs_attn32_kernel(const AttnArgs a) {
         int inner_n2[CP], blk_n1[CP];
 #pragma unroll
         for (int j = 0; j < CP; ++j) {
-            inner_n2[j] = s2 + j < n ? a.uni_inner[p0 + s2 + j] : 0;
-            blk_n1[j] = s1 + j < n ? a.uni_blk[(long)(p0 + s1 + j) * NW + w] : -1;
+            inner_n2[j] = s2 + j < n ? table_entry(a.uni_inner + p0 + s2 + j) : 0;
+            blk_n1[j] = s1 + j < n ? table_entry(a.uni_blk + (long)(p0 + s1 + j) * NW + w) : -1;
         }
 #pragma unroll
         for (int j = 0; j < CP; ++j)
@@ -2683,21 +2685,24 @@ struct AttnBwdArgs {
     const float* key_mask; long km_stride; const float* attn_mask; long am_stride;
 };
 
-// (registers for three waves per SIMD: the key-major form at 64 dims takes 176 without the bound, two waves per SIMD,
-//  and runs 7 % slower; with the dropout hashes it would spill 24 registers inside the loop at that bound -- 703 us
-//  against 365 without dropout -- and keeps two waves; a two-step register prefetch of the tiles costs more registers
-//  than it hides latency)
+// Bound by the vector ALU (70 % of the cycles query-major with dropout, 60 % key-major) and the matrix pipe (26 - 43 %) taking turns at
+// two to three waves per SIMD; LDS 15 - 27 %, without bank conflicts since the tiles go straight into LDS with swizzled rows.
+// B=8, 12 heads of 4096 tokens, 64 dims, training step in bfloat16: 797 -> 727 us, with dropout 1077 -> 1003 (tiles by way of
+// registers into padded rows, list entries by vector loads, a product per pair for the dropout scale before).
+// (registers for three waves per SIMD: the key-major form at 64 dims takes more without the bound, two waves per SIMD; with the
+//  dropout hashes it would spill inside the loop at that bound and keeps two.  Measured and not kept: tiles asked for two steps
+//  ahead, 2 % slower; one outer block after the other with fragment reads of its own, which leaves room for a fourth wave
+//  query-major, 5 % slower, as are four waves with spills)
 // MASKED: a variant of its own, so that the kernels without masks carry nothing of them (as a kernel-uniform branch the
 // mask code cost the key-major form 35 more spilled registers and the query-major form a wave per SIMD)
 template <typename T, int E, bool KEYMAJOR, bool DROP = false, bool MASKED = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR && (DROP || MASKED) ? 2 : 3, 8))) void bs_attn32_bwd_kernel(const AttnBwdArgs a) {
     static_assert(!(DROP && MASKED), "the forward with masks has no dropout");
     static_assert(sizeof(T) == 2 && E % 32 == 0, "2-byte inputs, whole MFMA steps");
-    constexpr int LD = E + 8, KS = E / 32, EB = E / 16;
-    constexpr int CPR = E / 8, NCH = (32 * CPR + 255) / 256;        // 16-byte chunks per tile row, per thread
+    constexpr int KS = E / 32, EB = E / 16, ROWB = 2 * E, TILE = 32 * ROWB;
     constexpr float LOG2E = 1.4426950408889634f;
-    __shared__ __attribute__((aligned(16))) uint16_t tiles[2][2][32 * LD];      // [stage][Y1 | Y2]
-    __shared__ __attribute__((aligned(16))) float rowv[2][3][32];              // key-major: [stage][lse2 | delta | row hash] of the tile's queries
+    __shared__ __attribute__((aligned(128))) char tiles[2][2][TILE];            // [stage][Y1 | Y2], rows as RowsToLds leaves them
+    __shared__ __attribute__((aligned(16))) float rowv[2][3][32];              // key-major: [stage][lse2 | delta (DROP: / drop_scale) | row hash] of the tile's queries
     const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     int unit, grp;
@@ -2721,8 +2726,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
     const long d1s = KEYMAJOR ? a.dk_sm : a.dq_sm;
     T* d2 = reinterpret_cast<T*>(a.dv) + z * a.dv_sz + head * a.dv_sh;
 
+    // dS = P (M g.v - delta), M = drop_scale or 0, is formed as -drop_scale P (delta / drop_scale - kept g.v): the sums start at
+    // delta / drop_scale and x2 goes in negated, so that a pair costs one select and one product, and the factor is the epilogue's
+    const float inv_drop = DROP ? 1.0f / a.drop_scale : 1.0f;
     uintx4 x1[2][KS], x2[2][KS];
-    float l_own[2] = {0.f, 0.f}, d_own[2] = {0.f, 0.f};
+    float l_own[2] = {0.f, 0.f}, d_own[2] = {0.f, 0.f};          // query-major: lse2 and delta of the lane's queries
     float km_own[2] = {0.f, 0.f};                     // key-major: the key mask entries of the lane's keys
     uint32_t h_own[2] = {0u, 0u};                     // DROP, query-major: hash of (seed, global row) of the lane's queries
     floatx4 acc1[2][EB], acc2[KEYMAJOR ? 2 : 1][KEYMAJOR ? EB : 1];     // d q | d k, and d v
@@ -2752,9 +2760,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
                     part += Elem<T>::to_f32(x) * Elem<T>::to_f32(y);
                 }
             }
-            d_own[qq] = group_sum(part);
-            if (have && g == 0) a.delta[qvec + row] = d_own[qq];
+            part = group_sum(part);
+            d_own[qq] = DROP ? part * inv_drop : part;
+            if (have && g == 0) a.delta[qvec + row] = part;
         }
+#pragma unroll
+        for (int c = 0; c < KS; ++c) x2[qq][c] ^= 0x80008000u;
 #pragma unroll
         for (int eb = 0; eb < EB; ++eb) acc1[qq][eb] = Frag<float>::zero();
     }
@@ -2765,66 +2776,71 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
             for (int eb = 0; eb < EB; ++eb) acc2[qq][eb] = Frag<float>::zero();
     }
 
-    uintx4 r1[NCH], r2[NCH];
+    RowsToLds<32, E, 256> r1, r2;
+    r1.init(y1p, y1s, 32 * a.inner_blocks - 1, w, lane);
+    r2.init(y2p, y2s, 32 * a.inner_blocks - 1, w, lane);
     float rl = 0.f, rd = 0.f;
     uint32_t rh = 0u;
-    auto fetch = [&](int inner) __attribute__((always_inline)) {
-        const long row0 = (long)inner * 32;
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            const int c = tid + 256 * i;
-            if (c < 32 * CPR) {
-                r1[i] = *reinterpret_cast<const uintx4*>(y1p + (row0 + c / CPR) * y1s + 8 * (c % CPR));
-                r2[i] = *reinterpret_cast<const uintx4*>(y2p + (row0 + c / CPR) * y2s + 8 * (c % CPR));
-            }
-        }
+    auto fetch = [&](int inner, int stage) __attribute__((always_inline)) {
+        r1.fetch(32 * inner, tiles[stage][0], w, lane);
+        r2.fetch(32 * inner, tiles[stage][1], w, lane);
         if (KEYMAJOR && tid < 32) {
-            rl = a.lse2[qvec + row0 + tid];
-            rd = a.delta[qvec + row0 + tid];
-            if (DROP) rh = drop_row_hash(a.drop_seed, (uint32_t)(qvec + row0 + tid));
+            const long at = qvec + (long)inner * 32 + tid;
+            rl = a.lse2[at];
+            rd = a.delta[at];
+            if (DROP) rh = drop_row_hash(a.drop_seed, (uint32_t)at);
         }
     };
-    auto stash = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            const int c = tid + 256 * i;
-            if (c < 32 * CPR) {
-                *reinterpret_cast<uintx4*>(&tiles[buf][0][(c / CPR) * LD + 8 * (c % CPR)]) = r1[i];
-                *reinterpret_cast<uintx4*>(&tiles[buf][1][(c / CPR) * LD + 8 * (c % CPR)]) = r2[i];
-            }
-        }
+    auto stash = [&](int stage) __attribute__((always_inline)) {
         if (KEYMAJOR && tid < 32) {
-            rowv[buf][0][tid] = rl;
-            rowv[buf][1][tid] = rd;
-            if (DROP) rowv[buf][2][tid] = __uint_as_float(rh);
+            rowv[stage][0][tid] = rl;
+            rowv[stage][1][tid] = DROP ? rd * inv_drop : rd;
+            if (DROP) rowv[stage][2][tid] = __uint_as_float(rh);
         }
     };
     const float sc = a.scale * LOG2E;
-    const int foff = (8 * (r16 >> 2) + (r16 & 3)) * LD + 8 * g;         // + 4 b LD + 32 c   (elements)
-    const int toff = (8 * g + (r16 >> 2)) * LD + 4 * (r16 & 3);         // (+ 4 LD) + 16 eb
+    // row fragments: chunk 4 c + g of row 16 hb + r16; transposing reads: rows 4 g + r16 / 4 (+ 16), half r16 % 2 of chunk
+    // 2 eb + (r16 % 4) / 2 (the swizzle depends on the row modulo 16 alone)
+    const int trow = 4 * g + (r16 >> 2);
+    int foff[KS], toff[EB];
+#pragma unroll
+    for (int c = 0; c < KS; ++c) foff[c] = r16 * ROWB + x3_swz(r16, 4 * c + g, ROWB) * 16;
+#pragma unroll
+    for (int eb = 0; eb < EB; ++eb) toff[eb] = trow * ROWB + x3_swz(trow, 2 * eb + ((r16 & 3) >> 1), ROWB) * 16 + 8 * (r16 & 1);
+    // (list entries a step ahead of their use)
+    int inner_cur = n > 0 ? table_entry(a.uni_inner + p0) : 0, inner_next = n > 1 ? table_entry(a.uni_inner + p0 + 1) : 0;
+    int blk_cur = n > 0 ? table_entry(a.uni_blk + (long)p0 * 4 + w) : -1;
     if (n > 0) {
-        fetch(a.uni_inner[p0]);
+        fetch(inner_cur, 0);
         stash(0);
     }
+    drain_loads();
     __syncthreads();
     for (int s = 0; s < n; ++s) {
         const int cur = s & 1;
         const bool more = s + 1 < n;
-        if (more) fetch(a.uni_inner[p0 + s + 1]);
-        const bool present = have && a.uni_blk[(long)(p0 + s) * 4 + w] >= 0;      // wave-uniform
+        if (more) fetch(inner_next, cur ^ 1);
+        const int blk_next = table_entry(a.uni_blk + (long)(p0 + min(s + 1, n - 1)) * 4 + w);
+        const int inner_after = table_entry(a.uni_inner + p0 + min(s + 2, n - 1));
+        const bool present = have && blk_cur >= 0;               // wave-uniform
         if (present) {
-            const uint16_t* Y1 = tiles[cur][0];
-            const uint16_t* Y2 = tiles[cur][1];
-            floatx4 s1[2][2], gp[2][2];                  // [outer block][inner block b]: scores (unscaled) and g.v
+            const char* Y1 = tiles[cur][0];
+            const char* Y2 = tiles[cur][1];
+            floatx4 s1[2][2], gp[2][2], nd[2];           // [outer block][inner block hb]: scores (unscaled) and delta - g.v
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq)
+            for (int hb = 0; hb < 2; ++hb) {
+                if (KEYMAJOR) nd[hb] = *reinterpret_cast<const floatx4*>(&rowv[cur][1][16 * hb + 4 * g]);
 #pragma unroll
-                for (int hb = 0; hb < 2; ++hb) { s1[qq][hb] = Frag<float>::zero(); gp[qq][hb] = Frag<float>::zero(); }
+                for (int qq = 0; qq < 2; ++qq) {
+                    s1[qq][hb] = Frag<float>::zero();
+                    gp[qq][hb] = KEYMAJOR ? nd[hb] : floatx4{d_own[qq], d_own[qq], d_own[qq], d_own[qq]};
+                }
+            }
 #pragma unroll
             for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
                 for (int c = 0; c < KS; ++c) {
-                    const int off = foff + 4 * hb * LD + 32 * c;
+                    const int off = 16 * hb * ROWB + foff[c];
                     const uintx4 f1 = *reinterpret_cast<const uintx4*>(Y1 + off);
                     const uintx4 f2 = *reinterpret_cast<const uintx4*>(Y2 + off);
 #pragma unroll
@@ -2833,23 +2849,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
                         gp[qq][hb] = mma32<T>(f2, x2[qq][c], gp[qq][hb]);
                     }
                 }
-            floatx4 ln4[2], dl4[2], hh4[2];              // key-major: the tile's queries' lse2, delta and row hashes, by block
+            floatx4 ln4[2], hh4[2];                      // key-major: the tile's queries' lse2 and row hashes, by block
             if (KEYMAJOR) {
 #pragma unroll
                 for (int hb = 0; hb < 2; ++hb) {
-                    ln4[hb] = *reinterpret_cast<const floatx4*>(&rowv[cur][0][8 * g + 4 * hb]);
-                    dl4[hb] = *reinterpret_cast<const floatx4*>(&rowv[cur][1][8 * g + 4 * hb]);
-                    if (DROP) hh4[hb] = *reinterpret_cast<const floatx4*>(&rowv[cur][2][8 * g + 4 * hb]);
+                    ln4[hb] = *reinterpret_cast<const floatx4*>(&rowv[cur][0][16 * hb + 4 * g]);
+                    if (DROP) hh4[hb] = *reinterpret_cast<const floatx4*>(&rowv[cur][2][16 * hb + 4 * g]);
                 }
             }
-            const int inner_cur = a.uni_inner[p0 + s];
             if constexpr (MASKED) {                                     // the masks, in units of the unscaled scores
                 const float inv_scale = 1.0f / a.scale;
 #pragma unroll
                 for (int qq = 0; qq < 2; ++qq)
 #pragma unroll
                     for (int hb = 0; hb < 2; ++hb) {
-                        const long in0 = (long)inner_cur * 32 + 8 * g + 4 * hb;        // the element's four inner rows
+                        const long in0 = (long)inner_cur * 32 + 16 * hb + 4 * g;        // the element's four inner rows
                         const long orow = (long)bo_c * 32 + 16 * qq + r16;             // its outer row
                         floatx4 add = Frag<float>::zero();
                         if (!KEYMAJOR) {
@@ -2875,23 +2889,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
                                               (uint32_t)bo_c * 32u + 16u * qq + r16, r01, r23);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const float lrow = KEYMAJOR ? ln4[hb][i] : l_own[qq], drow = KEYMAJOR ? dl4[hb][i] : d_own[qq];
+                        const float lrow = KEYMAJOR ? ln4[hb][i] : l_own[qq];
                         const float pr = __builtin_amdgcn_exp2f(fmaf(s1[qq][hb][i], sc, -lrow));   // (a row without scores: lse2 = +inf)
                         if (DROP) {
-                            // (query, key) of the element: the inner row 8 g + 4 hb + i of the tile, the outer row 16 qq + r16
+                            // (query, key) of the element: the inner row 16 hb + 4 g + i of the tile, the outer row 16 qq + r16
                             bool keep;
                             if (KEYMAJOR) {
                                 const uint32_t pair = i < 2 ? r01 : r23;
                                 keep = ((i & 1) ? pair >> 16 : pair & 0xffffu) >= a.drop_thresh;
                             } else {
-                                keep = drop_keep(h_own[qq], (uint32_t)inner_cur * 32u + 8u * g + 4u * hb + i, a.drop_thresh);
+                                keep = drop_keep(h_own[qq], (uint32_t)inner_cur * 32u + 16u * hb + 4u * g + i, a.drop_thresh);
                             }
-                            const float m = keep ? a.drop_scale : 0.f;
-                            s1[qq][hb][i] = m * pr;
-                            gp[qq][hb][i] = pr * (m * gp[qq][hb][i] - drow);
+                            s1[qq][hb][i] = keep ? pr : 0.f;
+                            gp[qq][hb][i] = pr * (keep ? gp[qq][hb][i] : KEYMAJOR ? nd[hb][i] : d_own[qq]);
                         } else {
                             s1[qq][hb][i] = pr;
-                            gp[qq][hb][i] = pr * (gp[qq][hb][i] - drow);
+                            gp[qq][hb][i] *= pr;
                         }
                     }
                 }
@@ -2906,30 +2919,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
             }
 #pragma unroll
             for (int eb = 0; eb < EB; ++eb) {
-                const uint16_t* p1 = Y1 + toff + 16 * eb;
-                const uintx4 t1 = lds_read_tr8(reinterpret_cast<const char*>(p1), reinterpret_cast<const char*>(p1 + 4 * LD));
+                const uintx4 t1 = lds_read_tr8(Y1 + toff[eb], Y1 + toff[eb] + 16 * ROWB);
 #pragma unroll
                 for (int qq = 0; qq < 2; ++qq) acc1[qq][eb] = mma32<T>(t1, sb[qq], acc1[qq][eb]);
                 if (KEYMAJOR) {
-                    const uint16_t* p2 = Y2 + toff + 16 * eb;
-                    const uintx4 t2 = lds_read_tr8(reinterpret_cast<const char*>(p2), reinterpret_cast<const char*>(p2 + 4 * LD));
+                    const uintx4 t2 = lds_read_tr8(Y2 + toff[eb], Y2 + toff[eb] + 16 * ROWB);
 #pragma unroll
                     for (int qq = 0; qq < 2; ++qq) acc2[qq][eb] = mma32<T>(t2, pb[qq], acc2[qq][eb]);
                 }
             }
         }
         if (more) stash(cur ^ 1);
+        inner_cur = inner_next;
+        inner_next = inner_after;
+        blk_cur = blk_next;
+        drain_loads();                                   // this wave's share of the next tile is in LDS
         __syncthreads();
     }
+    const float d1_scale = DROP ? -a.scale * a.drop_scale : -a.scale;
     if (have) {
 #pragma unroll
         for (int qq = 0; qq < 2; ++qq) {
             const long row = (long)bo * 32 + 16 * qq + r16;
 #pragma unroll
-            for (int eb = 0; eb < EB; ++eb) store4_f32(d1 + row * d1s + 16 * eb + 4 * g, acc1[qq][eb] * a.scale);
+            for (int eb = 0; eb < EB; ++eb) store4_f32(d1 + row * d1s + 16 * eb + 4 * g, acc1[qq][eb] * d1_scale);
             if (KEYMAJOR) {
 #pragma unroll
-                for (int eb = 0; eb < EB; ++eb) store4_f32(d2 + row * a.dv_sm + 16 * eb + 4 * g, acc2[qq][eb]);
+                for (int eb = 0; eb < EB; ++eb) store4_f32(d2 + row * a.dv_sm + 16 * eb + 4 * g, DROP ? acc2[qq][eb] * a.drop_scale : acc2[qq][eb]);
             }
         }
     }

@@ -403,6 +403,13 @@ inline DropArgs drop_args(float p, uint64_t seed) {
     return d;
 }
 
+// An entry of a table that no kernel writes, at a wave-uniform address: a scalar load.  Behind a transfer into LDS (assembly that
+// clobbers memory) the compiler otherwise takes a vector load, whose wait also covers every transfer in flight.
+template <typename I>
+__device__ __forceinline__ I table_entry(const I* p) {
+    return *(const __attribute__((address_space(4))) I*)(uintptr_t)p;
+}
+
 // One wave's 1024 bytes straight from global memory into LDS (lane l's 16 bytes land at wave_base + 16 l), issued as
 // assembly: the compiler then does not know of a transfer in flight, and does not drain the load counter in front of
 // LDS reads of the other stage (it does so before every transposing read, whose address it cannot tell from the
@@ -429,12 +436,22 @@ __device__ __forceinline__ void dma_to_lds_at(const void* base, uint32_t lane_of
                  : "=&s"(saved_m0) : "v"(lane_off), "s"(base), "s"(dst) : "memory");
 }
 
+// one float per active lane, lane l's to wave_base + 4 l
+__device__ __forceinline__ void dma_float_to_lds(const float* lane_src, const void* wave_base) {
+    typedef __attribute__((address_space(3))) const char* lds_ptr;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)wave_base);
+    uint32_t saved_m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved_m0) : "v"(lane_src), "s"(dst) : "memory");
+}
+
 // ROWS rows of W 2-byte elements straight into LDS by NT threads, chunk c of a row stored where x3_swz puts it: the transfers
 // fill LDS linearly, so the swizzle is in the addresses they read.  Row indices are clamped to the last row, as in Tile16.
 template <int ROWS, int W, int NT>
 struct RowsToLds {
-    static constexpr int CH = W / 8, N = ROWS * CH / NT, ROWB = 2 * W;
-    static_assert(ROWS * CH % NT == 0, "whole wave transfers");
+    // (fewer chunks than threads: the last waves have nothing to do)
+    static constexpr int CH = W / 8, N = (ROWS * CH + NT - 1) / NT, ROWB = 2 * W;
+    static_assert(ROWS * CH % (ROWS * CH < NT ? 64 : NT) == 0, "whole wave transfers");
     uint32_t off[N];
     const uint16_t* src; long stride; int last;
     __device__ __forceinline__ void init(const uint16_t* src_, long stride_, int last_row, int w, int lane) {
@@ -446,6 +463,7 @@ struct RowsToLds {
         }
     }
     __device__ __forceinline__ void fetch(int row0, const char* dst, int w, int lane) const {
+        if (ROWS * CH < NT && w >= ROWS * CH / 64) return;
         // (uniform) all rows exist and the offsets fit 32 bits
         if (row0 + ROWS - 1 <= last && stride < (1 << 24)) {
             const uint16_t* base = src + row0 * stride;
