@@ -555,10 +555,18 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
         if (nx == e0) nx = max(nx, e1);                                             // (over the chunks inside the band)
         if (AHEAD && nx < c1) t.fetch(a, KEYMAJOR, xip, xis, yip, yis, bh, nx * FC, len_i, base, kappa, tid);
         __syncthreads();
+        // (uniform) do the pairs of inner rows 32 st .. + 31 and outer rows 16 ob .. + 15 all lie in the band: a quarter of a chunk at a
+        // window that is a multiple of 128, half on average otherwise.  (16 heads of 16384 tokens, window 1024, 256 features, training step:
+        // 2108 -> 2071 us without their products)
+        auto band_only = [&](int st, int ob) __attribute__((always_inline)) {
+            const int rel = n0 + 32 * st - (o0 + 16 * ob);
+            return rel - 15 >= -A && rel + 31 < Bq;
+        };
         // df = g.v - c on the pairs outside the band, 0 inside: inner rows 32 st + 16 hb + 4 g + i, outer row 16 ob + r16 --
         // eight contraction slots of the products below -- in pieces
         for (int it = w; it < 8; it += NW) {
             const int st = it >> 2, ob = it & 3;
+            if (band_only(st, ob)) continue;
             floatx4 s[2] = {Frag<float>::zero(), Frag<float>::zero()};
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
@@ -602,6 +610,7 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int ob = 0; ob < 4; ++ob) {
+                if (band_only(st, ob)) continue;
                 const Pieces df = {{DF[(4 * st + ob) * 64 + lane], DF[(8 + 4 * st + ob) * 64 + lane], DF[(16 + 4 * st + ob) * 64 + lane]}};
 #pragma unroll
                 for (int sg = 0; sg < 2; ++sg) acc2[sg][ob] = mma_pieces(fp[sg], df, acc2[sg][ob]);
@@ -633,6 +642,7 @@ __global__ __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(!KEYMAJOR
                 __builtin_amdgcn_sched_barrier(0);          // (the steps' operands do not fit the registers side by side)
 #pragma unroll
                 for (int ob = 0; ob < 4; ++ob) {
+                    if (band_only(st, ob)) continue;
                     floatx4 wt[2];
                     const PiecesOf<NF> own = own_pieces(ob);
 #pragma unroll
