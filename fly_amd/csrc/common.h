@@ -403,7 +403,7 @@ inline DropArgs drop_args(float p, uint64_t seed) {
     return d;
 }
 
-// An entry of a table that no kernel writes, at a wave-uniform address: a scalar load.  Behind a transfer into LDS (assembly that
+// An entry of a table that nothing writes while the kernel runs, at a wave-uniform address: a scalar load.  Behind a transfer into LDS (assembly that
 // clobbers memory) the compiler otherwise takes a vector load, whose wait also covers every transfer in flight.
 template <typename I>
 __device__ __forceinline__ I table_entry(const I* p) {

@@ -3656,7 +3656,7 @@ __global__ __launch_bounds__(NT) void sblocal_fwd_x3_kernel(FwdArgs a) {
     char* lds = reinterpret_cast<char*>(smem);
     float* Ps = smem;                                  // only live before the key loop
 
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
     const int n_qt = (a.T + TQ - 1) / TQ;
     // (LIST: every workgroup has an item of the lists below; n_items = 0 keeps the band's mapping out of the way)
     const int n_items = LIST ? 0 : a.B * a.H * n_qt * a.n_parts;
@@ -3746,8 +3746,8 @@ __global__ __launch_bounds__(NT) void sblocal_fwd_x3_kernel(FwdArgs a) {
         }
         tl_inner = a.tl_inner + lp0;
         tl_blk = a.tl_blk + 4 * (long)lp0 + w;              // four masks per entry, one per wave
-        if (kt_hi > 0) { tile_cur = tl_inner[0]; pres_cur = tl_blk[0] & 3; }
-        if (kt_hi > 1) { tile_next = tl_inner[1]; pres_next = tl_blk[4] & 3; }
+        if (kt_hi > 0) { tile_cur = table_entry(tl_inner); pres_cur = table_entry(tl_blk) & 3; }
+        if (kt_hi > 1) { tile_next = table_entry(tl_inner + 1); pres_next = table_entry(tl_blk + 4) & 3; }
     }
     const int first_tile = LIST ? tile_cur : kt_lo;
 
@@ -3857,8 +3857,9 @@ __global__ __launch_bounds__(NT) void sblocal_fwd_x3_kernel(FwdArgs a) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const bool ok = 16 * fb + 4 * g + i < a.mh_valid;
-                    qf[fb][i] = ok ? quant16(__expf(dd[i] - qmax)) : 0.f;
-                    qf[FB + fb][i] = ok ? quant16(__expf(-dd[i] - qmax)) : 0.f;
+                    const float ep = quant16(__expf(dd[i] - qmax)), en = quant16(__expf(-dd[i] - qmax));
+                    qf[fb][i] = ok ? ep : 0.f;
+                    qf[FB + fb][i] = ok ? en : 0.f;
                 }
             }
             __syncthreads();      // Ps is dead; the tile buffers may overwrite it
@@ -3910,11 +3911,11 @@ __global__ __launch_bounds__(NT) void sblocal_fwd_x3_kernel(FwdArgs a) {
         float cscale_next = cscale;
         // LIST: the entry after the next one (tile, presence) is requested now
         int tile_n2 = 0, pres_n2 = 0;
-        if (LIST && kt + 2 < kt_hi) { tile_n2 = tl_inner[kt + 2]; pres_n2 = tl_blk[4 * (kt + 2)] & 3; }
+        if (LIST && kt + 2 < kt_hi) { tile_n2 = table_entry(tl_inner + kt + 2); pres_n2 = table_entry(tl_blk + 4 * (kt + 2)) & 3; }
         if (more) {                                      // next tile's transfer flies during the MFMAs (every wave is past
             const int nxt = LIST ? tile_next : kt + 1;   // the barrier that ended the last use of that stage)
             transfer(nxt, cur ^ 1);
-            cscale_next = csp[nxt * TK / CH];
+            cscale_next = table_entry(csp + nxt * TK / CH);
         }
         const float wc = __builtin_amdgcn_exp2f((cscale - kmax) * LOG2E);
         const bool any = LIST ? pres_cur != 0
@@ -4024,7 +4025,8 @@ __global__ __launch_bounds__(NT) void sblocal_fwd_x3_kernel(FwdArgs a) {
                         mx = fmaxf(mx, ok[kb][i] ? s1[kb][i] : -INFINITY);
                     }
                 mx = group_max(mx);
-                if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0) {      // wave-uniform
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0, 0)) {      // wave-uniform
+                    asm volatile("");                              // (stays a branch: the compiler would do the multiplications always)
                     const float m_new = fmaxf(m_run, mx);
                     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
                     m_run = m_new;
@@ -5129,8 +5131,8 @@ static int plan_parts(int B, int H, int T, int S, int lc) {
 }
 
 // workgroups of the key pass that a compute unit holds together: the fp32 pass that writes the bf16 operand images
-// (sb_kfeat_x3_kernel: more than 256 registers a lane and 108 KB of LDS) runs one, the others two
-static int key_pass_wgs_per_cu(int dtype, int E, int mh) { return (dtype == F32 && E <= 64 && 2 * mh <= 128) ? 1 : 2; }
+// (sb_kfeat_x3_kernel) runs one at 64 dims and 128 features (more than 256 registers a lane and 108 KB of LDS), all others two
+static int key_pass_wgs_per_cu(int dtype, int E, int mh) { return (dtype == F32 && E == 64 && mh == 64) ? 1 : 2; }
 
 static int plan(int B, int H, int S, int wgs_per_cu, int* n_chunks, int* n_split) {
     const int nc = (S + CH - 1) / CH;

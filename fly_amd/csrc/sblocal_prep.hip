@@ -14,6 +14,7 @@
 //   pass 3  sb_prep_reduce_kernel  partials -> KV, ksum, QG, qc
 // Everything is float32; nothing here is summed with atomics, so results do not depend on scheduling.
 #include "common.h"
+#include <type_traits>
 
 namespace flyhip {
 
@@ -84,11 +85,11 @@ __device__ __forceinline__ void prep_load(const float* xrow, int g, floatx4 (&xb
 #pragma unroll
     for (int cc = 0; cc < DIM / 16; ++cc) xb[cc] = *reinterpret_cast<const floatx4*>(xrow + 16 * cc + 4 * g);
 }
-template <int DIM, int FB>
+template <int DIM, int FB, int LDP = DIM>     // LDP: floats from one row of P to the next
 __device__ __forceinline__ void prep_project(floatx4 (&xb)[DIM / 16], const float* proj, float st, int r16, int g,
                                              floatx4 (&dd)[FB], float& sq) {
     constexpr int EC = DIM / 16;
-    const float* pp = proj + r16 * DIM + 4 * g;
+    const float* pp = proj + r16 * LDP + 4 * g;
     sq = 0.f;
 #pragma unroll
     for (int cc = 0; cc < EC; ++cc) {
@@ -102,7 +103,7 @@ __device__ __forceinline__ void prep_project(floatx4 (&xb)[DIM / 16], const floa
     for (int cc = 0; cc < EC; ++cc) {
         floatx4 pa[FB];
 #pragma unroll
-        for (int fb = 0; fb < FB; ++fb) pa[fb] = *reinterpret_cast<const floatx4*>(pp + 16 * fb * DIM + 16 * cc);
+        for (int fb = 0; fb < FB; ++fb) pa[fb] = *reinterpret_cast<const floatx4*>(pp + 16 * fb * LDP + 16 * cc);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -138,21 +139,17 @@ __global__ __launch_bounds__(PREP_NT) void sb_prep_kmax_kernel(PrepArgs a) {
     if (tid == 0) a.pmax[(long)bh * a.n_kblk + blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-// (at least two workgroups per compute unit: the kernel streams, and at 128 features the registers it would like to take
-//  leave room for one only; the few it spills instead cost less)
-template <int DIM, int MK, bool WRITE_F>     // WRITE_F: the float32 feature arrays are wanted (not only the images)
-__global__ __launch_bounds__(PREP_NT) __attribute__((amdgpu_waves_per_eu(2, 8))) void sb_prep_kernel(PrepArgs a) {
+// One role of sb_prep_kernel.  (A template of the role, and P in LDS: with the role a run-time value and the fragments of P in
+// registers across the chunks the loop spilled, and every reload waited for all the loads and stores in flight.  Training step at
+// B=64, 3136 tokens, window 256, 128 features, with the other changes to the band kernels of this precision: 1089 -> 1032 us; on
+// the block-sparse support with 32 features 659 -> 608 us.)
+template <int DIM, int MK, bool WRITE_F, bool KEYS>
+__device__ __forceinline__ void prep_role(const PrepArgs& a, float* Fs, float* Ys, float* red, const float* Ps, int bh, int sp, int n_split) {
     constexpr int MH = MK / 2, FB = MK / 32, RBN = MK / 16, RB = (RBN + 3) / 4, DB = DIM / 16;
-    constexpr int LDF = MK + 4, LDY = DIM + 4;
-    __shared__ float Fs[PREP_ROWS * LDF];         // features of the current rows
-    __shared__ float Ys[PREP_ROWS * LDY];         // their V (keys) or d out (queries)
-    __shared__ float red[4];
-
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, g = lane >> 4;
-    const int bh = blockIdx.y, b = bh / a.H;
-    const bool key_role = (int)blockIdx.x < a.n_split_k;
-    const int sp = key_role ? blockIdx.x : blockIdx.x - a.n_split_k;
-    const int n_split = key_role ? a.n_split_k : a.n_split_q;
+    constexpr int LDF = MK + 4, LDY = DIM + 4, LDP = DIM + 4;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    constexpr bool key_role = KEYS;
+    const int b = bh / a.H;
     const int rows = key_role ? a.S : a.T;
     const int len = key_role ? (a.lens ? min((int)a.lens[b], a.S) : a.S) : a.T;
     const float* X = (key_role ? a.k : a.q) + (long)bh * rows * DIM;
@@ -200,6 +197,7 @@ __global__ __launch_bounds__(PREP_NT) __attribute__((amdgpu_waves_per_eu(2, 8)))
         if (!key_role) ln_n = a.ln[(long)bh * rows + row];
     };
     if (c0 < c1) fetch(c0);
+    drain_loads();                                // (see there: the loop's waits would count the loads of the first chunk without its stores)
 
     for (int c = c0; c < c1; ++c) {
         const int base = c * PREP_ROWS;
@@ -239,7 +237,8 @@ __global__ __launch_bounds__(PREP_NT) __attribute__((amdgpu_waves_per_eu(2, 8)))
         const bool valid = row < len;
         const float wrow = key_role ? 1.f : crow[16 * w + r16];
         using TL = BwdTile<DIM, MK>;
-        char* img = key_role ? a.kimg : a.qimg;
+        char* img = key_role ? a.kimg : a.qimg;   // (without the feature arrays there are images)
+        if (!WRITE_F) __builtin_assume(img != nullptr);
         const int trow = (16 * w + r16) & 31;     // this lane's row inside its 32-row tile
         char* img0 = nullptr;                     // the chunk's first tile
         if (img) {
@@ -265,7 +264,7 @@ __global__ __launch_bounds__(PREP_NT) __attribute__((amdgpu_waves_per_eu(2, 8)))
         }
         floatx4 dd[FB];
         float sq;
-        prep_project<DIM, FB>(xb, a.proj, st, r16, g, dd, sq);
+        prep_project<DIM, FB, LDP>(xb, Ps, st, r16, g, dd, sq);
         float bias;
         if (key_role) bias = -0.5f * a.temp * sq - off - kappa;
         else bias = kappa - ln_row - 0.5f * a.temp * sq - off;
@@ -346,6 +345,21 @@ __global__ __launch_bounds__(PREP_NT) __attribute__((amdgpu_waves_per_eu(2, 8)))
         }
     __syncthreads();
     if (tid < MK) part[MK * DIM + tid] = (sums[tid] + sums[MK + tid]) + (sums[2 * MK + tid] + sums[3 * MK + tid]);
+}
+
+// (two workgroups per compute unit, as many as its LDS holds at 128 features)
+template <int DIM, int MK, bool WRITE_F>     // WRITE_F: the float32 feature arrays are wanted (not only the images)
+__global__ __launch_bounds__(PREP_NT) __attribute__((amdgpu_waves_per_eu(2, 8))) void sb_prep_kernel(PrepArgs a) {
+    constexpr int LDF = MK + 4, LDY = DIM + 4, LDP = DIM + 4, MH = MK / 2;
+    __shared__ __attribute__((aligned(16))) float Fs[PREP_ROWS * LDF];      // features of the current rows
+    __shared__ __attribute__((aligned(16))) float Ys[PREP_ROWS * LDY];      // their V (keys) or d out (queries)
+    __shared__ __attribute__((aligned(16))) float Ps[MH * LDP];
+    __shared__ float red[4];
+    for (int i = threadIdx.x; i < MH * DIM / 4; i += PREP_NT)
+        *reinterpret_cast<floatx4*>(Ps + i / (DIM / 4) * LDP + 4 * (i % (DIM / 4))) = *reinterpret_cast<const floatx4*>(a.proj + 4 * i);
+    // (the first barrier of the role lies before the first read of Ps)
+    if ((int)blockIdx.x < a.n_split_k) prep_role<DIM, MK, WRITE_F, true>(a, Fs, Ys, red, Ps, blockIdx.y, blockIdx.x, a.n_split_k);
+    else prep_role<DIM, MK, WRITE_F, false>(a, Fs, Ys, red, Ps, blockIdx.y, blockIdx.x - a.n_split_k, a.n_split_q);
 }
 
 // element (r, d) of the matrices (d == DIM: the vectors) = sum over the role's partials, in order
@@ -590,8 +604,13 @@ __device__ __forceinline__ void bwd_x3_epilogue(const BwdX3Args& a, char* smem, 
     }
 }
 
+// waves per SIMD: a third workgroup per compute unit where its stages fit LDS and the registers do without spills
+// (B=64, 3136 tokens, window 256, head dim and features 32: training step 402 -> 377 us; spilling ones lose 5 - 15 %)
+template <int E, int M, bool KEYMAJOR>
+constexpr int bwd_x3_waves() { return M == 32 && (E == 32 || !KEYMAJOR) ? 3 : 2; }
+
 template <int E, int M, bool KEYMAJOR, bool PARTS, bool LIST = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void sblocal_bwd_x3_kernel(BwdX3Args a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_x3_waves<E, M, KEYMAJOR>(), bwd_x3_waves<E, M, KEYMAJOR>()))) void sblocal_bwd_x3_kernel(BwdX3Args a) {
     using TL = BwdTile<E, M>;
     constexpr int NT = 256, TQ = 64, TK = 32, KB = 2;
     constexpr int D = E, KS1 = E / 32, KS2 = M / 32, EC = E / 16, FC = M / 16, DB = D / 16, MH = M / 2;
@@ -599,7 +618,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr float LOG2E = 1.4426950408889634f;
     static_assert(bwd_x3_epilogue_bytes<E, M>() <= 2 * STAGE, "epilogue operands must fit the tile stages");
     extern __shared__ __attribute__((aligned(256))) char smem[];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
     const int Lo = KEYMAJOR ? a.S : a.T, Li = KEYMAJOR ? a.T : a.S;
     const int n_ot = (Lo + TQ - 1) / TQ;
     const int n_parts = PARTS ? a.n_parts : 1;
@@ -642,7 +661,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         i_lo = min(i_hi, part * per);
         i_hi = min(i_hi, i_lo + per);
     }
-    auto tile_at = [&](int i) __attribute__((always_inline)) { return LIST ? a.tl_inner[e_lo + i] : kt_lo + i; };
+    auto tile_at = [&](int i) __attribute__((always_inline)) { return LIST ? table_entry(a.tl_inner + e_lo + i) : kt_lo + i; };
 
     if (i_lo < i_hi) bwd_tile_to_lds<TL::MAIN, KEYMAJOR>(itiles + (long)tile_at(i_lo) * TL::BYTES, smem, tid);
 
@@ -700,7 +719,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
         // wave-uniform: does this tile meet the band of any of the wave's 16 outer rows (is the block of the wave's
         // block-row and this block-column part of the support)?
-        const int pres = LIST ? a.tl_blk[4 * (e_lo + it) + w] & 3 : 3;      // (LIST: the wave's mask of this entry)
+        const int pres = LIST ? table_entry(a.tl_blk + 4 * (e_lo + it) + w) & 3 : 3;      // (LIST: the wave's mask of this entry)
         const bool any = LIST ? pres != 0
                               : !(n_base + TK - 1 - ow0 < lo || n_base - (ow0 + 15) >= hi || n_base >= n_limit || ow0 >= o_limit);
         if (any) {
@@ -743,50 +762,76 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             // lane holds the pair (outer row o, inner row n_base + 16kb + 4g + i)
             floatx4 wdm[KB], wdf[KB], wak[KB];
             const float* Ss = reinterpret_cast<const float*>(st + TL::S_OFF);
+            auto weights = [&](auto masked_tag, auto drop_tag) __attribute__((always_inline)) {
+                constexpr bool MASKED = decltype(masked_tag)::value, DROP = decltype(drop_tag)::value;
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb) {
-                floatx4 lnq, cq;
-                if (KEYMAJOR) {
-                    lnq = *reinterpret_cast<const floatx4*>(Ss + 16 * kb + 4 * g);
-                    cq = *reinterpret_cast<const floatx4*>(Ss + TK + 16 * kb + 4 * g);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int n = n_base + 16 * kb + 4 * g + i;
-                    const bool ok = LIST ? (ovalid && ((pres >> kb) & 1) != 0) : (unsigned)(n - nmin) < span;      // (a present half tile is whole)
-                    const float av = ok ? __builtin_amdgcn_exp2f(s1[kb][i] * sc - (KEYMAJOR ? lnq[i] : ln_o)) : 0.f;
-                    const float cc = KEYMAJOR ? cq[i] : c_o;
-                    const float df = ok ? s3[kb][i] - cc : 0.f;
-                    // with dropout D (0 or 1 / (1 - p)) on the exact weight: out = sum (D a - kb) v + ..., and the
-                    // normaliser sees no dropout: dm = a (D g.v - c), the weight of g in d v is D a - kb
-                    float dk = 1.f;
-                    if (drop_on) {
-                        const uint32_t rh = KEYMAJOR ? drop_row_hash(a.drop_seed, (uint32_t)(bh * a.T + n)) : drop_row;
-                        dk = drop_keep(rh, (uint32_t)(KEYMAJOR ? o : n), a.drop_thresh) ? a.drop_scale : 0.f;
+                for (int kb = 0; kb < KB; ++kb) {
+                    floatx4 lnq, cq;
+                    if (KEYMAJOR) {
+                        lnq = *reinterpret_cast<const floatx4*>(Ss + 16 * kb + 4 * g);
+                        cq = *reinterpret_cast<const floatx4*>(Ss + TK + 16 * kb + 4 * g);
                     }
-                    wdm[kb][i] = drop_on ? av * (ok ? dk * s3[kb][i] - cc : 0.f) : av * df;
-                    wdf[kb][i] = df;
-                    wak[kb][i] = av * dk - (ok ? s2[kb][i] : 0.f);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int n = n_base + 16 * kb + 4 * g + i;
+                        const bool ok = !MASKED || (LIST ? (ovalid && ((pres >> kb) & 1) != 0) : (unsigned)(n - nmin) < span);      // (a present half tile is whole)
+                        const float ex = __builtin_amdgcn_exp2f(s1[kb][i] * sc - (KEYMAJOR ? lnq[i] : ln_o));
+                        const float av = ok ? ex : 0.f;
+                        const float cc = KEYMAJOR ? cq[i] : c_o;
+                        const float df = ok ? s3[kb][i] - cc : 0.f;
+                        // with dropout D (0 or 1 / (1 - p)) on the exact weight: out = sum (D a - kb) v + ..., and the
+                        // normaliser sees no dropout: dm = a (D g.v - c), the weight of g in d v is D a - kb
+                        if (DROP) {
+                            const uint32_t rh = KEYMAJOR ? drop_row_hash(a.drop_seed, (uint32_t)(bh * a.T + n)) : drop_row;
+                            const float dk = drop_keep(rh, (uint32_t)(KEYMAJOR ? o : n), a.drop_thresh) ? a.drop_scale : 0.f;
+                            wdm[kb][i] = av * (ok ? dk * s3[kb][i] - cc : 0.f);
+                            wak[kb][i] = av * dk - (ok ? s2[kb][i] : 0.f);
+                        } else {
+                            wdm[kb][i] = av * df;
+                            wak[kb][i] = av - (ok ? s2[kb][i] : 0.f);
+                        }
+                        wdf[kb][i] = df;
+                    }
                 }
-            }
+            };
+            // (wave-uniform) every pair of the tile and the wave's rows counts, as on most tiles; no dropout
+            const bool whole = LIST ? pres == 3 && ow0 + 15 < o_limit
+                                    : n_base - (ow0 + 15) >= lo && n_base + TK - 1 - ow0 < hi && n_base + TK <= n_limit && ow0 + 15 < o_limit;
+            if (drop_on) weights(std::true_type{}, std::true_type{});
+            else if (whole) weights(std::false_type{}, std::false_type{});
+            else weights(std::true_type{}, std::false_type{});
             uintx4 dmh, dml, dfh, dfm, dfl, akh, akm, akl;
             split2(wdm[0], wdm[1], dmh, dml);
             split3(wdf[0], wdf[1], dfh, dfm, dfl);
             if (KEYMAJOR) split3(wak[0], wak[1], akh, akm, akl);
-            // out^T[col][outer] += sum_inner Y[inner][col] w[inner][outer]
+            // out^T[col][outer] += sum_inner Y[inner][col] w[inner][outer], the fragments of a 16-column block asked for before the
+            // products of the one in front of it (at two waves per SIMD nothing else hides the reads)
+            auto cols = [&](int off, int row_bytes, int c) __attribute__((always_inline)) {
+                const char* p = st + off + tr_row * row_bytes + x3_swz(tr_row, 2 * c + (tr_cb >> 1), row_bytes) * 16 + 8 * (tr_cb & 1);
+                return lds_read_tr8(p, p + 16 * row_bytes);
+            };
+            constexpr int NY = KEYMAJOR ? 5 : 2;
+            uintx4 yf[2][NY], ff[2][2];
+            auto read_y = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+                for (int n = 0; n < NY; ++n) yf[c & 1][n] = cols((n < 2 ? TL::X_OFF + n * TL::X_PIECE : TL::Y_OFF + (n - 2) * TL::X_PIECE), TL::X_ROW, c);
+            };
+            auto read_f = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+                for (int n = 0; n < 2; ++n) ff[c & 1][n] = cols(TL::F_OFF + n * TL::F_PIECE, TL::F_ROW, c);
+            };
+            read_y(0);
 #pragma unroll
             for (int c = 0; c < EC; ++c) {
-                const char* p = st + tr_row * TL::X_ROW + x3_swz(tr_row, 2 * c + (tr_cb >> 1), TL::X_ROW) * 16 + 8 * (tr_cb & 1);
-                const uintx4 yh = lds_read_tr8(p + TL::X_OFF, p + TL::X_OFF + 16 * TL::X_ROW);
-                const uintx4 yl = lds_read_tr8(p + TL::X_OFF + TL::X_PIECE, p + TL::X_OFF + TL::X_PIECE + 16 * TL::X_ROW);
+                if (c + 1 < EC) read_y(c + 1); else read_f(0);
+                __builtin_amdgcn_sched_barrier(0x47f);
+                const uintx4 yh = yf[c & 1][0], yl = yf[c & 1][1];
                 acc1[c] = mma_bf16(yl, dmh, acc1[c]);
                 acc1[c] = mma_bf16(yh, dml, acc1[c]);
                 acc1[c] = mma_bf16(yh, dmh, acc1[c]);
                 if (KEYMAJOR) {
                     // (a - kb) g: the band's low-rank part cancels against the per-head sum Q'^T g, so all six products
-                    const uintx4 vh = lds_read_tr8(p + TL::Y_OFF, p + TL::Y_OFF + 16 * TL::X_ROW);
-                    const uintx4 vm = lds_read_tr8(p + TL::Y_OFF + TL::X_PIECE, p + TL::Y_OFF + TL::X_PIECE + 16 * TL::X_ROW);
-                    const uintx4 vl = lds_read_tr8(p + TL::Y_OFF + 2 * TL::X_PIECE, p + TL::Y_OFF + 2 * TL::X_PIECE + 16 * TL::X_ROW);
+                    const uintx4 vh = yf[c & 1][KEYMAJOR ? 2 : 0], vm = yf[c & 1][KEYMAJOR ? 3 : 0], vl = yf[c & 1][KEYMAJOR ? 4 : 0];
                     acc3[c] = mma_bf16(vl, akh, acc3[c]);
                     acc3[c] = mma_bf16(vh, akl, acc3[c]);
                     acc3[c] = mma_bf16(vm, akm, acc3[c]);
@@ -794,17 +839,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     acc3[c] = mma_bf16(vh, akm, acc3[c]);
                     acc3[c] = mma_bf16(vh, akh, acc3[c]);
                 }
+                __builtin_amdgcn_sched_barrier(0x47f);
             }
 #pragma unroll
             for (int c = 0; c < FC; ++c) {
-                const char* p = st + TL::F_OFF + tr_row * TL::F_ROW + x3_swz(tr_row, 2 * c + (tr_cb >> 1), TL::F_ROW) * 16 + 8 * (tr_cb & 1);
-                const uintx4 fh = lds_read_tr8(p, p + 16 * TL::F_ROW);
-                const uintx4 fl = lds_read_tr8(p + TL::F_PIECE, p + TL::F_PIECE + 16 * TL::F_ROW);
+                if (c + 1 < FC) read_f(c + 1);
+                __builtin_amdgcn_sched_barrier(0x47f);
+                const uintx4 fh = ff[c & 1][0], fl = ff[c & 1][1];
                 acc2[c] = mma_bf16(fl, dfm, acc2[c]);
                 acc2[c] = mma_bf16(fh, dfl, acc2[c]);
                 acc2[c] = mma_bf16(fl, dfh, acc2[c]);
                 acc2[c] = mma_bf16(fh, dfm, acc2[c]);
                 acc2[c] = mma_bf16(fh, dfh, acc2[c]);
+                __builtin_amdgcn_sched_barrier(0x47f);
             }
         }
         drain_loads();                                     // this wave's share of the next tile is in LDS

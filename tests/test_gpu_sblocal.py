@@ -1375,3 +1375,25 @@ def test_bf16_gradients_leave_out_exactly_the_band(window, mh, monkeypatch):
         share = float((a.cpu() != r.bfloat16()).double().mean())
         print(name, share)
         assert share <= 1e-2, (name, share)
+
+
+@pytest.mark.parametrize('E,mh', [(32, 16), (32, 32), (64, 16), (64, 64)])
+@pytest.mark.parametrize('window,T,S', [(160, 333, 333), (95, 200, 257), (96, 257, 130)])
+def test_float32_gradients_on_whole_and_cut_tiles(E, mh, window, T, S):
+    """Tiles of which every pair counts and tiles that the band, the last row or the key lengths cut, at each number of waves per
+    SIMD of the band gradients' kernel, against autograd through the oracle in float64."""
+    from fly_amd import sblocal_attention_fn
+    dev = torch.device('cuda:0')
+    B, H = 2, 2
+    q, k, v, P = make_inputs(B, T, S, H, E, E, mh, seed=T + mh)
+    w = torch.randn(B, T, H, E, generator=torch.Generator().manual_seed(T))
+    lens = torch.tensor([S, S - 77])
+    qg, kg, vg = (x.to(dev).requires_grad_() for x in (q, k, v))
+    out, _ = sblocal_attention_fn(qg, kg, vg, P.to(dev), window, None, lens.to(dev))
+    got = torch.autograd.grad(out, (qg, kg, vg), w.to(dev))
+    qd, kd, vd = (x.double().requires_grad_() for x in (q, k, v))
+    ref_out, _ = osb.sblocal_attention(qd, kd, vd, P.double(), window, key_lengths=lens)
+    ref = torch.autograd.grad(ref_out, (qd, kd, vd), w.double())
+    assert rel_err(out, ref_out.detach()) <= 1e-4
+    for a, r in zip(got, ref):
+        assert rel_err(a, r) <= 2e-4, rel_err(a, r)
