@@ -8,6 +8,7 @@
 // the output columns on the MFMA "A" side, so a lane ends up with four consecutive output
 // columns of one row and writes them with a single vector store.
 #include "common.h"
+#include <type_traits>
 #include <math.h>
 
 namespace flyhip {
@@ -1601,209 +1602,227 @@ __global__ __launch_bounds__(512) void bs_dds32d_kernel(DdsGroupArgs a, int n_st
 }
 
 // The same per-wave scheme for reduction lists that do not fit the LDS (layers that narrow: 36 input blocks per output
-// block in the second linear of a channel MLP).  The group's weights pass through LDS in chunks of DDS_CK list entries
-// (32 KB), double-buffered and shared by the eight waves: a thread asks for its 64 bytes of the next chunk at the head
-// of a chunk, parks them in the other buffer at its end, and one barrier per chunk (two steps of 64 MFMAs per wave)
-// publishes them -- the tiled kernel pays a barrier, eight LDS writes and the wait for its loads per 32 MFMAs.  The
-// activations go through a stage per wave exactly as in bs_dds32d_kernel.  The weights are fetched again for every tile
-// of 512 tokens (from L2: a quarter of what the tiled kernel's 128-token tiles fetch).
-constexpr int DDS_CK = 4;
-typedef unsigned int uintx2 __attribute__((ext_vector_type(2)));
+// block in the second linear of a channel MLP, and the input gradients of layers that widen).  The group's weights pass
+// through LDS two list entries (16 KB) at a time, double-buffered and shared by the eight waves, the activations through two
+// stages per wave: a step's 8 KB are asked for two steps ahead, its weights one, all straight into LDS.  What bounds it is
+// the latency of those transfers between two barriers -- with one stage per wave, weights through registers and [k][n] blocks
+// transposed by 16-bit LDS writes a step took 5500 cycles for 1536 of MFMA on its SIMD, now 4400.  (Even shares of the tokens with a
+// lower last tile, 256 workgroups for 200 in the case below, made the kernel alone 9 % shorter and the training step no faster.)
+// Input gradient of 768 -> 3072 features, 50176 tokens: training step 443 -> 418 us; forward of 3072 -> 768: 492 -> 470 us a step.
+// The 160 KB of LDS are full, so the lists are read as scalars.  Weight blocks lie as in memory, 64 bytes a row with 16-byte
+// chunk c at c ^ ((row >> 2) & 3), and are the row operand of the products: [n][k] blocks by 16-byte reads, [k][n] blocks by
+// transposing reads.  A lane ends up with four consecutive outputs of a token in each tile of 16; a row swap makes eight of two.
+constexpr int DDS_PIPE_LDS = 2 * 16384 + 2 * 8 * 8192;
 
-template <typename T, bool WT>
-__global__ __launch_bounds__(512) void bs_dds32c_kernel(DdsGroupArgs a, int n_streams) {
-    constexpr int STEP = 8 * 16 * 32;                       // elements of an entry's eight weight tiles
-    constexpr int CHUNK = DDS_CK * STEP;                    // elements of a chunk buffer
-    extern __shared__ __attribute__((aligned(1024))) uint16_t wres[];   // 2 x [entry][tile n][row r][32 k], then 8 stages of 8 KB
-    __shared__ int s_inner[DDS_MAX_STEPS];
-    __shared__ int s_blk[4][DDS_MAX_STEPS];
+// One group of GN output blocks (a constant: a branch per output block would wait for its weights in turn)
+template <typename T, bool WT, int GN>
+__device__ __forceinline__ void dds32c_group(const DdsGroupArgs& a, char* lds, int grp, int ty, int gy) {
+    constexpr int NT = 2 * GN, TM = 4, NX = 2 * TM;         // NX: a step's transfers of activations per wave
+    const int n_tiles = ((a.M + 511) / 512 - ty + gy - 1) / gy;
     const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int z = blockIdx.y;
-    const int per_xcd = (int)gridDim.x / a.n_xcd;
-    const int pair = ((int)blockIdx.x % a.n_xcd) * per_xcd + (int)blockIdx.x / a.n_xcd;
-    const int n_grp = a.n_grp;
-    if (pair >= n_streams * n_grp) return;                  // workgroup-uniform
-    const int ty = pair / n_grp, grp = pair % n_grp, gy = n_streams;
-    const int tiles_all = (a.M + 511) / 512;
-    if (ty >= tiles_all) return;
-    const int my_tiles = (tiles_all - ty + gy - 1) / gy;
-    const int row0 = a.grp_row0[grp], gn = a.grp_n[grp];
+    const int row0 = a.grp_row0[grp];
     const int head = row0 / a.per_head, bcol0 = row0 % a.per_head;
     const int p0 = a.seg_ptr[row0], nin = a.seg_ptr[row0 + 1] - p0;
-    const uint16_t* spz = reinterpret_cast<const uint16_t*>(a.sp) + z * a.sp_sz;
-    const uint16_t* xp = reinterpret_cast<const uint16_t*>(a.dn) + z * a.dn_sz + head * a.dn_sh;
-    T* cp = reinterpret_cast<T*>(a.c) + z * a.c_sz + head * a.c_sh;
+    const char* spz = reinterpret_cast<const char*>(reinterpret_cast<const uint16_t*>(a.sp) + z * a.sp_sz);
+    const char* xb = reinterpret_cast<const char*>(reinterpret_cast<const uint16_t*>(a.dn) + z * a.dn_sz + head * a.dn_sh);
+    T* cp = reinterpret_cast<T*>(a.c) + z * a.c_sz + head * a.c_sh + (long)bcol0 * 32;
 
-    for (int i = tid; i < nin; i += 512) s_inner[i] = a.seg_inner[p0 + i];
-    for (int i = tid; i < 4 * nin; i += 512) {
-        const int ob = i / nin, t = i % nin;
-        s_blk[ob][t] = ob < gn ? a.seg_blk[a.seg_ptr[row0 + ob] + t] : -1;
-    }
-    __syncthreads();
-
-    floatx4 acc[4][8];
-    // The group's 32 gn outputs are dealt to NT = 2 gn tiles of 16: tile n holds outputs NT r + n (r = 0..15), so no MFMA
-    // column is padding whatever the group's size, and a lane ends up with NT consecutive outputs of four tokens.
-    const int NT = 2 * gn;
-    // what the sums start from (WT: zero -- eight registers more would spill, and gradients have no bias)
-    float bias[8];
+    // outputs 16 n + 4 g .. + 3 of the group, tokens 16 tm + r16
+    floatx4 acc[TM][NT];
+    // what the sums start from, as it lies in memory (WT: zero, gradients have no bias)
+    uint2 bias[WT ? 1 : NT];
 #pragma unroll
-    for (int n = 0; n < 8; ++n)
-        bias[n] = !WT && a.bias && n < NT ? Elem<T>::to_f32(reinterpret_cast<const T*>(a.bias)[((long)head * a.per_head + bcol0) * 32 + NT * r16 + n]) : 0.f;
+    for (int n = 0; n < (WT ? 0 : NT); ++n) {
+        bias[n] = make_uint2(0u, 0u);
+        if (a.bias) {
+            const uint16_t* b = reinterpret_cast<const uint16_t*>(a.bias) + ((long)head * a.per_head + bcol0) * 32 + 16 * n + 4 * g;
+            bias[n] = make_uint2(b[0] | ((uint32_t)b[1] << 16), b[2] | ((uint32_t)b[3] << 16));
+        }
+    }
     auto reset = [&](int tm) __attribute__((always_inline)) {
 #pragma unroll
-        for (int n = 0; n < 8; ++n) acc[tm][n] = floatx4{bias[n], bias[n], bias[n], bias[n]};
+        for (int n = 0; n < NT; ++n) {
+            if (WT) acc[tm][n] = Frag<float>::zero();
+            else {
+                const uint2 b = bias[WT ? 0 : n];
+                auto one = [](uint32_t bits) __attribute__((always_inline)) { return Elem<T>::to_f32(__builtin_bit_cast(T, (uint16_t)bits)); };
+                acc[tm][n] = floatx4{one(b.x & 0xffffu), one(b.x >> 16), one(b.y & 0xffffu), one(b.y >> 16)};
+            }
+        }
     };
 #pragma unroll
-    for (int tm = 0; tm < 4; ++tm) reset(tm);
+    for (int tm = 0; tm < TM; ++tm) reset(tm);
     auto store_tile = [&](int tile) __attribute__((always_inline)) {
-        const long m0 = ((long)ty + (long)tile * gy) * 512 + 64 * w + 4 * g;
-        T* base = cp + (long)bcol0 * 32 + NT * r16;
+        const long m0 = ((long)ty + (long)tile * gy) * 512 + 64 * w + r16;
+        T* base = cp + 16 * (g & 1) + 8 * (g >> 1);
 #pragma unroll
-        for (int tm = 0; tm < 4; ++tm) {
+        for (int tm = 0; tm < TM; ++tm) {
+            const long m = m0 + 16 * tm;
+            uint32_t* dst = reinterpret_cast<uint32_t*>(base + m * a.c_sm);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const long m = m0 + 16 * tm + i;
-                if (m < a.M) {
-                    uint32_t* dst = reinterpret_cast<uint32_t*>(base + m * a.c_sm);
-                    const uint32_t p0_ = pack2<T>(acc[tm][0][i], acc[tm][1][i]), p1_ = pack2<T>(acc[tm][2][i], acc[tm][3][i]);
-                    const uint32_t p2_ = pack2<T>(acc[tm][4][i], acc[tm][5][i]), p3_ = pack2<T>(acc[tm][6][i], acc[tm][7][i]);
-                    if (NT == 8) __builtin_nontemporal_store(uintx4{p0_, p1_, p2_, p3_}, reinterpret_cast<uintx4*>(dst));
-                    else if (NT == 6) { __builtin_nontemporal_store(uintx2{p0_, p1_}, reinterpret_cast<uintx2*>(dst)); __builtin_nontemporal_store(p2_, dst + 2); }
-                    else if (NT == 4) __builtin_nontemporal_store(uintx2{p0_, p1_}, reinterpret_cast<uintx2*>(dst));
-                    else __builtin_nontemporal_store(p0_, dst);
-                }
+            for (int ob = 0; ob < GN; ++ob) {
+                const floatx4 t0 = acc[tm][2 * ob], t1 = acc[tm][2 * ob + 1];
+                const auto s0 = __builtin_amdgcn_permlane16_swap(pack2<T>(t0[0], t0[1]), pack2<T>(t1[0], t1[1]), false, false);
+                const auto s1 = __builtin_amdgcn_permlane16_swap(pack2<T>(t0[2], t0[3]), pack2<T>(t1[2], t1[3]), false, false);
+                if (m < a.M) __builtin_nontemporal_store(uintx4{s0[0], s1[0], s0[1], s1[1]}, reinterpret_cast<uintx4*>(dst + 16 * ob));
             }
             reset(tm);
         }
     };
     if (nin == 0) {                                         // no input block: zero rows
-        for (int tile = 0; tile < my_tiles; ++tile) store_tile(tile);
+        for (int tile = 0; tile < n_tiles; ++tile) store_tile(tile);
         return;
     }
 
-    const int npair = (nin + 1) / 2, nchunk = (npair + DDS_CK / 2 - 1) / (DDS_CK / 2);      // steps and chunks per tile
-    const int n_steps = my_tiles * npair, n_chunks = my_tiles * nchunk;
-    // the weights of a chunk: this thread's 16 bytes of each of its DDS_CK entries -- row `wrow` (its 8 inputs `wch`..) of
-    // output block `wob`, parked at the place the MFMAs read (see bs_dds32s_kernel)
-    const int wch = tid & 3, wrow = (tid >> 2) & 31, wob = (tid >> 7) & 3;
-    const uint32_t wsrc = (uint32_t)((wrow * 32 + wch * 8) * 2);
-    // where they go: output o of the group sits in tile o % NT, row o / NT
-    int wdst[WT ? 8 : 1];
-    if (!WT) {
-        const int o = 32 * wob + wrow;
-        wdst[0] = (o % NT) * 512 + (o / NT) * 32 + 8 * wch;
-    } else {
+    const int npair = (nin + 1) / 2, n_steps = n_tiles * npair;
+    // weights: the wave's transfers of 16 rows (1 KB) of a step's 4 GN half blocks
+    const uint32_t wlane = (uint32_t)((lane >> 2) * 64 + 16 * ((lane & 3) ^ (lane >> 4)));
+    const int32_t* wlist[2];
+    int whf[2], wdst[2], whalf[2], wblk[2];
+    bool wlive[2];
 #pragma unroll
-        for (int e = 0; e < (WT ? 8 : 1); ++e) {
-            const int o = 32 * wob + 8 * wch + e;
-            wdst[e] = (o % NT) * 512 + (o / NT) * 32 + wrow;
-        }
+    for (int j = 0; j < 2; ++j) {
+        const int u = w + 8 * j, hf = u >= NT, rem = u - NT * hf;
+        wlive[j] = u < 2 * NT;
+        whf[j] = hf;
+        whalf[j] = (rem & 1) * 1024;
+        wdst[j] = hf * 8192 + rem * 1024;
+        wlist[j] = a.seg_blk + (wlive[j] ? a.seg_ptr[row0 + (rem >> 1)] : p0);
+        wblk[j] = table_entry(wlist[j] + min(hf, nin - 1));
     }
-    uintx4 rwq[DDS_CK];
-    bool wlive[DDS_CK];
-    auto fetch_w = [&](int q) __attribute__((always_inline)) {
-        const int e0 = DDS_CK * (q % nchunk);
+    int w_t = 0;                                            // weight cursor: pair of entries inside the tile
+    auto transfer_w = [&](int buf) __attribute__((always_inline)) {
+        if (++w_t == npair) w_t = 0;
 #pragma unroll
-        for (int j = 0; j < DDS_CK; ++j) {
-            const int blk_id = e0 + j < nin ? s_blk[wob][e0 + j] : -1;
-            wlive[j] = blk_id >= 0;
-            rwq[j] = *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(spz + (long)max(blk_id, 0) * 1024) + wsrc);
+        for (int j = 0; j < 2; ++j) {
+            if (wlive[j]) dma_to_lds_at(spz + (long)wblk[j] * 2048 + whalf[j], wlane, lds + buf * 16384 + wdst[j]);
+            wblk[j] = table_entry(wlist[j] + min(2 * w_t + whf[j], nin - 1));       // (an odd list's last step: the last entry twice)
         }
     };
-    auto stash_w = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < DDS_CK; ++j) {
-            const uintx4 v = wlive[j] ? rwq[j] : uintx4{0, 0, 0, 0};
-            uint16_t* dst = wres + (size_t)buf * CHUNK + (size_t)j * STEP;
-            if (wob < gn) {                                 // (an output block the group lacks has no place in the tiles)
-                if (!WT) {
-                    *reinterpret_cast<uintx4*>(dst + wdst[0]) = v;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < (WT ? 8 : 1); ++e) dst[wdst[e]] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-                }
-            }
-        }
-    };
-
-    char* stage = reinterpret_cast<char*>(wres) + 2 * CHUNK * 2 + 8192 * w;
+    // activations, as in bs_dds32d_kernel: chunk 4 hf + c of token t lies at chunk (4 hf + c) ^ ((t >> 1) & 7)
+    char* stage = lds + 32768 + 8192 * w;                   // the second stage 64 KB behind the first
     const int tl = lane >> 3;
-    uint32_t xoff[8];
-    int sel[8];
+    uint32_t xoff[NX];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) { xoff[j] = 0; sel[j] = 0; }
+    for (int j = 0; j < NX; ++j) xoff[j] = 0;
     int f_tile = 0, f_t = 0;                                // transfer cursor: (token tile, pair of entries inside it)
-    auto transfer = [&]() __attribute__((always_inline)) {  // (see bs_dds32d_kernel)
+    int in0 = table_entry(a.seg_inner + p0), in1 = table_entry(a.seg_inner + p0 + min(1, nin - 1));
+    uint32_t xeven = 0, xodd = 0;
+    auto transfer_head = [&]() __attribute__((always_inline)) {
         if (f_t == 0) {
             const long m0 = ((long)ty + (long)f_tile * gy) * 512 + 64 * w;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
+            for (int j = 0; j < NX; ++j) {
                 const int t = 8 * j + tl, c = (lane & 7) ^ ((t >> 1) & 7);
-                const long m = min(m0 + t, (long)a.M - 1);
+                const long m = min(m0 + t, (long)a.M - 1);   // clamped: masked at the store (past the last tile: never read)
                 xoff[j] = (uint32_t)((m * a.dn_sm + 8 * (c & 3)) * 2);
-                sel[j] = c >> 2;
             }
         }
-        const int in0 = __builtin_amdgcn_readfirstlane(s_inner[2 * f_t]);
-        const int in1 = __builtin_amdgcn_readfirstlane(s_inner[min(2 * f_t + 1, nin - 1)]);
-        const char* xb = reinterpret_cast<const char*>(xp);
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            dma_to_lds(xb + xoff[j] + (uint32_t)((sel[j] ? in1 : in0) * 64), stage + 1024 * j);
+        const uint32_t b0 = (uint32_t)in0 * 64u, b1 = (uint32_t)in1 * 64u;
+        const bool second = (((lane & 7) ^ (tl >> 1)) >> 2) != 0;             // even j: which of the two blocks the lane's chunk belongs to
+        xeven = second ? b1 : b0;
+        xodd = second ? b0 : b1;
         if (++f_t == npair) { f_t = 0; ++f_tile; }
+        in0 = table_entry(a.seg_inner + p0 + 2 * f_t);
+        in1 = table_entry(a.seg_inner + p0 + min(2 * f_t + 1, nin - 1));
     };
-    const int wfrag = r16 * 32 + 8 * g;
-    int xfrag[2][4];
+    auto transfer_row = [&](int st, int j) __attribute__((always_inline)) {
+        dma_to_lds_at(xb, xoff[j] + ((j & 1) ? xodd : xeven), stage + 65536 * st + 1024 * j);
+    };
+    int xfrag[2][TM];
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-        for (int tm = 0; tm < 4; ++tm) {
+        for (int tm = 0; tm < TM; ++tm) {
             const int t = 16 * tm + r16;
             xfrag[hf][tm] = t * 128 + 16 * ((4 * hf + g) ^ ((t >> 1) & 7));
         }
+    // the row operand of tile 2 ob + h of an entry: outputs 16 h + r16, contraction slots 8 g .. 8 g + 7
+    int wfrag[WT ? 4 : 1];
+    if (WT) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int part = 0; part < 2; ++part) {
+                const int row = 8 * g + 4 * part + (r16 >> 2), c = 2 * h + ((r16 & 3) >> 1);
+                wfrag[WT ? 2 * h + part : 0] = row * 64 + 16 * (c ^ ((row >> 2) & 3)) + 8 * (r16 & 1);
+            }
+    } else wfrag[0] = r16 * 64 + 16 * (g ^ (r16 >> 2));
 
-    fetch_w(0);
-    stash_w(0);
-    __syncthreads();
-    transfer();
-    int c_tile = 0, c_t = 0, q = 0;                         // compute cursor: tile, step inside it; chunks done so far
+    transfer_w(0);
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+        transfer_head();
+#pragma unroll
+        for (int j = 0; j < NX; ++j) transfer_row(st, j);
+    }
+    int c_tile = 0, c_t = 0;                                // compute cursor: tile, step inside it
     for (int step = 0; step < n_steps; ++step) {
-        drain_loads();                                      // this step's activations are in the stage
-        const bool chunk_head = (c_t & (DDS_CK / 2 - 1)) == 0;
-        if (chunk_head && q + 1 < n_chunks) fetch_w(q + 1); // (workgroup-uniform) parked at the chunk's end
-        uintx4 fx[2][4];
+        const int cur = step & 1;
+        drain_loads_but<NX>();                              // all but the next step's activations (stores of a tile wait too)
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();                       // the step's weights are there, the other buffer is free
+        asm volatile("" ::: "memory");
+        transfer_w(cur ^ 1);                                // (the last step's are not used)
+        uintx4 fx[2][TM];
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-            for (int tm = 0; tm < 4; ++tm) fx[hf][tm] = *reinterpret_cast<const uintx4*>(stage + xfrag[hf][tm]);
+            for (int tm = 0; tm < TM; ++tm) fx[hf][tm] = *reinterpret_cast<const uintx4*>(stage + 65536 * cur + xfrag[hf][tm]);
         __builtin_amdgcn_s_waitcnt(0xC07F);                 // lgkmcnt(0): the fragments are in registers, the stage is free
-        if (step + 1 < n_steps) transfer();
-        const uint16_t* wbuf = wres + (size_t)(q & 1) * CHUNK + (size_t)(2 * (c_t & (DDS_CK / 2 - 1))) * STEP + wfrag;
+        transfer_head();
+        // the transfers of step + 2 go out between the products: eight waves that ask for everything behind the barrier wait in
+        // line with idle matrix cores
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
             if (2 * c_t + hf < nin) {                       // workgroup-uniform
-                const uint16_t* wt = wbuf + (size_t)hf * STEP;
+                const char* wb = lds + 16384 * cur + hf * 8192;
+                uintx4 fw[2];
+                auto weights = [&](int n) __attribute__((always_inline)) {
+                    const char* p = wb + (n >> 1) * 2048;
+                    if (WT) fw[n & 1] = lds_read_tr8(p + wfrag[WT ? 2 * (n & 1) : 0], p + wfrag[WT ? 2 * (n & 1) + 1 : 0]);
+                    else fw[n & 1] = *reinterpret_cast<const uintx4*>(p + (n & 1) * 1024 + wfrag[0]);
+                };
+                weights(0);
 #pragma unroll
-                for (int n = 0; n < 8; ++n) {
-                    if (n < NT) {                           // workgroup-uniform
-                        const uint4 fw = *reinterpret_cast<const uint4*>(wt + n * 512);
+                for (int n = 0; n < NT; ++n) {
+                    if (n + 1 < NT) weights(n + 1);
+                    __builtin_amdgcn_sched_barrier(0x47f);  // (reads stay in front of the products before those that need them)
 #pragma unroll
-                        for (int tm = 0; tm < 4; ++tm)
-                            acc[tm][n] = Frag32<T>::mma(__builtin_bit_cast(uint4, fx[hf][tm]), fw, acc[tm][n]);
-                    }
+                    for (int tm = 0; tm < TM; ++tm)
+                        acc[tm][n] = Frag32<T>::mma(__builtin_bit_cast(uint4, fw[n & 1]), __builtin_bit_cast(uint4, fx[hf][tm]), acc[tm][n]);
+#pragma unroll
+                    for (int j = 0; j < TM; ++j)
+                        if (j * NT / TM == n) transfer_row(cur, TM * hf + j);
+                    __builtin_amdgcn_sched_barrier(0x47f);
                 }
+            } else {
+#pragma unroll
+                for (int j = 0; j < TM; ++j) transfer_row(cur, TM * hf + j);
             }
         }
-        bool chunk_end = false;
-        if (++c_t == npair) { store_tile(c_tile); c_t = 0; ++c_tile; chunk_end = true; }
-        else chunk_end = (c_t & (DDS_CK / 2 - 1)) == 0;
-        if (chunk_end) {                                    // (workgroup-uniform)
-            if (q + 1 < n_chunks) stash_w((q + 1) & 1);
-            __syncthreads();
-            ++q;
-        }
+        if (++c_t == npair) { store_tile(c_tile); c_t = 0; ++c_tile; }
+    }
+    drain_loads();                                          // (transfers past the last step)
+}
+
+template <typename T, bool WT>
+__global__ __launch_bounds__(512) void bs_dds32c_kernel(DdsGroupArgs a, int n_streams) {
+    extern __shared__ __attribute__((aligned(1024))) uint16_t wres[];   // 2 x [entry][output block][row][32], then 2 x 8 stages of 8 KB
+    char* lds = reinterpret_cast<char*>(wres);
+    const int per_xcd = (int)gridDim.x / a.n_xcd;
+    const int pair = ((int)blockIdx.x % a.n_xcd) * per_xcd + (int)blockIdx.x / a.n_xcd;
+    if (pair >= n_streams * a.n_grp) return;                // workgroup-uniform
+    const int ty = pair / a.n_grp, grp = pair % a.n_grp;
+    if (ty >= (a.M + 511) / 512) return;
+    switch (a.grp_n[grp]) {
+        case 4: dds32c_group<T, WT, 4>(a, lds, grp, ty, n_streams); break;
+        case 3: dds32c_group<T, WT, 3>(a, lds, grp, ty, n_streams); break;
+        case 2: dds32c_group<T, WT, 2>(a, lds, grp, ty, n_streams); break;
+        default: dds32c_group<T, WT, 1>(a, lds, grp, ty, n_streams); break;
     }
 }
 
@@ -3220,7 +3239,7 @@ extern "C" int flyhip_bs_dds_bias(const void* a, const void* b_sp, const void* b
         }
         if (FLY_DDS_STATIONARY == 2 && max_seg_len > DDS_STAT_STEPS && max_seg_len <= DDS_MAX_STEPS && (long)M >= 512L * 8 &&
             (trans_b || !bias)) {
-            // longer lists: the same workgroup shape with the weights passing through LDS in chunks ([k][n] blocks: no bias)
+            // longer lists: the same workgroup shape with the weights passing through LDS ([k][n] blocks: no bias)
             const long tiles = (M + 511) / 512;
             long n_streams = 1, best = -1;
             for (long n = 1; n <= tiles && n * n_grp * Z <= 4L * mach.cus + (long)n_grp * Z; ++n) {
@@ -3229,7 +3248,7 @@ extern "C" int flyhip_bs_dds_bias(const void* a, const void* b_sp, const void* b
             }
             const long pairs = n_streams * n_grp;
             const long gx = (pairs + mach.xcds - 1) / mach.xcds * mach.xcds;
-            const size_t smem = (size_t)2 * DDS_CK * 8192 + 8 * 8192;
+            const size_t smem = DDS_PIPE_LDS;
             dim3 grid((unsigned)gx, Z);
 #define DDS_CHUNKED(TT, WTT)                                                                                       \
     {                                                                                                              \

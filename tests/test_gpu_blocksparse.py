@@ -654,6 +654,50 @@ def test_dds_staged_kernel_with_weights_in_chunks(trans_b, dtype):
     assert rel_err(out, ref) <= TOL[dtype]
 
 
+@pytest.mark.parametrize('trans_b', [True, False])
+@pytest.mark.parametrize('M', [128 * 33 - 5, 128 * 41 + 64, 128 * 50 - 3])
+def test_dds_long_lists_past_the_last_tile(M, trans_b):
+    """The dds kernel for long reduction lists asks for activations two steps and for weights one step ahead, also past the end
+    of its tokens: last tiles of a few tokens, of half a tile and of nearly a whole one, lists of odd and even length."""
+    from fly_amd import matmul
+    print('case', M, trans_b, flush=True)
+    Z, H, block, n_out, n_in = 2, 2, 32, 9, 15
+    g = torch.Generator().manual_seed(47)
+    seg = (torch.rand(H, n_out, n_in, generator=g) < 0.8).long()
+    seg[0, 0] = (torch.arange(n_in) != 3).long()
+    seg[0, 1:4] = seg[0, 0]
+    seg[1, 5:7] = seg[1, 4]
+    assert int(seg.sum(-1).max()) > 9
+    layout = seg if trans_b else seg.transpose(1, 2).contiguous()
+    w = torch.randn(Z, int(layout.sum()), block, block, generator=g).bfloat16()
+    x = torch.randn(Z, H, M, n_in * block, generator=g).bfloat16()
+    out = matmul(layout, block, 'dds', trans_a=False, trans_b=trans_b)(x.to(DEV), w.to(DEV))
+    ref = ob.dds(x.double(), w.double(), layout, block, False, trans_b)
+    assert out.shape == ref.shape
+    assert rel_err(out, ref) <= TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_narrowing_linear_with_bias_and_long_lists(dtype):
+    """Bias inside the dds kernel for long reduction lists (36 blocks a row), forward and gradients against the dense product."""
+    from fly_amd import BlockSparseLinear, FlatBlockButterflySparsityConfig
+    torch.manual_seed(3)
+    layer = BlockSparseLinear(1536, 384, FlatBlockButterflySparsityConfig(4, 2, block=32), bias=True).to(DEV).to(dtype)
+    x, w = (torch.randn(4096 + 130, n, device=DEV).to(dtype) for n in (1536, 384))
+    x.requires_grad_()
+    layer.bias.data.normal_()
+    out = layer(x)
+    gx, = torch.autograd.grad(out, x, w)
+    lay = layer.layout.cpu()
+    dense = torch.zeros(lay.shape[0], 32, lay.shape[1], 32, dtype=torch.float64, device=DEV)
+    for n, (i, j) in enumerate(lay.nonzero().tolist()):
+        dense[i, :, j] = layer.weight[0, n].double()
+    mat = dense.view(384, 1536).t()
+    ref = x.detach().double() @ mat + layer.bias.double()
+    assert rel_err(out.double(), ref) <= TOL[dtype]
+    assert rel_err(gx.double(), w.double() @ mat.t()) <= TOL[dtype]
+
+
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize('p,r,N', [(8, 8, 64), (11, 6, 72), (5, 13, 128)])
 def test_dsd_with_transposed_sparse_operand(p, r, N, dtype):
