@@ -67,12 +67,15 @@ class _SBBlockSparseFn(torch.autograd.Function):
         ctx.save_for_backward(query, key, value, projection_matrix, out, log_norm)
         ctx.support, ctx.softmax_temp, ctx.dropout = support, softmax_temp, dropout
         ctx.mark_non_differentiable(log_norm)
+        ctx.set_materialize_grads(False)         # (no zeros for the log-normaliser: a launch per step)
         return out, log_norm
 
     @staticmethod
     def backward(ctx, grad_out, _grad_log_norm):
         from .sblocal_backward import sblocal_backward
         query, key, value, projection_matrix, out, log_norm = ctx.saved_tensors
+        if grad_out is None:
+            grad_out = torch.zeros_like(out)
         dq, dk, dv = sblocal_backward(query, key, value, projection_matrix, 1, ctx.softmax_temp, None, out, log_norm,
                                       grad_out, support=ctx.support, dropout=ctx.dropout)
         return dq, dk, dv, None, None, None, None, None, None

@@ -446,6 +446,7 @@ class _SBLocalFn(torch.autograd.Function):
         ctx.args = (local_context, softmax_temp, key_lengths)
         ctx.dropout = (float(dropout_p), int(dropout_seed))
         ctx.mark_non_differentiable(log_norm)
+        ctx.set_materialize_grads(False)         # (no zeros for the log-normaliser: a launch per step)
         return out, log_norm
 
     @staticmethod
@@ -453,6 +454,8 @@ class _SBLocalFn(torch.autograd.Function):
         from .sblocal_backward import sblocal_backward
         query, key, value, projection_matrix, out, log_norm = ctx.saved_tensors
         local_context, softmax_temp, key_lengths = ctx.args
+        if grad_out is None:
+            grad_out = torch.zeros_like(out)
         dq, dk, dv = sblocal_backward(query, key, value, projection_matrix, local_context, softmax_temp,
                                       key_lengths, out, log_norm, grad_out, dropout=ctx.dropout)
         return dq, dk, dv, None, None, None, None, None, None, None, None

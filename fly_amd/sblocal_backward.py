@@ -175,26 +175,27 @@ def _backward_hip(Q, K, V, G, O, LN, P, lens_b, H, local_context, t, dims, piece
     psi_ = phik_ = qimg = kimg = part_ws = None
     if pieces:
         images = torch.empty(sizes['qimg'] + sizes['kimg'], dtype=torch.uint8, device=Q.device)
-        qimg, kimg = images[:sizes['qimg']], images[sizes['qimg']:]
+        qimg = images.data_ptr()
+        kimg = qimg + sizes['qimg']
     else:
         psi_, phik_ = new(BH, T, mk), new(BH, S, mk)
-    # the small operands and the scratch as pieces of one allocation (each a multiple of 64 floats long)
-    want = [BH * T, BH * mk * dim, BH * mk, BH * mk * dim, BH * mk, sizes['scratch'], n_ws if pieces else 0]
+    # the small operands and the scratch as pieces of one allocation (each a multiple of 64 floats long), as addresses: small
+    # calls are bound by the host, and every view is a microsecond of it
+    want = (BH * T, BH * mk * dim, BH * mk, BH * mk * dim, BH * mk, sizes['scratch'], n_ws if pieces else 0)
     offs = [0]
     for n in want:
         offs.append(offs[-1] + (n + 63) // 64 * 64)
     pool = new(offs[-1])
-    c_, kv, ksum, qg, qc, scratch, ws = (pool[a:a + n] for a, n in zip(offs, want))
-    kv, qg = kv.view(BH, mk, dim), qg.view(BH, mk, dim)
+    c_, kv, ksum, qg, qc, scratch, ws = (pool.data_ptr() + 4 * o for o in offs[:-1])
     if pieces and n_ws > 0:
         part_ws = ws
     dq, dk, dv = new(BH, T, dim), new(BH, S, dim), new(BH, S, dim)
     with torch.cuda.device(Q.device):
         st = _lib.stream_ptr(Q.device)
         _lib.call('flyhip_sblocal_bwd_prep', q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), g_.data_ptr(), o_.data_ptr(),
-                  ln_.data_ptr(), proj.data_ptr(), _lib.ptr(lens_b), _lib.ptr(psi_), _lib.ptr(phik_), c_.data_ptr(),
-                  kv.data_ptr(), ksum.data_ptr(), qg.data_ptr(), qc.data_ptr(), _lib.ptr(qimg), _lib.ptr(kimg),
-                  scratch.data_ptr(), scratch.numel(), BH, H, T, S, dim, mk, mh, float(t), st)
+                  ln_.data_ptr(), proj.data_ptr(), _lib.ptr(lens_b), _lib.ptr(psi_), _lib.ptr(phik_), c_,
+                  kv, ksum, qg, qc, qimg, kimg,
+                  scratch, sizes['scratch'], BH, H, T, S, dim, mk, mh, float(t), st)
         if support is not None:
             passes = ((qimg, kimg, q_, kv, ksum, dq, None), (kimg, qimg, k_, qg, qc, dk, dv))
             for key_major, (tabs, (oimg, iimg, x1, gmat, gvec, d1, d3)) in enumerate(zip(support, passes)):
@@ -206,28 +207,28 @@ def _backward_hip(Q, K, V, G, O, LN, P, lens_b, H, local_context, t, dims, piece
                     n_heavy = heavy.numel()
                     n_hws = _lib.load().flyhip_sbblocksparse_bwd_parts_floats(BH // H, n_heavy, parts, dim, mk, key_major)
                     hws = new(n_hws)
-                _lib.call('flyhip_sbblocksparse_bwd_pieces', oimg.data_ptr(), iimg.data_ptr(), x1.data_ptr(), ln_.data_ptr(),
-                          c_.data_ptr(), gmat.data_ptr(), gvec.data_ptr(), proj.data_ptr(), d1.data_ptr(), _lib.ptr(d3),
+                _lib.call('flyhip_sbblocksparse_bwd_pieces', oimg, iimg, x1.data_ptr(), ln_.data_ptr(),
+                          c_, gmat, gvec, proj.data_ptr(), d1.data_ptr(), _lib.ptr(d3),
                           tl_ptr.data_ptr(), _lib.table_ptr(tl_inner), _lib.table_ptr(tl_blk), _lib.ptr(skip), _lib.ptr(heavy),
                           n_heavy, parts, _lib.ptr(hws), n_hws, BH, H, T, S, dim, mk, float(t), key_major,
                           float(dropout[0]), int(dropout[1]), st)
         elif pieces:
-            _lib.call('flyhip_sblocal_bwd_pieces', qimg.data_ptr(), kimg.data_ptr(), q_.data_ptr(),
-                      ln_.data_ptr(), c_.data_ptr(), _lib.ptr(lens_b), kv.data_ptr(), ksum.data_ptr(), proj.data_ptr(),
-                      dq.data_ptr(), None, _lib.ptr(part_ws), n_ws, BH, H, T, S, dim, mk, local_context, float(t), 0,
+            _lib.call('flyhip_sblocal_bwd_pieces', qimg, kimg, q_.data_ptr(),
+                      ln_.data_ptr(), c_, _lib.ptr(lens_b), kv, ksum, proj.data_ptr(),
+                      dq.data_ptr(), None, part_ws, n_ws, BH, H, T, S, dim, mk, local_context, float(t), 0,
                       float(dropout[0]), int(dropout[1]), st)
-            _lib.call('flyhip_sblocal_bwd_pieces', kimg.data_ptr(), qimg.data_ptr(), k_.data_ptr(),
-                      ln_.data_ptr(), c_.data_ptr(), _lib.ptr(lens_b), qg.data_ptr(), qc.data_ptr(), proj.data_ptr(),
-                      dk.data_ptr(), dv.data_ptr(), _lib.ptr(part_ws), n_ws, BH, H, T, S, dim, mk, local_context, float(t), 1,
+            _lib.call('flyhip_sblocal_bwd_pieces', kimg, qimg, k_.data_ptr(),
+                      ln_.data_ptr(), c_, _lib.ptr(lens_b), qg, qc, proj.data_ptr(),
+                      dk.data_ptr(), dv.data_ptr(), part_ws, n_ws, BH, H, T, S, dim, mk, local_context, float(t), 1,
                       float(dropout[0]), int(dropout[1]), st)
         else:
             _lib.call('flyhip_sblocal_bwd', q_.data_ptr(), psi_.data_ptr(), g_.data_ptr(), k_.data_ptr(), phik_.data_ptr(),
-                      v_.data_ptr(), ln_.data_ptr(), c_.data_ptr(), _lib.ptr(lens_b), kv.data_ptr(), ksum.data_ptr(),
+                      v_.data_ptr(), ln_.data_ptr(), c_, _lib.ptr(lens_b), kv, ksum,
                       proj.data_ptr(), dq.data_ptr(), None, BH, H, T, S, dim, mk, local_context, float(t), 0, st)
             _lib.call('flyhip_sblocal_bwd', k_.data_ptr(), phik_.data_ptr(), v_.data_ptr(), q_.data_ptr(), psi_.data_ptr(),
-                      g_.data_ptr(), ln_.data_ptr(), c_.data_ptr(), _lib.ptr(lens_b), qg.data_ptr(), qc.data_ptr(),
+                      g_.data_ptr(), ln_.data_ptr(), c_, _lib.ptr(lens_b), qg, qc,
                       proj.data_ptr(), dk.data_ptr(), dv.data_ptr(), BH, H, T, S, dim, mk, local_context, float(t), 1, st)
-    return dq[..., :E], dk[..., :E], dv[..., :D]
+    return tuple(x if width == dim else x[..., :width] for x, width in ((dq, E), (dk, E), (dv, D)))
 
 
 # (head dim, features) of the kernels of flyhip_sblocal_bwd_far
@@ -310,9 +311,11 @@ def _backward_far(query, key, value, P, local_context, t, key_lengths, out, log_
         for b0 in range(0, B, nb):
             for h0 in range(0, H, nh):
                 b1, h1 = min(B, b0 + nb), min(H, h0 + nh)
-                part = [x[b0:b1, :, h0:h1] for x in (q, k, v, o, g, dq, dk, dv)]
-                ln_ = ln[b0:b1, h0:h1].contiguous()
-                lens_ = None if lens is None else lens[b0:b1]
+                part, ln_, lens_ = (q, k, v, o, g, dq, dk, dv), ln, lens
+                if b1 - b0 < B or h1 - h0 < H:
+                    part = [x[b0:b1, :, h0:h1] for x in part]
+                    ln_ = ln[b0:b1, h0:h1].contiguous()
+                    lens_ = None if lens is None else lens[b0:b1]
                 qs, ks, vs, os_, gs, dqs, dks, dvs = part
                 _lib.call('flyhip_sblocal_bwd_far', qs.data_ptr(), ks.data_ptr(), vs.data_ptr(), os_.data_ptr(), gs.data_ptr(),
                           ln_.data_ptr(), proj.data_ptr(), _lib.ptr(lens_), dqs.data_ptr(), dks.data_ptr(), dvs.data_ptr(),
@@ -320,7 +323,7 @@ def _backward_far(query, key, value, P, local_context, t, key_lengths, out, log_
                           *strides(q), *strides(k), *strides(v), *strides(o), *strides(g), *strides(dq), *strides(dk),
                           *strides(dv), float(t), st)
     # (contiguous in the inputs' shapes also where the head dim was padded, as the other routes return them)
-    return dq[..., :E].contiguous(), dk[..., :E].contiguous(), dv[..., :D].contiguous()
+    return tuple(x if width == dim else x[..., :width].contiguous() for x, width in ((dq, E), (dk, E), (dv, D)))
 
 
 def _band_terms_hip(Q, K, V, G, psi, phik, LN, c, lens_b, H, local_context, t, dims, dropout=(0.0, 0), attn_mask=None):
@@ -438,6 +441,8 @@ def sblocal_backward(query, key, value, projection_matrix, local_context, softma
     wdt = torch.float64 if query.dtype == torch.float64 else torch.float32
 
     def bh(x):                                   # (B,L,H,C) -> (B*H, L, C)
+        if H == 1 and x.dtype == wdt:            # (one call of the host's where three do the same)
+            return x.squeeze(2)
         return x.permute(0, 2, 1, 3).reshape(B * H, x.shape[1], x.shape[3]).to(wdt)
     Q, K, V, G, O = bh(query), bh(key), bh(value), bh(grad_out), bh(out)
     LN = log_normalization.reshape(B * H, T, 1).to(wdt)
@@ -496,6 +501,8 @@ def sblocal_backward(query, key, value, projection_matrix, local_context, softma
         dK += st * ((uk[..., :mh] - uk[..., mh:]) @ P) - t * K * uk.sum(-1, keepdim=True)
 
     def back(x, like):                           # (B*H, L, C) -> (B,L,H,C)
+        if H == 1 and x.dtype == like.dtype:
+            return x.unsqueeze(2)
         # (in the inputs' own memory order: autograd then accumulates the gradient without another copy)
         return x.reshape(B, H, x.shape[1], x.shape[2]).permute(0, 2, 1, 3).to(like.dtype, memory_format=torch.contiguous_format)
     return back(dQ, query), back(dK, key), back(dV, value)

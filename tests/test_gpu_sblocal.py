@@ -1397,3 +1397,25 @@ def test_float32_gradients_on_whole_and_cut_tiles(E, mh, window, T, S):
     assert rel_err(out, ref_out.detach()) <= 1e-4
     for a, r in zip(got, ref):
         assert rel_err(a, r) <= 2e-4, rel_err(a, r)
+
+
+@pytest.mark.parametrize('H,dtype', [(1, torch.float32), (2, torch.float32), (1, torch.bfloat16)])
+def test_an_output_without_a_gradient_counts_as_zero(H, dtype):
+    """A consumer that returns no gradient for the output: query, key and value get zeros."""
+    from fly_amd import SBLocalAttention
+
+    class Silent(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+
+    dev = torch.device('cuda:0')
+    q, k, v, _ = make_inputs(1, 130, 130, H, 64, 64, 32, seed=5, dtype=dtype)
+    leaves = [x.to(dev).requires_grad_() for x in (q, k, v)]
+    out, _ = SBLocalAttention(33, dim_heads=64, nb_features=64).to(dev)(*leaves)
+    for g in torch.autograd.grad(Silent.apply(out).sum(), leaves):
+        assert float(g.abs().max()) == 0.0
