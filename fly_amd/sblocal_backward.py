@@ -249,19 +249,21 @@ def _far_pays(rows, heads, local_context, dims):
     (head dim, features).  The subtracting kernels form M-wide products on every pair of the band, in proportion to the window,
     and several heads cost them a permuting copy of every tensor.  The far path costs the chunk sums, two edge chunks per 64
     rows where the window is a multiple of 128 and up to four otherwise, and a fixed share per wave that does not shrink with
-    the features.  us, far / subtracting (windows 12, 96 or 97, 128, 200, 300, 512, 600 unless given):
-      (64, 128)  one head, 8000 rows: 96/98, 95/97, -, 110/105, 116/106, -, 126/118; 16384: 100/114 .. 131/164;
-                 200704: 677/738, 680/793, 617/796, 774/913, 798/975, 717/1172, 865/1281
-      (64, 64)   one head, 8000: 93/106, 93/105, -, 110/106, 116/105, -, 126/108; 50176: 203/163, 205/181, 181/181, -, -,
-                 209/293; 100352: 342/304, 346/332, -, 403/383, 413/409, -, 438/529; eight heads, 65536: 226/244 .. 242/365
-      (64, 32)   one head, 8000: 108/112, 108/145, -, 129/112, 136/110, -, 147/135; 50176: 231/147, 232/163, 199/163, -, -,
-                 228/242; 100352: 396/272, 397/295, -, 462/343, 478/364, -, 476/475; eight heads, 8000: 110/138 .. 110/127;
-                 65536: 245/223, 244/240, 212/244; twelve, 120000: 466/417, 464/452, -, 554/502, 577/533, -, 630/677
-      (32, 64)   one head, 16384: 72/104 .. 97/105; 100352: 197/180, 202/202, -, 231/243, 238/266, -, 267/362; 31360: 94/99,
-                 95/99, -, 112/106, 118/106, -, 130/140; twelve heads, 120000: 265/288 .. 365/515
-      (32, 32)   one head, 16384: 80/103 .. 109/103; 100352: 213/153, 215/173, -, 247/212, 254/226, -, 277/307; 200704: 354/296,
-                 356/331, 298/332; eight heads, 32768: 89/121 .. 125/147; twelve, 120000: 283/253, 283/274, -, 339/320,
-                 357/343, -, 392/451."""
+    the features.  us, far / subtracting at windows 12, 97, 128, 200, 300, 512, 600:
+      (64, 128)  one head, 8000 rows: 100/88, 94/92, 86/93, 106/101, 115/102, 100/109, 120/113; 15680: 109/110 .. 130/157;
+                 200704: 691/696, 654/739, 609/743, 718/846, 762/907, 679/1071, 791/1179
+      (64, 64)   one head, 8000: 97/86, 92/87, 82/86, 105/87, 115/87, 96/90, 118/93; 50176: 206/160, 192/176, 173/176, 216/202,
+                 233/214, 196/252, 240/279; 100352: 350/304, 325/329, 288/330, 364/373, 389/394, 317/458, 387/502; eight heads,
+                 64000: 235/256 .. 285/387
+      (64, 32)   one head, 8000: 115/87, 105/89, 92/88, 121/86, 131/86, 104/86, 133/86; 50176: 235/142, 216/154, 191/155,
+                 248/174, 266/184, 213/214, 272/238; 200704: 737/480, -, 578/510, -, -, 631/716, 806/785; twelve heads, 120000:
+                 474/406, 434/426, 384/428, 503/473, 542/497, 443/569, 562/614
+      (32, 64)   one head, 15680: 81/86 .. 95/97; 50176: 130/106, 122/117, 107/118, 125/136, 130/148, 117/176, 138/196; 100352:
+                 198/165, 184/186, 163/188, 202/220, 218/237, 188/284, 230/321; 200704: 329/332, 300/362, 265/364, 347/430,
+                 385/463, 326/556, 403/619; twelve heads, 120000: 267/277 .. 321/468
+      (32, 32)   one head, 15680: 91/96, 83/95, 74/94, 95/96, 104/93, 84/92, 105/93; 100352: 217/136, 194/148, 171/150, 217/172,
+                 230/185, 191/217, 241/245; 200704: 360/270, 322/292, 280/293, 374/336, 408/361, 333/429, 427/471; twelve heads,
+                 120000: 288/236, 261/250, 234/252, 301/281, 330/298, 276/343, 345/373."""
     dim, m = dims
     whole = local_context % 128 == 0
     few_edges = whole or local_context < 192
@@ -274,6 +276,8 @@ def _far_pays(rows, heads, local_context, dims):
         return True
     if heads == 1 and (dim, m) == (64, 32):
         return local_context >= (512 if whole else 768)
+    if heads == 1 and (dim, m) == (32, 64):
+        return local_context >= (128 if whole else 192) or (rows > 150000 and local_context >= 96)
     return local_context >= (128 if whole else 512)
 
 
