@@ -2721,7 +2721,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
     constexpr int KS = E / 32, EB = E / 16, ROWB = 2 * E, TILE = 32 * ROWB;
     constexpr float LOG2E = 1.4426950408889634f;
     __shared__ __attribute__((aligned(128))) char tiles[2][2][TILE];            // [stage][Y1 | Y2], rows as RowsToLds leaves them
-    __shared__ __attribute__((aligned(16))) float rowv[2][3][32];              // key-major: [stage][lse2 | delta (DROP: / drop_scale) | row hash] of the tile's queries
+    __shared__ __attribute__((aligned(16))) float rowv[2][3][32];              // key-major: [stage][lse2 (DROP: - log2 drop_scale) | delta (DROP: / drop_scale) | row hash] of the tile's queries
     const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     int unit, grp;
@@ -2745,11 +2745,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
     const long d1s = KEYMAJOR ? a.dk_sm : a.dq_sm;
     T* d2 = reinterpret_cast<T*>(a.dv) + z * a.dv_sz + head * a.dv_sh;
 
-    // dS = P (M g.v - delta), M = drop_scale or 0, is formed as -drop_scale P (delta / drop_scale - kept g.v): the sums start at
-    // delta / drop_scale and x2 goes in negated, so that a pair costs one select and one product, and the factor is the epilogue's
-    const float inv_drop = DROP ? 1.0f / a.drop_scale : 1.0f;
+    // dS = P (M g.v - delta), M = drop_scale or 0, is formed as -P' (delta / drop_scale - kept g.v) with P' = drop_scale P: the sums
+    // start at delta / drop_scale, x2 goes in negated and the factor of P' is in the rows' exponents, so that a pair costs one
+    // select and one product.  (The second products read M P and dS themselves rounded to the input type: float16 without the factor
+    // would put them log2(drop_scale) bits deeper into its subnormal range.)
+    const float inv_drop = DROP ? 1.0f / a.drop_scale : 1.0f, log_drop = DROP ? log2f(a.drop_scale) : 0.f;
     uintx4 x1[2][KS], x2[2][KS];
-    float l_own[2] = {0.f, 0.f}, d_own[2] = {0.f, 0.f};          // query-major: lse2 and delta of the lane's queries
+    float l_own[2] = {0.f, 0.f}, d_own[2] = {0.f, 0.f};          // query-major: lse2 and delta of the lane's queries, as in rowv
     float km_own[2] = {0.f, 0.f};                     // key-major: the key mask entries of the lane's keys
     uint32_t h_own[2] = {0u, 0u};                     // DROP, query-major: hash of (seed, global row) of the lane's queries
     floatx4 acc1[2][EB], acc2[KEYMAJOR ? 2 : 1][KEYMAJOR ? EB : 1];     // d q | d k, and d v
@@ -2763,7 +2765,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
         }
         if (MASKED && KEYMAJOR && a.key_mask) km_own[qq] = a.key_mask[z * a.km_stride + row];
         if (!KEYMAJOR) {
-            l_own[qq] = a.lse2[qvec + row];
+            l_own[qq] = a.lse2[qvec + row] - log_drop;
             if (DROP) h_own[qq] = drop_row_hash(a.drop_seed, (uint32_t)(qvec + row));
             // delta of the query, g . out, from the output row in the layout of the gradient row; kept for the key-major launch
             const uint16_t* orow = reinterpret_cast<const uint16_t*>(a.out) + z * a.o_sz + head * a.o_sh + row * a.o_sm;
@@ -2812,7 +2814,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
     };
     auto stash = [&](int stage) __attribute__((always_inline)) {
         if (KEYMAJOR && tid < 32) {
-            rowv[stage][0][tid] = rl;
+            rowv[stage][0][tid] = rl - log_drop;
             rowv[stage][1][tid] = DROP ? rd * inv_drop : rd;
             if (DROP) rowv[stage][2][tid] = __uint_as_float(rh);
         }
@@ -2955,16 +2957,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
         drain_loads();                                   // this wave's share of the next tile is in LDS
         __syncthreads();
     }
-    const float d1_scale = DROP ? -a.scale * a.drop_scale : -a.scale;
     if (have) {
 #pragma unroll
         for (int qq = 0; qq < 2; ++qq) {
             const long row = (long)bo * 32 + 16 * qq + r16;
 #pragma unroll
-            for (int eb = 0; eb < EB; ++eb) store4_f32(d1 + row * d1s + 16 * eb + 4 * g, acc1[qq][eb] * d1_scale);
+            for (int eb = 0; eb < EB; ++eb) store4_f32(d1 + row * d1s + 16 * eb + 4 * g, acc1[qq][eb] * -a.scale);
             if (KEYMAJOR) {
 #pragma unroll
-                for (int eb = 0; eb < EB; ++eb) store4_f32(d2 + row * a.dv_sm + 16 * eb + 4 * g, DROP ? acc2[qq][eb] * a.drop_scale : acc2[qq][eb]);
+                for (int eb = 0; eb < EB; ++eb) store4_f32(d2 + row * a.dv_sm + 16 * eb + 4 * g, acc2[qq][eb]);
             }
         }
     }

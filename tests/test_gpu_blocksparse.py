@@ -982,6 +982,43 @@ def test_blocksparse_attention_dropout_inside_the_kernels(E, dtype, p_drop):
     assert rel_err(plain, torch.einsum('bhts,bshd->bthd', prob, vd).detach()) <= tol
 
 
+@pytest.mark.parametrize('E', [32, 64])
+def test_float16_dropout_gradients_at_a_high_rate(E):
+    """The second products of the backward take M P and dS = P (M g.v - delta), M = 1 / (1 - p) = 100 here, rounded to float16.  With
+    output gradients of 1e-4 dS lies around 4e-4, in float16's normal range; dS / M, around 4e-6, lies deep in the subnormal one, where
+    a rounding to multiples of 2^-24 costs half a percent.  Bound: dS, delta's output row and the result are rounded, each by
+    2^-12 of its value in the 2-norm, sqrt(3) 2^-12 together; about twice that."""
+    from fly_amd import BlockSparseAttention
+    from oracle.sblocal import dropout_keep
+
+    class Cfg:
+        block = 32
+
+        def make_layout(self, seqlen):
+            return ob.band_layout(seqlen // 32, seqlen // 32, 3).unsqueeze(0).repeat(2, 1, 1)
+
+    B, T, H, p_drop = 2, 352, 2, 0.99
+    print('case', E, flush=True)
+    g = torch.Generator().manual_seed(23)
+    q, k, v = (torch.randn(B, T, H, E, generator=g).half() for _ in range(3))
+    w = (torch.randn(B, T, H, E, generator=g) * 1e-4).half()
+    mod = BlockSparseAttention(Cfg(), attention_dropout=p_drop, max_seq_length=T).to(DEV).train()
+    xs = [x.to(DEV).requires_grad_() for x in (q, k, v)]
+    torch.manual_seed(5)
+    out, _ = mod(*xs)
+    grads = torch.autograd.grad(out, xs, w.to(DEV))
+
+    qd, kd, vd = (x.double().requires_grad_() for x in (q, k, v))
+    lay = ob.densify_tensor(torch.ones(1, int(mod.master_layout.sum()), 32, 32), mod.master_layout.cpu())[0].bool()
+    s = torch.einsum('bthe,bshe->bhts', qd, kd) / math.sqrt(E)
+    prob = torch.softmax(s.masked_fill(~lay.unsqueeze(0), float('-inf')), -1)
+    ref = torch.einsum('bhts,bshd->bthd', prob * dropout_keep(mod.last_dropout_seed, p_drop, B, H, T, T), vd)
+    for got, want, name in zip(grads, torch.autograd.grad(ref, (qd, kd, vd), w.double()), 'qkv'):
+        err = float((got.cpu().double() - want).norm() / want.norm())
+        print('d' + name, err, flush=True)
+        assert err <= 1e-3, (name, err)
+
+
 def test_probabilities_from_log_denominators():
     """flyhip_bs_attn_lse + flyhip_bs_sdd_prob: the one-kernel attention's per-row log-denominators
     turn an sdd into the softmax probabilities (what the training path's backward starts from); against
