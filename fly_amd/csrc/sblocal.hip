@@ -24,6 +24,7 @@
 // consecutive keys/features -- which is exactly the operand layout the next product needs.
 #include "common.h"
 #include "local.h"
+#include "band_tiles.h"
 #include <hip/hip_ext.h>
 #include <math.h>
 #include <type_traits>
@@ -2741,9 +2742,8 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
     const int len = a.lens ? min((int)a.lens[b], a.S) : a.S;
     const int lc_lo = a.lc / 2, lc_hi = (a.lc + 1) / 2;    // band: -lc_lo <= s - i < lc_hi
 
-    const int q_last = min(q0 + TQB - 1, a.T - 1);
-    const int lo = max(0, q0 - lc_lo), hi = min(len, q_last + lc_hi);
-    const int kt_lo = lo / TKL, kt_hi = (hi > lo) ? (hi + TKL - 1) / TKL : kt_lo;
+    const TileRange all = band_tiles(q0, min(q0 + TQB, a.T), lc_lo, lc_hi, len, TKL);
+    const int kt_lo = all.lo, kt_hi = all.hi;
     RowsToLds<TKL, E, NT> rk, rv;
     rk.init(kptr, a.k_ss, a.S - 1, w, lane);
     rv.init(vptr, a.v_ss, a.S - 1, w, lane);
@@ -2786,9 +2786,7 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
     __syncthreads();
     // the tiles that touch the band of one of the wave's queries lie in a row (wave-uniform, scalar: w is): the loop over them
     // has no branch around its products, which would cost a copy of every accumulator per tile
-    const int w_last = min(qw0 + QW, a.T) - 1;
-    const int w_lo = w_last < qw0 ? kt_hi : max(kt_lo, max(0, qw0 - lc_lo) / TKL);
-    const int w_hi = w_last < qw0 ? kt_hi : min(kt_hi, (max(0, min(len, w_last + lc_hi)) + TKL - 1) / TKL);
+    const TileRange own = wave_tiles(all, qw0, min(qw0 + QW, a.T), lc_lo, lc_hi, len, TKL);
     int kt = kt_lo;
     auto begin_tile = [&]() __attribute__((always_inline)) {
         if (kt + 1 < kt_hi) fetch(kt + 1, (kt + 1 - kt_lo) & 1);
@@ -2797,8 +2795,8 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
         drain_loads();                                       // this wave's share of the next tile is in LDS
         __syncthreads();
     };
-    for (; kt < w_lo; ++kt) { begin_tile(); end_tile(); }
-    for (; kt < w_hi; ++kt) {
+    for (; kt < own.lo; ++kt) { begin_tile(); end_tile(); }
+    for (; kt < own.hi; ++kt) {
         const int s_base = kt * TKL;
         const char* Ks = lds + ((kt - kt_lo) & 1) * 2 * TILE;
         const char* Vs = Ks + TILE;
@@ -2986,9 +2984,8 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
     const int A = KEYMAJOR ? lc_hi - 1 : lc_lo, Bq = KEYMAJOR ? lc_lo + 1 : lc_hi;
     const int Lo = KEYMAJOR ? len : a.T, Ln = KEYMAJOR ? a.T : len;
 
-    const int o_last = min(min(o0 + TQB - 1, R_out - 1), Lo - 1);
-    const int lo = max(0, o0 - A), hi = o_last >= o0 ? min(Ln, o_last + Bq) : 0;
-    const int it_lo = lo / TKL, it_hi = (hi > lo) ? (hi + TKL - 1) / TKL : it_lo;
+    const TileRange all = band_tiles(o0, min(o0 + TQB, min(R_out, Lo)), A, Bq, Ln, TKL);
+    const int it_lo = all.lo, it_hi = all.hi;
     RowsToLds<TKL, E, NT> r1, r2;
     r1.init(y1p, y1s, R_in - 1, w, lane);
     r2.init(y2p, y2s, R_in - 1, w, lane);
@@ -3072,9 +3069,7 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
     __syncthreads();
     // the tiles that touch the band of one of the wave's outer rows lie in a row (wave-uniform, scalar): the loop over them has
     // no branch around its products, which would cost a copy of every accumulator per tile
-    const int w_last = min(ow0 + QW, Lo) - 1;
-    const int w_lo = w_last < ow0 ? it_hi : max(it_lo, (max(0, ow0 - A)) / TKL);
-    const int w_hi = w_last < ow0 ? it_hi : min(it_hi, (max(0, min(Ln, w_last + Bq)) + TKL - 1) / TKL);
+    const TileRange own = wave_tiles(all, ow0, min(ow0 + QW, Lo), A, Bq, Ln, TKL);
     int it = it_lo;
     auto begin_tile = [&]() __attribute__((always_inline)) {
         if (it + 1 < it_hi) fetch(it + 1, (it + 1 - it_lo) & 1);
@@ -3084,8 +3079,8 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
         drain_loads();                                     // this wave's share of the next tile is in LDS
         __syncthreads();
     };
-    for (; it < w_lo; ++it) { begin_tile(); end_tile(); }
-    for (; it < w_hi; ++it) {
+    for (; it < own.lo; ++it) { begin_tile(); end_tile(); }
+    for (; it < own.hi; ++it) {
         const char* Y1 = lds + ((it - it_lo) & 1) * STAGE_BYTES;
         const char* Y2 = Y1 + TILE;
         const float* Ls = reinterpret_cast<const float*>(Y2 + TILE);

@@ -4,6 +4,7 @@ header declares.  Nothing here launches a kernel."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 import torch
@@ -418,3 +419,56 @@ def test_route_of_the_bfloat16_scatterbrain_gradients():
     assert not far(8000, 1, 300, 64, 32) and far(50176, 1, 512, 64, 32) and not far(100352, 1, 600, 64, 32) and far(65536, 8, 128, 64, 32)
     assert far(16384, 1, 12, 32, 64) and not far(100352, 1, 12, 32, 64) and far(100352, 1, 600, 32, 64)
     assert far(32768, 8, 12, 32, 32) and not far(120000, 12, 300, 32, 32) and far(120000, 12, 600, 32, 32)
+
+
+_BAND_TILES_CHECK = r"""
+#include "band_tiles.h"
+#include <cstdio>
+using namespace flyhip;
+int main() {
+    const int tile = 64, sizes[] = {1, 17, 64, 130, 333, 784}, windows[] = {1, 2, 12, 50, 129, 130, 257, 1024};
+    long checked = 0;
+    for (int T : sizes) for (int S : sizes) for (int len = 0; len <= S; len += len < 70 || len > S - 3 ? 1 : 23) for (int lc : windows)
+    for (int key_major = 0; key_major < 2; ++key_major) for (int wave_rows = 16; wave_rows <= 32; wave_rows += 16) {
+        // (the band -lc / 2 <= key - query < (lc + 1) / 2 seen from either side)
+        const int below = key_major ? (lc + 1) / 2 - 1 : lc / 2, above = key_major ? lc / 2 + 1 : (lc + 1) / 2;
+        const int outer = key_major ? len : T, rows = key_major ? S : T, inner = key_major ? T : len;
+        for (int o0 = 0; o0 < rows; o0 += 4 * wave_rows) {
+            const int end = o0 + 4 * wave_rows < outer ? o0 + 4 * wave_rows : outer;
+            const TileRange all = band_tiles(o0, end, below, above, inner, tile);
+            if (all.lo < 0 || all.hi < all.lo) return printf("workgroup %d: tiles %d .. %d\n", o0, all.lo, all.hi), 1;
+            if (all.lo < all.hi && (all.hi - 1) * tile >= inner) return printf("workgroup %d: tile %d past the inner rows\n", o0, all.hi - 1), 1;
+            for (int w = 0; w < 4; ++w, ++checked) {
+                const int w0 = o0 + wave_rows * w, w1 = w0 + wave_rows < outer ? w0 + wave_rows : outer;
+                const TileRange own = wave_tiles(all, w0, w1, below, above, inner, tile);
+                // the loops of a wave: up to own.lo, up to own.hi, up to all.hi, a barrier in each of their iterations
+                int t = all.lo, barriers = 0;
+                for (; t < own.lo; ++t) ++barriers;
+                for (; t < own.hi; ++t) ++barriers;
+                for (; t < all.hi; ++t) ++barriers;
+                if (barriers != all.hi - all.lo)
+                    return printf("T %d S %d len %d window %d key_major %d rows %d o0 %d wave %d: %d barriers, %d tiles\n",
+                                  T, S, len, lc, key_major, wave_rows, o0, w, barriers, all.hi - all.lo), 1;
+                // no pair of the band outside the wave's own tiles
+                for (int o = w0; o < w1; ++o) {
+                    const int n0 = o - below > 0 ? o - below : 0, n1 = (o + above < inner ? o + above : inner) - 1;
+                    if (n0 <= n1 && (n0 / tile < own.lo || n1 / tile >= own.hi)) return printf("row %d sees a tile outside %d .. %d\n", o, own.lo, own.hi), 1;
+                }
+            }
+        }
+    }
+    return checked > 100000 ? 0 : 1;
+}
+"""
+
+
+def test_waves_of_local_attention_pass_the_same_barriers(tmp_path):
+    """The 2-byte kernels of plain local attention walk a workgroup's tiles in three loops per wave (before, inside and behind the
+    tiles that its own rows see) with a barrier in every iteration: the four waves of a workgroup have to make the same number,
+    also where the queries lie past the last valid key.  Over odd and even windows, both orientations, 16 and 32 rows a wave."""
+    src = tmp_path / 'check.cpp'
+    src.write_text(_BAND_TILES_CHECK)
+    exe = str(tmp_path / 'check')
+    subprocess.run(['g++', '-std=c++17', '-O2', '-I', os.path.join(ROOT, 'fly_amd', 'csrc'), str(src), '-o', exe], check=True)
+    res = subprocess.run([exe], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout
