@@ -12,6 +12,9 @@ from .sblocal_attention import rows_for_vectors
 UNION_MIN_SHARING = 1.5
 # sdd with both operands contraction-major (a^T b) takes the split-K kernel from this contraction length on
 KMAJOR_MIN_K = 512
+# dds from this many rows of the dense operand on may bring the sparse blocks into LDS by 16-byte transfers, which want them to
+# start at a multiple of 16 bytes; below it every kernel reads them by ordinary loads
+DDS_TRANSFER_MIN_M = 4096
 
 _BLOCKS = (16, 32, 64, 128)
 
@@ -262,6 +265,8 @@ class matmul:
         N = per_head * self.block
         Z = a.shape[0]
         M = a.shape[3 if trans_a else 2]
+        if M >= DDS_TRANSFER_MIN_M and b.data_ptr() % 16 != 0:
+            b = b.clone()
         a_sm, a_sk = (a.stride(3), a.stride(2)) if trans_a else (a.stride(2), a.stride(3))
         c = torch.empty((Z, H, N, M) if trans_c else (Z, H, M, N), dtype=a.dtype, device=a.device)
         c_sm, c_sn = (c.stride(3), c.stride(2)) if trans_c else (c.stride(2), c.stride(3))

@@ -3239,8 +3239,9 @@ extern "C" int flyhip_bs_dds_bias(const void* a, const void* b_sp, const void* b
             return check_launch("bs_dds32d_kernel");
         }
         if (FLY_DDS_STATIONARY == 2 && max_seg_len > DDS_STAT_STEPS && max_seg_len <= DDS_MAX_STEPS && (long)M >= 512L * 8 &&
-            (trans_b || !bias)) {
-            // longer lists: the same workgroup shape with the weights passing through LDS ([k][n] blocks: no bias)
+            (trans_b || !bias) && reinterpret_cast<uintptr_t>(b_sp) % 16 == 0) {
+            // longer lists: the same workgroup shape with the weights passing through LDS, by transfers of 16 bytes that have to start
+            // at a multiple of that ([k][n] blocks: no bias)
             const long tiles = (M + 511) / 512;
             long n_streams = 1, best = -1;
             for (long n = 1; n <= tiles && n * n_grp * Z <= 4L * mach.cus + (long)n_grp * Z; ++n) {

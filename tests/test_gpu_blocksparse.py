@@ -677,6 +677,45 @@ def test_dds_long_lists_past_the_last_tile(M, trans_b):
     assert rel_err(out, ref) <= TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize('trans_b', [True, False])
+@pytest.mark.parametrize('offset', [1, 4])
+def test_dds_long_lists_with_blocks_off_a_16_byte_boundary(offset, trans_b, monkeypatch):
+    """Sparse blocks that are a view into a larger buffer, 2 or 8 bytes off a 16-byte boundary, at a size whose kernel moves them into
+    LDS by 16-byte transfers: matmul hands the kernels an aligned copy (checked before the launch), and the C entry, given the
+    misaligned pointer itself, takes a kernel with ordinary loads."""
+    from fly_amd import matmul, _lib
+    print('case', offset, trans_b, flush=True)
+    Z, H, block, n_out, n_in, M = 1, 2, 32, 5, 12, 4096 + 40
+    g = torch.Generator().manual_seed(53)
+    seg = torch.ones(H, n_out, n_in, dtype=torch.long)
+    seg[1, 2, :] = 0
+    seg[1, 2, 1:12] = 1                                    # 11 entries
+    layout = seg if trans_b else seg.transpose(1, 2).contiguous()
+    w = torch.randn(Z, int(layout.sum()), block, block, generator=g).bfloat16()
+    x = torch.randn(Z, H, M, n_in * block, generator=g).bfloat16().to(DEV)
+    flat = torch.zeros(w.numel() + offset, dtype=w.dtype, device=DEV)
+    view = flat[offset:].view(w.shape)
+    view.copy_(w)
+    assert view.data_ptr() % 16 == 2 * offset and view.is_contiguous()
+    launch, calls = _lib.call, []
+
+    def call(name, *args):
+        if name == 'flyhip_bs_dds_bias':
+            assert args[1] % 16 == 0, 'misaligned blocks would reach the transfers into LDS'
+            calls.append(args)
+        return launch(name, *args)
+
+    monkeypatch.setattr(_lib, 'call', call)
+    out = matmul(layout, block, 'dds', trans_a=False, trans_b=trans_b)(x, view)
+    ref = ob.dds(x.cpu().double(), w.double(), layout, block, False, trans_b)
+    assert len(calls) == 1 and rel_err(out, ref) <= TOL[torch.bfloat16]
+    again = torch.empty_like(out)
+    args = list(calls[0])
+    args[1], args[3] = view.data_ptr(), again.data_ptr()
+    launch('flyhip_bs_dds_bias', *args)
+    assert rel_err(again, ref) <= TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 def test_narrowing_linear_with_bias_and_long_lists(dtype):
     """Bias inside the dds kernel for long reduction lists (36 blocks a row), forward and gradients against the dense product."""
