@@ -19,6 +19,7 @@ touch -- all chunks at once as batched products over overlapping windows of the 
 Everything is ordinary tensor algebra (library GEMMs on whatever device the tensors live on); the
 clamp of the low-rank normaliser (sblocal_attention.py:111) is taken as inactive.
 """
+import functools
 import math
 
 import torch
@@ -243,42 +244,74 @@ def _far_kernel_dims(E, D, M):
     return None
 
 
-def _far_pays(rows, heads, local_context, dims):
+# What the two routes of the bfloat16 gradients take on an MI355X, by (head dim, features), in us.  Fitted to 2403 measured pairs
+# (64 to 200000 rows, 1 to 128 pairs of batch and head, windows 8 to 1024); of 1301 other pairs the route with the smaller of the two
+# figures is 0.4 % slower than the better one on average and more than 5 % slower on 36, where both are within some 10 % of each
+# other.
+#   chunk sums: a chain of launches; more of it per 128 of the window; a step of the scan per segment of a sequence; per 1000 rows
+#               what streams, and per 1000 rows and 128 of the window the band; per 1000 rows of whole rounds of resident
+#               workgroups the low-rank kernels, and what eight 32 x 16 blocks of pairs at the band's edges add to them; resident
+#               workgroups of those per compute unit
+#   subtracting: the host's launches, and what several heads add to them (permuting copies); the kernels' chain, more of it per 128 of
+#               the window, per 64 rows of a sequence; per 1000 rows, per 1000 rows and 128 of the window, per 1000 rows of several heads
+_ROUTE_COSTS = {
+    (64, 128): ((51.0, 3.65, 0.158, 0.908, 0.151, 0.614, 0.519, 1), (89.7, 35.8, 61.0, 3.89, 0.024, 2.674, 0.606, 0.833)),
+    (64, 64): ((31.5, 4.47, 0.199, 1.042, 0.131, 0.396, 0.460, 2), (92.3, 26.7, 40.7, 4.55, 0.019, 2.245, 0.446, 0.835)),
+    (64, 32): ((27.3, 5.06, 0.214, 0.755, 0.129, 0.696, 0.616, 2), (92.2, 25.2, 33.1, 5.29, 0.030, 1.996, 0.349, 0.830)),
+    (32, 64): ((27.9, 3.68, 0.212, 0.694, 0.092, 0.000, 0.256, 3), (92.1, 25.1, 35.4, 3.66, 0.016, 1.193, 0.339, 0.519)),
+    (32, 32): ((19.5, 3.81, 0.207, 0.367, 0.091, 0.264, 0.324, 3), (92.4, 24.1, 21.2, 5.39, 0.022, 1.039, 0.232, 0.516)),
+}
+_COMPUTE_UNITS = 256
+
+
+def _edge_blocks(local_context, chunks):
+    """Blocks of 32 x 16 pairs outside the band, or cut by it, in the chunks that the band's two edges cross, per 64 outer rows:
+    what the chunk-sum kernels form pair by pair (of a sequence of `chunks` chunks, on average)."""
+    lo, hi = local_context // 2, (local_context + 1) // 2
+    n = 0.0
+    for d in {-lo // 64, (63 - lo) // 64, (hi - 1) // 64, (hi + 62) // 64}:
+        if abs(d) < chunks:
+            rels = [64 * d + 32 * i - 16 * o for i in range(2) for o in range(4)]
+            n += (1 - abs(d) / chunks) * sum(not (rel - 15 >= -lo and rel + 31 < hi) for rel in rels)
+    return n
+
+
+@functools.lru_cache(maxsize=1024)
+def _far_pays(rows, heads, local_context, dims, length=None):
     """Whether bfloat16 tensors go to _backward_far where the kernels that subtract the band from the sums over all keys
-    (_backward_hip, on widened copies) could take them too; rows = batch x heads x the longer sequence, dims = the padded
+    (_backward_hip, on widened copies) could take them too: by the smaller of the two costs above.  rows = batch x heads x the
+    longer sequence, length = that sequence (unless given: images of 48 x 48 tokens where there is one head), dims = the padded
     (head dim, features).  The subtracting kernels form M-wide products on every pair of the band, in proportion to the window,
-    and several heads cost them a permuting copy of every tensor.  The far path costs the chunk sums, two edge chunks per 64
-    rows where the window is a multiple of 128 and up to four otherwise, and a fixed share per wave that does not shrink with
-    the features.  us, far / subtracting at windows 12, 97, 128, 200, 300, 512, 600:
-      (64, 128)  one head, 8000 rows: 100/88, 94/92, 86/93, 106/101, 115/102, 100/109, 120/113; 15680: 109/110 .. 130/157;
-                 200704: 691/696, 654/739, 609/743, 718/846, 762/907, 679/1071, 791/1179
-      (64, 64)   one head, 8000: 97/86, 92/87, 82/86, 105/87, 115/87, 96/90, 118/93; 50176: 206/160, 192/176, 173/176, 216/202,
-                 233/214, 196/252, 240/279; 100352: 350/304, 325/329, 288/330, 364/373, 389/394, 317/458, 387/502; eight heads,
-                 64000: 235/256 .. 285/387
-      (64, 32)   one head, 8000: 115/87, 105/89, 92/88, 121/86, 131/86, 104/86, 133/86; 50176: 235/142, 216/154, 191/155,
-                 248/174, 266/184, 213/214, 272/238; 200704: 737/480, -, 578/510, -, -, 631/716, 806/785; twelve heads, 120000:
-                 474/406, 434/426, 384/428, 503/473, 542/497, 443/569, 562/614
-      (32, 64)   one head, 15680: 81/86 .. 95/97; 50176: 130/106, 122/117, 107/118, 125/136, 130/148, 117/176, 138/196; 100352:
-                 198/165, 184/186, 163/188, 202/220, 218/237, 188/284, 230/321; 200704: 329/332, 300/362, 265/364, 347/430,
-                 385/463, 326/556, 403/619; twelve heads, 120000: 267/277 .. 321/468
-      (32, 32)   one head, 15680: 91/96, 83/95, 74/94, 95/96, 104/93, 84/92, 105/93; 100352: 217/136, 194/148, 171/150, 217/172,
-                 230/185, 191/217, 241/245; 200704: 360/270, 322/292, 280/293, 374/336, 408/361, 333/429, 427/471; twelve heads,
-                 120000: 288/236, 261/250, 234/252, 301/281, 330/298, 276/343, 345/373."""
+    and several heads cost them a permuting copy of every tensor.  The far path costs the chunk sums, a scan over each sequence,
+    the chunks that the band's edges cross, and a share per wave that does not shrink with the features.  us, far / subtracting, at
+    windows 12, 128, 300, 600:
+      (64, 128)  one head, 64 images of 3136: 692/697, 606/743, 763/912, 803/1188; one sequence of 79046, window 127: 379/331
+      (64, 64)   8 images of 1000: 97/94, 81/95, 113/94, 117/95; 16 of 3136: 205/159, 172/178, 231/216, 241/283
+      (64, 32)   16 images of 3136: 234/141, 191/154, 264/184, 272/236; 8 heads of 8000: 261/231, 218/246, 302/281, 311/343
+      (32, 64)   16 images of 3136: 130/105, 107/117, 129/147, 138/196; one sequence of 111902, window 87: 556/225
+      (32, 32)   5 images of 3136: 91/94, 73/95, 103/94, 105/95; 64 of 3136: 361/270, 279/293, 408/364, 434/484."""
     dim, m = dims
-    whole = local_context % 128 == 0
-    few_edges = whole or local_context < 192
-    if m > 64:
-        return m > 128 or rows > 8192 or heads > 1 or few_edges             # (above 128 features there is no other kernel)
-    if heads > 1:
-        if m == 64 or rows <= (49152 if dim == 32 else 16384):
-            return True
-    elif rows <= 16384 and (dim == 32 or (m == 64 and few_edges)):
+    if m > 128:                                  # (there is no other kernel)
         return True
-    if heads == 1 and (dim, m) == (64, 32):
-        return local_context >= (512 if whole else 768)
-    if heads == 1 and (dim, m) == (32, 64):
-        return local_context >= (128 if whole else 192) or (rows > 150000 and local_context >= 96)
-    return local_context >= (128 if whole else 512)
+    if length is None:
+        length = rows // heads if heads > 1 else min(rows, 2304)
+    length = max(1, length)
+    pairs = max(1, rows // length)
+    chunks = (length + 63) // 64
+    segment = 16                                 # chunks per segment, as the launch chooses them
+    while segment > 1 and 2 * pairs * -(-chunks // segment) * (m // 32) < 16 * _COMPUTE_UNITS:
+        segment //= 2
+    base, chain, scan, row, band, rounds, edge, resident = _ROUTE_COSTS[dims][0]
+    wide, k_rows = min(local_context, 2 * length) / 128, rows / 1000
+    k_rounds = -(-pairs * chunks // (_COMPUTE_UNITS * resident)) * _COMPUTE_UNITS * resident * 64 / 1000
+    far = (base + chain * wide + scan * -(-chunks // segment) + k_rows * (row + band * wide)
+           + k_rounds * (rounds + edge * _edge_blocks(local_context, chunks) / 8))
+    host, host_heads, base, chain, scan, row, band, row_heads = _ROUTE_COSTS[dims][1]
+    several = heads > 1
+    wide = max(wide, 96 / 128)                   # (as many tiles at the least)
+    kernels = base + chain * wide + scan * length / 64 + k_rows * (row + band * wide + row_heads * several)
+    subtracting = ((host + host_heads * several) ** 8 + kernels ** 8) ** 0.125       # (the larger of the two; they overlap)
+    return far <= 1.01 * subtracting             # (a tie: without the widened copies)
 
 
 def _backward_far(query, key, value, P, local_context, t, key_lengths, out, log_norm, grad_out, dims):
@@ -439,7 +472,7 @@ def sblocal_backward(query, key, value, projection_matrix, local_context, softma
     if (query.dtype == torch.bfloat16 and query.is_cuda and band_kernel is None and support is None and dropout[0] == 0
             and key.dtype == value.dtype == out.dtype == grad_out.dtype == query.dtype):
         far_dims = _far_kernel_dims(E, D, 2 * projection_matrix.shape[0])
-        if far_dims is not None and _far_pays(B * H * max(T, S), H, local_context, far_dims):
+        if far_dims is not None and _far_pays(B * H * max(T, S), H, local_context, far_dims, max(T, S)):
             return _backward_far(query, key, value, projection_matrix.float(), local_context, t, key_lengths, out,
                                  log_normalization, grad_out, far_dims)
     wdt = torch.float64 if query.dtype == torch.float64 else torch.float32
