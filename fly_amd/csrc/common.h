@@ -436,15 +436,6 @@ __device__ __forceinline__ void dma_to_lds_at(const void* base, uint32_t lane_of
                  : "=&s"(saved_m0) : "v"(lane_off), "s"(base), "s"(dst) : "memory");
 }
 
-// one float per active lane, lane l's to wave_base + 4 l
-__device__ __forceinline__ void dma_float_to_lds(const float* lane_src, const void* wave_base) {
-    typedef __attribute__((address_space(3))) const char* lds_ptr;
-    const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)wave_base);
-    uint32_t saved_m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved_m0) : "v"(lane_src), "s"(dst) : "memory");
-}
-
 // ROWS rows of W 2-byte elements straight into LDS by NT threads, chunk c of a row stored where x3_swz puts it: the transfers
 // fill LDS linearly, so the swizzle is in the addresses they read.  Row indices are clamped to the last row, as in Tile16.
 template <int ROWS, int W, int NT>

@@ -1725,7 +1725,6 @@ struct B32Loads {
     }
 };
 
-template <int E, int M> constexpr size_t fwd_b32_smem() { return fwd_bf16_smem<E, M>(); }
 // Four waves per workgroup (two workgroups per compute unit, which then overlap by themselves).  Eight with the skew
 // below measured the same at 64 and 128 features and slower at 256, where the skewed form spills registers.
 #ifndef B32_WAVES
