@@ -5136,16 +5136,19 @@ static int plan(int B, int H, int S, int wgs_per_cu, int* n_chunks, int* n_split
     if (want < 1) want = 1;
     if (want > nc) want = nc;
     int per = (nc + (int)want - 1) / (int)want;
-    const long resident = (long)machine().cus * wgs_per_cu;
-    if ((long)B * H * nc > resident) {
-        // more work than one residency round: the pass takes about rounds x chunks per workgroup, and a round that
-        // is full costs no more than one that is not; among equals the larger share wins (fewer partial reductions
-        // to combine)
+    const long cus = machine().cus;
+    if ((long)B * H * nc > cus) {
+        // more work than one workgroup per compute unit: the pass takes about rounds x chunks per workgroup (and a sixth of a chunk to
+        // begin), where a round of one workgroup per compute unit costs 90 / 142 of one of two, and combining takes about 1/18 of a
+        // chunk's time per workgroup of a (batch, head) (its loop over the partial sums is serial); among equals the larger share wins.  Forward with 32 features, float32, us
+        // here / without the last two terms: one sequence of 50000 tokens 61 / 87, 16 heads of 4096 44 / 48, 64 images of 3136 both 109
         long best = -1;
         for (int p = 1; p <= nc; ++p) {
-            const long wgs = (long)B * H * ((nc + p - 1) / p);
-            const long cost = ((wgs + resident - 1) / resident) * p;
-            if (best < 0 || cost <= best) { best = cost; per = p; }
+            const long split = (nc + p - 1) / p, wgs = (long)B * H * split, rest = wgs % (wgs_per_cu * cus);
+            const long rounds = wgs / (wgs_per_cu * cus) * (wgs_per_cu == 2 ? 142 : 90) + (rest == 0 ? 0 : rest <= cus ? 90 : 142);
+            const long cost = rounds * (6 * p + 1) + 30 * split;
+            if (split <= MAX_SPLIT && (best < 0 || cost <= best)) { best = cost; per = p; }
+            if (wgs <= cus && 18L * p * p > nc) break;          // (from here on longer shares cost more than they save)
         }
     }
     *n_chunks = nc;
