@@ -3650,7 +3650,12 @@ __global__ __launch_bounds__(NT) void sblocal_fwd_x3_kernel(FwdArgs a) {
     char* lds = reinterpret_cast<char*>(smem);
     float* Ps = smem;                                  // only live before the key loop
 
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    // float inputs: list entries by scalar loads, query features selected behind their exponentials.  With 2-byte inputs, whose
+    // rows are widened on the way, both forms lose (us, 64 images of 768 tokens, 32 x 32 blocks, 64 features: 60.3 against 57.0, with 128
+    // features on 16 x 16 blocks of 784 77.0 / 73.3; float 55.4 / 57.4 and 69.8 / 72.3, 3136 tokens and 128 features 228 / 238)
+    constexpr bool FIO = sizeof(TIO) == 4;
+    auto list_entry = [](const int32_t* p) __attribute__((always_inline)) { return FIO ? table_entry(p) : *p; };
+    const int tid = threadIdx.x, lane = tid & 63, w = FIO ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, r16 = lane & 15, g = lane >> 4;
     const int n_qt = (a.T + TQ - 1) / TQ;
     // (LIST: every workgroup has an item of the lists below; n_items = 0 keeps the band's mapping out of the way)
     const int n_items = LIST ? 0 : a.B * a.H * n_qt * a.n_parts;
@@ -3740,8 +3745,8 @@ __global__ __launch_bounds__(NT) void sblocal_fwd_x3_kernel(FwdArgs a) {
         }
         tl_inner = a.tl_inner + lp0;
         tl_blk = a.tl_blk + 4 * (long)lp0 + w;              // four masks per entry, one per wave
-        if (kt_hi > 0) { tile_cur = table_entry(tl_inner); pres_cur = table_entry(tl_blk) & 3; }
-        if (kt_hi > 1) { tile_next = table_entry(tl_inner + 1); pres_next = table_entry(tl_blk + 4) & 3; }
+        if (kt_hi > 0) { tile_cur = list_entry(tl_inner); pres_cur = list_entry(tl_blk) & 3; }
+        if (kt_hi > 1) { tile_next = list_entry(tl_inner + 1); pres_next = list_entry(tl_blk + 4) & 3; }
     }
     const int first_tile = LIST ? tile_cur : kt_lo;
 
@@ -3851,9 +3856,14 @@ __global__ __launch_bounds__(NT) void sblocal_fwd_x3_kernel(FwdArgs a) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const bool ok = 16 * fb + 4 * g + i < a.mh_valid;
-                    const float ep = quant16(__expf(dd[i] - qmax)), en = quant16(__expf(-dd[i] - qmax));
-                    qf[fb][i] = ok ? ep : 0.f;
-                    qf[FB + fb][i] = ok ? en : 0.f;
+                    if constexpr (FIO) {
+                        const float ep = quant16(__expf(dd[i] - qmax)), en = quant16(__expf(-dd[i] - qmax));
+                        qf[fb][i] = ok ? ep : 0.f;
+                        qf[FB + fb][i] = ok ? en : 0.f;
+                    } else {
+                        qf[fb][i] = ok ? quant16(__expf(dd[i] - qmax)) : 0.f;
+                        qf[FB + fb][i] = ok ? quant16(__expf(-dd[i] - qmax)) : 0.f;
+                    }
                 }
             }
             __syncthreads();      // Ps is dead; the tile buffers may overwrite it
@@ -3905,7 +3915,7 @@ __global__ __launch_bounds__(NT) void sblocal_fwd_x3_kernel(FwdArgs a) {
         float cscale_next = cscale;
         // LIST: the entry after the next one (tile, presence) is requested now
         int tile_n2 = 0, pres_n2 = 0;
-        if (LIST && kt + 2 < kt_hi) { tile_n2 = table_entry(tl_inner + kt + 2); pres_n2 = table_entry(tl_blk + 4 * (kt + 2)) & 3; }
+        if (LIST && kt + 2 < kt_hi) { tile_n2 = list_entry(tl_inner + kt + 2); pres_n2 = list_entry(tl_blk + 4 * (kt + 2)) & 3; }
         if (more) {                                      // next tile's transfer flies during the MFMAs (every wave is past
             const int nxt = LIST ? tile_next : kt + 1;   // the barrier that ended the last use of that stage)
             transfer(nxt, cur ^ 1);
