@@ -2825,9 +2825,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEYMAJOR &&
     const int trow = 4 * g + (r16 >> 2);
     int foff[KS], toff[EB];
 #pragma unroll
-    for (int c = 0; c < KS; ++c) foff[c] = r16 * ROWB + x3_swz(r16, 4 * c + g, ROWB) * 16;
+    for (int c = 0; c < KS; ++c) foff[c] = r16 * ROWB + rows_swz(r16, 4 * c + g, ROWB) * 16;
 #pragma unroll
-    for (int eb = 0; eb < EB; ++eb) toff[eb] = trow * ROWB + x3_swz(trow, 2 * eb + ((r16 & 3) >> 1), ROWB) * 16 + 8 * (r16 & 1);
+    for (int eb = 0; eb < EB; ++eb) toff[eb] = trow * ROWB + rows_swz(trow, 2 * eb + ((r16 & 3) >> 1), ROWB) * 16 + 8 * (r16 & 1);
     // (list entries a step ahead of their use)
     int inner_cur = n > 0 ? table_entry(a.uni_inner + p0) : 0, inner_next = n > 1 ? table_entry(a.uni_inner + p0 + 1) : 0;
     int blk_cur = n > 0 ? table_entry(a.uni_blk + (long)p0 * 4 + w) : -1;

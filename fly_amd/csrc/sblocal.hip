@@ -2703,7 +2703,7 @@ __global__ __launch_bounds__(NT) void local_fwd_kernel(LocalArgs a) {
 //   out^T[d][query] += V^T[d][key] P[key][query], 32 keys (two blocks) per step, contraction slots {4 g + i, 16 + 4 g + i}: the
 //       weights go from registers into it, V^T fragments come by transposing LDS reads (ds_read_b64_tr_b16: column d of
 //       four consecutive key rows per read).
-// With the 16-byte chunks of a row swizzled (x3_swz) neither kind of read meets a bank conflict; rows padded by 16 bytes with
+// With the 16-byte chunks of a row swizzled (rows_swz) neither kind of read meets a bank conflict; rows padded by 16 bytes with
 // eight consecutive keys per lane left 27 % of the gradients' and 11 % of this kernel's cycles in conflicts.  B=2, 12 heads of 10007
 // tokens in a padded batch, window 1024, forward and gradients: 434 -> 348 us, of which the layout and the transfers 60, the
 // loop without a branch around its products 16, two blocks of queries in the query-major gradient 8.
@@ -2743,7 +2743,7 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
 
     const TileRange all = band_tiles(q0, min(q0 + TQB, a.T), lc_lo, lc_hi, len, TKL);
     const int kt_lo = all.lo, kt_hi = all.hi;
-    RowsToLds<TKL, E, NT> rk, rv;
+    RowsToLds<TKL, E, NT, true> rk, rv;
     rk.init(kptr, a.k_ss, a.S - 1, w, lane);
     rv.init(vptr, a.v_ss, a.S - 1, w, lane);
     auto fetch = [&](int kt, int stage) __attribute__((always_inline)) {
@@ -2778,9 +2778,9 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
     const int trow = 4 * g + (r16 >> 2);
     int koff[KS], voff[DB];
 #pragma unroll
-    for (int c = 0; c < KS; ++c) koff[c] = r16 * ROWB + x3_swz(r16, 4 * c + g, ROWB) * 16;
+    for (int c = 0; c < KS; ++c) koff[c] = r16 * ROWB + rows_swz(r16, 4 * c + g, ROWB) * 16;
 #pragma unroll
-    for (int db = 0; db < DB; ++db) voff[db] = trow * ROWB + x3_swz(trow, 2 * db + ((r16 & 3) >> 1), ROWB) * 16 + 8 * (r16 & 1);
+    for (int db = 0; db < DB; ++db) voff[db] = trow * ROWB + rows_swz(trow, 2 * db + ((r16 & 3) >> 1), ROWB) * 16 + 8 * (r16 & 1);
     drain_loads();
     __syncthreads();
     // the tiles that touch the band of one of the wave's queries lie in a row (wave-uniform, scalar: w is): the loop over them
@@ -3060,9 +3060,9 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
     const int trow = 4 * g + (r16 >> 2);
     int foff[KS], toff[EB];
 #pragma unroll
-    for (int c = 0; c < KS; ++c) foff[c] = r16 * ROWB + x3_swz(r16, 4 * c + g, ROWB) * 16;
+    for (int c = 0; c < KS; ++c) foff[c] = r16 * ROWB + rows_swz(r16, 4 * c + g, ROWB) * 16;
 #pragma unroll
-    for (int eb = 0; eb < EB; ++eb) toff[eb] = trow * ROWB + x3_swz(trow, 2 * eb + ((r16 & 3) >> 1), ROWB) * 16 + 8 * (r16 & 1);
+    for (int eb = 0; eb < EB; ++eb) toff[eb] = trow * ROWB + rows_swz(trow, 2 * eb + ((r16 & 3) >> 1), ROWB) * 16 + 8 * (r16 & 1);
     if (it_lo < it_hi) stash(0);
     drain_loads();
     __syncthreads();

@@ -1419,3 +1419,36 @@ def test_an_output_without_a_gradient_counts_as_zero(H, dtype):
     out, _ = SBLocalAttention(33, dim_heads=64, nb_features=64).to(dev)(*leaves)
     for g in torch.autograd.grad(Silent.apply(out).sum(), leaves):
         assert float(g.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('L,lc,far_apart', [(333, 70, False), (64, 300, False), (197, 33, False), (83, 50, True)])
+def test_local_attention_with_128_dims(L, lc, far_apart, dtype):
+    """Rows of 256 bytes, whose sixteen 16-byte chunks are swizzled over all sixteen places: forward and gradients with whole tiles, a last
+    tile cut by the rows' end, key lengths, and rows too far apart in memory for 32-bit offsets.  Bounds as for the other head dims."""
+    from fly_amd import LocalAttention, LengthMask
+    dev = torch.device('cuda:0')
+    B, H, E = 2, 2, 128
+    print('case', L, lc, far_apart, dtype, flush=True)
+    if far_apart:
+        B = 1
+    g = torch.Generator().manual_seed(71)
+    q, k, v, w = (torch.randn(B, L, H, E, generator=g).to(dtype) for _ in range(4))
+    lens = torch.full((B,), L)
+    lens[B - 1] = L * 3 // 4
+
+    def place(x):
+        if not far_apart:
+            return x.to(dev)
+        return torch.zeros(L << 24, dtype=x.dtype, device=dev).as_strided((B, L, H, E), (0, 1 << 24, E, 1)).copy_(x)
+
+    leaves = [place(x).requires_grad_() for x in (q, k, v)]
+    out, _ = LocalAttention(lc).to(dev)(*leaves, key_padding_mask=LengthMask(lens.to(dev), max_len=L))
+    grads = torch.autograd.grad(out, leaves, place(w))
+    ref = [x.double().requires_grad_() for x in (q, k, v)]
+    ref_out = osb.local_attention(*ref, lc, key_lengths=lens)
+    ref_grads = torch.autograd.grad(ref_out, ref, w.double())
+    tol = 2e-2 if dtype == torch.bfloat16 else 3e-3
+    assert rel_err(out.float(), ref_out.detach()) <= tol
+    for got, r in zip(grads, ref_grads):
+        assert rel_err(got.float(), r) <= 1.5 * tol
