@@ -627,22 +627,21 @@ def test_dds_weight_stationary_kernel(M, trans_b, dtype):
 @pytest.mark.parametrize('trans_b', [True, False])
 def test_dds_staged_kernel_with_weights_in_chunks(trans_b, dtype):
     """Reduction lists longer than nine blocks and more than 4096 tokens: the staged dds kernel whose group weights
-    pass through LDS in double-buffered chunks of four list entries.  Lists of 10 to 21 entries (the last chunk of a
-    list holds one to four entries, odd lengths end on a step with one entry), groups of one to four output blocks
-    (the lanes of a short group store fewer outputs), two batch entries, two heads, a token count that ends inside a
-    tile, both block orientations."""
+    pass through LDS two list entries at a time, double-buffered.  Lists of 10 to 21 entries (odd lengths end on a step with one
+    entry), groups of one to four output blocks (a kernel body of its own each), two batch entries, two heads, a token count that
+    ends inside a tile, both block orientations."""
     from fly_amd import matmul
     print('case', trans_b, dtype, flush=True)
     Z, H, block, n_out, n_in, M = 2, 2, 32, 10, 21, 4096 + 1024 + 77
     g = torch.Generator().manual_seed(43)
     seg = (torch.rand(H, n_out, n_in, generator=g) < 0.7).long()    # (head, output block, input block)
-    seg[0, 0] = 1                                          # 21 entries: five chunks and one entry more
+    seg[0, 0] = 1                                          # 21 entries: ten steps and one entry more
     seg[0, 1:4] = seg[0, 0]                                # a full group of four
     seg[0, 4] = (torch.arange(n_in) % 2 == 0).long()       # 11 entries, none with a neighbour
     seg[1, 0, :] = 0
-    seg[1, 0, :10] = 1                                     # 10 entries: two chunks and half a chunk
+    seg[1, 0, :10] = 1                                     # 10 entries: five steps
     seg[1, 1:3] = seg[1, 0]                                # a group of three
-    seg[1, 3] = (torch.arange(n_in) < 17).long()           # 17 entries: the last chunk holds one
+    seg[1, 3] = (torch.arange(n_in) < 17).long()           # 17 entries: the last step has one
     lens = seg.sum(-1)
     assert int(lens.max()) == 21 and all(bool((lens % 4 == k).any()) for k in range(4))
     layout = seg if trans_b else seg.transpose(1, 2).contiguous()
@@ -718,7 +717,8 @@ def test_dds_long_lists_with_blocks_off_a_16_byte_boundary(offset, trans_b, monk
 
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 def test_narrowing_linear_with_bias_and_long_lists(dtype):
-    """Bias inside the dds kernel for long reduction lists (36 blocks a row), forward and gradients against the dense product."""
+    """Bias inside the dds kernel for long reduction lists (36 blocks a row) against the dense product; the input gradient has lists of
+    nine blocks and another kernel."""
     from fly_amd import BlockSparseLinear, FlatBlockButterflySparsityConfig
     torch.manual_seed(3)
     layer = BlockSparseLinear(1536, 384, FlatBlockButterflySparsityConfig(4, 2, block=32), bias=True).to(DEV).to(dtype)
@@ -734,6 +734,31 @@ def test_narrowing_linear_with_bias_and_long_lists(dtype):
     mat = dense.view(384, 1536).t()
     ref = x.detach().double() @ mat + layer.bias.double()
     assert rel_err(out.double(), ref) <= TOL[dtype]
+    assert rel_err(gx.double(), w.double() @ mat.t()) <= TOL[dtype]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('tokens', [4096, 4096 + 130])
+def test_widening_linear_gradient_over_long_lists(tokens, dtype):
+    """The input gradient of a layer that widens has the long reduction lists (36 blocks) and reads the weight blocks transposed, the
+    [k][n] form of that kernel; the weight gradient rides along.  Against the dense products."""
+    from fly_amd import BlockSparseLinear, FlatBlockButterflySparsityConfig
+    torch.manual_seed(4)
+    layer = BlockSparseLinear(384, 1536, FlatBlockButterflySparsityConfig(4, 2, block=32), bias=True).to(DEV).to(dtype)
+    x, w = (torch.randn(tokens, n, device=DEV).to(dtype) for n in (384, 1536))
+    x.requires_grad_()
+    out = layer(x)
+    gx, gw = torch.autograd.grad(out, (x, layer.weight), w)
+    lay = layer.layout.cpu()
+    assert int(lay.sum(0).max()) == 36
+    dense = torch.zeros(lay.shape[0], 32, lay.shape[1], 32, dtype=torch.float64, device=DEV)
+    want = (w.double().t() @ x.detach().double()).view(lay.shape[0], 32, lay.shape[1], 32)
+    for n, (i, j) in enumerate(lay.nonzero().tolist()):
+        dense[i, :, j] = layer.weight[0, n].double()
+        if n % 7 == 0:
+            assert rel_err(gw[0, n].double(), want[i, :, j]) <= TOL[dtype]
+    mat = dense.view(1536, 384).t()
+    assert rel_err(out.double(), x.detach().double() @ mat + layer.bias.double()) <= TOL[dtype]
     assert rel_err(gx.double(), w.double() @ mat.t()) <= TOL[dtype]
 
 
