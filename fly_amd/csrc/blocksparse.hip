@@ -2682,9 +2682,9 @@ extern "C" int flyhip_bs_sdd_prob_dsoftmax_dropout(const void* dout, const void*
 // of which writes P or dS: a workgroup owns four block-rows (query-major: d q, and delta on the way) or four
 // block-columns (key-major: d k and d v), a wave one of them with its two operands in registers (q and g rows; k and v
 // rows), and walks the union of their lists (union_table, transposed for key-major), every 32-row tile of the other
-// side (K with V; Q with g, lse2 and delta) staged once in LDS for the four waves.  Per block S^T = Y1 . x1 and
-// G^T = Y2 . x2 (the tile's rows picked so that a lane's results over the two 16-row blocks are eight consecutive
-// inner rows, the contraction slots of what follows), then d x^T[e][outer] += Y^T[e][inner] . {dS, P}[inner][outer]
+// side (K with V; Q with g, lse2 and delta) moved once straight into LDS for the four waves.  Per block S^T = Y1 . x1 and
+// delta - G^T = delta - Y2 . x2 (x2 negated, the sums start at delta; a lane's results over the two 16-row blocks are inner rows
+// 4 g + i and 16 + 4 g + i, the contraction slots of what follows), then d x^T[e][outer] += Y^T[e][inner] . {-dS, P}[inner][outer]
 // with Y^T fragments by transposing LDS reads of the same tiles.
 struct AttnBwdArgs {
     const void* q; const void* k; const void* v; const void* go; const void* out;

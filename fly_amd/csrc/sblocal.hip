@@ -2932,8 +2932,8 @@ __global__ __launch_bounds__(NT) void local_fwd_b16_kernel(LocalArgs a) {
 // d k_s = t sum_i dS_is q_i.  One kernel in two orientations, built like local_fwd_b16_kernel: a wave owns QB blocks
 // of 16 "outer" rows (queries, or keys when KEYMAJOR) whose two operands stay in registers, and walks 64-row tiles of
 // the "inner" side (keys with values, or queries with their output gradients) through LDS.
-//   S^T  = Y1 . x1  and  G^T = Y2 . x2   (inner rows of a 16-row block picked so that a lane's results over two
-//                                         blocks are eight consecutive inner rows, the contraction slots below)
+//   S^T  = Y1 . x1  and  G^T = Y2 . x2   (a lane's results over the two 16-row blocks of 32 inner rows are rows 4 g + i and
+//                                         16 + 4 g + i, i = 0 .. 3: the contraction slots below; G starts at -delta)
 //   P = exp2(sc S - lse log2e) where the pair is in the band, dS = P (G - delta)   (lse, delta: of the query)
 //   d x^T[e][outer] += Y^T[e][inner] . {P, dS}[inner][outer]   (Y^T fragments by transposing LDS reads)
 // Query-major: d q from (K, dS).  Key-major: d v from (d out, P) and d k from (Q, dS).
@@ -2988,7 +2988,7 @@ __global__ __launch_bounds__(NT) void local_bwd_b16_kernel(LocalBwdArgs a) {
     RowsToLds<TKL, E, NT> r1, r2;
     r1.init(y1p, y1s, R_in - 1, w, lane);
     r2.init(y2p, y2s, R_in - 1, w, lane);
-    float rl = 0.f, rd = 0.f;                          // key-major: lse log2e and -delta of inner row tid (threads 0 .. 63)
+    float rl = 0.f, rd = 0.f;                          // key-major: lse and delta of inner row tid (threads 0 .. 63)
     auto fetch = [&](int it, int stage) __attribute__((always_inline)) {
         char* st = lds + stage * STAGE_BYTES;
         r1.fetch(it * TKL, st, w, lane);
